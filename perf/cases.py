@@ -134,28 +134,22 @@ def _late_embedding(label, c, g):
     return torch.cat([48.0 * torch.cos(at) + radius * torch.cos(angle), 48.0 * torch.sin(at) + radius * torch.sin(angle)])
 
 
-def prepare(case, seed):
+def _neighbours(case, seed):
+    """Points renumbered by locality first, as the estimator does and the loop expects of its callers: the clusters'
+    labels in that order, and the neighbour lists."""
     x, label, g = _points(case, seed)
-    n, k = case["n"], min(case["k"], case["n"])
-    if case["kind"] == "fit":
-        # Host arrays, as a program has them after reading a file, and the estimator.
-        y0 = 1e-4 * torch.randn(2, n, generator=g, device="cuda")
-        model = TSNE(perplexity=case["perplexity"], num_neighbors=k, learning_rate=case["lr"], n_iter=case["steps"])
-        return {"case": case, "x": x.cpu().numpy(), "y0": np.asfortranarray(y0.cpu().numpy().T), "model": model}
-    if case["kind"] == "knn":
-        return {"case": case, "x": x, "k": k}
-    # Points renumbered by locality first, as the estimator does and the loop expects of its callers.
     order = stages.locality_order(x)
     x = stages.gather_rows(x, order)
-    label = label[order.long()]
-    idx, d2 = stages.knn(x, k)
-    del x
-    if case["kind"] == "affinities":
-        return {"case": case, "idx": idx, "d2": d2, "work": torch.empty_like(d2)}
+    idx, d2 = stages.knn(x, min(case["k"], case["n"]))
+    return label[order.long()], g, idx, d2
+
+
+def _loop_inputs(case, seed):
+    """The symmetric probabilities over the neighbour lists, and where the loop starts: positions, gains, momenta."""
+    label, g, idx, d2 = _neighbours(case, seed)
     stages.max_normalize_(d2)
     p = stages.symmetrize(stages.perplexity(d2, case["perplexity"], 1e-4), idx)
-    plan = stages.Plan(n, k)
-    plan.prepare_attractive(p, idx)
+    n = case["n"]
     if case["phase"] == "start":
         y0 = 1e-4 * torch.randn(2 * n, generator=g, device="cuda")
         gains0, old0 = torch.ones_like(y0), torch.zeros_like(y0)
@@ -163,7 +157,26 @@ def prepare(case, seed):
         y0 = _late_embedding(label, _clusters(case), g)
         gains0 = torch.empty_like(y0).uniform_(0.2, 3.0, generator=g)
         old0 = 1e-2 * torch.randn(2 * n, generator=g, device="cuda")
-    return {"case": case, "plan": plan, "start": (y0, gains0, old0), "now": tuple(torch.empty_like(y0) for _ in range(3))}
+    return p, idx, y0, gains0, old0
+
+
+def prepare(case, seed):
+    n, k = case["n"], min(case["k"], case["n"])
+    if case["kind"] == "fit":
+        # Host arrays, as a program has them after reading a file, and the estimator.
+        x, _, g = _points(case, seed)
+        y0 = 1e-4 * torch.randn(2, n, generator=g, device="cuda")
+        model = TSNE(perplexity=case["perplexity"], num_neighbors=k, learning_rate=case["lr"], n_iter=case["steps"])
+        return {"case": case, "x": x.cpu().numpy(), "y0": np.asfortranarray(y0.cpu().numpy().T), "model": model}
+    if case["kind"] == "knn":
+        return {"case": case, "x": _points(case, seed)[0], "k": k}
+    if case["kind"] == "affinities":
+        _, _, idx, d2 = _neighbours(case, seed)
+        return {"case": case, "idx": idx, "d2": d2, "work": torch.empty_like(d2)}
+    p, idx, *start = _loop_inputs(case, seed)
+    plan = stages.Plan(n, k)
+    plan.prepare_attractive(p, idx)
+    return {"case": case, "plan": plan, "start": tuple(start), "now": tuple(torch.empty_like(v) for v in start)}
 
 
 # ---- one pass ----------------------------------------------------------------------------------------------------
@@ -188,6 +201,131 @@ def run(state):
     begin = 0 if case["phase"] == "start" else 500
     z = state["plan"].iterate_(None, None, y, gains, old, begin, begin + case["steps"], eta=case["lr"])
     return {"y": y, "gains": gains, "old": old, "z": z}
+
+
+# ---- the same in 64 bits, in plain torch ---------------------------------------------------------------------------
+
+
+def _neighbours64(x, k):
+    """(idx, squared distances) of the k nearest rows, the row itself first."""
+    x = x.double()
+    x -= x.mean(0)
+    square = (x * x).sum(1)
+    idx, d2 = [], []
+    for at in range(0, x.shape[0], 4096):
+        d = square[at:at + 4096, None] + square - 2.0 * (x[at:at + 4096] @ x.T)
+        rows = torch.arange(d.shape[0], device=d.device)
+        d[rows, rows + at] = -1e30
+        found, j = d.topk(k, dim=1, largest=False)
+        found[:, 0] = 0.0
+        idx.append(j)
+        d2.append(found)
+    return torch.cat(idx), torch.cat(d2)
+
+
+def _affinities64(d2, idx, perplexity, epsilon):
+    d2 = d2.double()
+    d2 = d2 / d2.abs().max()
+    n, k = d2.shape
+    is_self = d2[:, 0] == 0.0
+    beta = torch.ones(n, 1, dtype=torch.float64, device=d2.device)
+    lo, hi = torch.full_like(beta, -math.inf), torch.full_like(beta, math.inf)
+    p, searching = torch.empty_like(d2), torch.arange(n, device=d2.device)
+    for trial in range(200):
+        d, b = d2[searching], beta[searching]
+        v = torch.exp(-b * d)
+        v[is_self[searching], 0] = 0.0
+        total = v.sum(1, keepdim=True)
+        over = -torch.special.xlogy(v, v).sum(1, keepdim=True) / total + total.log() - math.log(perplexity)
+        p[searching] = v / total
+        wide, on = over > 0.0, (over.abs() >= epsilon).squeeze(1)
+        low, high = torch.where(wide, b, lo[searching]), torch.where(wide, hi[searching], b)
+        lo[searching], hi[searching] = low, high
+        beta[searching] = torch.where(wide, torch.where(high.isinf(), 2.0 * b, 0.5 * (b + high)),
+                                      torch.where(low.isinf(), 0.5 * b, 0.5 * (b + low)))
+        searching = searching[on]
+        if not searching.numel():
+            break
+    # Own entry plus what the neighbour's list holds of this row, over 2n.
+    i = torch.arange(n, device=d2.device)[:, None].expand(n, k)
+    key, order = (i * n + idx).flatten().sort()
+    wanted = (idx.long() * n + i).flatten()
+    at = torch.searchsorted(key, wanted).clamp_(max=key.numel() - 1)
+    back = torch.where(key[at] == wanted, p.flatten()[order[at]], torch.zeros((), dtype=torch.float64, device=d2.device))
+    return (p + back.view(n, k)) / (2.0 * n)
+
+
+def _repulsive64(y, boxes=130):
+    """Repulsive numerator and normalisation by interpolation: three nodes a box and dimension, the Cauchy kernel's
+    square between nodes, summed by transforms."""
+    n, side, length = y.shape[1], 3 * boxes, 800
+    low = y.min()
+    width = (y.max() - low) / boxes
+    box = ((y - low) / width).long().clamp_(0, boxes - 1)
+    t = (y - low) / width - box
+    node = (torch.arange(3, dtype=torch.float64, device=y.device) + 0.5) / 3.0
+    base = []
+    for j in range(3):
+        a, b = [node[m] for m in range(3) if m != j]
+        base.append((t - a) * (t - b) / ((node[j] - a) * (node[j] - b)))
+    charge = torch.stack([torch.ones_like(y[0]), y[0], y[1], (y * y).sum(0)])
+    grid = torch.zeros(4, side * side, dtype=torch.float64, device=y.device)
+    at = lambda a, b: (3 * box[0] + a) * side + 3 * box[1] + b  # noqa: E731
+    for a in range(3):
+        for b in range(3):
+            grid.index_add_(1, at(a, b), charge * (base[a][0] * base[b][1]))
+    step = torch.arange(length, device=y.device)
+    step = torch.where(step < side, step, length - step).double() * (width / 3.0)
+    kernel = (1.0 + step[:, None] ** 2 + step ** 2) ** -2
+    far = torch.fft.irfft2(torch.fft.rfft2(grid.view(4, side, side), s=(length, length)) * torch.fft.rfft2(kernel),
+                           s=(length, length))[:, :side, :side].reshape(4, -1)
+    phi = sum(far[:, at(a, b)] * (base[a][0] * base[b][1]) for a in range(3) for b in range(3))
+    z = (1.0 + (y * y).sum(0)) * phi[0] - 2.0 * (y * phi[1:3]).sum(0) + phi[3]
+    return y * phi[0] - phi[1:3], z.sum() - n
+
+
+def _loop64(p, idx, y, gains, old, begin, end, eta):
+    y, gains, old = (v.double().view(2, -1) for v in (y, gains, old))
+    p, idx, z = p.double(), idx.long(), None
+    for step in range(begin, end):
+        early = step < 250
+        repulsive, z = _repulsive64(y)
+        between = [c[:, None] - c[idx] for c in y]
+        w = p / (1.0 + between[0] ** 2 + between[1] ** 2)
+        force = (12.0 if early else 1.0) * torch.stack([(w * c).sum(1) for c in between]) - repulsive / z
+        gains = torch.where(force.signbit() != old.signbit(), gains + 0.2, gains * 0.8).clamp(min=0.01)
+        old = (0.5 if early else 0.8) * old - eta * gains * force
+        y = y + old
+    return y, gains, old, z
+
+
+def exact(case, seed):
+    n, k = case["n"], min(case["k"], case["n"])
+    if case["kind"] == "affinities":
+        _, _, idx, d2 = _neighbours(case, seed)
+        return {"p": _affinities64(d2, idx, case["perplexity"], 1e-4)}
+    if case["kind"] == "loop":
+        first = 0 if case["phase"] == "start" else 500
+        y, gains, old, z = _loop64(*_loop_inputs(case, seed), first, first + case["steps"], case["lr"])
+        if case["phase"] == "late":  # (branches on the signs of forces that are zero to rounding: see tolerance)
+            gains = old = None
+        return {"y": y.flatten(), "gains": None if gains is None else gains.flatten(),
+                "old": None if old is None else old.flatten(), "z": z.view(1)}
+    if n > 60000:  # (every pair's distance is formed)
+        return None
+    if case["kind"] == "knn":
+        return {"idx": None, "d2": _neighbours64(_points(case, seed)[0], k)[1]}
+    if case["lr"] > 10.0:  # (two correct fits drift apart)
+        return None
+    state = prepare(case, seed)
+    idx, d2 = _neighbours64(torch.from_numpy(state["x"]).cuda(), k)
+    p = _affinities64(d2, idx, case["perplexity"], 1e-3)
+    y = torch.from_numpy(np.ascontiguousarray(state["y0"].T)).cuda().double()
+    y = _loop64(p, idx, y, torch.ones_like(y), torch.zeros_like(y), 0, case["steps"], case["lr"])[0]
+    z = _repulsive64(y)[1]
+    apart = sum((c[:, None] - c[idx]) ** 2 for c in y)
+    kl = (torch.special.xlogy(p, p) + p * (apart.log1p() + z.log())).sum()
+    return {"embedding": y.T, "kl": kl.item()}
 
 
 # ---- what a pass cannot do without, and how near two correct ones are --------------------------------------------
