@@ -1113,3 +1113,31 @@ def test_loop_is_bit_repeatable(stages, c0_problem, monkeypatch, n_points):
         for a, b in zip(got[:3], want[:3]):
             assert same_bits(a, b), (graph, overlap, keep)
         assert got[3] == want[3]
+
+
+@pytest.mark.parametrize("n,d,k,kind", [
+    (3, 1, 2, "plain"), (64, 3, 64, "plain"), (65, 4, 20, "plain"), (127, 17, 127, "plain"), (129, 16, 91, "plain"),
+    (257, 33, 129, "plain"), (300, 7, 130, "plain"), (1025, 20, 257, "plain"), (1025, 5, 258, "plain"),
+    (1203, 20, 32, "cycle4"), (2051, 6, 65, "cycle16"), (1500, 2, 40, "equal"), (1301, 3, 129, "grid"),
+    (4500, 31, 90, "plain"), (10300, 3, 10, "grid")])
+def test_knn_small_problems(stages, n, d, k, kind):
+    """The search that writes the distances out and selects row by row: tile and chunk remainders, the most
+    neighbours each selection takes (129, 257) and one more, clusters that come in turn, many equal distances, one
+    and several blocks of rows.  The oracle's rows, bit for bit."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    if kind.startswith("cycle"):
+        c = int(kind[5:])
+        X += (10.0 * rng.standard_normal((c, d)).astype(np.float32))[np.arange(n) % c]
+    elif kind == "equal":
+        X[:] = X[0]
+    elif kind == "grid":
+        X = np.round(X).astype(np.float32)
+    idx, d2 = stages.knn(dev(X), k)
+    if n <= 4500:
+        idx_o, d2_o = oracle.knn(X, k)
+        assert np.array_equal(idx.cpu().numpy(), idx_o)
+        assert np.array_equal(d2.cpu().numpy(), d2_o)
+    else:
+        idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+        assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)

@@ -358,6 +358,27 @@ __device__ __forceinline__ void bitonic_sort(u64 *sortbuf, int cap, int tid) {
     }
 }
 
+// Bitonic sort of one wave's own keys in LDS (sort_n a power of two, at least 64): no workgroup barrier, a wave's
+// LDS operations execute in order and the wavefront fences only keep the compiler from reordering them.
+__device__ __forceinline__ void wave_sort(u64 *keys, int sort_n, int lane) {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    for (int k = 2; k <= sort_n; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int t = lane; t < sort_n / 2; t += kWave) {
+                const int lo = ((t & ~(j - 1)) << 1) | (t & (j - 1));
+                const int hi = lo | j;
+                const bool up = (lo & k) == 0;
+                const u64 a = keys[lo], b = keys[hi];
+                if ((a > b) == up) {
+                    keys[lo] = b;
+                    keys[hi] = a;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        }
+    }
+}
+
 // Keeps the `want` best entries of query slot qq and tightens its threshold.
 __device__ __forceinline__ void compact_query(u64 *list, int cap, int want, int *cnt, u64 *thr, int qq,
                                               u64 *sortbuf, int tid) {
@@ -781,6 +802,233 @@ __global__ __launch_bounds__(256) void knn_merge_slices_kernel(const u64 *__rest
         }
         out_idx[(size_t)q * K + e] = j;
         out_d[(size_t)q * K + e] = d;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Direct search (small problems): every canonical distance of a block of query rows is written to memory
+// (pair_distances_kernel), then one wave per query reads its row and keeps the K - 1 smallest keys
+// (select_row_kernel).  The sweeps above and below give a query tile to one workgroup, which walks all the
+// candidates by itself: 47 workgroups at 3000 points, on a chip that holds hundreds.  Here the pairs are spread
+// over the chip, and the selection has no barrier.
+// ---------------------------------------------------------------------------
+constexpr int kDirectDims = 16;  // dimensions staged per chunk
+
+// Distances of query rows row0 .. row0 + rows - 1 (rows of `dist`, pitch floats each, pitch a multiple of the
+// tile's side 16 R and at least N) to all points; columns from N on are left as distances to a point at 0.
+// A workgroup computes a square tile, R x R distances per thread, both operands staged in LDS a chunk of
+// dimensions ahead; same fma chain as everywhere (dimensions past D are zeros on both sides, which leave a sum
+// as it is).  Bound by the vector ALU, two instructions per pair and dimension.
+template <int R>
+__global__ __launch_bounds__(256) void pair_distances_kernel(const float *__restrict__ X, int N, int D, int row0,
+                                                             int rows, int pitch, float *__restrict__ dist) {
+    constexpr int kSide = 16 * R;
+    constexpr int kRow = kSide + 4;              // LDS row: 16-byte aligned, chunk rows off each other's banks
+    constexpr int kLoads = kSide * kDirectDims / (4 * 256);  // pieces of four dimensions per thread and operand
+    __shared__ __attribute__((aligned(16))) float xs[2][2][kDirectDims][kRow];
+    const int tid = threadIdx.x, tq = tid >> 4, tc = tid & 15;
+    const int q0 = row0 + blockIdx.y * kSide, c0 = blockIdx.x * kSide;
+    const bool wide = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    float4 ahead[2][kLoads];
+    auto load = [&](int d0) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                const int e = tid + u * 256, p = (o ? c0 : q0) + (e >> 2), d = d0 + 4 * (e & 3);
+                float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+                if (p < N && d < D) {
+                    const float *x = X + (size_t)p * D + d;
+                    if (wide) {
+                        v = *reinterpret_cast<const float4 *>(x);
+                    } else {
+                        v.x = x[0];
+                        if (d + 1 < D) v.y = x[1];
+                        if (d + 2 < D) v.z = x[2];
+                        if (d + 3 < D) v.w = x[3];
+                    }
+                }
+                ahead[o][u] = v;
+            }
+    };
+    auto stage = [&](int buffer) {
+#pragma unroll
+        for (int o = 0; o < 2; ++o)
+#pragma unroll
+            for (int u = 0; u < kLoads; ++u) {
+                const int e = tid + u * 256, p = e >> 2, dd = 4 * (e & 3);
+                xs[buffer][o][dd][p] = ahead[o][u].x;
+                xs[buffer][o][dd + 1][p] = ahead[o][u].y;
+                xs[buffer][o][dd + 2][p] = ahead[o][u].z;
+                xs[buffer][o][dd + 3][p] = ahead[o][u].w;
+            }
+    };
+    float acc[R][R];
+#pragma unroll
+    for (int a = 0; a < R; ++a)
+#pragma unroll
+        for (int b = 0; b < R; ++b) acc[a][b] = 0.0f;
+    load(0);
+    stage(0);
+    for (int d0 = 0, buffer = 0; d0 < D; d0 += kDirectDims, buffer ^= 1) {
+        const bool more = d0 + kDirectDims < D;
+        if (more) load(d0 + kDirectDims);
+        // One barrier per chunk: the buffer written below was last read before this barrier.
+        __syncthreads();
+        const int dn = min(kDirectDims, D - d0);
+#pragma unroll 2
+        for (int dd = 0; dd < dn; ++dd) {
+            float qs[R], cs[R];
+#pragma unroll
+            for (int a = 0; a < R; a += 4) {
+                const float4 v = *reinterpret_cast<const float4 *>(&xs[buffer][0][dd][tq * R + a]);
+                const float4 w = *reinterpret_cast<const float4 *>(&xs[buffer][1][dd][tc * 4 + 16 * a]);
+                qs[a] = v.x, qs[a + 1] = v.y, qs[a + 2] = v.z, qs[a + 3] = v.w;
+                cs[a] = w.x, cs[a + 1] = w.y, cs[a + 2] = w.z, cs[a + 3] = w.w;
+            }
+#pragma unroll
+            for (int a = 0; a < R; ++a)
+#pragma unroll
+                for (int b = 0; b < R; ++b) {
+                    const float df = qs[a] - cs[b];
+                    acc[a][b] = fmaf(df, df, acc[a][b]);
+                }
+        }
+        if (more) stage(buffer ^ 1);
+    }
+#pragma unroll
+    for (int a = 0; a < R; ++a) {
+        const int r = blockIdx.y * kSide + tq * R + a;
+        if (r >= rows) break;
+        float *dst = dist + (size_t)r * pitch + c0 + tc * 4;
+#pragma unroll
+        for (int b = 0; b < R; b += 4)
+            *reinterpret_cast<float4 *>(dst + 16 * b) = float4{acc[a][b], acc[a][b + 1], acc[a][b + 2], acc[a][b + 3]};
+    }
+}
+
+// The K - 1 smallest keys (distance, number) of every row of `dist`, in order, after the point itself; one wave
+// per row.  First reading: the row is cut into 64 S groups, which leave their minima; the (K-1)-th smallest
+// minimum bounds the (K-1)-th smallest distance, because every minimum is an entry of its own.  A group takes
+// pieces of four neighbouring entries, S 256 entries apart and one lane further each time, so that points whose
+// clusters come in turn (any period) spread over the groups.  Second reading: the entries within the bound (1.4
+// (K-1) of them where 64 S is 2 (K-1) and the order is random) go to LDS and are sorted.  If there are more than
+// LDS has room for, the (K-1)-th smallest of those that found room is a better bound for another reading; if it
+// is no better (many equal distances), the (K-1)-th smallest distance is found bit by bit and the entries equal
+// to it are taken by number.  Needs 2 (K-1) <= 64 S.
+template <int S>
+__global__ __launch_bounds__(256) void select_row_kernel(const float *__restrict__ dist, int N, int row0, int rows,
+                                                         int pitch, int K, int *__restrict__ out_idx,
+                                                         float *__restrict__ out_d) {
+    constexpr int kRoom = 128 * S;
+    __shared__ u64 keys_all[4][kRoom];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = blockIdx.x * 4 + wave, q = row0 + r, want = K - 1;
+    if (r >= rows) return;  // (no barrier below)
+    u64 *keys = keys_all[wave];
+    const float *row = dist + (size_t)r * pitch;
+    const float4 *row4 = reinterpret_cast<const float4 *>(row);
+    const int n4 = (N + 3) / 4;
+    const u64 below = (1ull << lane) - 1ull;
+
+    unsigned int least[S];
+#pragma unroll
+    for (int s = 0; s < S; ++s) least[s] = ~0u;
+    for (int e0 = 0, turn = 0; e0 < n4; e0 += kWave * S, ++turn) {
+        float4 v[S];  // (S loads in flight; past the end the last piece again, which is not counted)
+#pragma unroll
+        for (int s = 0; s < S; ++s) v[s] = row4[min(e0 + s * kWave + ((lane + turn) & (kWave - 1)), n4 - 1)];
+#pragma unroll
+        for (int s = 0; s < S; ++s) {
+            const int e = e0 + s * kWave + ((lane + turn) & (kWave - 1));
+            const float f[4] = {v[s].x, v[s].y, v[s].z, v[s].w};
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int j = e * 4 + c;
+                if (j < N && j != q) least[s] = min(least[s], float_to_ordered(f[c]));
+            }
+        }
+    }
+    unsigned int bound = 0u;  // the want-th smallest minimum: the largest value with fewer than `want` below it
+    for (int b = 31; b >= 0; --b) {
+        const unsigned int trial = bound | (1u << b);
+        int c = 0;
+#pragma unroll
+        for (int s = 0; s < S; ++s) c += __popcll(__ballot(least[s] < trial));
+        if (c < want) bound = trial;
+    }
+    int n = 0;
+    for (;;) {
+        n = 0;
+        for (int e0 = 0; e0 < n4; e0 += 4 * kWave) {
+            float4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = row4[min(e0 + u * kWave + lane, n4 - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                const int e = e0 + u * kWave + lane;
+                const float f[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int j = e * 4 + c;
+                    const bool in = j < N && j != q && float_to_ordered(f[c]) <= bound;
+                    const u64 m = __ballot(in);
+                    if (m) {
+                        const int p = n + __popcll(m & below);
+                        if (in && p < kRoom) keys[p] = pack_key(f[c], j);
+                        n += __popcll(m);
+                    }
+                }
+            }
+        }
+        if (n <= kRoom) break;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        unsigned int better = 0u;  // the want-th smallest distance of the kRoom entries in LDS
+        for (int b = 31; b >= 0; --b) {
+            const unsigned int trial = better | (1u << b);
+            int c = 0;
+            for (int p = lane; p < kRoom; p += kWave) c += __popcll(__ballot((unsigned int)(keys[p] >> 32) < trial));
+            if (c < want) better = trial;
+        }
+        if (better == bound) break;
+        bound = better;
+    }
+    if (n > kRoom) {
+        unsigned int kth = 0u;
+        for (int b = 31; b >= 0; --b) {
+            const unsigned int trial = kth | (1u << b);
+            int c = 0;
+            for (int j = lane; j < N; j += kWave) c += j != q && float_to_ordered(row[j]) < trial;
+#pragma unroll
+            for (int m = kWave / 2; m > 0; m >>= 1) c += __shfl_xor(c, m, kWave);
+            if (c < want) kth = trial;
+        }
+        int closer = 0;  // entries below the want-th smallest distance
+        for (int j = lane; j < N; j += kWave) closer += j != q && float_to_ordered(row[j]) < kth;
+#pragma unroll
+        for (int m = kWave / 2; m > 0; m >>= 1) closer += __shfl_xor(closer, m, kWave);
+        int n_closer = 0, n_equal = 0;
+        for (int j0 = 0; j0 < N; j0 += kWave) {
+            const int j = j0 + lane;
+            const float f = row[min(j, N - 1)];
+            const bool valid = j < N && j != q;
+            const bool lt = valid && float_to_ordered(f) < kth, eq = valid && float_to_ordered(f) == kth;
+            const u64 m_lt = __ballot(lt), m_eq = __ballot(eq);
+            if (lt) keys[n_closer + __popcll(m_lt & below)] = pack_key(f, j);
+            const int at = closer + n_equal + __popcll(m_eq & below);
+            if (eq && at < want) keys[at] = pack_key(f, j);
+            n_closer += __popcll(m_lt);
+            n_equal += __popcll(m_eq);
+        }
+        n = want;
+    }
+    int sort_n = kWave;
+    while (sort_n < n) sort_n <<= 1;
+    for (int e = n + lane; e < sort_n; e += kWave) keys[e] = ~0ull;
+    wave_sort(keys, sort_n, lane);
+    for (int e = lane; e < K; e += kWave) {
+        out_idx[(size_t)q * K + e] = e == 0 ? q : key_index(keys[e - 1]);
+        out_d[(size_t)q * K + e] = e == 0 ? 0.0f : key_distance(keys[e - 1]);
     }
 }
 
@@ -1741,24 +1989,7 @@ __global__ __launch_bounds__(256) void knn_rerank_kernel(const float *__restrict
         }
         keys[c] = key;
     }
-    // Bitonic sort of each wave's own keys: no workgroup barrier, a wave's LDS operations execute in
-    // order and the wavefront fences only keep the compiler from reordering them.
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    for (int k = 2; k <= sort_n; k <<= 1) {
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int t = lane; t < sort_n / 2; t += kWave) {
-                const int lo = ((t & ~(j - 1)) << 1) | (t & (j - 1));
-                const int hi = lo | j;
-                const bool up = (lo & k) == 0;
-                const u64 a = keys[lo], b = keys[hi];
-                if ((a > b) == up) {
-                    keys[lo] = b;
-                    keys[hi] = a;
-                }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        }
-    }
+    wave_sort(keys, sort_n, lane);
     if (!live) return;
     // Sweep on floats: every candidate outside the list has an approximate distance >= tau (without
     // |q|^2), so its canonical distance is >= tau + |q|^2 - g.  g bounds |approximate - canonical|: both are
@@ -1873,6 +2104,49 @@ int valu_cap(int K) {
     int cap = 256;
     while (cap < K - 1 + kCT) cap <<= 1;
     return cap;
+}
+
+// Direct search: distances and their selection, by blocks of query rows.  Measured (points in an order with
+// locality, ms, direct / sweep): 3000 x 64, 91 neighbours 0.13 / 3.9; 5000 x 50, 90: 0.21 / 4.9; 8000 x 126, 151:
+// 0.68 / 4.8; 8192 x 30, 45: 0.35 / 0.93; 12000 x 1024, 45: 6.3 / 18.4; 16384 x 126, 90: 2.1 / 2.6; 20000 x 32, 50:
+// 1.6 / 1.9; 20000 x 784, 45: 13.1 / 14.1; 32000 x 8, 30: 2.8 / 2.7; 32000 x 50, 90: 4.3 / 2.7.  It forms every pair,
+// where the matrix sweep skips tiles and multiplies on the matrix pipe: the line lies where the two are near each other.
+constexpr int kDirectPoints = 16384;
+constexpr int kDirectNeighbors = 256;  // most K - 1 that select_row_kernel<8> takes
+// Floats per block: 64 MiB are cheap to allocate (5000 x 50: 0.21 ms; 0.47 with the whole 100 MB at once), but
+// beyond 10240 points hold too few rows to fill the chip with their selection (16000 x 50: 1.6 ms with 64 MiB, 1.3
+// with 256).
+inline size_t direct_floats(int N) { return (size_t)1 << (N <= 10240 ? 24 : 26); }
+
+int run_direct_search(const float *points, int N, int D, int K, int cus, int *indices, float *sq_dist, hipStream_t s) {
+    const int pitch = div_up(N, 128) * 128;
+    // Tiles of 128 points a side where they fill the chip, of 64 otherwise.
+    const bool large = (int64_t)(pitch / 128) * (pitch / 128) >= 2 * (int64_t)cus;
+    const int side = large ? 128 : 64;
+    const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(direct_floats(N) / pitch) / 128 * 128));
+    DeviceMem dist;
+    if (!dist.alloc(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
+        set_error("knn: out of device memory for the distances");
+        return 1;
+    }
+    for (int row0 = 0; row0 < N; row0 += block) {
+        const int rows = std::min(block, N - row0);
+        const dim3 grid(div_up(N, side), div_up(rows, side));
+        if (large)
+            pair_distances_kernel<8><<<grid, 256, 0, s>>>(points, N, D, row0, rows, pitch, dist.as<float>());
+        else
+            pair_distances_kernel<4><<<grid, 256, 0, s>>>(points, N, D, row0, rows, pitch, dist.as<float>());
+        TSNE_TRY(hipGetLastError());
+        if (2 * (K - 1) <= 64 * 4)
+            select_row_kernel<4><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, indices,
+                                                                 sq_dist);
+        else
+            select_row_kernel<8><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, indices,
+                                                                 sq_dist);
+        TSNE_TRY(hipGetLastError());
+    }
+    TSNE_TRY(hipStreamSynchronize(s));
+    return 0;
 }
 
 // VALU sweep over all points (qlist == nullptr) or over the nq listed queries.
@@ -2008,6 +2282,8 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         TSNE_TRY(hipGetLastError());
         return 0;
     };
+    if (mode == 0 && N <= kDirectPoints && K - 1 <= kDirectNeighbors)
+        return run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
     if (!use_mfma) {
         if (build_transposed()) return 1;
         return run_valu_sweep(points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
