@@ -1141,3 +1141,21 @@ def test_knn_small_problems(stages, n, d, k, kind):
     else:
         idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
         assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("n,d,k,kind", [(16500, 6, 20, "plain"), (17003, 5, 33, "grid"), (20011, 200, 25, "plain"),
+                                        (16640, 140, 20, "far"), (16511, 3, 600, "plain")])
+def test_knn_of_points_in_no_order(stages, n, d, k, kind):
+    """Clusters that come in turn: the search renumbers the points for itself and answers in the caller's
+    numbering - also where equal distances are ordered by it, where queries fail the verification, where no margin
+    verifies and where the neighbours are too many for the matrix sweep.  The vector sweep's rows, bit for bit."""
+    rng = np.random.default_rng(n)
+    X = (rng.standard_normal((n, d)) + (6.0 * rng.standard_normal((5, d)))[np.arange(n) % 5]).astype(np.float32)
+    if kind == "grid":
+        X = np.round(X).astype(np.float32)
+    elif kind == "far":
+        X = (X * np.float32(1e-3) + np.float32(100.0)).astype(np.float32)
+    dX = dev(X)
+    idx, d2 = stages.knn(dX, k)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)

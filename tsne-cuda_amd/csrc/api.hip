@@ -285,7 +285,7 @@ const char *tsne_hip_last_error(void) { return last_error(); }
 int tsne_hip_knn(const float *points, int num_points, int num_dims, int num_neighbors, int *indices,
                  float *sq_dist, void *stream) {
     TSNE_REQUIRE(points && indices && sq_dist, "knn: null pointer argument");
-    return run_knn(points, num_points, num_dims, num_neighbors, indices, sq_dist, (hipStream_t)stream);
+    return run_knn_any_order(points, num_points, num_dims, num_neighbors, indices, sq_dist, (hipStream_t)stream, nullptr);
 }
 
 int tsne_hip_knn_select(const float *points, int num_points, int num_dims, int num_neighbors, int *indices,
@@ -293,6 +293,9 @@ int tsne_hip_knn_select(const float *points, int num_points, int num_dims, int n
     TSNE_REQUIRE(points && indices && sq_dist, "knn: null pointer argument");
     TSNE_REQUIRE(sweep >= 0 && sweep <= 3, "knn: sweep must be 0 (choose), 1 (vector), 2 (matrix) or 3 (matrix on floats), got %d",
                  sweep);
+    if (sweep == 0)
+        return run_knn_any_order(points, num_points, num_dims, num_neighbors, indices, sq_dist, (hipStream_t)stream,
+                                 stats);
     return run_knn_mode(points, num_points, num_dims, num_neighbors, indices, sq_dist, (hipStream_t)stream, sweep,
                         stats);
 }

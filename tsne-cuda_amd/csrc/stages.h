@@ -21,8 +21,17 @@ struct KnnProbes {
 };
 // probes != nullptr: only the matrix sweep's register-resident form can take it (error otherwise); queries whose
 // candidates fail the sweep's verification are then answered by the exact vector sweep over all points.
+// renumbered != nullptr: `points` are a renumbered copy (point i is the caller's order[i]) and the result is in
+// the caller's numbering.
+struct KnnRenumbered {
+    const int *order;            // device
+    const float *caller_points;  // device
+};
 int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
-                 int *stats, const KnnProbes *probes = nullptr);
+                 int *stats, const KnnProbes *probes = nullptr, const KnnRenumbered *renumbered = nullptr);
+// run_knn for points in any order: where the numbering has no locality, the search makes one for itself.
+int run_knn_any_order(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
+                      int *stats);
 // Inverted-file search (ivf.hip).  Trains nlist centroids (Lloyd iterations on a sample) into centroids (device,
 // nlist x D).
 int ivf_train(const float *points, int N, int D, int nlist, int iterations, float *centroids, hipStream_t s);
