@@ -1159,3 +1159,33 @@ def test_knn_of_points_in_no_order(stages, n, d, k, kind):
     idx, d2 = stages.knn(dX, k)
     idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("n,k", [(2, 2), (63, 5), (65, 1), (130, 129), (1203, 32), (2049, 33), (20011, 50), (300, 300)])
+def test_small_step_forms(stages, n, k):
+    """The step of a small problem takes its attractive forces in spare workgroups of the inverse row pass and
+    launches the grouping kernels every fourth step only; with per-kernel timing on it launches every kernel by
+    itself on every step.  Same bits, at the remainders of the rows of a workgroup and of the entries of a lane."""
+    rng = np.random.default_rng(n)
+    idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
+    idx[:, 0] = np.arange(n)
+    P = (rng.random((n, k)) / (n * k)).astype(np.float32)
+    y0 = rng.standard_normal(2 * n).astype(np.float32)
+
+    def run(timed):
+        plan = stages.Plan(n, k)
+        plan.prepare_attractive(dev(P), dev(idx))
+        if timed:
+            plan.profile_begin()
+        y = dev(y0).clone()
+        gains, old = torch.ones_like(y), torch.zeros_like(y)
+        for first in (0, 3, 12):  # (calls that take up where the one before left off)
+            z = plan.iterate_(None, None, y, gains, old, first, {0: 3, 3: 12, 12: 23}[first], eta=50.0)
+        torch.cuda.synchronize()
+        if timed:
+            assert plan.profile_end()["attractive_kernel"][1] == 23
+        plan.close()
+        return [v.cpu().numpy() for v in (y, gains, old, z)]
+
+    for a, b in zip(run(False), run(True)):
+        assert same_bits(a, b)

@@ -102,12 +102,6 @@ int check_plan(const tsne_hip_plan *p, const char *who) {
 
 namespace tsnehip {
 
-// Up to this many points a step is a chain of short dependent kernels that the attractive kernel hardly
-// lengthens: one stream without events and without a captured graph is then the fastest form (fits of 5000, 60000
-// and 50000 points 5 %, 3.5 % and 2.7 % shorter than with two streams and graphs, whose events cost 7-10 us per
-// step and whose instantiation 4 ms per stretch of constant parameters; at 100000 points two streams are 4 % ahead).
-constexpr int kSingleStreamPoints = 65536;
-
 // TSNE_OVERLAP: 0 never, 1 always, unset: by the size of the problem.
 static bool overlap_enabled(const tsne_hip_plan *p) {
     const char *v = std::getenv("TSNE_OVERLAP");  // read on every call, like TSNE_GRAPH
@@ -142,6 +136,12 @@ static int launch_step_attractive(tsne_hip_plan *p, const float *pij, const int 
     if (p->csr_row_ptr) return launch_attractive_csr(p, p->csr_row_ptr, p->csr_col_idx, p->csr_values, p->attr, s);
     return launch_attractive_blocked(p, p->attr, s);
 }
+
+// The kernels that group the points by tile exit at once while an earlier step's grouping is kept, 2 us each on every
+// step; launched less often, a grouping that has become poor is kept until then and costs the spread kernel strays.
+// 20011 points x 50 neighbours from the start of a fit at learning rate 200, us per step: launched every step 79.7
+// (with the attractive kernel by itself), every second 68.4, every fourth 73.6 (spread 12.8 -> 19.8).
+constexpr int kGroupingInterval = 2;
 
 static bool overlap_active(const tsne_hip_plan *p) {
     return overlap_enabled(p) && !p->profiling && p->side_stream != nullptr;
@@ -183,6 +183,18 @@ int launch_step(tsne_hip_plan *p, const float *pij, const int *indices, float *e
                 float *old_forces, float eta, float momentum, float exaggeration, int slot, float *normalization,
                 hipStream_t s) {
     if (!overlap_active(p)) {
+        // A small problem's step is its launches one after the other.  Its attractive forces ride along with the
+        // inverse row pass, whose workgroups leave most of the chip idle (kernel alone, us: 1203 points x 32 neighbours
+        // 5.1 -> 0; 20011 x 50 8.3 -> 1.5; 50000 x 90 13.4 -> 12.8, the positions' cache lines), and the two kernels
+        // that group the points by tile are only launched every kGroupingInterval steps.
+        if (!pij && !p->csr_row_ptr && p->row_entries && !p->profiling && !p->profiling_attractive) {
+            const SmallStep small = {p->attr, p->steps_to_grouping <= 0};
+            p->steps_to_grouping = (small.may_group ? kGroupingInterval : p->steps_to_grouping) - 1;
+            if (launch_repulsive(p, embedding, slot, p->rep, nullptr, nullptr, s, true, &small)) return 1;
+            if (normalization && launch_finish_z(p, normalization, s)) return 1;
+            return launch_update(p, embedding, p->attr, p->rep, gains, old_forces, eta, nullptr, momentum, exaggeration,
+                                 slot ^ 1, s);
+        }
         if (launch_repulsive(p, embedding, slot, p->rep, nullptr, nullptr, s, true)) return 1;
         if (launch_step_attractive(p, pij, indices, s)) return 1;
         if (normalization && launch_finish_z(p, normalization, s)) return 1;
@@ -732,6 +744,7 @@ int tsne_hip_plan_set_boxes(tsne_hip_plan *plan, int n_boxes_per_dim) {
     plan->n_nodes = n_boxes_per_dim * kInterp;
     // (a grouping of the points by tile belongs to the grid it was made on)
     TSNE_TRY(hipMemset(&plan->scalars->reuse_sort, 0, sizeof(int)));
+    plan->steps_to_grouping = 0;
     return 0;
 }
 

@@ -32,6 +32,7 @@
 #include <cstdlib>
 #include <vector>
 
+#include "pair_force.h"
 #include "plan.h"
 #include "stages.h"
 
@@ -44,7 +45,6 @@ constexpr int kPartPoints = 2048;   // == 1 << kColBits; 16 KB of (x, y) pairs, 
 constexpr int kStripMax = 3968;     // rows per strip: 31 KB of positions + 62 KB of accumulators; with the two
                                     // partitions 125 KB, which leaves 35 KB of a CU's LDS to the kernels of the
                                     // repulsive chain that run beside this one
-constexpr double kRoundMagic = 6755399441055744.0;  // 1.5 * 2^52: adding it rounds a double to an integer
 constexpr int kBlock = 1024;
 constexpr int kMaxParts = 8192;     // column partitions: up to 16.7 M points
 constexpr int kPrefetch = 4;        // entries per thread in one work item
@@ -272,15 +272,10 @@ __global__ void clear_pmax_kernel(float *p_max) {
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ void add_force(unsigned long long *acc, unsigned int rl, float vx, float vy,
                                           double scale, int y_offset = kStripMax) {
-    // magic + v * scale is a double in [2^52, 2^53), where doubles are the integers: its bit pattern is the
-    // magic's plus round(v * scale).  The patterns themselves are summed; every row has exactly K entries, so
-    // its accumulators start at -K times the magic's pattern (mod 2^64) and end at the sum of the integers.
-    const double tx = fma((double)vx, scale, kRoundMagic);
-    const double ty = fma((double)vy, scale, kRoundMagic);
     // x sums and y sums live in separate arrays: consecutive rows then fall
     // into consecutive 8-byte slots and the atomics of a wave spread over all banks.
-    atomicAdd(&acc[rl], (unsigned long long)__double_as_longlong(tx));
-    atomicAdd(&acc[y_offset + rl], (unsigned long long)__double_as_longlong(ty));
+    atomicAdd(&acc[rl], fixed_force(vx, scale));
+    atomicAdd(&acc[y_offset + rl], fixed_force(vy, scale));
 }
 
 // Polls *counter until it reaches `need`; after kSpinLimit polls the wave sets *gave_up and goes on (the
@@ -343,10 +338,10 @@ __global__ __launch_bounds__(kBlock, 8) void attractive_blocked_kernel(const flo
     ConstWords run_start = hdr + 4;  // ~0 after the last run
     ConstWords fresh_parts = run_start + list_words;
     const float pm = scalars->vmax;
-    const double scale = pm > 0.0f ? 2251799813685248.0 / (double)pm : 1.0;  // 2^51 / p_max
+    const double scale = force_scale(pm);
 
     const unsigned long long acc_start =
-        0ull - (unsigned long long)K * (unsigned long long)__double_as_longlong(kRoundMagic);
+        fixed_force_start(K);
     for (int r = tid; r < nrows; r += kBlock) {
         yi[r] = yxy[row0 + r];
         acc[r] = acc_start;
@@ -626,9 +621,9 @@ __global__ __launch_bounds__(kDirectThreads) void attractive_direct_kernel(const
     const int nrows = (int)hdr[2];
     ConstWords window_start = hdr + 4;  // the count after the last window, then ~0
     const float pm = scalars->vmax;
-    const double scale = pm > 0.0f ? 2251799813685248.0 / (double)pm : 1.0;  // 2^51 / p_max
+    const double scale = force_scale(pm);
     const unsigned long long acc_start =
-        0ull - (unsigned long long)K * (unsigned long long)__double_as_longlong(kRoundMagic);
+        fixed_force_start(K);
     for (int r = tid; r < nrows; r += kDirectThreads) {
         yi[r] = yxy[row0 + r];
         acc[r] = acc_start;
@@ -756,6 +751,12 @@ __global__ __launch_bounds__(256) void micro_strip_parts_kernel(const int *__res
     for (int w = threadIdx.x; w < words; w += 256) bitmaps[(size_t)blockIdx.x * words + w] = bits[w];
 }
 
+__global__ __launch_bounds__(256) void row_entries_kernel(const float *__restrict__ pij, const int *__restrict__ indices,
+                                                          int64_t n, uint2 *__restrict__ entries) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e < n) entries[e] = make_uint2(__float_as_uint(pij[e]), (unsigned int)indices[e]);
+}
+
 }  // namespace
 
 // row0 (n_strips + 1 entries, ascending, row0[0] = 0, row0[n_strips] = N) of strips with at most kStripMax rows
@@ -822,7 +823,9 @@ void release_blocked(tsne_hip_plan *p) {
     (void)hipFree(p->seg);
     (void)hipFree(p->strip_row0);
     (void)hipFree(p->wseg);
+    (void)hipFree(p->row_entries);
     p->wseg = nullptr;
+    p->row_entries = nullptr;
     p->blocked_direct = false;
     p->ent_p = nullptr;
     p->seg = nullptr;
@@ -992,6 +995,15 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBlockedLds));
     p->spin_limit = kSpinLimit;
     if (const char *v = std::getenv("TSNE_ATTRACTIVE_SPIN_LIMIT")) p->spin_limit = std::max(0, std::atoi(v));
+    if (N <= kSingleStreamPoints && K <= kRowEntriesNeighbors) {
+        if (hipMalloc(&p->row_entries, sizeof(uint2) * (size_t)N * K) != hipSuccess) {
+            release_blocked(p);
+            set_error("attractive_prepare: out of device memory for the row-ordered pattern");
+            return 1;
+        }
+        row_entries_kernel<<<div_up((int64_t)N * K, 256), 256, 0, s>>>(pij, indices, (int64_t)N * K, p->row_entries);
+        TSNE_LAUNCHED(s);
+    }
     p->blocked_ready = true;
     return 0;
 }

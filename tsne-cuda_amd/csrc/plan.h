@@ -38,6 +38,13 @@ struct LagrangeMonomials {
     double c[kInterp][3];
 };
 
+// Up to this many points a step is a chain of short dependent kernels that the attractive kernel hardly
+// lengthens: one stream without events and without a captured graph is then the fastest form (fits of 5000, 60000
+// and 50000 points 5 %, 3.5 % and 2.7 % shorter than with two streams and graphs, whose events cost 7-10 us per
+// step and whose instantiation 4 ms per stretch of constant parameters; at 100000 points two streams are 4 % ahead).
+constexpr int kSingleStreamPoints = 65536;
+constexpr int kRowEntriesNeighbors = 512;  // most neighbours the row-ordered copy of such a problem's pattern is made for
+
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
     kKernelTileCount = 0,
@@ -108,6 +115,10 @@ struct tsne_hip_plan {
     bool blocked_direct = false;
     unsigned int *wseg = nullptr;
     int wseg_stride = 0, n_windows = 0;
+    // Small problems (one stream, see api.hip): the pattern once more, row by row, {probability, neighbour} in the
+    // caller's order of neighbours; the inverse row pass computes the attractive forces from it in spare workgroups.
+    uint2 *row_entries = nullptr;
+    int steps_to_grouping = 0;      // steps of that form until the grouping kernels are launched again
     int spin_limit = 0;             // polls before a wave of the attractive kernel gives up a wait
     bool blocked_ready = false;
     // Optional CSR pattern (borrowed pointers; tsne_hip_plan_set_csr_pattern): when set, steps without an explicit
@@ -179,8 +190,16 @@ int launch_bounds_reset(tsne_hip_plan *p, int slot, hipStream_t s, bool new_embe
 int launch_bounds(tsne_hip_plan *p, const float *embedding, int slot, hipStream_t s, bool new_embedding = true);
 // keep_grouping: the call is a step of a gradient loop over this embedding buffer, so the grouping of the points by
 // spreading tile may be carried over from the step before (the kernels decide on the device); otherwise it is redone.
+// How launch_repulsive is used by the loop of a small problem (see launch_step): attractive forces (2N) computed in
+// spare workgroups of the inverse row pass from the plan's row_entries, and whether the points may be grouped
+// afresh by this step.
+struct SmallStep {
+    float *attr;
+    bool may_group;
+};
 int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *rep, float *point_potentials,
-                     float *charges_out, hipStream_t s, bool keep_grouping = false);
+                     float *charges_out, hipStream_t s, bool keep_grouping = false,
+                     const SmallStep *small = nullptr);
 // Writes Z = z_sum - N to the device scalar *normalization.
 int launch_finish_z(tsne_hip_plan *p, float *normalization, hipStream_t s);
 int launch_pack_xy(tsne_hip_plan *p, const float *embedding, hipStream_t s);

@@ -22,6 +22,7 @@
 //     planes of a pair in proportion to the larger one, so planes of like
 //     magnitude are paired: (1, r^2 / m^2) and (x, y), with m the largest
 //     absolute coordinate.
+#include "pair_force.h"
 #include "plan.h"
 
 #include <algorithm>
@@ -610,6 +611,9 @@ __device__ __forceinline__ float box_lower(int b, const Bounds &bd) {
 constexpr int kHalo = 1;
 constexpr int kRegionBoxes = kTileBoxes + 2 * kHalo;
 constexpr int kRegionBoxes2 = kRegionBoxes * kRegionBoxes;
+// keep_grouping of the chain's kernels: 0 never, 1 while the flag on the device says so, kKeepAlways whatever it
+// says (a step that does not launch the grouping kernels).
+constexpr int kKeepAlways = 2;
 constexpr int kMaxSortAge = 32;  // steps a grouping is kept at most
 constexpr int kStrayShift = 10;  // ... and only while at most N / 2^10 points strayed in the last step (36 global atomics each),
 constexpr int kStrayFloor = 128; // or 128 of a small problem's
@@ -639,7 +643,7 @@ __global__ __launch_bounds__(kSpreadThreads, 4) void spread_kernel(const float2 
     const int c0 = (int)((long long)share * nc / gridDim.x);
     const int c1 = (int)((long long)(share + 1) * nc / gridDim.x);
     if (share < 0 || c0 >= c1) return;
-    const bool reuse = keep_grouping && sc->reuse_sort;
+    const bool reuse = keep_grouping == kKeepAlways || (keep_grouping && sc->reuse_sort);
     const int tid = threadIdx.x;
     for (int e = tid; e < kMoments * kRegionBoxes2; e += kSpreadThreads) acc[e] = 0ull;
     const int tiles_per_dim = (n_boxes + kTileBoxes - 1) / kTileBoxes;
@@ -1117,12 +1121,65 @@ __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *_
 // Inverse row pass for x nodes m0, m0+1: consumes digit-reversed positions,
 // produces node potentials in natural order, scaled by 1 / (transform length)^2.
 // ---------------------------------------------------------------------------
+
+// Attractive forces of kRowThreads / kForceLanes rows from the row-ordered pattern: kForceLanes lanes per row, four
+// entries of a lane in flight, the same fixed-point sums as the re-blocked kernel's (the same bits).
+constexpr int kForceLanes = 8;
+struct RowForces {
+    const uint2 *entries;  // null: no workgroups of this kind
+    const float2 *yxy;
+    float *attr;
+    int N, K;
+    int first_block;  // (a multiple of the XCD count: the workgroups before it are the row pass's)
+};
+__device__ __forceinline__ void row_forces_block(const RowForces &f, int block, float p_max) {
+    const int row = block * (kRowThreads / kForceLanes) + (int)threadIdx.x / kForceLanes;
+    const int lane = threadIdx.x % kForceLanes;
+    const bool live = row < f.N;
+    const uint2 *mine = f.entries + (size_t)(live ? row : 0) * f.K;
+    const float2 yi = f.yxy[live ? row : 0];
+    const double scale = force_scale(p_max);
+    unsigned long long ax = 0ull, ay = 0ull;
+    for (int k0 = lane; k0 < f.K; k0 += 4 * kForceLanes) {
+        uint2 en[4];
+        float2 yj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) en[u] = mine[min(k0 + u * kForceLanes, f.K - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) yj[u] = f.yxy[en[u].y];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            if (k0 + u * kForceLanes < f.K) {
+                const float2 v = pair_force(__uint_as_float(en[u].x), yi, yj[u]);
+                ax += fixed_force(v.x, scale);
+                ay += fixed_force(v.y, scale);
+            }
+        }
+    }
+#pragma unroll
+    for (int m = kForceLanes / 2; m > 0; m >>= 1) {
+        ax += __shfl_xor(ax, m, kWave);
+        ay += __shfl_xor(ay, m, kWave);
+    }
+    if (live && lane < 2) {
+        const unsigned long long sum = (lane ? ay : ax) + fixed_force_start(f.K);
+        f.attr[(size_t)lane * f.N + row] = (float)((double)(long long)sum * (1.0 / scale));
+    }
+}
+
+// With rows.entries set, the workgroups from rows.first_block on compute the attractive forces of a small problem
+// (nothing of this step but the update waits for either).
 template <int NFFT>
 __global__ __launch_bounds__(kRowThreads) void conv_rows_inverse_kernel(const float2 *__restrict__ col_results, int G,
                                                                 const LoopScalars *sc, int slot,
                                                                 const float2 *__restrict__ twiddles,
-                                                                float4 *__restrict__ node_potentials) {
+                                                                float4 *__restrict__ node_potentials,
+                                                                RowForces rows) {
     using T = Transform<NFFT>;
+    if (rows.entries && (int)blockIdx.x >= rows.first_block) {
+        row_forces_block(rows, blockIdx.x - rows.first_block, sc->vmax);
+        return;
+    }
     __shared__ float2 s[4][NFFT];  // [row * 2 + pair]
     const float2 *tw = twiddles;
     const int tid = threadIdx.x;
@@ -1166,7 +1223,7 @@ __global__ __launch_bounds__(256) void gather_forces_kernel(const float *__restr
     // Last kernel of the chain: whether the next step keeps this step's grouping of the points by tile.  (The
     // spread kernel has finished counting; the chain's kernels of this step have all read the flag.)
     if (blockIdx.x == 0 && threadIdx.x == 0) {
-        const bool reused = keep_grouping && sc->reuse_sort;
+        const bool reused = keep_grouping == kKeepAlways || (keep_grouping && sc->reuse_sort);
         const int age = reused ? sc->sort_age + 1 : 0;
         const unsigned int strays = sc->strays;
         sc->strays = 0u;
@@ -1235,6 +1292,7 @@ int launch_finish_z(tsne_hip_plan *p, float *normalization, hipStream_t s) {
 }
 
 int launch_bounds_reset(tsne_hip_plan *p, int slot, hipStream_t s, bool new_embedding) {
+    if (new_embedding) p->steps_to_grouping = 0;
     bounds_reset_kernel<<<1, 64, 0, s>>>(p->scalars, slot, new_embedding ? 1 : 0);
     TSNE_LAUNCHED(s);
     return 0;
@@ -1255,24 +1313,28 @@ int launch_bounds(tsne_hip_plan *p, const float *embedding, int slot, hipStream_
 // `embedding` in `slot`; leaves sum_i z_i in scalars->z_part and resets the other
 // bounds slot.  charges_out (optional) receives a copy of the node charges.
 int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *rep, float *point_potentials,
-                     float *charges_out, hipStream_t s, bool keep_grouping) {
-    const int keep = keep_grouping && p->keep_grouping ? 1 : 0;
+                     float *charges_out, hipStream_t s, bool keep_grouping, const SmallStep *small) {
+    int keep = keep_grouping && p->keep_grouping ? 1 : 0;
+    const bool group = !small || small->may_group || !keep;
+    if (!group) keep = kKeepAlways;
     const int N = p->num_points, G = p->n_nodes, nb = p->n_boxes;
     const int tiles_per_dim = (nb + kTileBoxes - 1) / kTileBoxes;
     // Few, large workgroups: every workgroup ends with one global atomic per tile counter, and
     // same-address atomics serialise (about a thousand per counter cost ~20 us).
     // (one point per thread until that many workgroups are in use)
     const int sort_blocks = std::min(div_up(N, 1024), kSortBlocks);
-    if (profile_mark(p, kKernelTileCount, s)) return 1;
-    TSNE_LOOP_KERNEL(p, (tile_count_kernel), sort_blocks, 1024, 0, s, embedding, N, p->scalars, slot, slot ^ 1, nb, p->tile_count,
-                                                   p->tile_cursor, p->chunks, p->num_chunks, p->num_chunks + 1,
-                                                   p->point_code, p->wg_tile_base, keep);
-    TSNE_LAUNCHED(s);
-    if (profile_mark(p, kKernelTileScatter, s)) return 1;
-    TSNE_LOOP_KERNEL(p, (tile_scatter_kernel), sort_blocks, 1024, 0, s, embedding, N, tiles_per_dim * tiles_per_dim, p->tile_cursor,
-                                                     p->point_code, p->wg_tile_base, p->tile_xy, p->tile_perm,
-                                                     p->scalars, keep);
-    TSNE_LAUNCHED(s);
+    if (group) {
+        if (profile_mark(p, kKernelTileCount, s)) return 1;
+        TSNE_LOOP_KERNEL(p, (tile_count_kernel), sort_blocks, 1024, 0, s, embedding, N, p->scalars, slot, slot ^ 1, nb, p->tile_count,
+                                                       p->tile_cursor, p->chunks, p->num_chunks, p->num_chunks + 1,
+                                                       p->point_code, p->wg_tile_base, keep);
+        TSNE_LAUNCHED(s);
+        if (profile_mark(p, kKernelTileScatter, s)) return 1;
+        TSNE_LOOP_KERNEL(p, (tile_scatter_kernel), sort_blocks, 1024, 0, s, embedding, N, tiles_per_dim * tiles_per_dim, p->tile_cursor,
+                                                         p->point_code, p->wg_tile_base, p->tile_xy, p->tile_perm,
+                                                         p->scalars, keep);
+        TSNE_LAUNCHED(s);
+    }
     if (profile_mark(p, kKernelSpread, s)) return 1;
     // Resident workgroups share the chunk list (its length is only known on the device; with fewer chunks
     // than workgroups the surplus ones exit at once).
@@ -1314,12 +1376,18 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
                                                                   p->col_results, p->box_moments, moment_words);
     TSNE_LAUNCHED(s);
     if (profile_mark(p, kKernelConvRowsInverse, s)) return 1;
+    RowForces rows = {nullptr, nullptr, nullptr, 0, 0, 0};
+    int inverse_grid = row_grid;
+    if (small) {
+        rows = {p->row_entries, p->yxy, small->attr, N, p->num_neighbors, row_grid};
+        inverse_grid += div_up(N, kRowThreads / kForceLanes);
+    }
     if (short_fft)
-        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFftShort>), row_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
-                                                                            p->twiddles_short, p->node_potentials);
+        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFftShort>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
+                                                                            p->twiddles_short, p->node_potentials, rows);
     else
-        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFft>), row_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
-                                                                       p->twiddles, p->node_potentials);
+        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFft>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
+                                                                       p->twiddles, p->node_potentials, rows);
     TSNE_LAUNCHED(s);
     if (profile_mark(p, kKernelGather, s)) return 1;
     TSNE_LOOP_KERNEL(p, (gather_forces_kernel), std::min(div_up(N, 256), 1024), 256, 0, s, embedding, N, p->scalars, slot, nb, p->lagrange,
