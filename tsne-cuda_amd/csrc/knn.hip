@@ -814,13 +814,14 @@ __global__ __launch_bounds__(256) void knn_merge_slices_kernel(const u64 *__rest
 // ---------------------------------------------------------------------------
 constexpr int kDirectDims = 16;  // dimensions staged per chunk
 
-// Distances of query rows row0 .. row0 + rows - 1 (rows of `dist`, pitch floats each, pitch a multiple of the
-// tile's side 16 R and at least N) to all points; columns from N on are left as distances to a point at 0.
+// Distances of rows row0 .. row0 + rows - 1 of Q (NQ x D; rows of `dist`, pitch floats each, pitch a multiple of the
+// tile's side 16 R and at least N) to the N rows of X; columns from N on are left as distances to a point at 0.
 // A workgroup computes a square tile, R x R distances per thread, both operands staged in LDS a chunk of
 // dimensions ahead; same fma chain as everywhere (dimensions past D are zeros on both sides, which leave a sum
 // as it is).  Bound by the vector ALU, two instructions per pair and dimension.
 template <int R>
-__global__ __launch_bounds__(256) void pair_distances_kernel(const float *__restrict__ X, int N, int D, int row0,
+__global__ __launch_bounds__(256) void pair_distances_kernel(const float *__restrict__ Q, int NQ,
+                                                             const float *__restrict__ X, int N, int D, int row0,
                                                              int rows, int pitch, float *__restrict__ dist) {
     constexpr int kSide = 16 * R;
     constexpr int kRow = kSide + 4;              // LDS row: 16-byte aligned, chunk rows off each other's banks
@@ -828,7 +829,8 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__rest
     __shared__ __attribute__((aligned(16))) float xs[2][2][kDirectDims][kRow];
     const int tid = threadIdx.x, tq = tid >> 4, tc = tid & 15;
     const int q0 = row0 + blockIdx.y * kSide, c0 = blockIdx.x * kSide;
-    const bool wide = (D & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+    const bool wide =
+        (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Q)) & 15) == 0;
     float4 ahead[2][kLoads];
     auto load = [&](int d0) {
 #pragma unroll
@@ -837,8 +839,8 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__rest
             for (int u = 0; u < kLoads; ++u) {
                 const int e = tid + u * 256, p = (o ? c0 : q0) + (e >> 2), d = d0 + 4 * (e & 3);
                 float4 v = {0.0f, 0.0f, 0.0f, 0.0f};
-                if (p < N && d < D) {
-                    const float *x = X + (size_t)p * D + d;
+                if (p < (o ? N : NQ) && d < D) {
+                    const float *x = (o ? X : Q) + (size_t)p * D + d;
                     if (wide) {
                         v = *reinterpret_cast<const float4 *>(x);
                     } else {
@@ -1036,6 +1038,8 @@ struct SweepArgs {
     const float4 *Xp;
     const float *X;  // the points as given (bf16 sweep: the query side is formed from them)
     const float *centres_p, *tile_coef;  // chunked bf16 sweep: tile centres by chunk, error coefficients
+    const float *centre_dist;  // chunked bf16 sweep, TABLE: |query - tile centre|^2, a row of centre_pitch per tile
+    int centre_pitch;
     int N, D, Dnorm, want, cap;
     u64 *lists;
     int num_qtiles;
@@ -1536,7 +1540,11 @@ constexpr int kChunkSteps = 32;
 constexpr int kChunkS4 = kChunkSteps / 4;            // float4 per lane, block and chunk
 constexpr int kChunkFloat4 = 4 * kChunkS4 * 64;      // float4 per tile chunk
 
-template <bool BF16>
+// TABLE (bf16): |q - m|^2 comes from a table of all queries and tile centres, formed beforehand; otherwise every wave
+// forms it chunk by chunk from the query's own two terms and the centre's chunk, which is five vector instructions
+// per coordinate and 16 registers beside the matrix instructions (sweeps of 50000 x 1024: 27.5 -> 24.3 ms and 1.2 for
+// the table; 60000 x 784: 13.7 -> 11.9 and 1.1).
+template <bool BF16, bool TABLE>
 __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const SweepArgs args) {
     const int N = args.N, D = args.D, want = args.want, cap = args.cap;
     const int num_qtiles = args.num_qtiles, n_chunks = args.n_chunks;
@@ -1612,11 +1620,13 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             for (int b = 0; b < 4; ++b)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
-            float f_part = 0.0f;  // bf16: this lane's share of |q - m|^2 (m: the tile's centre)
+            // bf16: this lane's share of |q - m|^2 (m: the tile's centre), or all of it from the table
+            float f_part = 0.0f;
+            if constexpr (TABLE) f_part = args.centre_dist[(size_t)ct * args.centre_pitch + q];
             for (int c = 0; c < n_chunks; ++c) {
                 const bool last = c + 1 == n_chunks;
                 v4f mc[2 * kSteps16];  // bf16: the centre's 16 coordinates that go with this lane's 16 of the chunk
-                if constexpr (BF16) {
+                if constexpr (BF16 && !TABLE) {
                     const v4f *msrc = reinterpret_cast<const v4f *>(args.centres_p) + (size_t)ct * (8 * n_chunks) + 8 * c + 2 * kh;
 #pragma unroll
                     for (int step = 0; step < kSteps16; ++step) {
@@ -1650,18 +1660,20 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
 #pragma unroll
                         for (int b = 0; b < 4; ++b)
                             acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, xl[b]), qh, acc[b], 0, 0, 0);
-                        // |q - m|^2 from the query's two terms: q_d = -(high + low) / 2 to within 2^-16 |q_d|.
-                        const uint4 uh = __builtin_bit_cast(uint4, bcur[step]), ul = __builtin_bit_cast(uint4, bcur[kSteps16 + step]);
-                        const unsigned int wh[4] = {uh.x, uh.y, uh.z, uh.w}, wl[4] = {ul.x, ul.y, ul.z, ul.w};
-                        const float m[8] = {mc[2 * step][0], mc[2 * step][1], mc[2 * step][2], mc[2 * step][3],
-                                            mc[2 * step + 1][0], mc[2 * step + 1][1], mc[2 * step + 1][2], mc[2 * step + 1][3]};
+                        if constexpr (!TABLE) {
+                            // |q - m|^2 from the query's two terms: q_d = -(high + low) / 2 to within 2^-16 |q_d|.
+                            const uint4 uh = __builtin_bit_cast(uint4, bcur[step]), ul = __builtin_bit_cast(uint4, bcur[kSteps16 + step]);
+                            const unsigned int wh[4] = {uh.x, uh.y, uh.z, uh.w}, wl[4] = {ul.x, ul.y, ul.z, ul.w};
+                            const float m[8] = {mc[2 * step][0], mc[2 * step][1], mc[2 * step][2], mc[2 * step][3],
+                                                mc[2 * step + 1][0], mc[2 * step + 1][1], mc[2 * step + 1][2], mc[2 * step + 1][3]};
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) {
-                            const float s0 = __uint_as_float(wh[k] << 16) + __uint_as_float(wl[k] << 16);
-                            const float s1 = __uint_as_float(wh[k] & 0xffff0000u) + __uint_as_float(wl[k] & 0xffff0000u);
-                            const float e0 = fmaf(-0.5f, s0, -m[2 * k]), e1 = fmaf(-0.5f, s1, -m[2 * k + 1]);
-                            f_part = fmaf(e0, e0, f_part);
-                            f_part = fmaf(e1, e1, f_part);
+                            for (int k = 0; k < 4; ++k) {
+                                const float s0 = __uint_as_float(wh[k] << 16) + __uint_as_float(wl[k] << 16);
+                                const float s1 = __uint_as_float(wh[k] & 0xffff0000u) + __uint_as_float(wl[k] & 0xffff0000u);
+                                const float e0 = fmaf(-0.5f, s0, -m[2 * k]), e1 = fmaf(-0.5f, s1, -m[2 * k + 1]);
+                                f_part = fmaf(e0, e0, f_part);
+                                f_part = fmaf(e1, e1, f_part);
+                            }
                         }
                     }
                 } else {
@@ -1698,13 +1710,14 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             // has no threshold yet (a part can hold fewer than `want` real candidates, so nothing would
             // push them out of the list later).
             // bf16: the keys are lower bounds of the distances: product + `off`, off = |q - m|^2 rounded down
-            // (the rounding of its sum, and the 2^-16 |q| by which the query's two terms miss q) less the tile's
-            // error bound; the products are tested against the threshold less `off`, rounded up.
+            // (the rounding of its sum, and, formed from the query's two terms, the 2^-16 |q| by which they miss q)
+            // less the tile's error bound; the products are tested against the threshold less `off`, rounded up.
             float off = 0.0f, limit_acc = limit_d;
             if constexpr (BF16) {
-                const float f = f_part + __shfl_xor(f_part, 32);
-                off = f * (1.0f - (float)(D + 4) * 5.9604644775390625e-08f) - 2.1f / 65536.0f * q_len * sqrtf(f) -
-                      fmaf(q_len, args.tile_coef[2 * ct], args.tile_coef[2 * ct + 1]);
+                const float f = TABLE ? f_part : f_part + __shfl_xor(f_part, 32);
+                off = f * (1.0f - (float)(D + 4) * 5.9604644775390625e-08f);
+                if constexpr (!TABLE) off -= 2.1f / 65536.0f * q_len * sqrtf(f);
+                off -= fmaf(q_len, args.tile_coef[2 * ct], args.tile_coef[2 * ct + 1]);
                 limit_acc = limit_d - off;
                 limit_acc += 2.4e-7f * (fabsf(limit_d) + fabsf(off));
             }
@@ -2166,9 +2179,9 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
         const int rows = std::min(block, N - row0);
         const dim3 grid(div_up(N, side), div_up(rows, side));
         if (large)
-            pair_distances_kernel<8><<<grid, 256, 0, s>>>(points, N, D, row0, rows, pitch, dist.as<float>());
+            pair_distances_kernel<8><<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
         else
-            pair_distances_kernel<4><<<grid, 256, 0, s>>>(points, N, D, row0, rows, pitch, dist.as<float>());
+            pair_distances_kernel<4><<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
         TSNE_TRY(hipGetLastError());
         if (2 * (K - 1) <= 64 * 4)
             select_row_kernel<4><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, indices,
@@ -2359,7 +2372,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
                                                          num_tiles, Xp.as<float4>());
         TSNE_TRY(hipGetLastError());
     }
-    DeviceMem centres_p, tile_coef;
+    DeviceMem centres_p, tile_coef, centre_rows, centre_dist;
     if (bf16_chunked) {
         if (!centres_p.alloc(sizeof(float) * 32 * (size_t)n_chunks * num_tiles) ||
             !tile_coef.alloc(sizeof(float) * 2 * (size_t)num_tiles)) {
@@ -2376,6 +2389,17 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         pack_chunked_centres_kernel<<<num_tiles, 64, 0, s>>>(centers.as<float>(), radius.as<float>(), D, n_chunks,
                                                             num_tiles, centres_p.as<float>(), tile_coef.as<float>());
         TSNE_TRY(hipGetLastError());
+        // The table grows with the square of the points (80 MB at 50000) and is made where it takes up to 1 GB.
+        const size_t table_bytes = sizeof(float) * (size_t)num_tiles * Npad;
+        if (table_bytes <= (size_t)1 << 30 && centre_rows.alloc(sizeof(float) * (size_t)num_tiles * D) &&
+            centre_dist.alloc(table_bytes)) {
+            transpose_points_kernel<<<dim3(div_up(D, 32), div_up(num_tiles, 32)), 256, 0, s>>>(
+                centers.as<float>(), D, num_tiles, D, centre_rows.as<float>());
+            TSNE_TRY(hipGetLastError());
+            pair_distances_kernel<8><<<dim3(div_up(N, 128), div_up(num_tiles, 128)), 256, 0, s>>>(
+                centre_rows.as<float>(), num_tiles, points, N, D, 0, num_tiles, Npad, centre_dist.as<float>());
+            TSNE_TRY(hipGetLastError());
+        }
     }
 
     // Sweep + re-rank of `count` query tiles: those of tile_list (device), or first, first + step, ... without a
@@ -2408,6 +2432,8 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         args.X = points;
         args.centres_p = centres_p.as<float>();
         args.tile_coef = tile_coef.as<float>();
+        args.centre_dist = centre_dist.as<float>();
+        args.centre_pitch = Npad;
         args.N = N;
         args.D = D;
         args.Dnorm = Dnorm;
@@ -2437,15 +2463,12 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         args.probe_list_tiles = probes ? probes->list_tiles : nullptr;
         if (chunked) {
             const size_t lds = sweep_lds(keep);
-            if (bf16_chunked) {
-                TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(knn_mfma_chunked_sweep_kernel<true>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                knn_mfma_chunked_sweep_kernel<true><<<grid, 256, lds, s>>>(args);
-            } else {
-                TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(knn_mfma_chunked_sweep_kernel<false>),
-                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-                knn_mfma_chunked_sweep_kernel<false><<<grid, 256, lds, s>>>(args);
-            }
+            const auto sweep = !bf16_chunked          ? knn_mfma_chunked_sweep_kernel<false, false>
+                               : args.centre_dist ? knn_mfma_chunked_sweep_kernel<true, true>
+                                                  : knn_mfma_chunked_sweep_kernel<true, false>;
+            TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sweep),
+                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+            sweep<<<grid, 256, lds, s>>>(args);
             TSNE_TRY(hipGetLastError());
         } else if (bf16 ? dispatch_bf16_sweep(steps16, args, grid, s) : dispatch_mfma_sweep(ksteps, args, grid, s)) {
             return 1;
