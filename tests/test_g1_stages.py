@@ -1164,7 +1164,7 @@ def test_knn_of_points_in_no_order(stages, n, d, k, kind):
 @pytest.mark.parametrize("n,k", [(2, 2), (63, 5), (65, 1), (130, 129), (1203, 32), (2049, 33), (20011, 50), (300, 300)])
 def test_small_step_forms(stages, n, k):
     """The step of a small problem takes its attractive forces in spare workgroups of the inverse row pass and
-    launches the grouping kernels every fourth step only; with per-kernel timing on it launches every kernel by
+    launches the grouping kernels every second step only; with per-kernel timing on it launches every kernel by
     itself on every step.  Same bits, at the remainders of the rows of a workgroup and of the entries of a lane."""
     rng = np.random.default_rng(n)
     idx = rng.integers(0, n, size=(n, k), dtype=np.int32)

@@ -996,13 +996,13 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
     p->spin_limit = kSpinLimit;
     if (const char *v = std::getenv("TSNE_ATTRACTIVE_SPIN_LIMIT")) p->spin_limit = std::max(0, std::atoi(v));
     if (N <= kSingleStreamPoints && K <= kRowEntriesNeighbors) {
-        if (hipMalloc(&p->row_entries, sizeof(uint2) * (size_t)N * K) != hipSuccess) {
-            release_blocked(p);
-            set_error("attractive_prepare: out of device memory for the row-ordered pattern");
-            return 1;
+        if (hipMalloc(&p->row_entries, sizeof(uint2) * (size_t)N * K) == hipSuccess) {
+            row_entries_kernel<<<div_up((int64_t)N * K, 256), 256, 0, s>>>(pij, indices, (int64_t)N * K, p->row_entries);
+            TSNE_LAUNCHED(s);
+        } else {
+            p->row_entries = nullptr;  // (no room: the steps then launch the attractive kernel by itself)
+            (void)hipGetLastError();
         }
-        row_entries_kernel<<<div_up((int64_t)N * K, 256), 256, 0, s>>>(pij, indices, (int64_t)N * K, p->row_entries);
-        TSNE_LAUNCHED(s);
     }
     p->blocked_ready = true;
     return 0;

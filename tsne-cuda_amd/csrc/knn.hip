@@ -2162,6 +2162,7 @@ constexpr int kDirectNeighbors = 256;  // most K - 1 that select_row_kernel<8> t
 // Floats per block: 64 MiB are cheap to allocate (5000 x 50: 0.21 ms; 0.47 with the whole 100 MB at once), but
 // beyond 10240 points hold too few rows to fill the chip with their selection (16000 x 50: 1.6 ms with 64 MiB, 1.3
 // with 256).
+constexpr int kNoRoom = -1;  // run_direct_search: nothing done, the sweeps need less memory
 inline size_t direct_floats(int N) { return (size_t)1 << (N <= 10240 ? 24 : 26); }
 
 int run_direct_search(const float *points, int N, int D, int K, int cus, int *indices, float *sq_dist, hipStream_t s) {
@@ -2172,8 +2173,8 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
     const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(direct_floats(N) / pitch) / 128 * 128));
     DeviceMem dist;
     if (!dist.alloc(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
-        set_error("knn: out of device memory for the distances");
-        return 1;
+        (void)hipGetLastError();
+        return kNoRoom;
     }
     for (int row0 = 0; row0 < N; row0 += block) {
         const int rows = std::min(block, N - row0);
@@ -2330,8 +2331,10 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         TSNE_TRY(hipGetLastError());
         return 0;
     };
-    if (mode == 0 && N <= kDirectPoints && K - 1 <= kDirectNeighbors)
-        return run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
+    if (mode == 0 && N <= kDirectPoints && K - 1 <= kDirectNeighbors) {
+        const int rc = run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
+        if (rc != kNoRoom) return rc;
+    }
     if (!use_mfma) {
         if (build_transposed()) return 1;
         return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
@@ -2399,6 +2402,8 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
             pair_distances_kernel<8><<<dim3(div_up(N, 128), div_up(num_tiles, 128)), 256, 0, s>>>(
                 centre_rows.as<float>(), num_tiles, points, N, D, 0, num_tiles, Npad, centre_dist.as<float>());
             TSNE_TRY(hipGetLastError());
+        } else {
+            (void)hipGetLastError();  // (of an allocation that did not fit: the sweep then forms them itself)
         }
     }
 
@@ -2615,16 +2620,15 @@ int run_knn_any_order(const float *points, int N, int D, int K, int *indices, fl
     if (K > 1 && D > 0 && K <= N && N > kDirectPoints && locality_pivot_count(N) > 0 &&
         numbering_lacks_locality(points, N, D, &lacks, s))
         return 1;
-    DeviceMem order, sorted;
-    // (without room for a second copy of the points: as they come)
-    if (lacks && order.alloc(sizeof(int) * (size_t)N) && sorted.alloc(sizeof(float) * (size_t)N * D)) {
+    // (without room for a second copy of the points, or for the search beside it: as they come)
+    if (DeviceMem order, sorted; lacks && order.alloc(sizeof(int) * (size_t)N) && sorted.alloc(sizeof(float) * (size_t)N * D)) {
         std::vector<int> order_host;
         if (locality_order(points, N, D, order_host, s)) return 1;
         TSNE_TRY(hipMemcpyAsync(order.p, order_host.data(), sizeof(int) * (size_t)N, hipMemcpyHostToDevice, s));
         if (launch_gather_rows(points, order.as<int>(), N, D, sorted.as<float>(), s)) return 1;
         TSNE_TRY(hipStreamSynchronize(s));
         const KnnRenumbered renumbered = {order.as<int>(), points};
-        return run_knn_mode(sorted.as<float>(), N, D, K, indices, sq_dist, s, 0, stats, nullptr, &renumbered);
+        if (!run_knn_mode(sorted.as<float>(), N, D, K, indices, sq_dist, s, 0, stats, nullptr, &renumbered)) return 0;
     }
     (void)hipGetLastError();  // (of an allocation that did not fit)
     return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, stats, nullptr, nullptr);
