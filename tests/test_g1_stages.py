@@ -118,6 +118,30 @@ def test_perplexity_far_below_the_neighbour_count(stages, c0_problem, data, k, p
     assert np.array_equal(p.view(np.uint32), p_o.view(np.uint32))
 
 
+@pytest.mark.parametrize("k", [2, 15, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 256, 257, 512, 513, 1024])
+@pytest.mark.parametrize("perp,eps", [(30.0, 1e-4), (1.7, 1e-3), (12.0, 0.0), (5.0, 1e-6), (1.0, 1e-4)])
+def test_perplexity_search_path(stages, k, perp, eps):
+    """The search takes most of its steps from approximate evaluations; its path must be the one of exact
+    evaluations at every step.  The most neighbours each form of the kernel takes and one more, rows that leave
+    lanes and workgroups partly empty, narrow and wide rows, rows of equal distances, rows without the point
+    itself, a negative distance (exact evaluations only), tolerances that are never and barely met."""
+    rng = np.random.default_rng(k)
+    n = 67
+    d = rng.random((n, k)).astype(np.float32) * np.exp(rng.uniform(-9.0, 3.0, (n, 1))).astype(np.float32)
+    d[10:30] = 0.4 + 0.01 * d[10:30]
+    d.sort(axis=1)
+    d[:60, 0] = 0.0
+    d[30] = d[30, -1]
+    if k > 64:
+        d[40, 3] = -0.25
+    p, beta = stages.perplexity(dev(d), perp, eps, return_betas=True)
+    p_o, beta_o, _ = oracle.perplexity(d, perp, eps, return_search=True)
+    ok = np.isfinite(p_o).all(axis=1)
+    assert ok.sum() >= n // 2 and np.array_equal(np.isfinite(p.cpu().numpy()), np.isfinite(p_o))
+    assert same_bits(beta.cpu().numpy(), beta_o)
+    assert same_bits(p.cpu().numpy()[ok], p_o[ok])
+
+
 def test_symmetrize(stages, c0_problem):
     c = c0_problem
     P = stages.symmetrize(dev(c["p"]), dev(c["idx"])).cpu().numpy()

@@ -64,6 +64,24 @@ __device__ __forceinline__ float entropy_term(float v) {
     return (e != e || isinf(e)) ? 0.0f : e;
 }
 
+// v plus the value of the lane that DPP control CTRL names (every lane of a 16-lane row active).
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// group_sum's tree, bit for bit, its last four levels inside the vector instructions: rotations of a 16-lane row by
+// 8 and by 4 (after the level of 8 a value depends on the lane modulo 8 only, so 4 back is 4 across), then
+// permutations of four.
+template <int LANES>
+__device__ __forceinline__ float lanes_sum(float v) {
+#pragma unroll
+    for (int m = LANES / 2; m >= 16; m >>= 1) v += __shfl_xor(v, m, kWave);
+    v = dpp_add<0x128>(v);
+    v = dpp_add<0x124>(v);
+    v = dpp_add<0x4E>(v);
+    return dpp_add<0xB1>(v);
+}
+
 // The stated summation order for a group of LANES lanes whose lane l holds the slots l + v * LANES: a lane
 // owns 64 / LANES of the 64 partial sums (classes l + LANES * (v mod (64 / LANES))); it forms them one after
 // the other, combines them by the upper levels of the tree, and the lower levels run across the lanes.
@@ -81,10 +99,55 @@ __device__ __forceinline__ float ordered_row_sum(const float (&val)[VPL]) {
     for (int m = kClasses / 2; m > 0; m >>= 1)
 #pragma unroll
         for (int c = 0; c < m; ++c) q[c] += q[c + m];
-    return group_sum<LANES>(q[0]);
+    return lanes_sum<LANES>(q[0]);
+}
+
+// H - ln(perplexity) of a row by the hardware's exponential, logarithm and reciprocal, for 0 <= d < infinity, and
+// *slack, a bound of how far the same quantity evaluated by det_expf / det_logf in the stated order is from it.
+// In units of u = 2^-24, with a_i = beta d_i (rounded once, the same in both), A = sum p_i a_i, L = |ln sum|,
+// `depth` the additions a term goes through:
+//   exponentials: within 6 u each of e^-a_i on either side; H moves by sum p_i |ln p_i + H| <= 2 (A + L) times that;
+//   ln v_i against -a_i: 6 + 4 A, and A for the products;
+//   sums: depth (1 + 2 A) on either side, A for the fused ones; quotients and logarithms of the sums: 6 A + 9 L + 4;
+//   last additions: 3 (A + L) + 2 |ln perplexity|.
+// Terms below the smallest normal number count as zero, which the caller's limit on the sum makes harmless.
+template <int LANES, int VPL>
+__device__ __forceinline__ float approximate_excess(const float (&d)[VPL], const bool (&use)[VPL], float beta,
+                                                    float log_target, float *sum_out, float *slack) {
+#pragma clang fp contract(off)
+    constexpr int kDepth = VPL + 6;
+    float sum = 0.0f, weighted = 0.0f;
+#pragma unroll
+    for (int v = 0; v < VPL; ++v) {
+        const float a = beta * d[v];
+        const float x = a * -1.44269502f;  // log2 e, whose remaining 1.925963e-8 goes in with the product's rounding
+        float r = fmaf(a, -1.44269502f, -x);
+        r = fmaf(a, -1.925963e-8f, r);
+        float e = __builtin_amdgcn_exp2f(x);
+        e = fmaf(e, r * 0.693147181f, e);
+        e = use[v] ? e : 0.0f;
+        sum += e;
+        weighted = fmaf(e, a, weighted);
+    }
+    sum = lanes_sum<LANES>(sum);
+    weighted = lanes_sum<LANES>(weighted);
+    const float A = weighted * __builtin_amdgcn_rcpf(sum);
+    const float log_sum = __builtin_amdgcn_logf(sum) * 0.693147181f;  // (the builtin is log2)
+    const float L = fabsf(log_sum);
+    *sum_out = sum;
+    *slack = 5.9604644775390625e-08f *
+             ((float)(48 + 4 * kDepth) * (A + L) + (float)(16 + 2 * kDepth) + 4.0f * fabsf(log_target));
+    return (A + log_sum) - log_target;
 }
 
 // One row per LANES-lane group, VPL values per lane held in registers.
+// Bound by the vector ALU: an evaluation by det_expf / det_logf takes about 55 instructions per neighbour, and a row
+// evaluates 15 to 20 exponents.  But all that an evaluation decides, until the last, is a sign: so each exponent
+// is first evaluated by the hardware's functions (13 instructions), and where that is further from the target than
+// the tolerance plus a bound of the two evaluations' difference, the search goes on from its sign - the same path.
+// The rows of a wave that cannot tell wait for each other and are then evaluated exactly together.  Sixteen lanes
+// per row up to 128 neighbours: four rows share the search's scalar part, and sums stay inside a DPP row.
+// 1,000,000 x 90, tolerance 1e-4, us: every exponent exactly, 32 lanes per row 3647; this form 1442.
 template <int LANES, int VPL>
 __global__ __launch_bounds__(256) void perplexity_kernel(const float *__restrict__ sq_dist, int N, int K,
                                                          float log_target, float eps, float *__restrict__ pij,
@@ -97,46 +160,64 @@ __global__ __launch_bounds__(256) void perplexity_kernel(const float *__restrict
     const size_t base = (size_t)(live ? row : 0) * K;
 
     float d[VPL];
-    bool self[VPL];
+    bool use[VPL];
+    bool plain = true;
 #pragma unroll
     for (int v = 0; v < VPL; ++v) {
         const int s = lane + v * LANES;
         d[v] = (live && s < K) ? sq_dist[base + s] : 0.0f;
         // perplexity_search.cu:32: neighbour 0 at distance 0 is the point itself.
-        self[v] = (s == 0 && d[v] == 0.0f);
+        use[v] = s < K && !(s == 0 && d[v] == 0.0f);
+        plain = plain && d[v] >= 0.0f && d[v] < INFINITY;
     }
+    const bool filter = __all(plain);
 
     float beta = 1.0f, lo = -FLT_MAX, hi = FLT_MAX;
     float p[VPL];
     float sum = 1.0f;
     bool done = !live;
-    for (int it = 0; it < 200; ++it) {
+    int it = 0;
+    auto advance = [&](bool up) {
+        if (up) {
+            lo = beta;
+            beta = (hi == FLT_MAX || hi == -FLT_MAX) ? beta * 2.0f : (beta + hi) / 2.0f;
+        } else {
+            hi = beta;
+            beta = (lo == -FLT_MAX || lo == FLT_MAX) ? beta / 2.0f : (beta + lo) / 2.0f;
+        }
+        ++it;
+    };
+    // (every pass of either loop advances a row that is not done or ends its part; a row takes 199 at most)
+    while (!__all(done)) {
+        bool open = filter && !done && it < 199;
+        while (__any(open)) {
+            float s, slack;
+            const float diff = approximate_excess<LANES, VPL>(d, use, beta, log_target, &s, &slack);
+            if (open) {
+                open = s >= 1e-24f && fabsf(diff) > fmaxf(eps, 0.0f) + slack;  // (false where one is not a number)
+                if (open) {
+                    advance(diff > 0.0f);
+                    open = it < 199;
+                }
+            }
+        }
         if (!done) {
             float et[VPL];
 #pragma unroll
             for (int v = 0; v < VPL; ++v) {
-                const int s = lane + v * LANES;
-                float pv = 0.0f;
-                if (s < K && !self[v]) pv = det_expf(-beta * d[v]);
-                p[v] = pv;
-                et[v] = s < K ? entropy_term(pv) : 0.0f;
+                p[v] = use[v] ? det_expf(-beta * d[v]) : 0.0f;
+                et[v] = lane + v * LANES < K ? entropy_term(p[v]) : 0.0f;
             }
             sum = ordered_row_sum<LANES, VPL>(p);
             const float ent = ordered_row_sum<LANES, VPL>(et);
             const float H = (-ent / sum) + det_logf(sum);
             const float diff = H - log_target;
             const bool found = (diff < eps && -diff < eps);
-            if (found || it == 199) {
+            if (found || it == 199)
                 done = true;
-            } else if (diff > 0) {
-                lo = beta;
-                beta = (hi == FLT_MAX || hi == -FLT_MAX) ? beta * 2.0f : (beta + hi) / 2.0f;
-            } else {
-                hi = beta;
-                beta = (lo == -FLT_MAX || lo == FLT_MAX) ? beta / 2.0f : (beta + lo) / 2.0f;
-            }
+            else
+                advance(diff > 0);
         }
-        if (__all(done)) break;
     }
     if (live) {
 #pragma unroll
@@ -241,13 +322,13 @@ int launch_perplexity(const float *sq_dist, int N, int K, float perplexity, floa
     if (K <= 32) {
         TSNE_PERP(16, 2);
     } else if (K <= 64) {
-        TSNE_PERP(32, 2);
+        TSNE_PERP(16, 4);
     } else if (K <= 96) {
-        TSNE_PERP(32, 3);
+        TSNE_PERP(16, 6);
     } else if (K <= 128) {
-        TSNE_PERP(64, 2);
+        TSNE_PERP(16, 8);
     } else if (K <= 256) {
-        TSNE_PERP(64, 4);
+        TSNE_PERP(32, 8);
     } else if (K <= 512) {
         TSNE_PERP(64, 8);
     } else if (K <= 1024) {
