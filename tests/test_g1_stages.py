@@ -191,6 +191,23 @@ def test_symmetrize_hashed_and_scanning_forms(stages, c0_problem, monkeypatch, n
         stages.symmetrize(dev(p), dev(bad))
 
 
+@pytest.mark.parametrize("n,k", [(4096, 1), (4101, 12), (4096, 13), (4099, 102), (4096, 103), (4500, 204), (4096, 205),
+                                 (4097, 1638), (4096, 1639), (70001, 1000), (530000, 102)])
+def test_symmetrize_table_sizes(stages, monkeypatch, n, k):
+    """The fullest table of a size and the emptiest of the next (buckets that overflow), one bucket only, the most
+    neighbours of the tables and one more, tables large enough to have tags beside them: the scanning form's values,
+    bit for bit.  Bands of columns (most pairs in both directions), every second row strided (few)."""
+    g = torch.Generator(device="cuda").manual_seed(n + k)
+    i = torch.arange(n, device="cuda")[:, None]
+    stride = torch.where(i % 2 == 0, 1, max(1, n // k))
+    idx = ((i + (torch.arange(k, device="cuda") - k // 3) * stride) % n).int()
+    p = torch.rand(n, k, generator=g, device="cuda")
+    monkeypatch.delenv("TSNE_SYMMETRIZE_SCAN", raising=False)
+    got = stages.symmetrize(p, idx)
+    monkeypatch.setenv("TSNE_SYMMETRIZE_SCAN", "1")
+    assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
+
+
 @pytest.mark.parametrize("n,k", [(2, 2), (7, 3), (300, 300), (5000, 90), (70000, 20), (20000, 1)])
 def test_symmetrize_full_csr(stages, c0_problem, n, k):
     """(A + A^T) / 2N with the union pattern: the device radix sort + segmented reduce against the oracle's

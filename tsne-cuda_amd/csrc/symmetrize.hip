@@ -8,9 +8,10 @@
 // index reads, 32 GB at a million points and 90 neighbours.  Two forms here:
 //   * hashed (the default from 4096 points up): every row's (column, value)
 //     pairs go once into a small open-addressing table of the row's own (a power
-//     of two >= 1.25 K slots of 8 bytes, linear probing, built in LDS by a group
-//     of lanes per row); a non-zero then looks for its row number in the table of
-//     row j: one or two 64-byte sectors instead of the 720 bytes of row j;
+//     of two >= 1.25 K slots of 8 bytes, in buckets of 16 that overflow into the
+//     next, built in LDS by a group of lanes per row); a non-zero looks for its row
+//     number in the table of row j.  Beside large tables stands one byte of each
+//     column's hash: 16 bytes of a bucket then answer most lookups;
 //   * scanning (small problems, more than 1638 neighbours, rows that name a column
 //     twice, or when the tables do not fit in memory): a group of lanes owns row i
 //     and the whole group scans each row j
@@ -58,34 +59,48 @@ struct Slot {
     int key;  // column, -1: empty
     float value;
 };
-__device__ __forceinline__ unsigned int slot_of(int key, int log2_slots) {
-    return ((unsigned int)key * 0x9E3779B1u) >> (32 - log2_slots);
+constexpr int kBucket = 16;  // slots; their tags are one 16-byte load
+__device__ __forceinline__ unsigned int hash_of(int key) { return (unsigned int)key * 0x9E3779B1u; }
+// The tag of a column, 1 to 255 (0: an empty slot), from hash bits below those that choose the slot.
+__device__ __forceinline__ unsigned int tag_of(unsigned int hash) {
+    const unsigned int t = (hash >> 13) & 0xffu;
+    return t ? t : 1u;
+}
+
+// The slot after `at`, the seen-th looked at: round the bucket, then the next bucket.
+__device__ __forceinline__ unsigned int next_slot(unsigned int at, int seen, int log2_slots) {
+    at = (at & ~(kBucket - 1u)) | ((at + 1u) & (kBucket - 1u));
+    return (seen & (kBucket - 1)) ? at : (at + kBucket) & ((1u << log2_slots) - 1u);
 }
 
 // A group of LANES lanes per row builds the row's table in LDS (insertions race for empty slots with a
-// compare-and-swap; which slot a column ends up in does not matter to a lookup) and writes it out whole.  A row
-// that names a column twice raises *repeated: the caller then takes the scanning form, which adds such values up.
+// compare-and-swap; which slot of its bucket a column ends up in does not matter to a lookup, and it goes to the
+// next bucket only when its own is full) and writes it out whole, the tags as well (if any).  flags[0]: some row names a column
+// twice (the caller then takes the scanning form, which adds such values up); flags[1]: a column outside [0, N).
 template <int LANES>
 __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                            int N, int K, int log2_slots, Slot *__restrict__ table,
-                                                           int *__restrict__ repeated) {
+                                                           unsigned int *__restrict__ tags, int *__restrict__ flags) {
     extern __shared__ Slot lds_tables[];
     constexpr int kRows = 256 / LANES;
     const int slots = 1 << log2_slots;
-    const unsigned int mask = (unsigned int)slots - 1u;
     const int group = threadIdx.x / LANES, lane = threadIdx.x % LANES;
     const int row = blockIdx.x * kRows + group;
     Slot *mine = lds_tables + (size_t)group * slots;
     for (int e = lane; e < slots; e += LANES) mine[e] = Slot{-1, 0.0f};
     __syncthreads();
-    bool twice = false;
+    bool twice = false, outside = false;
     if (row < N) {
         const size_t base = (size_t)row * K;
         for (int t = lane; t < K; t += LANES) {
             const int key = idx[base + t];
             const float v = p[base + t];
-            unsigned int at = slot_of(key, log2_slots);
-            for (;;) {  // (more slots than pairs: an empty one is always met)
+            if ((unsigned int)key >= (unsigned int)N) {
+                outside = true;
+                continue;
+            }
+            unsigned int at = hash_of(key) >> (32 - log2_slots);
+            for (int seen = 1;; ++seen) {  // (more slots than pairs: an empty one is always met)
                 const int old = atomicCAS(&mine[at].key, -1, key);
                 if (old == -1) {
                     mine[at].value = v;
@@ -95,40 +110,98 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
                     twice = true;
                     break;
                 }
-                at = (at + 1u) & mask;
+                at = next_slot(at, seen, log2_slots);
             }
         }
     }
-    if (__any(twice) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(repeated, 1);
+    if (__any(twice) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(&flags[0], 1);
+    if (__any(outside) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(&flags[1], 1);
     __syncthreads();
     if (row < N) {
         Slot *out = table + ((size_t)row << log2_slots);
-        for (int e = lane; e < slots; e += LANES) out[e] = mine[e];
+        if (!tags) {
+            for (int e = lane; e < slots; e += LANES) out[e] = mine[e];
+            return;
+        }
+        unsigned int *out_tags = tags + ((size_t)row << (log2_slots - 2));
+        for (int e = lane; e < slots; e += LANES) {  // (whole groups of four lanes: slots and LANES are multiples of 16)
+            const Slot here = mine[e];
+            out[e] = here;
+            unsigned int four = (here.key < 0 ? 0u : tag_of(hash_of(here.key))) << (8 * (lane & 3));
+            four |= __builtin_amdgcn_update_dpp(0u, four, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+            four |= __builtin_amdgcn_update_dpp(0u, four, 0x4E, 0xf, 0xf, true);  // lane ^ 2
+            if ((lane & 3) == 0) out_tags[e / 4] = four;
+        }
     }
 }
 
+// 0x80 in every byte of w that is zero.
+__device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
+    return ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w | 0x7f7f7f7fu);
+}
+
+// Bound by the cache lines that the lookups touch, one random line each.  TAGS: a lookup reads its bucket's tags first
+// and ends there unless one matches.  The tags of a million rows of 90 neighbours are 128 MB, which the memory-side
+// cache holds; the slots are 1 GB, which it does not.  50-dimensional Gaussians, where one lookup in four finds a match:
+// 2970 -> 1547 us.  Where most do, a second line is read for most (8 dimensions, the whole stage, us, without / with
+// tags): 1,000,000 x 90 4500 / 4250, x 33 1429 / 1777, 100,000 x 150 856 / 978; hence kTaggedBytes.
+constexpr size_t kTaggedBytes = (size_t)512 << 20;  // slots of more bytes than this have tags
+template <bool TAGS>
 __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                                 int N, int K, int log2_slots,
-                                                                const Slot *__restrict__ table, float *__restrict__ P) {
+                                                                const Slot *__restrict__ table,
+                                                                const uint4 *__restrict__ tags, float *__restrict__ P) {
     const size_t nnz = (size_t)N * K;
     const double denom = 2.0 * (double)N;
-    const unsigned int mask = (1u << log2_slots) - 1u;
-    for (size_t e = (size_t)blockIdx.x * 256 + threadIdx.x; e < nnz; e += (size_t)gridDim.x * 256) {
-        const int row = (int)(e / K);
+    const unsigned int buckets = 1u << (log2_slots - 4);
+    for (size_t e0 = (size_t)blockIdx.x * 256; e0 < nnz; e0 += (size_t)gridDim.x * 256) {
+        const size_t row0 = e0 / (unsigned int)K, e = e0 + threadIdx.x;
+        if (e >= nnz) return;
+        const int row = (int)row0 + (int)((unsigned int)(e - row0 * K) / (unsigned int)K);
         const int j = idx[e];
-        const Slot *theirs = table + ((size_t)j << log2_slots);
+        const float own = p[e];
         float found = 0.0f;
-        unsigned int at = slot_of(row, log2_slots);
-        for (;;) {
-            const Slot here = theirs[at];
-            if (here.key == row) {
-                found = here.value;
-                break;
+        if (!TAGS && (unsigned int)j < (unsigned int)N) {
+            const Slot *theirs = table + ((size_t)j << log2_slots);
+            unsigned int at = hash_of(row) >> (32 - log2_slots);
+            for (int seen = 1;; ++seen) {  // (an empty slot is always met)
+                const Slot here = theirs[at];
+                if (here.key == row) {
+                    found = here.value;
+                    break;
+                }
+                if (here.key < 0) break;
+                at = next_slot(at, seen, log2_slots);
             }
-            if (here.key < 0) break;
-            at = (at + 1u) & mask;
         }
-        P[e] = (float)((double)(p[e] + found) / denom);
+        if (TAGS && (unsigned int)j < (unsigned int)N) {
+            const unsigned int hash = hash_of(row), tag = tag_of(hash) * 0x01010101u;
+            unsigned int bucket = (hash >> (32 - log2_slots)) / kBucket;
+            const uint4 *their_tags = tags + ((size_t)j << (log2_slots - 4));
+            const Slot *theirs = table + ((size_t)j << log2_slots);
+            for (unsigned int visited = 0; visited < buckets; ++visited) {
+                const uint4 t = their_tags[bucket];
+                const unsigned int w[4] = {t.x, t.y, t.z, t.w};
+                unsigned int empty = 0u, matches = 0u;  // (matches: a bit per slot of the bucket)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    empty |= zero_bytes(w[u]);
+                    matches |= (((zero_bytes(w[u] ^ tag) >> 7) * 0x10204080u) >> 28) << (4 * u);
+                }
+                bool hit = false;
+                while (matches && !hit) {
+                    const Slot here = theirs[bucket * kBucket + (__ffs((int)matches) - 1)];
+                    matches &= matches - 1u;
+                    if (here.key == row) {
+                        found = here.value;
+                        hit = true;
+                    }
+                }
+                if (hit || empty) break;
+                bucket = (bucket + 1u) & (buckets - 1u);
+            }
+        }
+        P[e] = (float)((double)(own + found) / denom);
     }
 }
 
@@ -166,49 +239,49 @@ int validate_indices(const int *idx, int64_t n, int N, const char *who, hipStrea
 }
 
 int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hipStream_t s) {
-    // Hashed form: tables of next_pow2(1.25 K) slots per row.  A column outside [0, N) would address another
-    // row's table, so the indices are checked first (the scanning form only compares them).
-    int log2_slots = 3;
+    // Hashed form: tables of next_pow2(1.25 K) slots per row (one bucket at least) and their tags.
+    int log2_slots = 4;
     while ((1 << log2_slots) < K + (K + 3) / 4) ++log2_slots;
-    const size_t table_bytes = ((size_t)N << log2_slots) * sizeof(Slot);
+    const size_t slots = (size_t)N << log2_slots;
     const bool scan_only = std::getenv("TSNE_SYMMETRIZE_SCAN") != nullptr;  // (for measurements and tests)
-    if (N >= 4096 && log2_slots <= 11 && table_bytes <= ((size_t)64 << 30) && !scan_only) {
+    if (N >= 4096 && log2_slots <= 11 && slots * sizeof(Slot) <= ((size_t)64 << 30) && !scan_only) {
         Slot *table = nullptr;
-        int *repeated = nullptr;
-        if (hipMalloc(&table, table_bytes) == hipSuccess && hipMalloc(&repeated, sizeof(int)) == hipSuccess) {
-            int rc = validate_indices(idx, (int64_t)N * K, N, "symmetrize", s);
-            int twice = 0;
-            if (!rc) {
-                hipError_t e = hipMemsetAsync(repeated, 0, sizeof(int), s);
-                if (e == hipSuccess) {
-                    if (log2_slots <= 8) {
-                        build_tables_kernel<16><<<div_up(N, 16), 256, sizeof(Slot) * 16 << log2_slots, s>>>(
-                            p, idx, N, K, log2_slots, table, repeated);
-                    } else {
-                        TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(build_tables_kernel<64>),
-                                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                                     (int)(sizeof(Slot) * 4 << 11)));
-                        build_tables_kernel<64><<<div_up(N, 4), 256, sizeof(Slot) * 4 << log2_slots, s>>>(
-                            p, idx, N, K, log2_slots, table, repeated);
-                    }
-                    symmetrize_hashed_kernel<<<(int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20), 256, 0,
-                                               s>>>(p, idx, N, K, log2_slots, table, P);
-                    e = hipGetLastError();
-                }
-                if (e == hipSuccess) e = hipMemcpyAsync(&twice, repeated, sizeof(int), hipMemcpyDeviceToHost, s);
-                if (e == hipSuccess) e = hipStreamSynchronize(s);  // the tables go
-                if (e != hipSuccess) {
-                    set_error("symmetrize: %s", hipGetErrorString(e));
-                    rc = 1;
-                }
+        const bool tagged = slots * sizeof(Slot) > kTaggedBytes;
+        const size_t table_bytes = slots * (sizeof(Slot) + (tagged ? 1 : 0));
+        if (hipMalloc(&table, table_bytes + 2 * sizeof(int)) == hipSuccess) {
+            unsigned int *tags = tagged ? reinterpret_cast<unsigned int *>(table + slots) : nullptr;
+            int *flags = reinterpret_cast<int *>(reinterpret_cast<char *>(table) + table_bytes);
+            int raised[2] = {0, 0};
+            hipError_t e = hipMemsetAsync(flags, 0, sizeof(raised), s);
+            if (e == hipSuccess && log2_slots > 8)
+                e = hipFuncSetAttribute(reinterpret_cast<const void *>(build_tables_kernel<64>),
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(Slot) * 4 << 11));
+            if (e == hipSuccess) {
+                if (log2_slots <= 8)
+                    build_tables_kernel<16><<<div_up(N, 16), 256, sizeof(Slot) * 16 << log2_slots, s>>>(
+                        p, idx, N, K, log2_slots, table, tags, flags);
+                else
+                    build_tables_kernel<64><<<div_up(N, 4), 256, sizeof(Slot) * 4 << log2_slots, s>>>(
+                        p, idx, N, K, log2_slots, table, tags, flags);
+                const auto look_up = tagged ? symmetrize_hashed_kernel<true> : symmetrize_hashed_kernel<false>;
+                look_up<<<(int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20), 256, 0, s>>>(
+                    p, idx, N, K, log2_slots, table, reinterpret_cast<const uint4 *>(tags), P);
+                e = hipGetLastError();
             }
+            if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
+            if (e == hipSuccess) e = hipStreamSynchronize(s);  // the tables go
             (void)hipFree(table);
-            (void)hipFree(repeated);
-            if (rc || !twice) return rc;
+            if (e != hipSuccess) {
+                set_error("symmetrize: %s", hipGetErrorString(e));
+                return 1;
+            }
+            if (raised[1]) {
+                set_error("symmetrize: a neighbour index lies outside [0, %d)", N);
+                return 1;
+            }
+            if (!raised[0]) return 0;
             // (some row names a column twice: the scanning form below adds those values up)
         } else {
-            (void)hipFree(table);
-            (void)hipFree(repeated);
             (void)hipGetLastError();  // no room for the tables: the scanning form needs none
         }
     }
