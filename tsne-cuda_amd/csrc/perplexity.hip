@@ -38,13 +38,27 @@ namespace tsnehip {
 
 namespace {
 
+// Bound by memory, and by the atomics on one address if there are many: one per workgroup (one per wave of 4096
+// workgroups: 90 M values 237 us, this form 93, 3.9 TB/s), and four values per load where the address allows it.
 __global__ __launch_bounds__(256) void abs_max_kernel(const float *__restrict__ v, int64_t n, float *out) {
+    __shared__ float partial[256 / kWave];
     float m = 0.0f;
-    for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (int64_t)gridDim.x * blockDim.x)
-        m = fmaxf(m, fabsf(v[t]));
+    const int64_t first = (int64_t)blockIdx.x * 256 + threadIdx.x, stride = (int64_t)gridDim.x * 256;
+    const int64_t quads = (reinterpret_cast<uintptr_t>(v) & 15) == 0 ? n / 4 : 0;
+    for (int64_t t = first; t < quads; t += stride) {
+        const float4 x = reinterpret_cast<const float4 *>(v)[t];
+        m = fmaxf(m, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
+    }
+    for (int64_t t = 4 * quads + first; t < n; t += stride) m = fmaxf(m, fabsf(v[t]));
     m = group_max<kWave>(m);
-    // Non-negative floats order like their bit patterns.
-    if ((threadIdx.x & (kWave - 1)) == 0) atomicMax(reinterpret_cast<unsigned int *>(out), __float_as_uint(m));
+    if ((threadIdx.x & (kWave - 1)) == 0) partial[threadIdx.x / kWave] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int w = 1; w < 256 / kWave; ++w) m = fmaxf(m, partial[w]);
+        // Non-negative floats order like their bit patterns.
+        atomicMax(reinterpret_cast<unsigned int *>(out), __float_as_uint(m));
+    }
 }
 
 __global__ __launch_bounds__(256) void divide_kernel(float *__restrict__ v, int64_t n, const float *denom) {
@@ -277,7 +291,7 @@ int launch_max_normalize(float *values, int64_t n, float *scratch, hipStream_t s
     zero_scalar_kernel<<<1, 64, 0, s>>>(scratch);
     TSNE_LAUNCHED(s);
     const int blocks = std::max(1, (int)std::min<int64_t>(div_up(n, 256 * 4), 4096));
-    abs_max_kernel<<<blocks, 256, 0, s>>>(values, n, scratch);
+    abs_max_kernel<<<std::min(blocks, 2048), 256, 0, s>>>(values, n, scratch);
     TSNE_LAUNCHED(s);
     divide_kernel<<<blocks, 256, 0, s>>>(values, n, scratch);
     TSNE_LAUNCHED(s);
