@@ -139,6 +139,7 @@ static_assert(kItemEntries % 128 == 0, "items hold whole groups of 64 entry pair
 // kBalancedParts partitions keeps the order of arrival instead (neighbour slot by neighbour slot).
 constexpr int kBalancedParts = 320;
 constexpr int kResidues = 32;
+constexpr int kSlotsAhead = 4;  // neighbour slots of a row that are loaded at once
 constexpr int kResidueStride = kResidues + 1;  // odd: the 32 counters of different partitions spread over the banks
 constexpr size_t kReblockLds = sizeof(unsigned int) * 2 * kBalancedParts * kResidueStride;
 
@@ -206,31 +207,61 @@ __global__ __launch_bounds__(kBlock) void reblock_kernel(const float *__restrict
     // Entries are visited neighbour slot by neighbour slot, so that the entries of one row lie far apart
     // in a partition's run (also within a residue's bucket): a wave of the force kernel never meets a row twice.
     float biggest = 0.0f;
-    for (unsigned int v = tid; v < count; v += kBlock) {
-        const unsigned int slot = v / (unsigned int)nrows;
-        const unsigned int row_local = v - slot * (unsigned int)nrows;
-        const unsigned int e = row_local * (unsigned int)K + slot;
-        const int col = idx[base + e];
-        const int part = col / kPartPoints;
-        unsigned int pos;
-        if (balanced) {
-            const unsigned int q = row_local & (kResidues - 1);
-            const unsigned int *counts = residue_count + fresh_of[part] * kResidueStride;
-            const unsigned int j = atomicAdd(&residue_cursor[fresh_of[part] * kResidueStride + q], 1u);
-            // Round j of the dealing: everything of the rounds before it, then the buckets before q that reach round j.
-            pos = cursor[part];
-#pragma unroll 8
-            for (unsigned int other = 0; other < (unsigned int)kResidues; ++other) {
-                const unsigned int c = counts[other];
-                pos += min(c, j) + ((other < q && c > j) ? 1u : 0u);
+    // A wave reads 64 rows at a time, a cache line each, which is gone from the L2 by the time the next slot is wanted:
+    // kSlotsAhead slots of all rows are therefore loaded at once (16 bytes per lane and row) and placed slot by slot.
+    // 1,000,000 x 90, ms: one slot at a time 5.9, four 2.7.
+    constexpr int kRowsPerLane = (kStripMax + kBlock - 1) / kBlock;
+    for (unsigned int slot0 = 0; slot0 < (unsigned int)K; slot0 += kSlotsAhead) {
+        int cols[kRowsPerLane][kSlotsAhead];
+        float values[kRowsPerLane][kSlotsAhead];
+#pragma unroll
+        for (int r = 0; r < kRowsPerLane; ++r) {
+            const unsigned int row_local = tid + r * kBlock;
+            if (row_local >= (unsigned int)nrows) break;
+            const size_t e = base + row_local * (unsigned int)K + slot0;
+            if (slot0 + kSlotsAhead <= (unsigned int)K) {
+                __builtin_memcpy(cols[r], idx + e, sizeof(cols[r]));  // (16-byte loads; rows start at any multiple of 4)
+                __builtin_memcpy(values[r], pij + e, sizeof(values[r]));
+            } else {
+#pragma unroll
+                for (int u = 0; u < kSlotsAhead; ++u) {
+                    const unsigned int over = slot0 + u < (unsigned int)K ? u : 0;
+                    cols[r][u] = idx[e + over];
+                    values[r][u] = pij[e + over];
+                }
             }
-        } else {
-            pos = atomicAdd(&cursor[part], 1u);
         }
-        const float pv = pij[base + e];
-        biggest = fmaxf(biggest, fabsf(pv));
-        reinterpret_cast<uint2 *>(ent_p)[entry_slot(pos, strip, (int)gridDim.x)] =
-            make_uint2(__float_as_uint(pv), (unsigned int)(col - part * kPartPoints) | (row_local << kColBits));
+#pragma unroll
+        for (int u = 0; u < kSlotsAhead; ++u) {
+            if (slot0 + u >= (unsigned int)K) break;
+#pragma unroll
+            for (int r = 0; r < kRowsPerLane; ++r) {
+                const unsigned int row_local = tid + r * kBlock;
+                if (row_local >= (unsigned int)nrows) break;
+                const int col = cols[r][u];
+                const int part = col / kPartPoints;
+                unsigned int pos;
+                if (balanced) {
+                    const unsigned int q = row_local & (kResidues - 1);
+                    const unsigned int *counts = residue_count + fresh_of[part] * kResidueStride;
+                    const unsigned int j = atomicAdd(&residue_cursor[fresh_of[part] * kResidueStride + q], 1u);
+                    // Round j of the dealing: everything of the rounds before it, then the buckets before q that reach
+                    // round j.
+                    pos = cursor[part];
+#pragma unroll 8
+                    for (unsigned int other = 0; other < (unsigned int)kResidues; ++other) {
+                        const unsigned int c = counts[other];
+                        pos += min(c, j) + ((other < q && c > j) ? 1u : 0u);
+                    }
+                } else {
+                    pos = atomicAdd(&cursor[part], 1u);
+                }
+                const float pv = values[r][u];
+                biggest = fmaxf(biggest, fabsf(pv));
+                reinterpret_cast<uint2 *>(ent_p)[entry_slot(pos, strip, (int)gridDim.x)] =
+                    make_uint2(__float_as_uint(pv), (unsigned int)(col - part * kPartPoints) | (row_local << kColBits));
+            }
+        }
     }
     biggest = group_max<kWave>(biggest);
     // Non-negative floats order like their bit patterns.
