@@ -10,8 +10,9 @@
 //     pairs go once into a small open-addressing table of the row's own (a power
 //     of two >= 1.25 K slots of 8 bytes, in buckets of 16 that overflow into the
 //     next, built in LDS by a group of lanes per row); a non-zero looks for its row
-//     number in the table of row j.  Beside large tables stands one byte of each
-//     column's hash: 16 bytes of a bucket then answer most lookups;
+//     number in the table of row j.  Large tables hold a byte of each column's hash
+//     and its place in the row instead: 16 bytes of a bucket answer most lookups,
+//     and the row itself the others;
 //   * scanning (small problems, more than 1638 neighbours, rows that name a column
 //     twice, or when the tables do not fit in memory): a group of lanes owns row i
 //     and the whole group scans each row j
@@ -22,6 +23,7 @@
 
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 namespace tsnehip {
 
@@ -73,14 +75,21 @@ __device__ __forceinline__ unsigned int next_slot(unsigned int at, int seen, int
     return (seen & (kBucket - 1)) ? at : (at + kBucket) & ((1u << log2_slots) - 1u);
 }
 
+// A neighbour's place in its row, in tables built by LANES lanes per row: up to 204 neighbours by 16, else 64.
+template <int LANES>
+using PlaceOf = std::conditional_t<LANES == 16, unsigned char, unsigned short>;
+
 // A group of LANES lanes per row builds the row's table in LDS (insertions race for empty slots with a
 // compare-and-swap; which slot of its bucket a column ends up in does not matter to a lookup, and it goes to the
-// next bucket only when its own is full) and writes it out whole, the tags as well (if any).  flags[0]: some row names a column
-// twice (the caller then takes the scanning form, which adds such values up); flags[1]: a column outside [0, N).
+// next bucket only when its own is full) and writes it out whole: the slots, or (tags != nullptr) the columns' tags
+// and their places in the row.  flags[0]: some row names a column twice (the caller then takes the scanning form,
+// which adds such values up); flags[1]: a column outside [0, N).
 template <int LANES>
 __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                            int N, int K, int log2_slots, Slot *__restrict__ table,
-                                                           unsigned int *__restrict__ tags, int *__restrict__ flags) {
+                                                           unsigned int *__restrict__ tags,
+                                                           PlaceOf<LANES> *__restrict__ places,
+                                                           int *__restrict__ flags) {
     extern __shared__ Slot lds_tables[];
     constexpr int kRows = 256 / LANES;
     const int slots = 1 << log2_slots;
@@ -94,7 +103,7 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
         const size_t base = (size_t)row * K;
         for (int t = lane; t < K; t += LANES) {
             const int key = idx[base + t];
-            const float v = p[base + t];
+            const float v = tags ? __int_as_float(t) : p[base + t];
             if ((unsigned int)key >= (unsigned int)N) {
                 outside = true;
                 continue;
@@ -118,15 +127,16 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
     if (__any(outside) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(&flags[1], 1);
     __syncthreads();
     if (row < N) {
-        Slot *out = table + ((size_t)row << log2_slots);
         if (!tags) {
+            Slot *out = table + ((size_t)row << log2_slots);
             for (int e = lane; e < slots; e += LANES) out[e] = mine[e];
             return;
         }
         unsigned int *out_tags = tags + ((size_t)row << (log2_slots - 2));
+        PlaceOf<LANES> *out_places = places + ((size_t)row << log2_slots);
         for (int e = lane; e < slots; e += LANES) {  // (whole groups of four lanes: slots and LANES are multiples of 16)
             const Slot here = mine[e];
-            out[e] = here;
+            out_places[e] = (PlaceOf<LANES>)__float_as_int(here.value);
             unsigned int four = (here.key < 0 ? 0u : tag_of(hash_of(here.key))) << (8 * (lane & 3));
             four |= __builtin_amdgcn_update_dpp(0u, four, 0xB1, 0xf, 0xf, true);  // lane ^ 1
             four |= __builtin_amdgcn_update_dpp(0u, four, 0x4E, 0xf, 0xf, true);  // lane ^ 2
@@ -140,17 +150,21 @@ __device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
     return ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w | 0x7f7f7f7fu);
 }
 
-// Bound by the cache lines that the lookups touch, one random line each.  TAGS: a lookup reads its bucket's tags first
-// and ends there unless one matches.  The tags of a million rows of 90 neighbours are 128 MB, which the memory-side
-// cache holds; the slots are 1 GB, which it does not.  50-dimensional Gaussians, where one lookup in four finds a match:
-// 2970 -> 1547 us.  Where most do, a second line is read for most (8 dimensions, the whole stage, us, without / with
-// tags): 1,000,000 x 90 4500 / 4250, x 33 1429 / 1777, 100,000 x 150 856 / 978; hence kTaggedBytes.
-constexpr size_t kTaggedBytes = (size_t)512 << 20;  // slots of more bytes than this have tags
-template <bool TAGS>
+// Bound by the cache lines that the lookups touch, random ones.  TAGS: a lookup reads its bucket's tags first and ends
+// there unless one matches (50-dimensional Gaussians: one lookup in four finds its column); the match's place leads to
+// the row's own column and value.  Tags and places of a million rows of 90 neighbours are 256 MB where slots are 1 GB.
+// What that saves is not the kernels' time alone (lookups 2970 us in slots, 2580 in this form; 1547 with tags beside
+// the slots, 1.15 GB) but the memory: a call that takes and returns over a gigabyte waits for the driver to clear what
+// the call before returned.  1,000,000 x 90, affinities called one after the other: 17.3 ms with tags beside the slots
+// (4.6 for a single call), 5.7 in this form.
+constexpr size_t kTaggedBytes = (size_t)512 << 20;  // slots of more bytes than this are replaced by tags and places
+template <bool TAGS, typename PLACE>
 __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                                 int N, int K, int log2_slots,
                                                                 const Slot *__restrict__ table,
-                                                                const uint4 *__restrict__ tags, float *__restrict__ P) {
+                                                                const uint4 *__restrict__ tags,
+                                                                const PLACE *__restrict__ places,
+                                                                float *__restrict__ P) {
     const size_t nnz = (size_t)N * K;
     const double denom = 2.0 * (double)N;
     const unsigned int buckets = 1u << (log2_slots - 4);
@@ -178,7 +192,8 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
             const unsigned int hash = hash_of(row), tag = tag_of(hash) * 0x01010101u;
             unsigned int bucket = (hash >> (32 - log2_slots)) / kBucket;
             const uint4 *their_tags = tags + ((size_t)j << (log2_slots - 4));
-            const Slot *theirs = table + ((size_t)j << log2_slots);
+            const PLACE *their_places = places + ((size_t)j << log2_slots);
+            const size_t their_row = (size_t)j * K;
             for (unsigned int visited = 0; visited < buckets; ++visited) {
                 const uint4 t = their_tags[bucket];
                 const unsigned int w[4] = {t.x, t.y, t.z, t.w};
@@ -190,10 +205,12 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
                 }
                 bool hit = false;
                 while (matches && !hit) {
-                    const Slot here = theirs[bucket * kBucket + (__ffs((int)matches) - 1)];
+                    const size_t at = their_row + their_places[bucket * kBucket + (__ffs((int)matches) - 1)];
                     matches &= matches - 1u;
-                    if (here.key == row) {
-                        found = here.value;
+                    const int key = idx[at];
+                    const float value = p[at];
+                    if (key == row) {
+                        found = value;
                         hit = true;
                     }
                 }
@@ -245,32 +262,41 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
     const size_t slots = (size_t)N << log2_slots;
     const bool scan_only = std::getenv("TSNE_SYMMETRIZE_SCAN") != nullptr;  // (for measurements and tests)
     if (N >= 4096 && log2_slots <= 11 && slots * sizeof(Slot) <= ((size_t)64 << 30) && !scan_only) {
-        Slot *table = nullptr;
-        const bool tagged = slots * sizeof(Slot) > kTaggedBytes;
-        const size_t table_bytes = slots * (sizeof(Slot) + (tagged ? 1 : 0));
-        if (hipMalloc(&table, table_bytes + 2 * sizeof(int)) == hipSuccess) {
-            unsigned int *tags = tagged ? reinterpret_cast<unsigned int *>(table + slots) : nullptr;
-            int *flags = reinterpret_cast<int *>(reinterpret_cast<char *>(table) + table_bytes);
+        void *memory = nullptr;
+        const bool tagged = slots * sizeof(Slot) > kTaggedBytes, narrow = log2_slots <= 8;
+        const size_t table_bytes = slots * (!tagged ? sizeof(Slot) : 1 + (narrow ? sizeof(PlaceOf<16>) : sizeof(PlaceOf<64>)));
+        if (hipMalloc(&memory, table_bytes + 2 * sizeof(int)) == hipSuccess) {
+            Slot *table = tagged ? nullptr : static_cast<Slot *>(memory);
+            unsigned int *tags = tagged ? static_cast<unsigned int *>(memory) : nullptr;
+            void *places = tagged ? static_cast<char *>(memory) + slots : nullptr;
+            int *flags = reinterpret_cast<int *>(static_cast<char *>(memory) + table_bytes);
             int raised[2] = {0, 0};
             hipError_t e = hipMemsetAsync(flags, 0, sizeof(raised), s);
-            if (e == hipSuccess && log2_slots > 8)
+            if (e == hipSuccess && !narrow)
                 e = hipFuncSetAttribute(reinterpret_cast<const void *>(build_tables_kernel<64>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(Slot) * 4 << 11));
             if (e == hipSuccess) {
-                if (log2_slots <= 8)
+                auto *bytes = static_cast<PlaceOf<16> *>(places);
+                auto *words = static_cast<PlaceOf<64> *>(places);
+                if (narrow)
                     build_tables_kernel<16><<<div_up(N, 16), 256, sizeof(Slot) * 16 << log2_slots, s>>>(
-                        p, idx, N, K, log2_slots, table, tags, flags);
+                        p, idx, N, K, log2_slots, table, tags, bytes, flags);
                 else
                     build_tables_kernel<64><<<div_up(N, 4), 256, sizeof(Slot) * 4 << log2_slots, s>>>(
-                        p, idx, N, K, log2_slots, table, tags, flags);
-                const auto look_up = tagged ? symmetrize_hashed_kernel<true> : symmetrize_hashed_kernel<false>;
-                look_up<<<(int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20), 256, 0, s>>>(
-                    p, idx, N, K, log2_slots, table, reinterpret_cast<const uint4 *>(tags), P);
+                        p, idx, N, K, log2_slots, table, tags, words, flags);
+                const int grid = (int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20);
+                const auto *buckets = reinterpret_cast<const uint4 *>(tags);
+                if (!tagged)
+                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, bytes, P);
+                else if (narrow)
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, bytes, P);
+                else
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, words, P);
                 e = hipGetLastError();
             }
             if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipStreamSynchronize(s);  // the tables go
-            (void)hipFree(table);
+            (void)hipFree(memory);
             if (e != hipSuccess) {
                 set_error("symmetrize: %s", hipGetErrorString(e));
                 return 1;
