@@ -78,17 +78,22 @@ __device__ __forceinline__ unsigned int next_slot(unsigned int at, int seen, int
 // A neighbour's place in its row, in tables built by LANES lanes per row: up to 204 neighbours by 16, else 64.
 template <int LANES>
 using PlaceOf = std::conditional_t<LANES == 16, unsigned char, unsigned short>;
+// A bucket without slots: the columns' tags, one load, and their places in the row.
+template <typename PLACE>
+struct alignas(16) Tagged {
+    unsigned int tags[kBucket / 4];
+    PLACE places[kBucket];
+};
 
 // A group of LANES lanes per row builds the row's table in LDS (insertions race for empty slots with a
 // compare-and-swap; which slot of its bucket a column ends up in does not matter to a lookup, and it goes to the
-// next bucket only when its own is full) and writes it out whole: the slots, or (tags != nullptr) the columns' tags
+// next bucket only when its own is full) and writes it out whole: the slots, or (tagged != nullptr) the columns' tags
 // and their places in the row.  flags[0]: some row names a column twice (the caller then takes the scanning form,
 // which adds such values up); flags[1]: a column outside [0, N).
 template <int LANES>
 __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                            int N, int K, int log2_slots, Slot *__restrict__ table,
-                                                           unsigned int *__restrict__ tags,
-                                                           PlaceOf<LANES> *__restrict__ places,
+                                                           Tagged<PlaceOf<LANES>> *__restrict__ tagged,
                                                            int *__restrict__ flags) {
     extern __shared__ Slot lds_tables[];
     constexpr int kRows = 256 / LANES;
@@ -103,7 +108,7 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
         const size_t base = (size_t)row * K;
         for (int t = lane; t < K; t += LANES) {
             const int key = idx[base + t];
-            const float v = tags ? __int_as_float(t) : p[base + t];
+            const float v = tagged ? __int_as_float(t) : p[base + t];
             if ((unsigned int)key >= (unsigned int)N) {
                 outside = true;
                 continue;
@@ -127,20 +132,19 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
     if (__any(outside) && (threadIdx.x & (kWave - 1)) == 0) atomicOr(&flags[1], 1);
     __syncthreads();
     if (row < N) {
-        if (!tags) {
+        if (!tagged) {
             Slot *out = table + ((size_t)row << log2_slots);
             for (int e = lane; e < slots; e += LANES) out[e] = mine[e];
             return;
         }
-        unsigned int *out_tags = tags + ((size_t)row << (log2_slots - 2));
-        PlaceOf<LANES> *out_places = places + ((size_t)row << log2_slots);
+        Tagged<PlaceOf<LANES>> *out = tagged + ((size_t)row << (log2_slots - 4));
         for (int e = lane; e < slots; e += LANES) {  // (whole groups of four lanes: slots and LANES are multiples of 16)
             const Slot here = mine[e];
-            out_places[e] = (PlaceOf<LANES>)__float_as_int(here.value);
+            out[e / kBucket].places[e % kBucket] = (PlaceOf<LANES>)__float_as_int(here.value);
             unsigned int four = (here.key < 0 ? 0u : tag_of(hash_of(here.key))) << (8 * (lane & 3));
             four |= __builtin_amdgcn_update_dpp(0u, four, 0xB1, 0xf, 0xf, true);  // lane ^ 1
             four |= __builtin_amdgcn_update_dpp(0u, four, 0x4E, 0xf, 0xf, true);  // lane ^ 2
-            if ((lane & 3) == 0) out_tags[e / 4] = four;
+            if ((lane & 3) == 0) out[e / kBucket].tags[e % kBucket / 4] = four;
         }
     }
 }
@@ -162,8 +166,7 @@ template <bool TAGS, typename PLACE>
 __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                                 int N, int K, int log2_slots,
                                                                 const Slot *__restrict__ table,
-                                                                const uint4 *__restrict__ tags,
-                                                                const PLACE *__restrict__ places,
+                                                                const Tagged<PLACE> *__restrict__ tagged,
                                                                 float *__restrict__ P) {
     const size_t nnz = (size_t)N * K;
     const double denom = 2.0 * (double)N;
@@ -191,11 +194,10 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
         if (TAGS && (unsigned int)j < (unsigned int)N) {
             const unsigned int hash = hash_of(row), tag = tag_of(hash) * 0x01010101u;
             unsigned int bucket = (hash >> (32 - log2_slots)) / kBucket;
-            const uint4 *their_tags = tags + ((size_t)j << (log2_slots - 4));
-            const PLACE *their_places = places + ((size_t)j << log2_slots);
+            const Tagged<PLACE> *theirs = tagged + ((size_t)j << (log2_slots - 4));
             const size_t their_row = (size_t)j * K;
             for (unsigned int visited = 0; visited < buckets; ++visited) {
-                const uint4 t = their_tags[bucket];
+                const uint4 t = *reinterpret_cast<const uint4 *>(theirs[bucket].tags);
                 const unsigned int w[4] = {t.x, t.y, t.z, t.w};
                 unsigned int empty = 0u, matches = 0u;  // (matches: a bit per slot of the bucket)
 #pragma unroll
@@ -205,7 +207,7 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
                 }
                 bool hit = false;
                 while (matches && !hit) {
-                    const size_t at = their_row + their_places[bucket * kBucket + (__ffs((int)matches) - 1)];
+                    const size_t at = their_row + theirs[bucket].places[__ffs((int)matches) - 1];
                     matches &= matches - 1u;
                     const int key = idx[at];
                     const float value = p[at];
@@ -264,11 +266,10 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
     if (N >= 4096 && log2_slots <= 11 && slots * sizeof(Slot) <= ((size_t)64 << 30) && !scan_only) {
         void *memory = nullptr;
         const bool tagged = slots * sizeof(Slot) > kTaggedBytes, narrow = log2_slots <= 8;
-        const size_t table_bytes = slots * (!tagged ? sizeof(Slot) : 1 + (narrow ? sizeof(PlaceOf<16>) : sizeof(PlaceOf<64>)));
+        const size_t table_bytes = !tagged ? slots * sizeof(Slot) :
+                                   slots / kBucket * (narrow ? sizeof(Tagged<PlaceOf<16>>) : sizeof(Tagged<PlaceOf<64>>));
         if (hipMalloc(&memory, table_bytes + 2 * sizeof(int)) == hipSuccess) {
             Slot *table = tagged ? nullptr : static_cast<Slot *>(memory);
-            unsigned int *tags = tagged ? static_cast<unsigned int *>(memory) : nullptr;
-            void *places = tagged ? static_cast<char *>(memory) + slots : nullptr;
             int *flags = reinterpret_cast<int *>(static_cast<char *>(memory) + table_bytes);
             int raised[2] = {0, 0};
             hipError_t e = hipMemsetAsync(flags, 0, sizeof(raised), s);
@@ -276,22 +277,21 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
                 e = hipFuncSetAttribute(reinterpret_cast<const void *>(build_tables_kernel<64>),
                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)(sizeof(Slot) * 4 << 11));
             if (e == hipSuccess) {
-                auto *bytes = static_cast<PlaceOf<16> *>(places);
-                auto *words = static_cast<PlaceOf<64> *>(places);
+                auto *bytes = tagged ? static_cast<Tagged<PlaceOf<16>> *>(memory) : nullptr;
+                auto *words = tagged ? static_cast<Tagged<PlaceOf<64>> *>(memory) : nullptr;
                 if (narrow)
                     build_tables_kernel<16><<<div_up(N, 16), 256, sizeof(Slot) * 16 << log2_slots, s>>>(
-                        p, idx, N, K, log2_slots, table, tags, bytes, flags);
+                        p, idx, N, K, log2_slots, table, bytes, flags);
                 else
                     build_tables_kernel<64><<<div_up(N, 4), 256, sizeof(Slot) * 4 << log2_slots, s>>>(
-                        p, idx, N, K, log2_slots, table, tags, words, flags);
+                        p, idx, N, K, log2_slots, table, words, flags);
                 const int grid = (int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20);
-                const auto *buckets = reinterpret_cast<const uint4 *>(tags);
                 if (!tagged)
-                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, bytes, P);
+                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, P);
                 else if (narrow)
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, bytes, P);
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, P);
                 else
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, buckets, words, P);
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, words, P);
                 e = hipGetLastError();
             }
             if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
