@@ -206,11 +206,6 @@ def test_symmetrize_table_sizes(stages, monkeypatch, n, k):
     got = stages.symmetrize(p, idx)
     monkeypatch.setenv("TSNE_SYMMETRIZE_SCAN", "1")
     assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
-    if n * k > 5e7:  # tables with values in them: the result may take the place of the input
-        monkeypatch.delenv("TSNE_SYMMETRIZE_SCAN")
-        assert stages.lib().tsne_hip_symmetrize(p.data_ptr(), idx.data_ptr(), n, k, p.data_ptr(), None) == 0
-        torch.cuda.synchronize()
-        assert torch.equal(got.view(torch.int32), p.view(torch.int32))
 
 
 @pytest.mark.parametrize("n,k", [(2, 2), (7, 3), (300, 300), (5000, 90), (70000, 20), (20000, 1)])
