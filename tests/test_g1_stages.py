@@ -1230,3 +1230,68 @@ def test_small_step_forms(stages, n, k):
 
     for a, b in zip(run(False), run(True)):
         assert same_bits(a, b)
+
+
+def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch):
+    """Steps of a small problem that do not launch the grouping kernels only ever follow one of the same call that
+    does: a captured pair of steps replayed for a new start finds that start's grouping (no point strays), a call
+    that was captured and not run leaves the next one to group for itself, and replays of it start afresh each time."""
+    monkeypatch.setenv("TSNE_OVERLAP", "0")
+    n, k = 3000, 20
+    rng = np.random.default_rng(11)
+    idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
+    idx[:, 0] = np.arange(n)
+    P = (rng.random((n, k)) / (n * k)).astype(np.float32)
+    starts = [dev(rng.standard_normal(2 * n).astype(np.float32)) for _ in range(2)]
+    dP, di = dev(P), dev(idx)
+
+    def fresh():
+        plan = stages.Plan(n, k)
+        plan.prepare_attractive(dP, di)
+        return plan, torch.empty_like(starts[0]), torch.empty_like(starts[0]), torch.empty_like(starts[0])
+
+    def begin(start, y, gains, old):
+        y.copy_(start), gains.fill_(1.0), old.zero_()
+
+    monkeypatch.setenv("TSNE_GRAPH", "0")
+    plan, *state = fresh()
+    begin(starts[1], *state)
+    want = []
+    for first, last in ((0, 1), (1, 4)):
+        plan.iterate_(None, None, *state, first, last, eta=1e-3)
+        want.append([v.cpu().numpy() for v in state])
+    plan.close()
+
+    monkeypatch.setenv("TSNE_GRAPH", "1")
+    plan, *state = fresh()
+    begin(starts[0], *state)
+    plan.iterate_(None, None, *state, 0, 1, eta=1e-3)
+    plan.iterate_(None, None, *state, 1, 5, eta=1e-3)  # (captured after an odd number of steps)
+    torch.cuda.synchronize()
+    strays = plan.grouping_stats()[2]
+    begin(starts[1], *state)
+    plan.iterate_(None, None, *state, 0, 4, eta=1e-3)
+    torch.cuda.synchronize()
+    assert plan.grouping_stats()[2] == strays  # (steps too short for a point to leave its tile's neighbourhood)
+    for got, a in zip(state, want[1]):
+        assert same_bits(got.cpu().numpy(), a)
+    plan.close()
+
+    monkeypatch.setenv("TSNE_GRAPH", "0")
+    plan, *state = fresh()
+    begin(starts[1], *state)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.iterate_(None, None, *state, 0, 1, eta=1e-3)
+    plan.iterate_(None, None, *state, 1, 2, eta=1e-3)  # the captured step has not run: this one is the first
+    torch.cuda.synchronize()
+    for got, a in zip(state, want[0]):
+        assert same_bits(got.cpu().numpy(), a)
+    for start in (starts[0], starts[1], starts[1]):
+        begin(start, *state)
+        graph.replay()
+        torch.cuda.synchronize()
+        _ = (state[0] * 2.0).sum().item()  # eager work between the replays
+    for got, a in zip(state, want[0]):
+        assert same_bits(got.cpu().numpy(), a)
+    plan.close()

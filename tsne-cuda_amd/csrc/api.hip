@@ -259,6 +259,8 @@ int launch_steps(tsne_hip_plan *p, const float *pij, const int *indices, float *
             // Capture two steps (the bounds slot is back where it started) including the side stream's part.
             hipGraph_t graph = nullptr;
             TSNE_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
+            // (a captured step that kept the grouping unseen would do so at every replay: the first may always group)
+            p->steps_to_grouping = 0;
             const int rc =
                 launch_two_steps(p, pij, indices, embedding, gains, old_forces, eta, momentum, exaggeration, slot, s);
             const hipError_t end = hipStreamEndCapture(s, &graph);
@@ -601,6 +603,9 @@ int tsne_hip_iterate(tsne_hip_plan *plan, const float *pij, const int *indices, 
     plan->loop_embedding = embedding;
     plan->loop_next_step = step_end;
     int slot = 0;
+    // The first step of a call launches the grouping kernels: what the plan's arrays hold when it runs is only known
+    // on the device (the call before may have been captured and not run yet, or this one may be replayed).
+    plan->steps_to_grouping = 0;
     if (launch_bounds(plan, embedding, slot, s, !continues)) return 1;
     if (plan->recenter && launch_centre_sums(plan, embedding, slot, s)) return 1;
     if (launch_pack_xy(plan, embedding, s)) return 1;
@@ -744,7 +749,6 @@ int tsne_hip_plan_set_boxes(tsne_hip_plan *plan, int n_boxes_per_dim) {
     plan->n_nodes = n_boxes_per_dim * kInterp;
     // (a grouping of the points by tile belongs to the grid it was made on)
     TSNE_TRY(hipMemset(&plan->scalars->reuse_sort, 0, sizeof(int)));
-    plan->steps_to_grouping = 0;
     return 0;
 }
 

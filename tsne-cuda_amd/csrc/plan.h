@@ -118,7 +118,7 @@ struct tsne_hip_plan {
     // Small problems (one stream, see api.hip): the pattern once more, row by row, {probability, neighbour} in the
     // caller's order of neighbours; the inverse row pass computes the attractive forces from it in spare workgroups.
     uint2 *row_entries = nullptr;
-    int steps_to_grouping = 0;      // steps of that form until the grouping kernels are launched again
+    int steps_to_grouping = 0;      // steps of that form until the grouping kernels are launched again, in this call
     int spin_limit = 0;             // polls before a wave of the attractive kernel gives up a wait
     bool blocked_ready = false;
     // Optional CSR pattern (borrowed pointers; tsne_hip_plan_set_csr_pattern): when set, steps without an explicit

@@ -1292,7 +1292,6 @@ int launch_finish_z(tsne_hip_plan *p, float *normalization, hipStream_t s) {
 }
 
 int launch_bounds_reset(tsne_hip_plan *p, int slot, hipStream_t s, bool new_embedding) {
-    if (new_embedding) p->steps_to_grouping = 0;
     bounds_reset_kernel<<<1, 64, 0, s>>>(p->scalars, slot, new_embedding ? 1 : 0);
     TSNE_LAUNCHED(s);
     return 0;
