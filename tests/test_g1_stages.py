@@ -874,6 +874,25 @@ def test_locality_order(stages):
     assert np.array_equal(small, np.arange(1000))
 
 
+def locality_pivot(number, n):
+    """The point that pivot `number` of the locality ordering of n points is (locality.hip)."""
+    m = (1 << 64) - 1
+    z = ((number + 1) * 0x9E3779B97F4A7C15) & m
+    z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & m
+    z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & m
+    return (z ^ (z >> 31)) % n
+
+
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("n", [17003, 300000])
+def test_locality_order_of_points_that_are_not_numbers(stages, n, value):
+    """The pivot that the chain starts from and another hold a NaN or an infinity: still a permutation."""
+    X = np.random.default_rng(n).standard_normal((n, 4)).astype(np.float32)
+    X[[locality_pivot(0, n), locality_pivot(9, n)], 1] = value
+    order = stages.locality_order(dev(X)).cpu().numpy()
+    assert np.array_equal(np.sort(order), np.arange(n))
+
+
 def test_iterate_with_prepared_pattern(stages, c0_problem):
     c = c0_problem
     n = c["X"].shape[0]

@@ -16,9 +16,9 @@
 // locality from the FAISS IVF lists (src/util/distance_utils.cu:101-127).
 #include <algorithm>
 #include <cmath>
-#include <limits>
 #include <vector>
 
+#include "locality_chain.h"
 #include "stages.h"
 
 namespace tsnehip {
@@ -158,38 +158,7 @@ int locality_order(const float *points, int N, int D, std::vector<int> &order_ho
     TSNE_TRY(hipMemcpyAsync(h_labels.data(), labels.p, sizeof(int) * (size_t)N, hipMemcpyDeviceToHost, s));
     TSNE_TRY(hipStreamSynchronize(s));
 
-    // Greedy chain over the pivots: start at pivot 0, always continue with the
-    // nearest pivot not yet placed.
-    std::vector<int> chain_pos(M, -1);
-    {
-        std::vector<char> placed(M, 0);
-        int cur = 0;
-        for (int pos = 0; pos < M; ++pos) {
-            placed[cur] = 1;
-            chain_pos[cur] = pos;
-            double best = std::numeric_limits<double>::infinity();
-            int next = -1;
-            for (int j = 0; j < M; ++j) {
-                if (placed[j]) continue;
-                double d2 = 0.0;
-                for (int d = 0; d < D; ++d) {
-                    const double diff = (double)h_rows[(size_t)cur * D + d] - (double)h_rows[(size_t)j * D + d];
-                    d2 += diff * diff;
-                }
-                if (d2 < best) {
-                    best = d2;
-                    next = j;
-                }
-            }
-            if (next < 0) break;
-            cur = next;
-        }
-    }
-    // Stable counting sort of the points by chain position.
-    std::vector<int64_t> start(M + 1, 0);
-    for (int i = 0; i < N; ++i) start[chain_pos[h_labels[i]] + 1] += 1;
-    for (int c = 0; c < M; ++c) start[c + 1] += start[c];
-    for (int i = 0; i < N; ++i) order_host[start[chain_pos[h_labels[i]]]++] = i;
+    order_by_place(h_labels.data(), N, chain_pivots(h_rows.data(), M, D), order_host.data());
     return 0;
 }
 
