@@ -1314,3 +1314,51 @@ def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch):
     for got, a in zip(state, want[0]):
         assert same_bits(got.cpu().numpy(), a)
     plan.close()
+
+
+@pytest.mark.parametrize("n,d,k,order", [
+    (1203, 20, 32, "cycle"),    # direct search / vector sweep
+    (9001, 17, 60, "cycle"),    # direct search / matrix sweep
+    (20011, 37, 25, "cycle"),   # renumbered / as the points come
+    (16901, 127, 20, "runs"),   # chunked sweep with the table of centre distances / without
+    (20483, 261, 33, "runs"),
+    (17000, 129, 30, "far")])   # ... where no margin verifies
+def test_knn_without_room_for_the_faster_form(stages, monkeypatch, n, d, k, order):
+    """The same rows, bit for bit, with memory for the faster form of a search and without."""
+    rng = np.random.default_rng(n)
+    at = np.arange(n) % 5 if order == "cycle" else np.arange(n) * 5 // n
+    X = (rng.standard_normal((n, d)) + (4.0 * rng.standard_normal((5, d)))[at]).astype(np.float32)
+    if order == "far":
+        X = (X * np.float32(1e-3) + np.float32(100.0)).astype(np.float32)
+    dX = dev(X)
+    idx, d2 = stages.knn(dX, k)
+    monkeypatch.setenv("TSNE_SCRATCH_LIMIT", "0")
+    idx_0, d2_0 = stages.knn(dX, k)
+    assert torch.equal(idx, idx_0) and torch.equal(d2, d2_0)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("n,k", [(1203, 32), (20011, 50)])
+def test_loop_and_symmetrisation_without_room_for_the_faster_form(stages, monkeypatch, n, k):
+    rng = np.random.default_rng(n)
+    idx = (np.arange(n)[:, None] + np.sort(rng.permuted(np.tile(np.arange(1, 2 * k), (n, 1)), axis=1)[:, :k], axis=1)) % n
+    idx[:, 0] = np.arange(n)
+    p, idx = rng.random((n, k)).astype(np.float32), idx.astype(np.int32)
+    y0 = dev(rng.standard_normal(2 * n).astype(np.float32))
+
+    def run():
+        P = stages.symmetrize(dev(p), dev(idx))
+        plan = stages.Plan(n, k)
+        plan.prepare_attractive(P, dev(idx))
+        y = y0.clone()
+        gains, old = torch.ones_like(y), torch.zeros_like(y)
+        z = plan.iterate_(None, None, y, gains, old, 0, 11)
+        torch.cuda.synchronize()
+        plan.close()
+        return [v.cpu().numpy() for v in (P, y, gains, old, z)]
+
+    want = run()
+    monkeypatch.setenv("TSNE_SCRATCH_LIMIT", "0")
+    for a, b in zip(run(), want):
+        assert same_bits(a, b)

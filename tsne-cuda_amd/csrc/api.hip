@@ -33,6 +33,15 @@ bool sync_kernels_enabled() {
     return enabled;
 }
 
+hipError_t malloc_optional(void **p, size_t bytes) {
+    if (const char *v = std::getenv("TSNE_SCRATCH_LIMIT"))
+        if (bytes > std::strtoull(v, nullptr, 10)) {
+            *p = nullptr;
+            return hipErrorOutOfMemory;
+        }
+    return hipMalloc(p, bytes);
+}
+
 int profile_mark(tsne_hip_plan *p, int id, hipStream_t) {
     if (p->profiling || (p->profiling_attractive && id == kKernelAttractive)) p->pending_kernel = id;
     return 0;

@@ -19,6 +19,10 @@ const char *last_error();
 // TSNE_MAYBE_SYNC does (src/include/util/cuda_utils.h:46-70).
 bool sync_kernels_enabled();
 
+// hipMalloc for memory that a faster form of a stage uses and a slower one does without.  TSNE_SCRATCH_LIMIT=<bytes>
+// (read on every call; for measurements and tests of the slower forms): more than that is never there.
+hipError_t malloc_optional(void **p, size_t bytes);
+
 #define TSNE_TRY(expr)                                                                              \
     do {                                                                                            \
         hipError_t tsne_err_ = (expr);                                                              \

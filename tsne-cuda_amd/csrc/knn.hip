@@ -2082,6 +2082,8 @@ struct DeviceMem {
         if (p) (void)hipFree(p);
     }
     bool alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess; }
+    // (of a form that the call can do without)
+    bool alloc_optional(size_t bytes) { return malloc_optional(&p, bytes ? bytes : 1) == hipSuccess; }
     template <typename T>
     T *as() const {
         return static_cast<T *>(p);
@@ -2172,7 +2174,7 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
     const int side = large ? 128 : 64;
     const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(direct_floats(N) / pitch) / 128 * 128));
     DeviceMem dist;
-    if (!dist.alloc(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
+    if (!dist.alloc_optional(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
         (void)hipGetLastError();
         return kNoRoom;
     }
@@ -2394,8 +2396,8 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         TSNE_TRY(hipGetLastError());
         // The table grows with the square of the points (80 MB at 50000) and is made where it takes up to 1 GB.
         const size_t table_bytes = sizeof(float) * (size_t)num_tiles * Npad;
-        if (table_bytes <= (size_t)1 << 30 && centre_rows.alloc(sizeof(float) * (size_t)num_tiles * D) &&
-            centre_dist.alloc(table_bytes)) {
+        if (table_bytes <= (size_t)1 << 30 && centre_rows.alloc_optional(sizeof(float) * (size_t)num_tiles * D) &&
+            centre_dist.alloc_optional(table_bytes)) {
             transpose_points_kernel<<<dim3(div_up(D, 32), div_up(num_tiles, 32)), 256, 0, s>>>(
                 centers.as<float>(), D, num_tiles, D, centre_rows.as<float>());
             TSNE_TRY(hipGetLastError());
@@ -2621,7 +2623,8 @@ int run_knn_any_order(const float *points, int N, int D, int K, int *indices, fl
         numbering_lacks_locality(points, N, D, &lacks, s))
         return 1;
     // (without room for a second copy of the points, or for the search beside it: as they come)
-    if (DeviceMem order, sorted; lacks && order.alloc(sizeof(int) * (size_t)N) && sorted.alloc(sizeof(float) * (size_t)N * D)) {
+    if (DeviceMem order, sorted; lacks && order.alloc_optional(sizeof(int) * (size_t)N) &&
+                                 sorted.alloc_optional(sizeof(float) * (size_t)N * D)) {
         std::vector<int> order_host;
         if (locality_order(points, N, D, order_host, s)) return 1;
         TSNE_TRY(hipMemcpyAsync(order.p, order_host.data(), sizeof(int) * (size_t)N, hipMemcpyHostToDevice, s));

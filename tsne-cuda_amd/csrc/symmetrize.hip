@@ -268,7 +268,7 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
         const bool tagged = slots * sizeof(Slot) > kTaggedBytes, narrow = log2_slots <= 8;
         const size_t table_bytes = !tagged ? slots * sizeof(Slot) :
                                    slots / kBucket * (narrow ? sizeof(Tagged<PlaceOf<16>>) : sizeof(Tagged<PlaceOf<64>>));
-        if (hipMalloc(&memory, table_bytes + 2 * sizeof(int)) == hipSuccess) {
+        if (malloc_optional(&memory, table_bytes + 2 * sizeof(int)) == hipSuccess) {
             Slot *table = tagged ? nullptr : static_cast<Slot *>(memory);
             int *flags = reinterpret_cast<int *>(static_cast<char *>(memory) + table_bytes);
             int raised[2] = {0, 0};
