@@ -195,7 +195,7 @@ def test_symmetrize_hashed_and_scanning_forms(stages, c0_problem, monkeypatch, n
                                  (4097, 1638), (4096, 1639), (70001, 1000), (530000, 102), (263000, 204), (140000, 205)])
 def test_symmetrize_table_sizes(stages, monkeypatch, n, k):
     """The fullest table of a size and the emptiest of the next (buckets that overflow), one bucket only, the most
-    neighbours of the tables and one more, tables large enough to have tags beside them: the scanning form's values,
+    neighbours of the tables and one more, tables large enough to hold tags and places instead: the scanning form's values,
     bit for bit.  Bands of columns (most pairs in both directions), every second row strided (few)."""
     g = torch.Generator(device="cuda").manual_seed(n + k)
     i = torch.arange(n, device="cuda")[:, None]
@@ -206,6 +206,22 @@ def test_symmetrize_table_sizes(stages, monkeypatch, n, k):
     got = stages.symmetrize(p, idx)
     monkeypatch.setenv("TSNE_SYMMETRIZE_SCAN", "1")
     assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
+
+
+@pytest.mark.parametrize("n,k", [(5000, 30), (530000, 102), (140000, 205)])
+def test_symmetrize_refuses_before_it_writes(stages, n, k):
+    """Slots, and tags with places of either width: a column that names no point is an error that leaves the output as
+    it was, whatever else the row holds."""
+    idx = ((torch.arange(n, device="cuda")[:, None] + torch.arange(k, device="cuda")) % n).int()
+    p = torch.rand(n, k, device="cuda")
+    for bad, twice in ((n, False), (-1, True)):
+        idx[n // 2, k // 2] = bad
+        if twice:
+            idx[n // 3, 5] = idx[n // 3, 2]
+        out = torch.full_like(p, -3.0)
+        rc = stages.lib().tsne_hip_symmetrize(stages._ptr(p), stages._ptr(idx), n, k, stages._ptr(out), stages._stream())
+        assert rc != 0 and b"outside" in stages.lib().tsne_hip_last_error()
+        assert bool((out == -3.0).all())
 
 
 @pytest.mark.parametrize("n,k", [(2, 2), (7, 3), (300, 300), (5000, 90), (70000, 20), (20000, 1)])

@@ -167,7 +167,8 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
                                                                 int N, int K, int log2_slots,
                                                                 const Slot *__restrict__ table,
                                                                 const Tagged<PLACE> *__restrict__ tagged,
-                                                                float *__restrict__ P) {
+                                                                const int *__restrict__ flags, float *__restrict__ P) {
+    if (flags[0] | flags[1]) return;  // (a column out of range: P stays as it is; one named twice: the scan writes it)
     const size_t nnz = (size_t)N * K;
     const double denom = 2.0 * (double)N;
     const unsigned int buckets = 1u << (log2_slots - 4);
@@ -287,11 +288,11 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
                         p, idx, N, K, log2_slots, table, words, flags);
                 const int grid = (int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20);
                 if (!tagged)
-                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, P);
+                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, flags, P);
                 else if (narrow)
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, P);
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, flags, P);
                 else
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, words, P);
+                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, words, flags, P);
                 e = hipGetLastError();
             }
             if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
