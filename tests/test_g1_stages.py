@@ -1224,7 +1224,7 @@ def test_knn_small_problems(stages, n, d, k, kind):
 def test_knn_of_points_in_no_order(stages, n, d, k, kind):
     """Clusters that come in turn: the search renumbers the points for itself and answers in the caller's
     numbering - also where equal distances are ordered by it, where queries fail the verification, where no margin
-    verifies and where the neighbours are too many for the matrix sweep.  The vector sweep's rows, bit for bit."""
+    verifies and where many neighbours are wanted.  The vector sweep's rows, bit for bit."""
     rng = np.random.default_rng(n)
     X = (rng.standard_normal((n, d)) + (6.0 * rng.standard_normal((5, d)))[np.arange(n) % 5]).astype(np.float32)
     if kind == "grid":
@@ -1352,6 +1352,21 @@ def test_knn_without_room_for_the_faster_form(stages, monkeypatch, n, d, k, orde
     idx_0, d2_0 = stages.knn(dX, k)
     assert torch.equal(idx, idx_0) and torch.equal(d2, d2_0)
     idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("limit", [0, 20000, 100000, 1 << 40])
+@pytest.mark.parametrize("k", [25, 1500])
+def test_knn_of_points_in_no_order_without_room(stages, monkeypatch, k, limit):
+    """No room for the look at the numbering, for the ordering, for the renumbered copy: the points are searched as
+    they come, without an error.  1500 neighbours are more than the matrix sweep takes: nothing is renumbered."""
+    n, d = 20011, 37
+    rng = np.random.default_rng(n)
+    X = (rng.standard_normal((n, d)) + (6.0 * rng.standard_normal((5, d)))[np.arange(n) % 5]).astype(np.float32)
+    dX = dev(X)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    monkeypatch.setenv("TSNE_SCRATCH_LIMIT", str(limit))
+    idx, d2 = stages.knn(dX, k)
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 

@@ -43,6 +43,8 @@ hipError_t malloc_optional(void **p, size_t bytes);
 // Return code of the launchers that have a fallback: the shape is beyond what this form of the kernel holds
 // (as opposed to 1, a failure).
 constexpr int kShapeNotSupported = 2;
+// ... and of those that a caller can do without: their memory is not there, nothing else went wrong.
+constexpr int kNoRoom = 3;
 
 inline int div_up(int64_t a, int64_t b) { return (int)((a + b - 1) / b); }
 

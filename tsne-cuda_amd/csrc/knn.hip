@@ -55,6 +55,7 @@
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <new>
 #include <vector>
 
 namespace tsnehip {
@@ -2078,12 +2079,20 @@ __global__ __launch_bounds__(128) void sample_tiles_kernel(const float *__restri
 
 struct DeviceMem {
     void *p = nullptr;
-    ~DeviceMem() {
-        if (p) (void)hipFree(p);
+    ~DeviceMem() { release(); }
+    void release() {
+        if (p) (void)hipFree(p);  // (waits for the kernels that use it)
+        p = nullptr;
     }
-    bool alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess; }
+    bool alloc(size_t bytes) {
+        release();
+        return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess;
+    }
     // (of a form that the call can do without)
-    bool alloc_optional(size_t bytes) { return malloc_optional(&p, bytes ? bytes : 1) == hipSuccess; }
+    bool alloc_optional(size_t bytes) {
+        release();
+        return malloc_optional(&p, bytes ? bytes : 1) == hipSuccess;
+    }
     template <typename T>
     T *as() const {
         return static_cast<T *>(p);
@@ -2148,6 +2157,49 @@ int dispatch_mfma_sweep(int ksteps, const SweepArgs &args, int grid, hipStream_t
 #undef TSNE_MFMA_CASE
 }
 
+// Shape of the matrix-instruction sweep for N points of D dimensions.
+struct SweepGeometry {
+    int Dnorm;           // |x|^2 row: first even row after the real dimensions
+    int ksteps;          // k-steps incl. the augmented pair
+    bool chunked;        // more dimensions than one wave's registers hold
+    bool bf16, bf16_chunked;
+    int n_chunks, steps16, num_tiles, bitmap_words;
+    size_t tile_lds;
+
+    // Unless force_f32 asks for products of floats, the sweeps multiply bf16 terms (two per coordinate) of the
+    // points relative to their tile's centre; three more dimensions carry a per-point term.
+    SweepGeometry(int N, int D, bool force_f32) {
+        Dnorm = (D + 1) & ~1;
+        ksteps = (Dnorm + 2) / 2;
+        chunked = ksteps > kMfmaMaxSteps;
+        bf16 = !chunked && !force_f32 && D + 3 <= 128;
+        bf16_chunked = chunked && !force_f32;
+        n_chunks = chunked ? (bf16_chunked ? div_up(D + 3, 32) : div_up(ksteps, kChunkSteps)) : 0;
+        if (chunked) ksteps = n_chunks * (bf16_chunked ? kChunkSteps / 2 : kChunkSteps);  // (slots of 16 bytes per lane x 4)
+        else if (ksteps > 32) ksteps = (ksteps + 3) & ~3;
+        steps16 = div_up(D + 3, 16);
+        num_tiles = div_up(N, kCT);
+        bitmap_words = div_up(num_tiles, 32);
+        tile_lds = chunked ? sizeof(float4) * kChunkFloat4 + sizeof(float) * D  // (bf16: two chunks of half the size)
+                           : sizeof(float4) * (bf16 ? 512 * steps16 + 64 : 4 * ((ksteps + 3) / 4) * 64);
+    }
+    size_t lds_with(int cap) const {
+        return tile_lds + sizeof(u64) * 4 * cap + sizeof(unsigned int) * bitmap_words;
+    }
+    // Room for the candidates kept, as many again and one more tile where the LDS sort buffers of that
+    // size fit: a list that is nearly full right after a selection would be selected again after every tile.
+    int list_cap(int want) const {
+        int cap = next_pow2(2 * want + kCT);
+        if (cap > 4096 || lds_with(cap) > 150 * 1024) cap = next_pow2(want + kCT);
+        return cap < 256 ? 256 : cap;
+    }
+    size_t sweep_lds(int want) const { return lds_with(list_cap(want)); }
+    bool fits(int want) const { return list_cap(want) <= 4096 && sweep_lds(want) <= 150 * 1024; }
+};
+constexpr int kMatrixPoints = 8192;  // fewer points: vector sweep
+// K' candidates kept per query.
+inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2)); }
+
 int valu_cap(int K) {
     int cap = 256;
     while (cap < K - 1 + kCT) cap <<= 1;
@@ -2164,9 +2216,9 @@ constexpr int kDirectNeighbors = 256;  // most K - 1 that select_row_kernel<8> t
 // Floats per block: 64 MiB are cheap to allocate (5000 x 50: 0.21 ms; 0.47 with the whole 100 MB at once), but
 // beyond 10240 points hold too few rows to fill the chip with their selection (16000 x 50: 1.6 ms with 64 MiB, 1.3
 // with 256).
-constexpr int kNoRoom = -1;  // run_direct_search: nothing done, the sweeps need less memory
 inline size_t direct_floats(int N) { return (size_t)1 << (N <= 10240 ? 24 : 26); }
 
+// (kNoRoom: nothing done, the sweeps need less memory)
 int run_direct_search(const float *points, int N, int D, int K, int cus, int *indices, float *sq_dist, hipStream_t s) {
     const int pitch = div_up(N, 128) * 128;
     // Tiles of 128 points a side where they fill the chip, of 64 otherwise.
@@ -2222,7 +2274,7 @@ int run_valu_sweep(const float *points, const float *Xt, int N, int Npad, int D,
         (slices > 1 && !slice_keys.alloc(sizeof(u64) * (size_t)num_qtiles * kQT * slices * (K - 1))) ||
         (prune && (!centers.alloc(sizeof(float) * (size_t)D * T) || !radius.alloc(sizeof(float) * T)))) {
         set_error("knn: out of device memory for the candidate lists");
-        return 1;
+        return kNoRoom;
     }
     if (prune) {
         tile_balls_kernel<<<T, 128, sizeof(float) * D, s>>>(points, N, D, T, centers.as<float>(), radius.as<float>());
@@ -2250,8 +2302,14 @@ int run_valu_sweep(const float *points, const float *Xt, int N, int Npad, int D,
 // 3 = as 2 with the products on floats where 2 multiplies bf16 terms (every dimension count but 126).
 // stats (optional, 3 ints): [0] = 1 if the matrix-instruction sweep ran, [1] = queries redone by the VALU sweep,
 // [2] = per mille of the (query tile, candidate tile) pairs the matrix sweep computed.
-int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
-                 int *stats, const KnnProbes *probes, const KnnRenumbered *renumbered) {
+// renumbered != nullptr: `points` are a renumbered copy (point i is the caller's order[i]) and the result is in
+// the caller's numbering.  Returns kNoRoom where memory is what it lacks.
+struct KnnRenumbered {
+    const int *order;            // device
+    const float *caller_points;  // device
+};
+static int search(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
+                  int *stats, const KnnProbes *probes, const KnnRenumbered *renumbered) {
     if (stats) stats[0] = stats[1] = stats[2] = 0;
     if (N <= 0 || D <= 0 || K <= 0) {
         set_error("knn: num_points, num_dims and num_neighbors must be positive (got %d, %d, %d)", N, D, K);
@@ -2275,39 +2333,15 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
     TSNE_TRY(hipGetDevice(&device));
     TSNE_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
 
-    // Matrix-instruction sweep geometry.
-    const int Dnorm = (D + 1) & ~1;        // |x|^2 row: first even row after the real dimensions
-    int ksteps = (Dnorm + 2) / 2;          // k-steps incl. the augmented pair
-    const bool chunked = ksteps > kMfmaMaxSteps;  // more dimensions than one wave's registers hold
-    // Unless mode 3 asks for products of floats, the sweeps multiply bf16 terms (two per coordinate) of the
-    // points relative to their tile's centre; three more dimensions carry a per-point term.
     const bool force_f32 = mode == 3;
     if (mode == 3) mode = 2;
-    const bool bf16 = !chunked && !force_f32 && D + 3 <= 128;
-    const bool bf16_chunked = chunked && !force_f32;
-    const int n_chunks = chunked ? (bf16_chunked ? div_up(D + 3, 32) : div_up(ksteps, kChunkSteps)) : 0;
-    if (chunked) ksteps = n_chunks * (bf16_chunked ? kChunkSteps / 2 : kChunkSteps);  // (slots of 16 bytes per lane x 4)
-    else if (ksteps > 32) ksteps = (ksteps + 3) & ~3;
-    const int steps16 = div_up(D + 3, 16);
-    const int num_tiles = div_up(N, kCT);
-    const int bitmap_words = div_up(num_tiles, 32);
-    // Room for the candidates kept, as many again and one more tile where the LDS sort buffers of that
-    // size fit: a list that is nearly full right after a selection would be selected again after every tile.
-    const size_t tile_lds = chunked ? sizeof(float4) * kChunkFloat4 + sizeof(float) * D  // (bf16: two chunks of half the size)
-                                    : sizeof(float4) * (bf16 ? 512 * steps16 + 64 : 4 * ((ksteps + 3) / 4) * 64);
-    auto lds_with = [&](int cap) -> size_t {
-        return tile_lds + sizeof(u64) * 4 * cap + sizeof(unsigned int) * bitmap_words;
-    };
-    auto list_cap = [&](int want) {
-        int cap = next_pow2(2 * want + kCT);
-        if (cap > 4096 || lds_with(cap) > 150 * 1024) cap = next_pow2(want + kCT);
-        return cap < 256 ? 256 : cap;
-    };
-    auto sweep_lds = [&](int want) -> size_t { return lds_with(list_cap(want)); };
-    auto sweep_fits = [&](int want) { return list_cap(want) <= 4096 && sweep_lds(want) <= 150 * 1024; };
-    int want = std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2));  // K' candidates kept per query
-    const bool mfma_fits = sweep_fits(want);
-    bool use_mfma = mode == 2 || (mode == 0 && mfma_fits && N >= 8192);
+    const SweepGeometry geometry(N, D, force_f32);
+    const bool chunked = geometry.chunked, bf16 = geometry.bf16, bf16_chunked = geometry.bf16_chunked;
+    const int Dnorm = geometry.Dnorm, ksteps = geometry.ksteps, n_chunks = geometry.n_chunks;
+    const int steps16 = geometry.steps16, num_tiles = geometry.num_tiles, bitmap_words = geometry.bitmap_words;
+    int want = candidates_kept(N, K);
+    const bool mfma_fits = geometry.fits(want);
+    bool use_mfma = mode == 2 || (mode == 0 && mfma_fits && N >= kMatrixPoints);
     if (mode == 2 && !mfma_fits) {
         set_error("knn: the matrix-instruction sweep does not fit %d dimensions / %d neighbours", D, K);
         return kShapeNotSupported;
@@ -2321,12 +2355,15 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
     const int Npad = div_up(N, kCT) * kCT;
     // Transposed points for the vector sweep (built only when that sweep runs).
     DeviceMem Xt;
+    // Table of centre distances (chunked sweep), which goes where another buffer finds no room beside it.
+    DeviceMem centre_dist;
     // (the points in the caller's numbering: equal distances are ordered by that)
     const float *caller_points = renumbered ? renumbered->caller_points : points;
     auto build_transposed = [&]() -> int {
+        centre_dist.release();
         if (!Xt.alloc(sizeof(float) * (size_t)D * Npad)) {
             set_error("knn: out of device memory for the transposed points");
-            return 1;
+            return kNoRoom;
         }
         dim3 tgrid(div_up(Npad, 32), div_up(D, 32));
         transpose_points_kernel<<<tgrid, 256, 0, s>>>(caller_points, N, D, Npad, Xt.as<float>());
@@ -2338,7 +2375,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         if (rc != kNoRoom) return rc;
     }
     if (!use_mfma) {
-        if (build_transposed()) return 1;
+        if (const int rc = build_transposed()) return rc;
         return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
     }
 
@@ -2351,7 +2388,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         !scal.alloc(4 * sizeof(int)) || !fail_list.alloc(sizeof(int) * N) ||
         !centers.alloc(sizeof(float) * (size_t)D * num_tiles) || !radius.alloc(sizeof(float) * num_tiles)) {
         set_error("knn: out of device memory for the candidate buffers");
-        return 1;
+        return kNoRoom;
     }
     TSNE_TRY(hipMemsetAsync(scal.p, 0, 4 * sizeof(int), s));  // [0] max |x|^2 (float bits), [1] fail count, [2..3] tiles swept (64-bit)
     norms_kernel<<<div_up(Npad, 256), 256, 0, s>>>(points, N, D, Npad, norms.as<float>(), scal.as<float>());
@@ -2377,12 +2414,12 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
                                                          num_tiles, Xp.as<float4>());
         TSNE_TRY(hipGetLastError());
     }
-    DeviceMem centres_p, tile_coef, centre_rows, centre_dist;
+    DeviceMem centres_p, tile_coef, centre_rows;
     if (bf16_chunked) {
         if (!centres_p.alloc(sizeof(float) * 32 * (size_t)n_chunks * num_tiles) ||
             !tile_coef.alloc(sizeof(float) * 2 * (size_t)num_tiles)) {
             set_error("knn: out of device memory for the tile centres");
-            return 1;
+            return kNoRoom;
         }
         const int64_t pieces = (int64_t)Npad * n_chunks * 8;
         pack_points_bf16_chunked_kernel<<<div_up(pieces, 256), 256, 0, s>>>(points, centers.as<float>(), N, D, n_chunks,
@@ -2414,7 +2451,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
     // failed (listed in fail_list), swept = tile pairs computed.
     auto sweep_and_rerank = [&](int keep, const int *tile_list, int first, int step, int count, int &failed,
                                 unsigned long long &swept) -> int {
-        const int cap = list_cap(keep);
+        const int cap = geometry.list_cap(keep);
         // One workgroup sweeps a query tile against all its candidate tiles, which takes long with hundreds
         // of dimensions, and the tiles differ in how many candidate tiles they can skip: unless there are
         // several query tiles per workgroup slot to even that out, the chunked kernel splits every tile's
@@ -2427,11 +2464,20 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         const int grid = std::min(count * parts, slots);
         const size_t n_slots = (size_t)(tile_list || step != 1 ? count * kMQ : N);
         DeviceMem lists, cand, tau, part_keys;
-        if (!lists.alloc(sizeof(u64) * (size_t)grid * kMQ * cap) || !cand.alloc(sizeof(int) * n_slots * keep) ||
-            !tau.alloc(sizeof(float) * n_slots) ||
-            (parts > 1 && !part_keys.alloc(sizeof(u64) * n_slots * parts * keep))) {
+        auto alloc_lists = [&]() -> bool {
+            return lists.alloc(sizeof(u64) * (size_t)grid * kMQ * cap) && cand.alloc(sizeof(int) * n_slots * keep) &&
+                   tau.alloc(sizeof(float) * n_slots) &&
+                   (parts == 1 || part_keys.alloc(sizeof(u64) * n_slots * parts * keep));
+        };
+        bool room = alloc_lists();
+        if (!room && centre_dist.p) {
+            centre_dist.release();
+            (void)hipGetLastError();
+            room = alloc_lists();
+        }
+        if (!room) {
             set_error("knn: out of device memory for the candidate lists");
-            return 1;
+            return kNoRoom;
         }
         TSNE_TRY(hipMemsetAsync(scal.as<int>() + 1, 0, 3 * sizeof(int), s));
         SweepArgs args;
@@ -2469,7 +2515,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         args.probe_nlist = probes ? probes->nlist : 0;
         args.probe_list_tiles = probes ? probes->list_tiles : nullptr;
         if (chunked) {
-            const size_t lds = sweep_lds(keep);
+            const size_t lds = geometry.sweep_lds(keep);
             const auto sweep = !bf16_chunked          ? knn_mfma_chunked_sweep_kernel<false, false>
                                : args.centre_dist ? knn_mfma_chunked_sweep_kernel<true, true>
                                                   : knn_mfma_chunked_sweep_kernel<true, false>;
@@ -2517,21 +2563,21 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
         const int sample_tiles = 16, step = num_qtiles / sample_tiles;
         bool verified = false;
         for (int attempt = 0; attempt < 3 && !verified; ++attempt) {
-            if (sweep_and_rerank(want, nullptr, step / 2, step, sample_tiles, failed, swept)) return 1;
+            if (const int rc = sweep_and_rerank(want, nullptr, step / 2, step, sample_tiles, failed, swept)) return rc;
             if (failed * 10 <= sample_tiles * kMQ) {
                 verified = true;
             } else {
                 const int wider = std::min(N - 1, 2 * want);
-                if (wider == want || !sweep_fits(wider)) break;
+                if (wider == want || !geometry.fits(wider)) break;
                 want = wider;
             }
         }
         if (!verified && mode == 0) {
-            if (build_transposed()) return 1;
+            if (const int rc = build_transposed()) return rc;
             return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
         }
     }
-    if (sweep_and_rerank(want, nullptr, 0, 1, num_qtiles, failed, swept)) return 1;
+    if (const int rc = sweep_and_rerank(want, nullptr, 0, 1, num_qtiles, failed, swept)) return rc;
     if (stats) {
         stats[0] = 1;
         stats[1] = failed;
@@ -2544,7 +2590,7 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
     // tiles); what fails again, and every failure of the register-resident sweep, goes to the vector sweep.
     if (failed > 4 * kQT && chunked && failed * 10 <= N) {
         const int wider = std::min(N - 1, 2 * want);
-        if (wider != want && sweep_fits(wider)) {
+        if (wider != want && geometry.fits(wider)) {
             std::vector<int> queries(failed), tiles;
             TSNE_TRY(hipMemcpy(queries.data(), fail_list.p, sizeof(int) * (size_t)failed, hipMemcpyDeviceToHost));
             for (int q : queries) tiles.push_back(q / kMQ);
@@ -2554,17 +2600,18 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
                 DeviceMem tile_list;
                 if (!tile_list.alloc(sizeof(int) * tiles.size())) {
                     set_error("knn: out of device memory for the retry list");
-                    return 1;
+                    return kNoRoom;
                 }
                 TSNE_TRY(hipMemcpy(tile_list.p, tiles.data(), sizeof(int) * tiles.size(), hipMemcpyHostToDevice));
                 unsigned long long swept_again = 0;
-                if (sweep_and_rerank(wider, tile_list.as<int>(), 0, 1, (int)tiles.size(), failed, swept_again))
-                    return 1;
+                if (const int rc =
+                        sweep_and_rerank(wider, tile_list.as<int>(), 0, 1, (int)tiles.size(), failed, swept_again))
+                    return rc;
             }
         }
     }
     if (failed > 0) {
-        if (build_transposed()) return 1;
+        if (const int rc = build_transposed()) return rc;
         if (renumbered) {
             rename_list_kernel<<<div_up(failed, 256), 256, 0, s>>>(renumbered->order, failed, fail_list.as<int>());
             TSNE_TRY(hipGetLastError());
@@ -2574,8 +2621,14 @@ int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *
     return 0;
 }
 
+int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
+                 int *stats, const KnnProbes *probes) {
+    const int rc = search(points, N, D, K, indices, sq_dist, s, mode, stats, probes, nullptr);
+    return rc == kNoRoom ? 1 : rc;
+}
+
 int run_knn(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s) {
-    return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, nullptr, nullptr, nullptr);
+    return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, nullptr);
 }
 
 // Whether consecutive points are no closer to each other than any points are: the mean squared distance of a
@@ -2585,9 +2638,9 @@ static int numbering_lacks_locality(const float *points, int N, int D, bool *lac
     DeviceMem out;
     *lacks = false;
     if (sampled < 2) return 0;
-    if (!out.alloc(sizeof(float) * (size_t)sampled * (D + 1))) {
+    if (!out.alloc_optional(sizeof(float) * (size_t)sampled * (D + 1))) {
         set_error("knn: out of device memory");
-        return 1;
+        return kNoRoom;
     }
     sample_tiles_kernel<<<sampled, 128, 0, s>>>(points, D, tiles / sampled, out.as<float>());
     TSNE_TRY(hipGetLastError());
@@ -2611,30 +2664,46 @@ static int numbering_lacks_locality(const float *points, int N, int D, bool *lac
     return 0;
 }
 
+// run_knn_any_order on a renumbered copy of the points (kNoRoom: nothing done).
+static int search_renumbered(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
+                             int *stats) {
+    std::vector<int> order_host;
+    if (const int rc = locality_order(points, N, D, order_host, s, true)) return rc;
+    DeviceMem order, sorted;
+    if (!order.alloc_optional(sizeof(int) * (size_t)N) || !sorted.alloc_optional(sizeof(float) * (size_t)N * D))
+        return kNoRoom;
+    TSNE_TRY(hipMemcpyAsync(order.p, order_host.data(), sizeof(int) * (size_t)N, hipMemcpyHostToDevice, s));
+    if (launch_gather_rows(points, order.as<int>(), N, D, sorted.as<float>(), s)) return 1;
+    TSNE_TRY(hipStreamSynchronize(s));
+    const KnnRenumbered renumbered = {order.as<int>(), points};
+    return search(sorted.as<float>(), N, D, K, indices, sq_dist, s, 0, stats, nullptr, &renumbered);
+}
+
 // The matrix sweep skips candidate tiles whose ball lies out of reach, which needs close points to have close
 // numbers.  Points that come in no such order are searched in the locality order and the rows written in the
 // caller's: the same rows, because distances do not depend on the numbering and the re-rank orders equal ones by
 // the caller's.  (199999 x 30 in four clusters that come in turn, 33 neighbours: 27.2 -> 12.3 ms; on points
-// that already are in order the look at the numbering costs 0.05 ms.)
+// that already are in order the look at the numbering costs 0.05 ms.)  Only where that sweep will run, and where
+// there is room for a second copy of the points and the search beside it.
 int run_knn_any_order(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
                       int *stats) {
-    bool lacks = false;
     if (K > 1 && D > 0 && K <= N && N > kDirectPoints && locality_pivot_count(N) > 0 &&
-        numbering_lacks_locality(points, N, D, &lacks, s))
-        return 1;
-    // (without room for a second copy of the points, or for the search beside it: as they come)
-    if (DeviceMem order, sorted; lacks && order.alloc_optional(sizeof(int) * (size_t)N) &&
-                                 sorted.alloc_optional(sizeof(float) * (size_t)N * D)) {
-        std::vector<int> order_host;
-        if (locality_order(points, N, D, order_host, s)) return 1;
-        TSNE_TRY(hipMemcpyAsync(order.p, order_host.data(), sizeof(int) * (size_t)N, hipMemcpyHostToDevice, s));
-        if (launch_gather_rows(points, order.as<int>(), N, D, sorted.as<float>(), s)) return 1;
-        TSNE_TRY(hipStreamSynchronize(s));
-        const KnnRenumbered renumbered = {order.as<int>(), points};
-        if (!run_knn_mode(sorted.as<float>(), N, D, K, indices, sq_dist, s, 0, stats, nullptr, &renumbered)) return 0;
+        SweepGeometry(N, D, false).fits(candidates_kept(N, K))) {
+        bool lacks = false;
+        int rc = 0;
+        try {
+            rc = numbering_lacks_locality(points, N, D, &lacks, s);
+            if (!rc && lacks) {
+                rc = search_renumbered(points, N, D, K, indices, sq_dist, s, stats);
+                if (!rc) return 0;
+            }
+        } catch (const std::bad_alloc &) {  // (host memory for the order)
+            rc = kNoRoom;
+        }
+        if (rc && rc != kNoRoom) return rc;
+        if (rc) (void)hipGetLastError();  // (of the allocation that did not fit)
     }
-    (void)hipGetLastError();  // (of an allocation that did not fit)
-    return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, stats, nullptr, nullptr);
+    return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, stats);
 }
 
 }  // namespace tsnehip

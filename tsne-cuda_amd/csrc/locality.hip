@@ -100,7 +100,10 @@ __global__ void gather_rows_kernel(const float *__restrict__ src, const int *__r
 struct Scratch {
     void *p = nullptr;
     ~Scratch() { (void)hipFree(p); }
-    bool alloc(size_t bytes) { return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess; }
+    bool alloc(size_t bytes, bool optional) {
+        if (!bytes) bytes = 1;
+        return (optional ? malloc_optional(&p, bytes) : hipMalloc(&p, bytes)) == hipSuccess;
+    }
     template <typename T>
     T *as() { return static_cast<T *>(p); }
 };
@@ -117,7 +120,7 @@ int locality_pivot_count(int N) {
 }
 
 // order_host[new] = old.  Synchronises the stream.
-int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s) {
+int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s, bool optional) {
     order_host.resize(N);
     const int M = locality_pivot_count(N);
     if (M == 0) {
@@ -125,10 +128,10 @@ int locality_order(const float *points, int N, int D, std::vector<int> &order_ho
         return 0;
     }
     Scratch pivots_t, rows, labels;
-    if (!pivots_t.alloc(sizeof(float) * (size_t)M * D) || !rows.alloc(sizeof(float) * (size_t)M * D) ||
-        !labels.alloc(sizeof(int) * (size_t)N)) {
+    if (!pivots_t.alloc(sizeof(float) * (size_t)M * D, optional) || !rows.alloc(sizeof(float) * (size_t)M * D, optional) ||
+        !labels.alloc(sizeof(int) * (size_t)N, optional)) {
         set_error("locality_order: out of device memory");
-        return 1;
+        return kNoRoom;
     }
     // Pivots: a fixed pseudo-random draw (splitmix64 of the pivot number), so that no regular
     // pattern in the caller's numbering can line up with it; the draw is the same on every call.

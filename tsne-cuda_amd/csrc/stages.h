@@ -21,14 +21,8 @@ struct KnnProbes {
 };
 // probes != nullptr: only the matrix sweep's register-resident form can take it (error otherwise); queries whose
 // candidates fail the sweep's verification are then answered by the exact vector sweep over all points.
-// renumbered != nullptr: `points` are a renumbered copy (point i is the caller's order[i]) and the result is in
-// the caller's numbering.
-struct KnnRenumbered {
-    const int *order;            // device
-    const float *caller_points;  // device
-};
 int run_knn_mode(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
-                 int *stats, const KnnProbes *probes = nullptr, const KnnRenumbered *renumbered = nullptr);
+                 int *stats, const KnnProbes *probes = nullptr);
 // run_knn for points in any order: where the numbering has no locality, the search makes one for itself.
 int run_knn_any_order(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
                       int *stats);
@@ -45,9 +39,11 @@ int run_knn_ivf(const float *points, int N, int D, int K, const float *centroids
                 int *order_out, int *indices, float *sq_dist, int *stats, hipStream_t s);
 // `count` distinct pseudo-random indices below n, ascending (all of them when count >= n).
 std::vector<int> sample_indices(int n, int count, unsigned int seed);
-// Locality ordering (locality.hip): order_host[new] = old; synchronises the stream.
+// Locality ordering (locality.hip): order_host[new] = old; synchronises the stream.  kNoRoom: its memory was not
+// there (optional: memory that the caller can do without).
 int locality_pivot_count(int N);
-int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s);
+int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s,
+                   bool optional = false);
 int launch_gather_rows(const float *src, const int *order, int N, int D, float *dst, hipStream_t s);
 int launch_max_normalize(float *values, int64_t n, float *scratch, hipStream_t s);
 int launch_perplexity(const float *sq_dist, int N, int K, float perplexity, float eps, float *pij, float *betas,
