@@ -1355,6 +1355,24 @@ def test_knn_without_room_for_the_faster_form(stages, monkeypatch, n, d, k, orde
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+@pytest.mark.parametrize("row", ["pivot 0", "another pivot", "no pivot"])
+def test_knn_of_points_in_no_order_that_are_not_numbers(stages, row, value):
+    """Points that come in no order, one of them with a NaN or an infinity and outside the tiles that the numbering is
+    judged by: the rows are those of the sweep over the caller's numbering."""
+    n, d, k = 17002, 9, 20
+    rng = np.random.default_rng(3)
+    X = (rng.standard_normal((n, d)) + (6.0 * rng.standard_normal((5, d)))[np.arange(n) % 5]).astype(np.float32)
+    at = {"pivot 0": locality_pivot(0, n), "another pivot": locality_pivot(5, n), "no pivot": n - 3}[row]
+    assert at // 128 not in n // 128 // 64 * np.arange(64)
+    assert row != "no pivot" or at not in [locality_pivot(j, n) for j in range(64)]
+    X[at, 3] = value
+    idx, d2 = stages.knn(dev(X), k)
+    idx_s, d2_s, stats = stages.knn_select(dev(X), k, 2)
+    assert stats[0] == 1
+    assert torch.equal(idx, idx_s) and torch.equal(d2.view(torch.int32), d2_s.view(torch.int32))
+
+
 @pytest.mark.parametrize("limit", [0, 20000, 100000, 1 << 40])
 @pytest.mark.parametrize("k", [25, 1500])
 def test_knn_of_points_in_no_order_without_room(stages, monkeypatch, k, limit):

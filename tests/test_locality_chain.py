@@ -21,7 +21,8 @@ int main(int, char **argv) {
     if (std::fread(rows.data(), sizeof(float), rows.size(), stdin) != rows.size()) return 2;
     if (std::fread(labels.data(), sizeof(int), labels.size(), stdin) != labels.size()) return 2;
     const std::vector<int> place = tsnehip::chain_pivots(rows.data(), M, D);
-    tsnehip::order_by_place(labels.data(), N, place, order.data());
+    const bool all_near = tsnehip::order_by_place(labels.data(), N, place, order.data());
+    if (all_near != (*std::min_element(labels.begin(), labels.end()) >= 0)) return 3;
     std::fwrite(place.data(), sizeof(int), place.size(), stdout);
     std::fwrite(order.data(), sizeof(int), order.size(), stdout);
     return 0;
@@ -35,7 +36,7 @@ def chain(tmp_path_factory):
         pytest.skip("no host compiler")
     folder = tmp_path_factory.mktemp("chain")
     source, program = folder / "chain.cpp", folder / "chain"
-    source.write_text("#include <cstdlib>\n" + PROGRAM)
+    source.write_text("#include <algorithm>\n#include <cstdlib>\n" + PROGRAM)
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address", "-static-libasan", "-D_GLIBCXX_ASSERTIONS", "-I",
                     os.path.join(ROOT, "tsne-cuda_amd", "csrc"), str(source), "-o", str(program)], check=True)
 
@@ -79,3 +80,6 @@ def test_every_pivot_and_every_point_has_a_place(chain, bad, value):
     assert np.array_equal(place, greedy(rows))
     assert np.array_equal(np.sort(place), np.arange(64))
     assert np.array_equal(order, np.argsort(place[labels], kind="stable"))
+    labels[[17, 999]] = -1  # points at no finite distance from a pivot go with pivot 0
+    place, order = chain(rows, labels)
+    assert np.array_equal(order, np.argsort(place[np.maximum(labels, 0)], kind="stable"))

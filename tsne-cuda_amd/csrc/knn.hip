@@ -2664,11 +2664,15 @@ static int numbering_lacks_locality(const float *points, int N, int D, bool *lac
     return 0;
 }
 
-// run_knn_any_order on a renumbered copy of the points (kNoRoom: nothing done).
+// run_knn_any_order on a renumbered copy of the points, unless they are searched as they come (*searched false).
 static int search_renumbered(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
-                             int *stats) {
+                             int *stats, bool *searched) {
     std::vector<int> order_host;
-    if (const int rc = locality_order(points, N, D, order_host, s, true)) return rc;
+    bool all_near = true;
+    if (const int rc = locality_order(points, N, D, order_host, s, true, &all_near)) return rc;
+    // The tile of a point that is not made of numbers has no centre, and the sweep loses the other points of that tile:
+    // the caller's numbering decides which those are.
+    if (!all_near) return 0;
     DeviceMem order, sorted;
     if (!order.alloc_optional(sizeof(int) * (size_t)N) || !sorted.alloc_optional(sizeof(float) * (size_t)N * D))
         return kNoRoom;
@@ -2676,6 +2680,7 @@ static int search_renumbered(const float *points, int N, int D, int K, int *indi
     if (launch_gather_rows(points, order.as<int>(), N, D, sorted.as<float>(), s)) return 1;
     TSNE_TRY(hipStreamSynchronize(s));
     const KnnRenumbered renumbered = {order.as<int>(), points};
+    *searched = true;
     return search(sorted.as<float>(), N, D, K, indices, sq_dist, s, 0, stats, nullptr, &renumbered);
 }
 
@@ -2689,13 +2694,13 @@ int run_knn_any_order(const float *points, int N, int D, int K, int *indices, fl
                       int *stats) {
     if (K > 1 && D > 0 && K <= N && N > kDirectPoints && locality_pivot_count(N) > 0 &&
         SweepGeometry(N, D, false).fits(candidates_kept(N, K))) {
-        bool lacks = false;
+        bool lacks = false, searched = false;
         int rc = 0;
         try {
             rc = numbering_lacks_locality(points, N, D, &lacks, s);
             if (!rc && lacks) {
-                rc = search_renumbered(points, N, D, K, indices, sq_dist, s, stats);
-                if (!rc) return 0;
+                rc = search_renumbered(points, N, D, K, indices, sq_dist, s, stats, &searched);
+                if (!rc && searched) return 0;
             }
         } catch (const std::bad_alloc &) {  // (host memory for the order)
             rc = kNoRoom;

@@ -43,7 +43,7 @@ __global__ void gather_pivots_kernel(const float *__restrict__ points, int D, in
     rows[t] = v;
 }
 
-// One wave labels one point at a time; lane l holds pivots l, l + 64, ...
+// One wave labels one point at a time; lane l holds pivots l, l + 64, ...  -1: no pivot at a finite distance.
 template <int PER_LANE>
 __global__ __launch_bounds__(kAssignThreads) void pivot_assign_kernel(const float *__restrict__ points, int N,
                                                                       int D, int M,
@@ -85,7 +85,7 @@ __global__ __launch_bounds__(kAssignThreads) void pivot_assign_kernel(const floa
                 best_j = oj;
             }
         }
-        if (lane == 0) labels[i] = best_j;
+        if (lane == 0) labels[i] = best < INFINITY ? best_j : -1;
     }
 }
 
@@ -120,7 +120,9 @@ int locality_pivot_count(int N) {
 }
 
 // order_host[new] = old.  Synchronises the stream.
-int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s, bool optional) {
+int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s, bool optional,
+                   bool *all_near) {
+    if (all_near) *all_near = true;
     order_host.resize(N);
     const int M = locality_pivot_count(N);
     if (M == 0) {
@@ -161,7 +163,8 @@ int locality_order(const float *points, int N, int D, std::vector<int> &order_ho
     TSNE_TRY(hipMemcpyAsync(h_labels.data(), labels.p, sizeof(int) * (size_t)N, hipMemcpyDeviceToHost, s));
     TSNE_TRY(hipStreamSynchronize(s));
 
-    order_by_place(h_labels.data(), N, chain_pivots(h_rows.data(), M, D), order_host.data());
+    const bool near = order_by_place(h_labels.data(), N, chain_pivots(h_rows.data(), M, D), order_host.data());
+    if (all_near) *all_near = near;
     return 0;
 }
 

@@ -37,12 +37,18 @@ inline std::vector<int> chain_pivots(const float *rows, int M, int D) {
     return place;
 }
 
-// Stable counting sort of N points by the place of their pivot (labels: a pivot in [0, place.size()) per point).
-inline void order_by_place(const int *labels, int N, const std::vector<int> &place, int *order) {
+// Stable counting sort of N points by the place of their pivot (labels: a pivot in [0, place.size()) per point, or
+// negative: no pivot is at a finite distance, the point goes with pivot 0).  Whether no label is negative.
+inline bool order_by_place(const int *labels, int N, const std::vector<int> &place, int *order) {
     std::vector<int64_t> start(place.size() + 1, 0);
-    for (int i = 0; i < N; ++i) start[place[labels[i]] + 1] += 1;
+    bool all_near = true;
+    for (int i = 0; i < N; ++i) {
+        all_near = all_near && labels[i] >= 0;
+        start[place[labels[i] < 0 ? 0 : labels[i]] + 1] += 1;
+    }
     for (size_t c = 0; c < place.size(); ++c) start[c + 1] += start[c];
-    for (int i = 0; i < N; ++i) order[start[place[labels[i]]]++] = i;
+    for (int i = 0; i < N; ++i) order[start[place[labels[i] < 0 ? 0 : labels[i]]]++] = i;
+    return all_near;
 }
 
 }  // namespace tsnehip

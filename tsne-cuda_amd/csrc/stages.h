@@ -40,10 +40,11 @@ int run_knn_ivf(const float *points, int N, int D, int K, const float *centroids
 // `count` distinct pseudo-random indices below n, ascending (all of them when count >= n).
 std::vector<int> sample_indices(int n, int count, unsigned int seed);
 // Locality ordering (locality.hip): order_host[new] = old; synchronises the stream.  kNoRoom: its memory was not
-// there (optional: memory that the caller can do without).
+// there (optional: memory that the caller can do without).  all_near: whether every point is at a finite distance from
+// some pivot, which a point with a NaN or an infinity is not.
 int locality_pivot_count(int N);
 int locality_order(const float *points, int N, int D, std::vector<int> &order_host, hipStream_t s,
-                   bool optional = false);
+                   bool optional = false, bool *all_near = nullptr);
 int launch_gather_rows(const float *src, const int *order, int N, int D, float *dst, hipStream_t s);
 int launch_max_normalize(float *values, int64_t n, float *scratch, hipStream_t s);
 int launch_perplexity(const float *sq_dist, int N, int K, float perplexity, float eps, float *pij, float *betas,
