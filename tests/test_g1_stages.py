@@ -1388,7 +1388,7 @@ def test_knn_of_points_in_no_order_without_room(stages, monkeypatch, k, limit):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
-@pytest.mark.parametrize("n,k", [(1203, 32), (20011, 50)])
+@pytest.mark.parametrize("n,k", [(1203, 32), (20011, 50), (20011, 199), (20011, 200)])
 def test_loop_and_symmetrisation_without_room_for_the_faster_form(stages, monkeypatch, n, k):
     rng = np.random.default_rng(n)
     idx = (np.arange(n)[:, None] + np.sort(rng.permuted(np.tile(np.arange(1, 2 * k), (n, 1)), axis=1)[:, :k], axis=1)) % n

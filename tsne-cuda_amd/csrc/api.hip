@@ -194,8 +194,8 @@ int launch_step(tsne_hip_plan *p, const float *pij, const int *indices, float *e
     if (!overlap_active(p)) {
         // A small problem's step is its launches one after the other.  Its attractive forces ride along with the
         // inverse row pass, whose workgroups leave most of the chip idle (kernel alone, us: 1203 points x 32 neighbours
-        // 5.1 -> 0; 20011 x 50 8.3 -> 1.5; 50000 x 90 13.4 -> 12.8, the positions' cache lines), and the two kernels
-        // that group the points by tile are only launched every kGroupingInterval steps.
+        // 5.1 -> 0; 20011 x 50 8.3 -> 1.5; 50000 x 90 13.4 -> 12.8, the positions' cache lines; see forces_ride_along),
+        // and the two kernels that group the points by tile are only launched every kGroupingInterval steps.
         if (!pij && !p->csr_row_ptr && p->row_entries && !p->profiling && !p->profiling_attractive) {
             const SmallStep small = {p->attr, p->steps_to_grouping <= 0};
             p->steps_to_grouping = (small.may_group ? kGroupingInterval : p->steps_to_grouping) - 1;

@@ -1026,7 +1026,7 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
                                  hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBlockedLds));
     p->spin_limit = kSpinLimit;
     if (const char *v = std::getenv("TSNE_ATTRACTIVE_SPIN_LIMIT")) p->spin_limit = std::max(0, std::atoi(v));
-    if (N <= kSingleStreamPoints && K <= kRowEntriesNeighbors) {
+    if (forces_ride_along(N, K)) {
         if (malloc_optional(reinterpret_cast<void **>(&p->row_entries), sizeof(uint2) * (size_t)N * K) == hipSuccess) {
             row_entries_kernel<<<div_up((int64_t)N * K, 256), 256, 0, s>>>(pij, indices, (int64_t)N * K, p->row_entries);
             TSNE_LAUNCHED(s);

@@ -43,7 +43,15 @@ struct LagrangeMonomials {
 // and 50000 points 5 %, 3.5 % and 2.7 % shorter than with two streams and graphs, whose events cost 7-10 us per
 // step and whose instantiation 4 ms per stretch of constant parameters; at 100000 points two streams are 4 % ahead).
 constexpr int kSingleStreamPoints = 65536;
-constexpr int kRowEntriesNeighbors = 512;  // most neighbours the row-ordered copy of such a problem's pattern is made for
+// Of such a problem, whether the attractive forces ride along with the inverse row pass, for which the pattern is
+// copied row by row.  They read the other point's position from memory, entry by entry, where the attractive kernel has
+// it in LDS, so they save a launch and two of the grouping's (8 us) and lose by the number of entries.  us per step,
+// riding / the kernel by itself, neighbours of all numbers (of close ones it is ahead to twice as many entries):
+// 5000 x 400 68 / 70, x 512 72 / 71; 10000 x 300 68 / 71, x 400 73 / 72; 25000 x 150 74 / 75, x 200 80 / 76;
+// 40000 x 110 80 / 82, x 130 84 / 81; 50000 x 100 83 / 86, x 120 87 / 87; 65536 x 90 86 / 90, x 110 93 / 92, x 512 239 / 113.
+inline bool forces_ride_along(int N, int K) {
+    return N <= kSingleStreamPoints && K <= 512 && (int64_t)N * K <= 3000000 + 50 * (int64_t)N;
+}
 
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
