@@ -208,6 +208,18 @@ def test_symmetrize_table_sizes(stages, monkeypatch, n, k):
     assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
 
 
+@pytest.mark.parametrize("n,k", [(4096, 2), (5003, 6), (5003, 7), (200000, 5)])
+def test_symmetrize_tables_of_half_a_bucket(stages, monkeypatch, n, k):
+    """Up to six neighbours have tables of eight slots (the fullest of them, and one neighbour more): the scanning
+    form's values, bit for bit."""
+    i = torch.arange(n, device="cuda")[:, None]
+    idx = ((i + torch.arange(k, device="cuda") * torch.where(i % 3 == 0, 1, n // 2 + 1)) % n).int()
+    p = torch.rand(n, k, device="cuda")
+    got = stages.symmetrize(p, idx)
+    monkeypatch.setenv("TSNE_SYMMETRIZE_SCAN", "1")
+    assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
+
+
 @pytest.mark.parametrize("n,k", [(5000, 30), (530000, 102), (140000, 205)])
 def test_symmetrize_refuses_before_it_writes(stages, n, k):
     """Slots, and tags with places of either width: a column that names no point is an error that leaves the output as
