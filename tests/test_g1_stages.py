@@ -1367,6 +1367,23 @@ def test_knn_without_room_for_the_faster_form(stages, monkeypatch, n, d, k, orde
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("n,d,k", [(12288, 5, 12), (12289, 5, 12), (12289, 5, 13), (16384, 30, 13), (16384, 127, 12),
+                                   (11003, 21, 257)])
+def test_knn_at_the_lines_of_the_direct_search(stages, n, d, k):
+    """Either side of the lines between the direct search and the sweeps, over several blocks of rows, with equal
+    distances and a few points that are not numbers (the vector sweep orders both as the direct search does)."""
+    rng = np.random.default_rng(n + d + k)
+    X = np.round(3.0 * rng.standard_normal((n, d))).astype(np.float32)
+    idx, d2 = stages.knn(dev(X), k)
+    idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+    if n <= 11003:
+        X[[5, n - 1], 2] = np.nan, -np.inf
+        idx, d2 = stages.knn(dev(X), k)
+        idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+        assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("row", ["pivot 0", "another pivot", "no pivot"])
 def test_knn_of_points_in_no_order_that_are_not_numbers(stages, row, value):

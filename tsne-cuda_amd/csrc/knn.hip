@@ -2206,17 +2206,21 @@ int valu_cap(int K) {
     return cap;
 }
 
-// Direct search: distances and their selection, by blocks of query rows.  Measured (points in an order with
-// locality, ms, direct / sweep): 3000 x 64, 91 neighbours 0.13 / 3.9; 5000 x 50, 90: 0.21 / 4.9; 8000 x 126, 151:
-// 0.68 / 4.8; 8192 x 30, 45: 0.35 / 0.93; 12000 x 1024, 45: 6.3 / 18.4; 16384 x 126, 90: 2.1 / 2.6; 20000 x 32, 50:
-// 1.6 / 1.9; 20000 x 784, 45: 13.1 / 14.1; 32000 x 8, 30: 2.8 / 2.7; 32000 x 50, 90: 4.3 / 2.7.  It forms every pair,
-// where the matrix sweep skips tiles and multiplies on the matrix pipe: the line lies where the two are near each other.
-constexpr int kDirectPoints = 16384;
+// Direct search: distances and their selection, by blocks of query rows.  Measured, ms, direct / sweep, points in an
+// order with locality: 3000 x 64, 91 neighbours 0.13 / 3.9; 5000 x 50, 90: 0.21 / 4.9; 8000 x 126, 151: 0.68 / 4.8;
+// 8192 x 30, 45: 0.35 / 0.93; 16384 x 50, 33: 1.5 / 1.4; 16384 x 125, 90: 2.4 / 3.0; 20000 x 32, 50: 1.6 / 1.9;
+// 32000 x 8, 30: 2.8 / 2.7; 32000 x 50, 90: 4.3 / 2.7.  It forms every pair, where the matrix sweep skips tiles and
+// multiplies on the matrix pipe: the line lies where the two are near each other.  Beyond 126 dimensions the sweep's
+// time depends on how well its margin verifies, the direct form's does not: 14336 x 784, 33: clustered pixels 7.2 / 16,
+// no structure 7.1 / 6.0; 16384 x 1024, 33: 11.6 / 44 and 11.4 / 7.5.  A sweep for few neighbours keeps few candidates,
+// and the line lies lower: 12288 x 125, 2: 1.35 / 1.53; 16384 x 125, 2: 2.27 / 1.77; 16384 x 50, 10: 1.39 / 1.31.
+constexpr int kDirectPoints = 16384, kDirectPointsFew = 12288, kFewNeighbors = 12;
+inline bool direct_search_pays(int N, int K) { return N <= (K <= kFewNeighbors ? kDirectPointsFew : kDirectPoints); }
 constexpr int kDirectNeighbors = 256;  // most K - 1 that select_row_kernel<8> takes
-// Floats per block: 64 MiB are cheap to allocate (5000 x 50: 0.21 ms; 0.47 with the whole 100 MB at once), but
-// beyond 10240 points hold too few rows to fill the chip with their selection (16000 x 50: 1.6 ms with 64 MiB, 1.3
-// with 256).
-inline size_t direct_floats(int N) { return (size_t)1 << (N <= 10240 ? 24 : 26); }
+// Floats per block: 64 MiB, which the driver hands out again at once.  Calls that took 128 or 256 MiB (a third fewer
+// launches, none of it measurable: 12288 x 50, 33 neighbours 0.89 ms with either) waited for it to clear what the call
+// before had returned, at times: 11000 x 50, medians of 12 calls in a row 0.72 / 7.5 / 15.1 ms with 64 / 128 / 256 MiB.
+constexpr size_t kDirectFloats = (size_t)1 << 24;
 
 // (kNoRoom: nothing done, the sweeps need less memory)
 int run_direct_search(const float *points, int N, int D, int K, int cus, int *indices, float *sq_dist, hipStream_t s) {
@@ -2224,7 +2228,7 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
     // Tiles of 128 points a side where they fill the chip, of 64 otherwise.
     const bool large = (int64_t)(pitch / 128) * (pitch / 128) >= 2 * (int64_t)cus;
     const int side = large ? 128 : 64;
-    const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(direct_floats(N) / pitch) / 128 * 128));
+    const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(kDirectFloats / pitch) / 128 * 128));
     DeviceMem dist;
     if (!dist.alloc_optional(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
         (void)hipGetLastError();
@@ -2370,7 +2374,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         TSNE_TRY(hipGetLastError());
         return 0;
     };
-    if (mode == 0 && N <= kDirectPoints && K - 1 <= kDirectNeighbors) {
+    if (mode == 0 && direct_search_pays(N, K) && K - 1 <= kDirectNeighbors) {
         const int rc = run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
         if (rc != kNoRoom) return rc;
     }
