@@ -1348,9 +1348,10 @@ def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch):
     (1203, 20, 32, "cycle"),    # direct search / vector sweep
     (9001, 17, 60, "cycle"),    # direct search / matrix sweep
     (20011, 37, 25, "cycle"),   # renumbered / as the points come
-    (16901, 127, 20, "runs"),   # chunked sweep with the table of centre distances / without
-    (20483, 261, 33, "runs"),
-    (17000, 129, 30, "far")])   # ... where no margin verifies
+    (16901, 127, 20, "runs"),   # chunked sweep
+    (20483, 785, 33, "runs"),   # ... with the table of centre distances / without
+    (24573, 511, 20, "cycle"),  # ... renumbered / as the points come
+    (48600, 129, 30, "far")])   # ... where no margin verifies
 def test_knn_without_room_for_the_faster_form(stages, monkeypatch, n, d, k, order):
     """The same rows, bit for bit, with memory for the faster form of a search and without."""
     rng = np.random.default_rng(n)

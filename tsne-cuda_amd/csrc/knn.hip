@@ -2196,6 +2196,13 @@ struct SweepGeometry {
     size_t sweep_lds(int want) const { return lds_with(list_cap(want)); }
     bool fits(int want) const { return list_cap(want) <= 4096 && sweep_lds(want) <= 150 * 1024; }
 };
+// Chunked sweep: the table of centre distances takes a pass of N^2 D / 128 and saves one in the sweep, and its launches
+// and memory (the square of the points: 80 MB at 50000) cost 0.2 ms.  Calls in a row without / with it, clustered and
+// structureless points: 17000 x 127 0.96, 0.97; 30000 x 127 0.92, 0.95; 45000 x 127 0.94, 0.98; 24576 x 400 1.00, 1.03;
+// 30000 x 400 1.00, 1.04; 45000 x 250 0.98, 1.03; 60000 x 784 1.03, 1.09; 150000 x 256 1.02, 1.12; 180000 x 256 (1 GB)
+// 1.02, 1.06.
+inline bool centre_table_pays(int N, int D) { return (double)N * N * D >= 3e11; }
+constexpr size_t kMaxCentreTable = (size_t)1 << 30;
 constexpr int kMatrixPoints = 8192;  // fewer points: vector sweep
 // K' candidates kept per query.
 inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2)); }
@@ -2435,9 +2442,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         pack_chunked_centres_kernel<<<num_tiles, 64, 0, s>>>(centers.as<float>(), radius.as<float>(), D, n_chunks,
                                                             num_tiles, centres_p.as<float>(), tile_coef.as<float>());
         TSNE_TRY(hipGetLastError());
-        // The table grows with the square of the points (80 MB at 50000) and is made where it takes up to 1 GB.
         const size_t table_bytes = sizeof(float) * (size_t)num_tiles * Npad;
-        if (table_bytes <= (size_t)1 << 30 && centre_rows.alloc_optional(sizeof(float) * (size_t)num_tiles * D) &&
+        if (centre_table_pays(N, D) && table_bytes <= kMaxCentreTable && centre_rows.alloc_optional(sizeof(float) * (size_t)num_tiles * D) &&
             centre_dist.alloc_optional(table_bytes)) {
             transpose_points_kernel<<<dim3(div_up(D, 32), div_up(num_tiles, 32)), 256, 0, s>>>(
                 centers.as<float>(), D, num_tiles, D, centre_rows.as<float>());
