@@ -1403,6 +1403,27 @@ def test_knn_of_points_in_no_order_that_are_not_numbers(stages, row, value):
     assert torch.equal(idx, idx_s) and torch.equal(d2.view(torch.int32), d2_s.view(torch.int32))
 
 
+@pytest.mark.parametrize("n,d,kind,renumbered", [
+    (16500, 3, "cycle", True), (30000, 30, "cycle", True), (33000, 140, "cycle", True), (100000, 2, "blob", True),
+    (16500, 30, "blob", False), (60000, 30, "blob", False), (30000, 30, "runs", False), (33000, 140, "blob", False)])
+def test_knn_renumbers_where_it_pays(stages, n, d, kind, renumbered):
+    """Clusters that come in turn are renumbered, which lets the sweep skip tiles, and so is one cloud of many points in
+    few dimensions; clusters one after the other, and one cloud in many dimensions, are swept as they come (as many
+    tile pairs as the sweep of the caller's order computes).  The same rows either way."""
+    rng = np.random.default_rng(d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    if kind != "blob":
+        at = np.arange(n) % 5 if kind == "cycle" else np.arange(n) * 5 // n
+        X += (6.0 * rng.standard_normal((5, d)))[at].astype(np.float32)
+    idx, d2, stats = stages.knn_select(dev(X), 20, 0)
+    idx_s, d2_s, stats_s = stages.knn_select(dev(X), 20, 2)
+    assert torch.equal(idx, idx_s) and torch.equal(d2, d2_s)
+    if renumbered:
+        assert stats[2] < 0.8 * stats_s[2]
+    else:
+        assert stats[2] == stats_s[2]
+
+
 @pytest.mark.parametrize("limit", [0, 20000, 100000, 1 << 40])
 @pytest.mark.parametrize("k", [25, 1500])
 def test_knn_of_points_in_no_order_without_room(stages, monkeypatch, k, limit):

@@ -2053,15 +2053,18 @@ __global__ __launch_bounds__(256) void rename_list_kernel(const int *__restrict_
     if (i < count) list[i] = order[list[i]];
 }
 
-// How far the points of a sampled tile (128 consecutive points) lie from the tile's mean: out[0 .. D-1] the mean,
-// out[D] the mean squared distance to it.  One workgroup of 128 threads per sampled tile, `step` tiles apart.
+// How far the points of a sampled tile (128 consecutive points) lie from the tile's mean, and how far a point of it
+// from the nearest of the other tiles' (one per tile, at a place that no regular numbering lines up with).  Per tile
+// out[0 .. D-1] the mean, out[D] the mean squared distance to it, out[D+1] the smallest squared distance.  One workgroup
+// of 128 threads per sampled tile, at most 64 of them, `step` tiles apart.
 __global__ __launch_bounds__(128) void sample_tiles_kernel(const float *__restrict__ X, int D, int step,
                                                            float *__restrict__ out) {
-    __shared__ float part[128 / kWave];
-    const float *x = X + (size_t)blockIdx.x * step * kCT * D;
-    float *dst = out + (size_t)blockIdx.x * (D + 1);
+    __shared__ float part[128 / kWave], between[128];
+    const int tile = blockIdx.x, tid = threadIdx.x;
+    const float *x = X + (size_t)tile * step * kCT * D;
+    float *dst = out + (size_t)tile * (D + 2);
     float within = 0.0f;
-    for (int d = threadIdx.x; d < D; d += 128) {  // (a lane per dimension: neighbouring lanes read neighbouring words)
+    for (int d = tid; d < D; d += 128) {  // (a lane per dimension: neighbouring lanes read neighbouring words)
         float sum = 0.0f;
         for (int p = 0; p < kCT; ++p) sum += x[(size_t)p * D + d];
         const float mean = sum * (1.0f / kCT);
@@ -2072,9 +2075,27 @@ __global__ __launch_bounds__(128) void sample_tiles_kernel(const float *__restri
         }
     }
     within = group_sum<kWave>(within);
-    if ((threadIdx.x & (kWave - 1)) == 0) part[threadIdx.x / kWave] = within;
+    if ((tid & (kWave - 1)) == 0) part[tid / kWave] = within;
+    auto member = [&](int t) { return ((size_t)t * step * kCT + ((unsigned int)t * 0x9E3779B1u >> 25)) * D; };
+    // (two threads per other tile, half of the dimensions each)
+    const int other = tid & (kWave - 1), d0 = tid < kWave ? 0 : D / 2, d1 = tid < kWave ? D / 2 : D;
+    const bool counts = other < (int)gridDim.x && other != tile;
+    const float *mine = X + member(tile), *theirs = X + member(counts ? other : tile);
+    float dist = 0.0f;
+#pragma unroll 8
+    for (int d = d0; d < d1; ++d) {
+        const float off = mine[d] - theirs[d];
+        dist = fmaf(off, off, dist);
+    }
+    between[tid] = dist;
     __syncthreads();
-    if (threadIdx.x == 0) dst[D] = (part[0] + part[1]) * (1.0f / kCT);
+    if (tid < kWave) {
+        const float nearest = group_min<kWave>(counts ? between[tid] + between[tid + kWave] : INFINITY);
+        if (tid == 0) {
+            dst[D] = (part[0] + part[1]) * (1.0f / kCT);
+            dst[D + 1] = nearest;
+        }
+    }
 }
 
 struct DeviceMem {
@@ -2641,36 +2662,53 @@ int run_knn(const float *points, int N, int D, int K, int *indices, float *sq_di
     return run_knn_mode(points, N, D, K, indices, sq_dist, s, 0, nullptr);
 }
 
-// Whether consecutive points are no closer to each other than any points are: the mean squared distance of a
+// Whether the points come in no order and an order would let the sweep skip tiles.
+// No order: consecutive points are no closer to each other than any points are, by the mean squared distance of a
 // sampled tile's points to the tile's mean against that of all sampled points to theirs.
-static int numbering_lacks_locality(const float *points, int N, int D, bool *lacks, hipStream_t s) {
+// An order pays where points have others much closer to them than points are on average, which a sample shows too:
+// `near`, the squared distance to the nearest of 63 others over the spread, is 0.02 for well separated clusters, 0.1 to
+// 0.4 in few dimensions, 1 and more for one cloud in many, where no tile can be skipped whatever the order.  Time as
+// they come / renumbered, 33 neighbours, 2 to 120 dimensions, by `near` (the ordering costs 0.3 ms and the larger
+// copies, so that small searches need more of it):
+//   20000 points  < 0.2 0.94-1.25   0.2-0.5 0.94-1.21   > 0.5 0.78-1.17
+//   30000         < 0.2 1.04-1.38   0.2-0.5 0.99-1.21   > 0.5 0.84-1.22
+//   60000         < 0.2 1.18-1.63   0.2-0.5 1.08-1.34   > 0.5 0.93-1.25
+//   100000        < 0.2 1.27-4.08   0.2-0.5 1.23-1.76   0.5-1.3 0.99-1.68   > 1.3 0.93-0.98
+//   500000                          0.2-0.5 1.19-1.57   0.5-1.3 1.05-1.50
+// (clustered pixels below 28672 points: 127 and 250 dimensions 0.87-0.95 for 15 neighbours, 1.0-1.5 for 90; 400 to 1024
+// dimensions 1.1-3.6).
+static int renumbering_pays(const float *points, int N, int D, bool *pays, hipStream_t s) {
     const int tiles = N / kCT, sampled = std::min(tiles, 64);  // (whole tiles only)
     DeviceMem out;
-    *lacks = false;
+    *pays = false;
     if (sampled < 2) return 0;
-    if (!out.alloc_optional(sizeof(float) * (size_t)sampled * (D + 1))) {
+    if (!out.alloc_optional(sizeof(float) * (size_t)sampled * (D + 2))) {
         set_error("knn: out of device memory");
         return kNoRoom;
     }
     sample_tiles_kernel<<<sampled, 128, 0, s>>>(points, D, tiles / sampled, out.as<float>());
     TSNE_TRY(hipGetLastError());
-    std::vector<float> host((size_t)sampled * (D + 1));
+    std::vector<float> host((size_t)sampled * (D + 2));
     TSNE_TRY(hipMemcpyAsync(host.data(), out.p, sizeof(float) * host.size(), hipMemcpyDeviceToHost, s));
     TSNE_TRY(hipStreamSynchronize(s));
-    double within = 0.0, between = 0.0;
-    for (int t = 0; t < sampled; ++t) within += host[(size_t)t * (D + 1) + D];
+    double within = 0.0, between = 0.0, nearest = 0.0;
+    for (int t = 0; t < sampled; ++t) {
+        within += host[(size_t)t * (D + 2) + D];
+        nearest += host[(size_t)t * (D + 2) + D + 1];
+    }
     for (int d = 0; d < D; ++d) {
         double mean = 0.0, square = 0.0;
-        for (int t = 0; t < sampled; ++t) mean += host[(size_t)t * (D + 1) + d];
+        for (int t = 0; t < sampled; ++t) mean += host[(size_t)t * (D + 2) + d];
         mean /= sampled;
         for (int t = 0; t < sampled; ++t) {
-            const double off = host[(size_t)t * (D + 1) + d] - mean;
+            const double off = host[(size_t)t * (D + 2) + d] - mean;
             square += off * off;
         }
         between += square;
     }
     // In a numbering without locality the means of 128 points lie within 1/128 of the points' own spread.
-    *lacks = between < 0.1 * within;
+    const double near = N < 28672 ? 0.2 : N < 90112 ? 0.5 : 1.3;
+    *pays = between < 0.1 * within && nearest < near * within;
     return 0;
 }
 
@@ -2704,11 +2742,11 @@ int run_knn_any_order(const float *points, int N, int D, int K, int *indices, fl
                       int *stats) {
     if (K > 1 && D > 0 && K <= N && N > kDirectPoints && locality_pivot_count(N) > 0 &&
         SweepGeometry(N, D, false).fits(candidates_kept(N, K))) {
-        bool lacks = false, searched = false;
+        bool pays = false, searched = false;
         int rc = 0;
         try {
-            rc = numbering_lacks_locality(points, N, D, &lacks, s);
-            if (!rc && lacks) {
+            rc = renumbering_pays(points, N, D, &pays, s);
+            if (!rc && pays) {
                 rc = search_renumbered(points, N, D, K, indices, sq_dist, s, stats, &searched);
                 if (!rc && searched) return 0;
             }
