@@ -220,6 +220,24 @@ def test_symmetrize_tables_of_half_a_bucket(stages, monkeypatch, n, k):
     assert torch.equal(got.view(torch.int32), stages.symmetrize(p, idx).view(torch.int32))
 
 
+@pytest.mark.parametrize("k", [5, 40, 130])
+def test_symmetrize_scan_follows_no_column_out_of_range(stages, k):
+    """Fewer than 4096 points are not checked: an entry whose column names no point keeps its own value over 2N, and
+    the others are what they would be without it."""
+    n = 300
+    rng = np.random.default_rng(k)
+    idx = np.stack([rng.permutation(n)[:k] for _ in range(n)]).astype(np.int32)
+    p = rng.random((n, k)).astype(np.float32)
+    want = oracle.symmetrize(p, idx)
+    bad = idx.copy()
+    bad[7, 2], bad[250, k - 1] = n + 5, -3
+    i, j = idx[7, 2], idx[250, k - 1]
+    want[7, 2], want[250, k - 1] = p[7, 2] / (2 * n), p[250, k - 1] / (2 * n)
+    want[i][idx[i] == 7] = p[i][idx[i] == 7] / (2 * n)
+    want[j][idx[j] == 250] = p[j][idx[j] == 250] / (2 * n)
+    np.testing.assert_allclose(stages.symmetrize(dev(p), dev(bad)).cpu().numpy(), want, rtol=1e-6, atol=0)
+
+
 @pytest.mark.parametrize("n,k", [(5000, 30), (530000, 102), (140000, 205)])
 def test_symmetrize_refuses_before_it_writes(stages, n, k):
     """Slots, and tags with places of either width: a column that names no point is an error that leaves the output as

@@ -47,7 +47,8 @@ __global__ __launch_bounds__(256) void symmetrize_kernel(const float *__restrict
             const int j = __shfl(my_j, t, LANES);
             const size_t jb = (size_t)j * K;
             float found = 0.0f;
-            for (int u = lane; u < K; u += LANES)
+            // (a column that names no point has no row to scan)
+            for (int u = (unsigned int)j < (unsigned int)N ? lane : K; u < K; u += LANES)
                 if (idx[jb + u] == row) found += p[jb + u];
             found = group_sum<LANES>(found);
             if (lane == t) my_acc += found;
