@@ -48,7 +48,7 @@ int tsne_hip_knn(const float *points, int num_points, int num_dims, int num_neig
  * shape (what tsne_hip_knn does), 1 = vector-ALU sweep, 2 = matrix-instruction
  * (MFMA) candidate sweep followed by an exact re-rank and verification (up to
  * 126 dimensions the queries stay in registers; beyond, both operands stream in
- * chunks of 64 dimensions; except at 126 dimensions the candidate distances are
+ * chunks of 32 dimensions; except at 126 dimensions the candidate distances are
  * products of bf16 terms, two per coordinate, on the bf16 matrix pipe), 3 = as 2
  * with the candidate distances as products of floats throughout.  Results are
  * identical whichever sweep runs.  stats
@@ -134,7 +134,8 @@ int tsne_hip_perplexity(const float *sq_dist, int num_points, int num_neighbors,
 
 /* Pattern-restricted symmetrisation P[i,s] = (p[i,s] + sum_{t: idx[j,t]==i} p[j,t]) / 2N,
  * j = idx[i,s].  Replaces tsnecuda::util::SymmetrizeMatrixV2
- * (src/util/math_utils.cu:269-308). */
+ * (src/util/math_utils.cu:269-308).  From 4096 points on an index outside
+ * [0, num_points) is an error, and pij is then as it was. */
 int tsne_hip_symmetrize(const float *pij_non_symmetric, const int *indices, int num_points,
                         int num_neighbors, float *pij, void *stream);
 

@@ -1,4 +1,5 @@
-// The attractive force of one stored pair, and how such forces are summed, for every kernel that does so (gfx950).
+// The attractive force of one stored pair, and how forces over a prepared pattern are summed (gfx950).  The kernels that
+// hold an entry in several pieces (attractive.hip, attractive_blocked.hip) spell the force out: the same operations.
 #ifndef TSNE_HIP_PAIR_FORCE_H_
 #define TSNE_HIP_PAIR_FORCE_H_
 

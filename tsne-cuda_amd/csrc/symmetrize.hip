@@ -160,8 +160,8 @@ __device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
 // there unless one matches (50-dimensional Gaussians: one lookup in four finds its column); the match's place leads to
 // the row's own column and value.  Tags and places of a million rows of 90 neighbours are 256 MB where slots are 1 GB.
 // What that saves is not the kernels' time alone (lookups 2970 us in slots, 2340 in this form, 2580 with tags and
-// places in two arrays; 1547 with tags beside the slots, 1.15 GB) but the memory: a call that takes and returns over a gigabyte waits for the driver to clear what
-// the call before returned.  1,000,000 x 90, affinities called one after the other: 17.3 ms with tags beside the slots
+// places in two arrays; 1547 with tags beside the slots, 1.15 GB) but the memory: a call that takes and returns over a
+// gigabyte waits for the driver to clear what the call before returned.  1,000,000 x 90, affinities called one after the other: 17.3 ms with tags beside the slots
 // (4.6 for a single call), 8.4 with slots alone, 5.4 in this form.
 constexpr size_t kTaggedBytes = (size_t)512 << 20;  // slots of more bytes than this are replaced by tags and places
 template <bool TAGS, typename PLACE>
