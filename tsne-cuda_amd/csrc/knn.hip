@@ -2220,10 +2220,11 @@ struct SweepGeometry {
 // Chunked sweep: the table of centre distances takes a pass of N^2 D / 128 and saves one in the sweep, and its launches
 // and memory (the square of the points: 80 MB at 50000) cost 0.2 ms.  Calls in a row without / with it, clustered and
 // structureless points: 17000 x 127 0.96, 0.97; 30000 x 127 0.92, 0.95; 45000 x 127 0.94, 0.98; 24576 x 400 1.00, 1.03;
-// 30000 x 400 1.00, 1.04; 45000 x 250 0.98, 1.03; 60000 x 784 1.03, 1.09; 150000 x 256 1.02, 1.12; 180000 x 256 (1 GB)
-// 1.02, 1.06.
+// 30000 x 400 1.00, 1.04; 45000 x 250 0.98, 1.03; 60000 x 784 1.03, 1.09.  Larger tables gain as much (150000 x 256 1.02,
+// 1.12) but are memory that the driver clears between calls: with 200 to 313 MB (80000 and 100000 points) about one call
+// in a hundred took 0.1 to 1.3 s longer, none without a table or with up to 153 MB.
 inline bool centre_table_pays(int N, int D) { return (double)N * N * D >= 3e11; }
-constexpr size_t kMaxCentreTable = (size_t)1 << 30;
+constexpr size_t kMaxCentreTable = (size_t)128 << 20;  // (64896 points)
 constexpr int kMatrixPoints = 8192;  // fewer points: vector sweep
 // K' candidates kept per query.
 inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2)); }
