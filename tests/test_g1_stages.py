@@ -1480,3 +1480,32 @@ def test_loop_and_symmetrisation_without_room_for_the_faster_form(stages, monkey
     monkeypatch.setenv("TSNE_SCRATCH_LIMIT", "0")
     for a, b in zip(run(), want):
         assert same_bits(a, b)
+
+
+@pytest.mark.parametrize("n,d,k,kind", [
+    (16500, 5, 2, "plain"), (16513, 16, 20, "grid"), (17003, 17, 33, "clusters"), (17003, 64, 172, "plain"),
+    (17003, 65, 173, "plain"), (16640, 126, 129, "clusters"), (16500, 127, 20, "grid"), (16500, 192, 20, "clusters"),
+    (16500, 193, 33, "plain"), (20000, 30, 25, "far"), (20000, 30, 25, "one far point"), (98304, 12, 60, "grid"),
+    (98433, 8, 20, "plain"), (100003, 20, 90, "clumps"), (131200, 24, 33, "clusters"), (100003, 3, 45, "clumps")])
+def test_knn_on_halves(stages, n, d, k, kind):
+    """The search's own choice of sweep - on halves relative to frames, beyond four dimensions - gives the vector sweep's
+    rows, bit for bit: at the remainders of a step of 16 dimensions and of a chunk of 64, at the most neighbours the
+    register-resident form keeps, with whole rounds of query tiles and what is left of one (from 98304 points on, where
+    thresholds are set ahead of the lists), with equal distances, neighbours that lie forty to a tile, points far from
+    the origin and one point far from all others."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    if kind == "clusters":
+        X += (8.0 * rng.standard_normal((5, d)))[np.arange(n) * 5 // n].astype(np.float32)
+    elif kind == "grid":
+        X = np.round(2.0 * X).astype(np.float32)
+    elif kind == "clumps":
+        X = (X[np.arange(n) // 40] + 1e-2 * X).astype(np.float32)
+    elif kind == "far":
+        X += np.float32(300.0)
+    elif kind == "one far point":
+        X[7] = 1e9
+    idx, d2, stats = stages.knn_select(dev(X), k, 0)
+    assert stats[0] == 1
+    idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)

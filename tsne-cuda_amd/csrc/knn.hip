@@ -28,8 +28,14 @@
 //    >= tau - g for a rigorous rounding bound g, and the query passes when its
 //    K-th canonical distance is below that.  Queries that do not pass are redone
 //    by the VALU sweep, so the result is exact either way.
-//    Except at 126 dimensions the products run on the bf16 matrix pipe instead
-//    (v_mfma_f32_32x32x16_bf16, two bf16 terms per coordinate, three products):
+//    By default the products run on halves relative to a few frames that the
+//    tiles are spread over (v_mfma_f32_32x32x16_f16, one product;
+//    knn_half_sweep_kernel, and the chunked sweep below), with the distances less
+//    a rigorous bound of what that loses as keys.  Where that bound is much larger
+//    than the next one's, or more than a few queries fail because of it, and where
+//    a caller asks for that sweep, they run on the bf16 matrix pipe
+//    (v_mfma_f32_32x32x16_bf16, two bf16 terms per coordinate, three products;
+//    not at 126 dimensions):
 //    the candidates are stored relative to the centre m of their own 128-point
 //    tile, which keeps what the split leaves out small, |q - m|^2 is added on
 //    the vector ALU per (query, tile), and the keys are the distances less the
@@ -66,6 +72,10 @@ typedef unsigned long long u64;
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+
+// What the matrix sweeps multiply: floats, two bf16 terms per coordinate, or one half each (see half_pack_kernel).
+enum class Products { kFloats, kBf16, kHalf };
 
 constexpr int kQT = 64;   // VALU sweep: queries per workgroup
 constexpr int kCT = 128;  // candidates per tile (both sweeps)
@@ -88,10 +98,33 @@ __device__ __forceinline__ float min2(float a, float b) {
     asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
     return r;
 }
+__device__ __forceinline__ float max3(float a, float b, float c) {
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+__device__ __forceinline__ float max2(float a, float b) {
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// The smaller of three, or the larger (MAX).
+template <bool MAX>
+__device__ __forceinline__ float extreme3(float a, float b, float c) {
+    return MAX ? max3(a, b, c) : min3(a, b, c);
+}
+template <bool MAX>
+__device__ __forceinline__ float extreme2(float a, float b) {
+    return MAX ? max2(a, b) : min2(a, b);
+}
 __device__ __forceinline__ float matrix_result(float x) { return __builtin_canonicalizef(x); }
 
 __device__ __forceinline__ u64 pack_key(float d, int j) {
     return ((u64)float_to_ordered(d) << 32) | (unsigned int)j;
+}
+// ... of a distance that is not negative (or of -0).
+__device__ __forceinline__ u64 pack_key_positive(float d, int j) {
+    return ((u64)(__float_as_uint(d) | 0x80000000u) << 32) | (unsigned int)j;
 }
 __device__ __forceinline__ float key_distance(u64 key) { return ordered_to_float((unsigned int)(key >> 32)); }
 __device__ __forceinline__ int key_index(u64 key) { return (int)(unsigned int)(key & 0xffffffffu); }
@@ -544,6 +577,108 @@ __device__ __forceinline__ int wave_select(u64 *list, int want, int *cnt, u64 *t
     return want;
 }
 
+// Smallest (MIN) or largest of a value over the wave, in every lane, by DPP (see wave_inclusive_scan).
+template <bool MIN>
+__device__ __forceinline__ unsigned int wave_extreme(unsigned int v) {
+    constexpr unsigned int none = MIN ? ~0u : 0u;
+    auto step = [](unsigned int a, unsigned int b) { return MIN ? min(a, b) : max(a, b); };
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x111, 0xf, 0xf, false));
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x112, 0xf, 0xf, false));
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x114, 0xf, 0xf, false));
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x118, 0xf, 0xf, false));
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x142, 0xa, 0xf, false));
+    v = step(v, (unsigned int)__builtin_amdgcn_update_dpp((int)none, (int)v, 0x143, 0xc, 0xf, false));
+    return (unsigned int)__builtin_amdgcn_readlane((int)v, kWave - 1);
+}
+
+// wave_select over a list of at most 64 NK entries that the wave holds in registers (load_halves): the want-th smallest
+// distance is found by counting how many lie below a trial value (a ballot per register), trial values by interpolation
+// between the counts at either end and by halving in turn.  The list is two regions of `half` entries, c0 and n - c0 of
+// them in use; the entries kept go back alternately into the two (entry p to region p & 1, position p >> 1).  Keeps the
+// `want` smallest, or with slack > 0 any want .. want + slack smallest; lowers *thr to a value that everything kept is
+// within and everything dropped at or beyond.  Fewer than `want` entries: all kept, dealt out afresh.
+// counted: the rank is taken among the entries without kNotCounted; fewer than `want` of those: all entries kept.
+// (A wave's loads find what its stores before them wrote: nothing is waited for but the loads themselves.)
+constexpr u64 kNotCounted = 0x80000000ull;  // in a key's point number
+template <int NK>
+__device__ __forceinline__ void load_halves(const u64 *list, int half, int c0, int n, int lane, u64 (&key)[NK]) {
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        const int e = u * kWave + lane;
+        key[u] = ~0ull;
+        if (e < n) key[u] = list[e < c0 ? e : half + e - c0];
+    }
+}
+template <int NK>
+__device__ __forceinline__ int select_halves(u64 *list, int want, int slack, bool counted, int half, int n, u64 *thr,
+                                             int lane, const u64 (&key)[NK]) {
+    unsigned int rated[NK];  // distances, the largest number for an entry that is not counted
+    int ranked = 0;
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        rated[u] = counted && (key[u] & kNotCounted) ? ~0u : (unsigned int)(key[u] >> 32);
+        ranked += __popcll(__ballot(rated[u] != ~0u));
+    }
+    const u64 below = (1ull << lane) - 1ull;
+    unsigned int limit = ~0u;  // distances up to this are kept ...
+    int ties = INT_MAX;        // ... of those equal to it so many
+    if (ranked >= want) {
+        unsigned int lo = ~0u, hi = 0u;
+#pragma unroll
+        for (int u = 0; u < NK; ++u) {
+            lo = min(lo, rated[u]);
+            hi = max(hi, rated[u] == ~0u ? 0u : rated[u]);
+        }
+        lo = wave_extreme<true>(lo);
+        hi = wave_extreme<false>(hi);
+        // Fewer than `want` lie below or at `lo - 1` (at_lo of them), at least `want` at or below hi (at_hi of them).
+        unsigned int under = lo - 1u;
+        int at_under = 0, at_hi = ranked;
+        for (int round = 0; at_hi > want + slack && hi - under > 1u; ++round) {
+            const float share = (round & 1) ? 0.5f : (float)(want + slack / 2 - at_under) / (float)(at_hi - at_under);
+            const unsigned int span = hi - under;
+            unsigned int step = (unsigned int)((float)span * share);
+            step = min(max(step, 1u), span - 1u);
+            const unsigned int trial = __builtin_amdgcn_readfirstlane(under + step);
+            int c = 0;
+#pragma unroll
+            for (int u = 0; u < NK; ++u) c += __popcll(__ballot(rated[u] <= trial));
+            if (c >= want) {
+                hi = trial;
+                at_hi = c;
+            } else {
+                under = trial;
+                at_under = c;
+            }
+        }
+        limit = hi;
+        if (at_hi > want + slack && !counted) ties = want - at_under;  // (equal distances: as many of them as there is room for)
+        if (lane == 0) *thr = ((u64)limit << 32) | 0xffffffffull;
+    }
+    int base = 0, equal = 0;
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        const unsigned int bits = (unsigned int)(key[u] >> 32);
+        bool keep = u * kWave + lane < n && bits <= limit;
+        if (ties != INT_MAX) {
+            const u64 eq = __ballot(keep && bits == limit);
+            if (keep && bits == limit && equal + __popcll(eq & below) >= ties) keep = false;
+            equal += __popcll(eq);
+        }
+        const u64 m = __ballot(keep);
+        const int p = base + __popcll(m & below);
+        if (keep) list[(p & 1) * half + (p >> 1)] = key[u];
+        base += __popcll(m);
+    }
+    return base;
+}
+
+__device__ __forceinline__ int group_sum_int(int v) {
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1) v += __shfl_xor(v, m, kWave);
+    return v;
+}
+
 // Bounding ball of every tile of kCT consecutive points: the centre is the tile's mean, the
 // radius the largest distance of a member to it, inflated by 1e-3 (far more than the fp32
 // rounding of the sums) so that it is an upper bound.  centers_t is D x T (dimension-major).
@@ -918,16 +1053,17 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__rest
 // (K-1) of them where 64 S is 2 (K-1) and the order is random) go to LDS and are sorted.  If there are more than
 // LDS has room for, the (K-1)-th smallest of those that found room is a better bound for another reading; if it
 // is no better (many equal distances), the (K-1)-th smallest distance is found bit by bit and the entries equal
-// to it are taken by number.  Needs 2 (K-1) <= 64 S.
+// to it are taken by number.  Needs 2 (K-1) <= 64 S.  listed (optional): the point every row is of.
 template <int S>
 __global__ __launch_bounds__(256) void select_row_kernel(const float *__restrict__ dist, int N, int row0, int rows,
-                                                         int pitch, int K, int *__restrict__ out_idx,
-                                                         float *__restrict__ out_d) {
+                                                         int pitch, int K, const int *__restrict__ listed,
+                                                         int *__restrict__ out_idx, float *__restrict__ out_d) {
     constexpr int kRoom = 128 * S;
     __shared__ u64 keys_all[4][kRoom];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int r = blockIdx.x * 4 + wave, q = row0 + r, want = K - 1;
+    const int r = blockIdx.x * 4 + wave, want = K - 1;
     if (r >= rows) return;  // (no barrier below)
+    const int q = listed ? listed[r] : row0 + r;
     u64 *keys = keys_all[wave];
     const float *row = dist + (size_t)r * pitch;
     const float4 *row4 = reinterpret_cast<const float4 *>(row);
@@ -1035,6 +1171,240 @@ __global__ __launch_bounds__(256) void select_row_kernel(const float *__restrict
     }
 }
 
+// ---------------------------------------------------------------------------
+// Operands of the sweeps on halves.  Every tile belongs to one of kFrames frames (the nearest of as many points, see
+// frame_kernel), and a point x of a tile of frame c is kept as x' = x - c, one half per coordinate, for either side of
+// the products.  With f the query's frame and c the candidate's,
+//   |q - x|^2 = |q - c|^2 + beta_f(x) - 2 q'.x',   beta_f(x) = |x'|^2 - 2 (f - c).x':
+// |q - c|^2 = beta_c(q) + |f - c|^2 is a number per query while the frame lasts, beta a number per candidate that the
+// accumulator starts from, and nothing but the products depends on the pair.  One product per pair and coordinate
+// where two bf16 terms take three, and half the operand bytes; what it loses is bounded below.
+// ---------------------------------------------------------------------------
+constexpr int kFrames = 16, kSeedFrames = 8;
+
+// What the frames and the choice between the sweeps take from the tiles.
+struct HalfScale {
+    unsigned int reach;     // float bits: most a point lies from its frame (an upper bound)
+    int not_finite;         // tiles without a finite ball
+    float bound, bound_bf16;  // sums over the tiles of about what a distance within the tile may be off by, on either operand
+    float log_reach;        // sum over the tiles of log2 of the most a point of theirs lies from the frame
+    float pad[3];
+};
+
+// Frames first .. last - 1: distances of all tile centres to them, and every tile's nearest frame so far.  The first
+// kSeedFrames are centres of tiles spread evenly over the numbering (where points have an order, as densely as the
+// points lie), the others each the centre that lies farthest from all frames before it, which reaches the parts of the
+// points that the even spread missed.  best[f]: that centre, by the launch whose last frame is f.  The launch of the last
+// frame also fills `scale`.  64 threads per tile.
+constexpr int kFrameTiles = 16;
+__global__ __launch_bounds__(1024) void frame_kernel(const float *__restrict__ centers_t, const float *__restrict__ radius,
+                                                     int D, int T, int first, int last, u64 *best, int *frame_tile,
+                                                     float *__restrict__ nearest, int *__restrict__ tile_frame,
+                                                     HalfScale *scale) {
+    __shared__ float part[64][kFrameTiles];
+    const int l = threadIdx.x % kFrameTiles, slice = threadIdx.x / kFrameTiles;
+    const int t = blockIdx.x * kFrameTiles + l, tc = min(t, T - 1);
+    const int per = (D + 63) / 64, d0 = slice * per, d1 = min(d0 + per, D);
+    float near2 = INFINITY;
+    int frame = 0;
+    if (first > 0) {
+        near2 = nearest[tc];
+        frame = tile_frame[tc];
+    }
+    for (int f = first; f < last; ++f) {
+        const int seed = f < kSeedFrames ? (int)((2 * f + 1) * (long long)T / (2 * kSeedFrames))
+                                         : min((int)(unsigned int)(best[f - 1] & 0xffffffffu), T - 1);
+        if (blockIdx.x == 0 && threadIdx.x == 0) frame_tile[f] = seed;
+        float sum = 0.0f;
+#pragma unroll 8
+        for (int d = d0; d < d1; ++d) {
+            const float diff = centers_t[(size_t)d * T + tc] - centers_t[(size_t)d * T + seed];
+            sum = fmaf(diff, diff, sum);
+        }
+        part[slice][l] = sum;
+        __syncthreads();
+        if (slice == 0) {
+            float d2 = 0.0f;
+#pragma unroll
+            for (int k = 0; k < 64; ++k) d2 += part[k][l];
+            if (d2 < near2) {
+                near2 = d2;
+                frame = f;
+            }
+        }
+        __syncthreads();
+    }
+    float m2 = 0.0f;  // (of the launch of the last frame)
+    if (last == kFrames) {
+        float sum = 0.0f;
+#pragma unroll 8
+        for (int d = d0; d < d1; ++d) {
+            const float m = centers_t[(size_t)d * T + tc];
+            sum = fmaf(m, m, sum);
+        }
+        part[slice][l] = sum;
+        __syncthreads();
+        if (slice == 0)
+#pragma unroll
+            for (int k = 0; k < 64; ++k) m2 += part[k][l];
+    }
+    if (threadIdx.x >= kWave) return;
+    const bool mine = slice == 0 && t < T;  // (the other lanes of the wave take part in its sums with nothing)
+    if (mine) {
+        nearest[t] = near2;
+        tile_frame[t] = frame;
+    }
+    const bool finite = mine && near2 < INFINITY;
+    u64 far = finite ? ((u64)__float_as_uint(near2) << 32) | (unsigned int)t : 0ull;
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1) {
+        const u64 other = __shfl_xor(far, m, kWave);
+        far = far > other ? far : other;
+    }
+    if (threadIdx.x == 0) atomicMax(&best[last - 1], far);
+    if (last < kFrames) return;
+    const float r = radius[tc], mlen = sqrtf(m2), reach = (sqrtf(near2) * (1.0f + 1e-3f) + r) * (1.0f + 1e-3f);
+    const bool good = finite && reach < 1e18f && mlen < 1e18f;  // (its square is a float)
+    const float acc = 4.0f * (float)(3 * D + 6) * 5.9604644775390625e-08f;
+    const float b = good ? 4.0f / 4096.0f * reach * reach : 0.0f;
+    const float b16 = good ? (6.2f / 65536.0f + 2.0f * acc) * r * (mlen + r) + acc * (r * r + 2.0f * mlen * r) : 0.0f;
+    const float sl = group_sum<kWave>(good ? log2f(fmaxf(reach, 1e-30f)) : 0.0f);
+    const float sb = group_sum<kWave>(b), sb16 = group_sum<kWave>(b16), top = group_max<kWave>(good ? reach : 0.0f);
+    const int bad = __popcll(__ballot(mine && !good));
+    if (threadIdx.x == 0) {
+        atomicMax(&scale->reach, __float_as_uint(top));
+        if (bad) atomicAdd(&scale->not_finite, bad);
+        atomicAdd(&scale->bound, sb);
+        atomicAdd(&scale->bound_bf16, sb16);
+        atomicAdd(&scale->log_reach, sl);
+    }
+}
+
+// frames[d][f]: coordinate d of frame f (rows of kFrames floats), and |frame f - frame g|^2.  One workgroup.
+__global__ __launch_bounds__(1024) void frame_rows_kernel(const float *__restrict__ centers_t, int D, int T,
+                                                          const int *__restrict__ frame_tile, float *__restrict__ frames,
+                                                          float *__restrict__ frame_d2) {
+    constexpr int kDims = 512;  // at a time
+    __shared__ float rows[kDims * kFrames];
+    __shared__ float part[4][kFrames * kFrames];
+    const int tid = threadIdx.x, pair = tid & 255, quarter = tid >> 8;
+    static_assert(kFrames * kFrames == 256, "four threads per pair of frames");
+    float sum = 0.0f;
+    for (int first = 0; first < D; first += kDims) {
+        const int dims = min(kDims, D - first);
+        __syncthreads();
+        for (int e = tid; e < dims * kFrames; e += 1024) {
+            rows[e] = centers_t[(size_t)(first + e / kFrames) * T + frame_tile[e % kFrames]];
+            frames[(size_t)first * kFrames + e] = rows[e];
+        }
+        __syncthreads();
+        for (int d = quarter; d < dims; d += 4) {
+            const float diff = rows[d * kFrames + pair / kFrames] - rows[d * kFrames + pair % kFrames];
+            sum = fmaf(diff, diff, sum);
+        }
+    }
+    part[quarter][pair] = sum;
+    __syncthreads();
+    if (quarter == 0) frame_d2[pair] = (part[0][pair] + part[1][pair]) + (part[2][pair] + part[3][pair]);
+}
+
+// Halves are kept times a power of two that brings the largest distance from a frame to at most 2^14; what would be
+// a subnormal half is kept as zero, so it does not matter what the matrix unit makes of those.
+__device__ __forceinline__ float half_scale_factor(const HalfScale *scale) {
+    const float reach = fmaxf(__uint_as_float(scale->reach), 1e-30f);
+    return ldexpf(1.0f, min(max(13 - ilogbf(reach), -60), 60));
+}
+
+// One workgroup per tile.  Xh: [tile][block of 32 points (4)][step of 16 dimensions (S)][lane (64)] 8 halves, lane = 32 *
+// (dimension % 16 / 8) + point % 32, element = dimension % 8 (the layout of pack_points_bf16_kernel, one term).
+// beta: row f of `pitch` floats holds beta_f of every point.  point_len: |x'| and |x' - what the halves stand for|,
+// rounded up.  tile_info: the largest of the second and of |x'| among a tile's points, and the tile's frame.
+__global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict__ X, int N, int D, int S,
+                                                        const float *__restrict__ frames, const int *__restrict__ tile_frame,
+                                                        const HalfScale *scale, int pitch, uint4 *__restrict__ Xh,
+                                                        float *__restrict__ beta, float2 *__restrict__ point_len,
+                                                        float4 *__restrict__ tile_info) {
+    __shared__ float wave_eps[4], wave_len[4];
+    const int tile = blockIdx.x, tid = threadIdx.x, lane = tid & 63, block = tid >> 6;
+    const int i = tile * kCT + block * 32 + (lane & 31), h = lane >> 5;
+    const int own = tile_frame[tile];
+    const float s = half_scale_factor(scale), inv = 1.0f / s;
+    const float *x = X + (size_t)(i < N ? i : 0) * D;
+    float dot[kFrames], len = 0.0f, eps = 0.0f;
+#pragma unroll
+    for (int f = 0; f < kFrames; ++f) dot[f] = 0.0f;
+    uint4 *dst = Xh + ((size_t)tile * 4 + block) * S * 64 + lane;
+    for (int step = 0; step < S; ++step) {
+        const int d0 = 16 * step + 8 * h;
+        unsigned int bits[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            bits[j] = 0u;
+            if (i < N && d0 + j < D) {
+                const float *fr = frames + (size_t)(d0 + j) * kFrames;
+                const float c = fr[own], v = x[d0 + j] - c, w = v * s;
+                const _Float16 hv = fabsf(w) < 6.103515625e-05f ? (_Float16)0.0f : (_Float16)w;  // (2^-14)
+                const float lost = v - (float)hv * inv;
+                bits[j] = (unsigned int)__builtin_bit_cast(unsigned short, hv);
+                len = fmaf(v, v, len);
+                eps = fmaf(lost, lost, eps);
+#pragma unroll
+                for (int f = 0; f < kFrames; ++f) dot[f] = fmaf(fr[f] - c, v, dot[f]);
+            }
+        }
+        dst[step * 64] = make_uint4(bits[0] | (bits[1] << 16), bits[2] | (bits[3] << 16), bits[4] | (bits[5] << 16),
+                                    bits[6] | (bits[7] << 16));
+    }
+    len += __shfl_xor(len, 32, kWave);
+    eps += __shfl_xor(eps, 32, kWave);
+#pragma unroll
+    for (int f = 0; f < kFrames; ++f) {
+        const float other = dot[f] + __shfl_xor(dot[f], 32, kWave);
+        if ((f & 1) == h) beta[(size_t)f * pitch + i] = fmaf(-2.0f, other, len);
+    }
+    const float xl = sqrtf(len) * (1.0f + 1e-3f), xe = sqrtf(eps) * (1.0f + 1e-3f);
+    if (h == 0) point_len[i] = make_float2(xl, xe);
+    const float me = group_max<kWave>(xe), ml = group_max<kWave>(xl);
+    if (lane == 0) {
+        wave_eps[block] = me;
+        wave_len[block] = ml;
+    }
+    __syncthreads();
+    if (tid == 0)
+        tile_info[tile] = make_float4(fmaxf(fmaxf(wave_eps[0], wave_eps[1]), fmaxf(wave_eps[2], wave_eps[3])),
+                                      fmaxf(fmaxf(wave_len[0], wave_len[1]), fmaxf(wave_len[2], wave_len[3])),
+                                      __int_as_float(own), 0.0f);
+}
+
+// A query's side of the bound: what is subtracted from a distance of the sweep on halves to make it a lower bound.
+//  - q' and x' are kept as halves: |q'.x' - (their halves)| <= |q'| e_x + e_q (|x'| + e_x), e what the halves lose;
+//  - D products are accumulated in fp32 onto -beta / 2, in the matrix unit's order, and beta itself is a sum of D
+//    rounded terms: 5 (D + 8) 2^-24 (the factor covers that order) times the magnitudes, 2 |q'||x'| + |x'|^2 + 2 |f - c||x'|;
+//  - |q - c|^2 is a sum of D rounded terms too, (|q'| + |f - c|)^2 at most, taken in a known order: 1.25 (D + 8) 2^-24.
+struct HalfQuery {
+    float len, eps, kap;      // |q'|, what its halves lose, 5 (D + 8) 2^-24
+    float off, frame_len;     // lower bound of |q - c|^2, and |f - c|, of the candidate frame at hand
+    int frame;                // that frame (-1: none yet)
+};
+// (d2, frame_len: |f - c|^2, and |f - c| rounded up)
+__device__ __forceinline__ void enter_frame(HalfQuery &hq, int frame, float beta_q, float d2, float frame_len) {
+    hq.frame = frame;
+    hq.frame_len = frame_len;
+    const float reach = hq.len + hq.frame_len;
+    hq.off = beta_q + d2 - 0.25f * hq.kap * reach * reach;
+}
+// |q - c|^2 less the bound for a tile (its tile_info).
+__device__ __forceinline__ float tile_offset(const HalfQuery &hq, float tile_eps, float tile_len) {
+    const float split = hq.len * tile_eps + hq.eps * (tile_len + tile_eps);
+    const float sums = tile_len * (2.0f * hq.len + tile_len + 2.0f * hq.frame_len);
+    return hq.off - (2.02f * split + hq.kap * sums);
+}
+
+constexpr int kRankRounds = 3;
+// Memory that no kernel writes while this one runs: with a uniform address, loads on the scalar unit.
+typedef const __attribute__((address_space(4))) float ConstFloat;
+__device__ __forceinline__ ConstFloat *as_const(const void *p) { return (ConstFloat *)p; }
+
 struct SweepArgs {
     const float4 *Xp;
     const float *X;  // the points as given (bf16 sweep: the query side is formed from them)
@@ -1071,6 +1441,14 @@ struct SweepArgs {
     const unsigned int *probe_tile_lists;
     int probe_list_words, probe_nlist;
     const int *probe_list_tiles;
+    // Sweeps on halves (see half_pack_kernel).
+    const float *beta;
+    int beta_pitch;
+    const float2 *point_len;
+    const float4 *tile_info;
+    const float *frame_d2;
+    const HalfScale *half_scale;
+    int ranks[kRankRounds];  // see knn_half_sweep_kernel
 };
 
 // ---------------------------------------------------------------------------
@@ -1521,6 +1899,411 @@ __global__ __launch_bounds__(256, (sweep_occupancy<KSTEPS, BF16>())) void knn_mf
 }
 
 // ---------------------------------------------------------------------------
+// The sweep on halves, up to 126 dimensions (see half_pack_kernel).  Query tiles, visiting order, tile skipping, lists and
+// output are those of knn_mfma_sweep_kernel; the accumulators start from the candidates' betas and fall as the
+// distance grows, so what is looked for is the largest.
+//
+// What bounds the kernel is the latency of a wave's own chain (the products are a sixth of its time): runs of results
+// in which some lane passes, stores to the lists, selections over them, the barrier that ends a tile.  So: three waves
+// per SIMD, nothing of the tile loop in scratch memory (a wait for a spilled register is a wait for the next tile's loads
+// too: four waves of 128 registers took 115 ms where three of 168 take 92), no sort buffers (a selection holds the list
+// in registers), two LDS tiles and one barrier per tile, what a tile's bound takes fetched a tile ahead.
+// Whole searches, ms, on two bf16 terms / here: 1,000,000 x 50 in four clusters, 90 neighbours 163 / 91; 300000 x 50 without
+// structure 57 / 30; 300000 x 100, 45 neighbours 41 / 24; 199999 x 30, 33 neighbours 11.7 / 9.3; 300000 x 10, 30 neighbours
+// 21.8 / 19.9.
+//
+// Thresholds ahead of the lists.  A list's own threshold, the `want`-th best of what has been seen, lets 133 ln(N / n)
+// candidates of a query with 90 neighbours through (more, as it is only lowered when a list is full), ten times what is
+// wanted in the end, and each costs a store and a share of the selections.  So after the neighbourhood the tiles are
+// visited in four rounds, every 64th, 16th and 4th tile first: the r-th nearest point of a share p of the tiles is
+// farther than the wanted number of all of them unless r or more of those lie in that share, and ranks[] has the r for
+// which that does not happen (p wanted + 5.5 sqrt(p wanted) + 5: about 1e-8).  Neighbours may lie many to a tile, so at
+// most one entry per query, tile and lane counts, the first that passes: r entries are in r halves of tiles then, and
+// all tiles have r / p with one at least as near.  A query for which it happens all the same is left with too few
+// candidates, fails its verification and is searched again.
+//
+// Parts: as in the chunked sweep (no rounds: a part's threshold must be that of a list that lacks nothing).
+// Dynamic LDS: two candidate tiles, each
+//   a[cand block (4)][step (S)][lane (64)] 8 halves, 128 betas (times -s^2 / 2)
+// and the visit bitmap.
+// ---------------------------------------------------------------------------
+constexpr int kRoundTiles = 256;  // fewer tiles to visit after the neighbourhood: no rounds
+// Entries of a list, which a selection holds in registers (eight per lane; with sixteen the tile loop's own go to
+// memory: 20000 x 8, 300 neighbours 3.1 ms on bf16 terms, 3.8), and the most candidates kept of them.
+constexpr int kHalfCap = 512, kHalfWant = 256;
+// Workgroups per compute unit the register budget is set for.
+constexpr int half_sweep_occupancy(int steps) { return steps <= 5 ? 3 : 2; }
+constexpr int half_tile_float4(int steps) { return 256 * steps + kCT / 4; }
+template <int S>
+__global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_kernel(const SweepArgs args) {
+    constexpr int cap = kHalfCap, half = cap / 2, NK = cap / kWave;
+    const int N = args.N, D = args.D, want = args.want;
+    constexpr int kMain = 256 * S, kTile = half_tile_float4(S);
+    // Arguments of the code outside the tile loop, read where they are used: kept in registers from the start, they push
+    // those of the loop out.
+    typedef const __attribute__((address_space(4))) SweepArgs ConstArgs;
+    auto cold = []() {
+        ConstArgs *p = (ConstArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+        asm volatile("" : "+s"(p));
+        return p;
+    };
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
+    v4f *tiles = reinterpret_cast<v4f *>(lds_raw);
+    unsigned int *bitmap = reinterpret_cast<unsigned int *>(tiles + 2 * kTile);
+    __shared__ u64 thr[kMQ];
+    __shared__ int fill[256];  // entries in each lane's region of its query's list, around a selection
+    __shared__ float qcenter[128];
+    __shared__ float tmax_part[2];
+
+    const int tid = threadIdx.x;
+    const int wave = tid >> 6, lane = tid & 63;
+    const int qn = lane & 31, kh = lane >> 5;
+    u64 *list = args.lists + (size_t)blockIdx.x * kMQ * cap;
+    const float s = half_scale_factor(cold()->half_scale), s2 = 0.5f * s * s, back = -1.0f / s2;  // (powers of two)
+    const int T = (N + kCT - 1) / kCT, P = args.parts;
+
+    v4f stage[S], stage_more;
+    const float *tile_beta = nullptr;  // of the query tile's frame
+    auto fetch = [&](int tile) {
+        const v4f *src = reinterpret_cast<const v4f *>(args.Xp) + (size_t)tile * kMain + tid;
+#pragma unroll
+        for (int r = 0; r < S; ++r) stage[r] = src[r * 256];
+        if (tid < kCT / 4) stage_more = reinterpret_cast<const v4f *>(tile_beta + (size_t)tile * kCT)[tid];
+    };
+    auto stash = [&](int buf) {
+        v4f *dst = tiles + buf * kTile + tid;
+#pragma unroll
+        for (int r = 0; r < S; ++r) dst[r * 256] = stage[r];
+        if (tid < kCT / 4) dst[kMain] = stage_more * -s2;
+    };
+
+    for (int w = blockIdx.x; w < args.num_qtiles * P; w += gridDim.x) {
+        const int qi = w / P, part = w - qi * P;
+        const int qt = cold()->qtile_first + qi * cold()->qtile_step;
+        const int q0 = qt * kMQ;
+        const int q = q0 + wave * 32 + qn;  // this lane's query (>= N in the last tile: padded zeros)
+        const bool live = q < N;
+        if (tid < kMQ) thr[tid] = ~0ull;
+        // A query's list is two regions of cap / 2 entries, one per lane of the pair that shares the query; a lane
+        // appends at my_at, a byte offset into the workgroup's lists.
+        const unsigned int region = (unsigned int)(((wave * 32 + qn) * cap + kh * half) * (int)sizeof(u64));
+        unsigned int my_at = region;
+        float limit_d = INFINITY;  // the query's threshold
+        unsigned int not_counted = (unsigned int)kNotCounted;  // of the next entry of this lane
+        bool home = true;
+        auto my_fill = [&]() { return (int)((my_at - region) / (unsigned int)sizeof(u64)); };
+        // Selections over the lists of this wave's queries in `mask`, the next list on its way into registers meanwhile.
+        auto select_queries = [&](unsigned int mask, int rank, int slack, bool counted) {
+            fill[tid] = my_fill();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            auto counts = [&](int b, int &c0, int &n) {
+                c0 = __builtin_amdgcn_readfirstlane(fill[wave * 64 + b]);
+                n = c0 + __builtin_amdgcn_readfirstlane(fill[wave * 64 + b + 32]);
+            };
+            u64 next[NK];
+            int c0, n, next_n = 0;
+            auto load = [&](int b) {
+                counts(b, c0, next_n);
+                load_halves<NK>(list + (size_t)(wave * 32 + b) * cap, half, c0, next_n, lane, next);
+            };
+            if (mask) load(__ffs((int)mask) - 1);
+            while (mask) {
+                const int b = __ffs((int)mask) - 1;
+                mask &= mask - 1u;
+                u64 key[NK];
+#pragma unroll
+                for (int u = 0; u < NK; ++u) key[u] = next[u];
+                n = next_n;
+                if (mask) load(__ffs((int)mask) - 1);
+                const int ql = wave * 32 + b;
+                const int kept = select_halves<NK>(list + (size_t)ql * cap, rank, slack, counted, half, n, &thr[ql], lane, key);
+                if (lane == 0) {
+                    fill[wave * 64 + b] = (kept + 1) >> 1;
+                    fill[wave * 64 + b + 32] = kept >> 1;
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            my_at = region + (unsigned int)(fill[tid] * (int)sizeof(u64));
+            const u64 limit = thr[wave * 32 + qn];
+            // ~0 is "no threshold yet": its distance field does not decode to a number.
+            limit_d = limit == ~0ull ? INFINITY : key_distance(limit);
+        };
+        const int valid = min(max(N - (q0 + wave * 32), 0), 32);  // this wave's queries
+        const unsigned int all_queries = valid == 32 ? ~0u : (1u << valid) - 1u;
+
+        v8h bq[S];
+        HalfQuery hq;
+        {
+            const v4f *src = reinterpret_cast<const v4f *>(args.Xp) + (size_t)qt * kMain + (size_t)wave * S * 64 + lane;
+#pragma unroll
+            for (int k = 0; k < S; ++k) bq[k] = __builtin_bit_cast(v8h, src[k * 64]);
+        }
+        const float2 len = cold()->point_len[q];
+        hq = {len.x, len.y, 5.0f * (float)(D + 8) * 5.9604644775390625e-08f, 0.0f, 0.0f, -1};
+        const int own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(args.tile_info[qt].z));
+        tile_beta = args.beta + (size_t)own_frame * args.beta_pitch;
+
+        int buf = 0;
+        // What the bound of a tile takes, and the query's distance from its frame: fetched a tile ahead.
+        float2 info, next_info;
+        int next_frame = -1;
+        float next_beta = 0.0f;
+        const float *const query_beta = args.beta + q;
+        const float my_d2 = args.frame_d2[own_frame * kFrames + (lane & (kFrames - 1))];  // a frame per lane
+        const float my_frame_len = sqrtf(my_d2) * (1.0f + 1e-3f);
+        auto fetch_info = [&](int tile) {
+            const int t = __builtin_amdgcn_readfirstlane(tile);
+            ConstFloat *of_tile = as_const(args.tile_info) + 4 * (size_t)t;  // (scalar loads)
+            next_info = make_float2(of_tile[0], of_tile[1]);
+            next_frame = __float_as_int(of_tile[2]);
+        };
+        auto fetch_beta = [&]() { next_beta = query_beta[(size_t)next_frame * args.beta_pitch]; };
+        // One tile: compute it from LDS buffer `buf` while the next one travels through registers into the other.
+        auto process = [&](int ct, int next_ct) {
+            const int c0 = ct * kCT;
+            info = next_info;
+            if (next_frame != hq.frame)
+                enter_frame(hq, next_frame, next_beta, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_d2), next_frame)),
+                            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_frame_len), next_frame)));
+            if (next_ct >= 0) {
+                fetch(next_ct);
+                fetch_info(next_ct);
+            }
+            const v4f *tile = tiles + buf * kTile;
+            // Distance less its bound = off + product * back; what is tested is the product.  (Never -inf: excluded
+            // elements must fail also while the query has no threshold.)
+            not_counted = home ? (unsigned int)kNotCounted : 0u;
+            const float off = tile_offset(hq, info.x, info.y);
+            const float limit_acc = ((off - limit_d) - 4e-7f * (fabsf(off) + fabsf(limit_d))) * s2;
+            const float lim = live ? fmaxf(limit_acc, -3.4028234663852886e38f) : INFINITY;
+            const bool edge = c0 + kCT > N || (unsigned int)(q0 - c0) < (unsigned int)kCT;
+            auto multiply = [&](int cb, v16f &acc0, v16f &acc1) {
+                const v4f *b0 = tile + (size_t)cb * S * 64 + lane, *b1 = b0 + S * 64;
+                // (register v of the result is candidate 8 (v / 4) + 4 (lane / 32) + v % 4 of the block)
+                const v4f *start = tile + kMain + 8 * cb + kh;
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const v4f t0 = start[2 * g], t1 = start[8 + 2 * g];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        acc0[4 * g + k] = t0[k];
+                        acc1[4 * g + k] = t1[k];
+                    }
+                }
+                v4f next[2] = {b0[0], b1[0]};
+#pragma unroll
+                for (int k = 0; k < S; ++k) {
+                    const v8h x = __builtin_bit_cast(v8h, next[0]), y = __builtin_bit_cast(v8h, next[1]);
+                    if (k + 1 < S) {
+                        next[0] = b0[(k + 1) * 64];
+                        next[1] = b1[(k + 1) * 64];
+                    }
+                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, bq[k], acc0, 0, 0, 0);
+                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(y, bq[k], acc1, 0, 0, 0);
+                }
+            };
+            auto filter = [&](int cb, v16f &acc0, v16f &acc1) {
+                // The largest of each run of eight results: a run in which no lane of the wave passes is skipped.
+                float run_max[4];
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const v16f &a = g < 2 ? acc0 : acc1;
+                    const int o = 8 * (g & 1);
+                    float m = matrix_result(a[o + 7]);
+                    m = max3(m, a[o], a[o + 1]);
+                    m = max3(m, a[o + 2], a[o + 3]);
+                    m = max3(m, a[o + 4], a[o + 5]);
+                    run_max[g] = max2(m, a[o + 6]);
+                }
+                const int jbase = c0 + cb * 32 + 4 * kh;  // element (half, v) is candidate jbase + 32 half + 8 (v / 4) + v % 4
+                // Only the last tile has candidates beyond N and only the query's own tile holds the query.
+                if (edge) {
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        int j = jbase + 8 * (e >> 2) + (e & 3);
+                        asm volatile("" : "+v"(j));  // (one after the other: thirty comparisons at a time take every register)
+                        if (j >= N || j == q) acc0[e] = -INFINITY;
+                        if (j + 32 >= N || j + 32 == q) acc1[e] = -INFINITY;
+                    }
+                }
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    // (the maxima are from before the exclusions: upper bounds, which is all this needs)
+                    if (__ballot(run_max[g] >= lim) == 0) continue;
+                    // All eight comparisons first: a branch on a comparison just made waits for it.
+                    u64 any[8];
+#pragma unroll
+                    for (int v = 0; v < 8; ++v) any[v] = __ballot((g < 2 ? acc0 : acc1)[8 * (g & 1) + v] >= lim);
+#pragma unroll
+                    for (int v = 0; v < 8; ++v) {
+                        if (any[v] == 0) continue;
+                        asm volatile("");  // (a scalar branch, not a condition more for the lanes)
+                        const int e = 8 * (g & 1) + v;
+                        const float p = (g < 2 ? acc0 : acc1)[e];
+                        if (p >= lim) {
+                            int jb = jbase;
+                            asm volatile("" : "+v"(jb));  // the index is formed here, not held in 32 registers
+                            *reinterpret_cast<u64 *>(reinterpret_cast<char *>(list) + my_at) =
+                                pack_key_positive(fmaxf(fmaf(p, back, off), 0.0f),
+                                                  (int)((unsigned int)(jb + 32 * (g >> 1) + 8 * (e >> 2) + (e & 3)) | not_counted));
+                            my_at += (unsigned int)sizeof(u64);
+                            not_counted = (unsigned int)kNotCounted;
+                        }
+                    }
+                }
+            };
+            v16f acc0, acc1;
+            multiply(0, acc0, acc1);
+            if (next_ct >= 0) fetch_beta();
+            filter(0, acc0, acc1);
+            multiply(2, acc0, acc1);
+            if (next_ct >= 0) stash(buf ^ 1);  // (last read a tile ago, before the barrier that ended that tile)
+            filter(2, acc0, acc1);
+            __syncthreads();
+            if (next_ct >= 0) buf ^= 1;
+        };
+
+        // Phase 1: the query tile's neighbourhood; phase 2: the tiles the bitmap keeps.
+        const int reach = max(kHomeTiles / P, 2) * P;  // (at least two tiles either side of every part)
+        const int h0 = max(qt - reach, 0), h1 = min(qt + reach, T - 1);
+        int word_idx = -1;
+        unsigned int cur_word = 0u;
+        // Next set bit of the bitmap, ascending within a round; every wave walks the same words.  Round k takes the
+        // tiles that are `first` modulo 64, 16, 4 and 1, without those of the rounds before it.
+        int round = kRankRounds;
+        bool in_rounds = false;
+        const int first = (int)((unsigned int)qt * 0x9E3779B1u >> 26);
+        auto round_mask = [&](int k, int word) -> unsigned int {
+            return k < 0   ? 0u
+                   : k == 0 ? ((word & 1) == first >> 5 ? 1u << (first & 31) : 0u)
+                   : k == 1 ? 0x00010001u << (first & 15)
+                   : k == 2 ? 0x11111111u << (first & 3)
+                            : ~0u;
+        };
+        bool round_over = false;  // the tile returned last was the last of its round
+        auto next_tile = [&]() -> int {
+            for (;;) {
+                while (cur_word == 0u) {
+                    ++word_idx;
+                    if (word_idx >= args.bitmap_words) {
+                        if (round == kRankRounds) return -1;
+                        ++round;
+                        round_over = true;
+                        word_idx = -1;
+                        continue;
+                    }
+                    cur_word = bitmap[word_idx];
+                    if (in_rounds) cur_word &= round_mask(round, word_idx) & ~round_mask(round - 1, word_idx);
+                }
+                const int b = __ffs((int)cur_word) - 1;
+                cur_word &= cur_word - 1u;
+                return word_idx * 32 + b;
+            }
+        };
+        int cur = h0 + (part - h0 % P + P) % P;  // this part's first tile of the neighbourhood
+        if (cur > h1) cur = -1;  // fewer tiles than parts: nothing for this part, its lists stay empty
+        if (cur >= 0) {
+            fetch(cur);
+            fetch_info(cur);
+            fetch_beta();
+        }
+        __syncthreads();
+        if (cur >= 0) stash(0);
+        __syncthreads();
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): see below
+        unsigned int swept = 0;
+        for (bool done = false; !done; ) {
+            int nxt = -1;
+            round_over = false;
+            if (cur >= 0) {
+                ++swept;
+                nxt = home ? (cur + P <= h1 ? cur + P : -1) : next_tile();
+                process(cur, nxt);
+            }
+            const bool home_done = cur >= 0 && nxt < 0 && home && (h0 > 0 || h1 < T - 1);
+            done = nxt < 0 && !home_done;
+            // Lists that a further tile could overflow are compacted by their own wave, right away (a region takes at
+            // most 64 entries per tile); all of them after the neighbourhood, for thresholds, and at the end.
+            unsigned int mask = all_queries;
+            if (nxt >= 0 && !round_over) {
+                const u64 crowded = __ballot(my_fill() > half - kCT / 2);
+                mask = (unsigned int)(crowded | (crowded >> 32));  // lanes l, l+32 share a query
+            }
+            const bool rank = round_over && nxt >= 0;
+            if (mask) {
+                const int slack = cold()->select_slack;
+                select_queries(mask, rank ? cold()->ranks[round - 1] : want, rank || nxt < 0 ? 0 : slack, rank);
+            }
+            if (home_done) {
+                home = false;
+                for (int k = tid; k < args.bitmap_words; k += 256) bitmap[k] = 0u;
+                if (tid < args.D) qcenter[tid] = cold()->centers_t[(size_t)tid * T + qt];
+                __syncthreads();
+                if (tid < kMQ) {
+                    // Largest squared distance any query of the tile would still accept (rounded up).
+                    float v = -INFINITY;
+                    if (q0 + tid < N) {
+                        const u64 t = thr[tid];
+                        v = t == ~0ull ? INFINITY : key_distance(t);
+                        v += 1e-5f * fabsf(v) + 1e-30f;
+                    }
+                    v = group_max<kWave>(v);
+                    if (lane == 0) tmax_part[wave] = v;
+                }
+                __syncthreads();
+                const float tmax = fmaxf(tmax_part[0], tmax_part[1]);
+                const float *radius = cold()->radius, *centers_t = cold()->centers_t;
+                const float ra = radius[qt];
+                for (int t = tid; t < T; t += 256)
+                    if ((t < h0 || t > h1) && t % P == part && tile_may_matter(qcenter, ra, centers_t, radius, D, T, t, tmax))
+                        atomicOr(&bitmap[t >> 5], 1u << (t & 31));
+                __syncthreads();
+                int visits = 0;
+                for (int k = lane; k < args.bitmap_words; k += kWave) visits += __popc(bitmap[k]);
+                visits = __builtin_amdgcn_readfirstlane(group_sum_int(visits));
+                if (P == 1 && visits >= kRoundTiles) {
+                    in_rounds = true;
+                    round = 0;
+                }
+                nxt = next_tile();
+                round_over = false;
+                done = nxt < 0;
+                if (nxt >= 0) {
+                    fetch(nxt);
+                    fetch_info(nxt);
+                    fetch_beta();
+                    stash(buf);  // the barrier that ended the last tile freed both buffers
+                    __syncthreads();
+                }
+                // (nothing left in flight as far as the compiler can tell, as in the kernel above)
+                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+            }
+            cur = nxt;
+        }
+        if (tid == 0) atomicAdd(cold()->tiles_swept, (unsigned long long)swept);
+        // Output, every wave for its own queries.
+        for (int b = 0; b < valid; ++b) {
+            const int ql = wave * 32 + b;
+            const int n = fill[wave * 64 + b] + fill[wave * 64 + b + 32];
+            const u64 *lq = list + (size_t)ql * cap;  // entry e of the n kept: region e & 1, position e >> 1
+            const size_t row = (size_t)qt * kMQ + ql;
+            if (P == 1) {
+                for (int e = lane; e < want; e += kWave)
+                    cold()->cand[row * want + e] = e < n ? key_index(lq[(e & 1) * half + (e >> 1)] & ~kNotCounted) : -1;
+                // Every candidate that was dropped, by a compaction or by the filter, had a distance >= the
+                // threshold of the moment, and thresholds only decrease.
+                if (lane == 0) cold()->tau[row] = thr[ql] == ~0ull ? INFINITY : key_distance(thr[ql]);
+            } else {
+                u64 *dst = cold()->part_keys + (((size_t)qi * kMQ + ql) * P + part) * want;
+                for (int e = lane; e < want; e += kWave)
+                    dst[e] = e < n ? lq[(e & 1) * half + (e >> 1)] & ~kNotCounted : ~0ull;
+            }
+        }
+        __syncthreads();  // before the next query tile re-initialises thr and the LDS tiles
+    }
+}
+
+// ---------------------------------------------------------------------------
 // MFMA sweep for more dimensions than one wave's registers hold (more than 126).
 // The k-steps are cut into chunks of kChunkSteps (64 dimensions).  Per candidate tile and chunk the
 // workgroup keeps the chunk of the tile in LDS (32 KB, layout [block (4)][step group (8)][lane (64)]
@@ -1545,8 +2328,9 @@ constexpr int kChunkFloat4 = 4 * kChunkS4 * 64;      // float4 per tile chunk
 // forms it chunk by chunk from the query's own two terms and the centre's chunk, which is five vector instructions
 // per coordinate and 16 registers beside the matrix instructions (sweeps of 50000 x 1024: 27.5 -> 24.3 ms and 1.2 for
 // the table; 60000 x 784: 13.7 -> 11.9 and 1.1).
-template <bool BF16, bool TABLE>
+template <Products PRODUCTS, bool TABLE>
 __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const SweepArgs args) {
+    constexpr bool BF16 = PRODUCTS == Products::kBf16, HALF = PRODUCTS == Products::kHalf;
     const int N = args.N, D = args.D, want = args.want, cap = args.cap;
     const int num_qtiles = args.num_qtiles, n_chunks = args.n_chunks;
     u64 *__restrict__ lists = args.lists;
@@ -1555,12 +2339,13 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     // Slots of 16 bytes per lane, block and chunk: 8 groups of four k-steps (64 dimensions) on floats; on bf16
     // terms 2 terms x 2 steps of 16 dimensions (32 dimensions: with 64 the chunk loop's registers did not fit
     // and the compiler spilled the prefetched chunks the moment they were loaded).
-    constexpr int kSlots = BF16 ? 4 : kChunkS4;
+    // halves 4 steps of 16 dimensions (64): sweeps of 50000 x 1024 21.8 -> 11.9 ms, of 60000 x 784 9.2 -> 5.7.
+    constexpr int kSlots = BF16 || HALF ? 4 : kChunkS4;
     constexpr int kSteps16 = 2;                     // bf16: steps of 16 dimensions per chunk
     constexpr int kChunkF4 = 4 * kSlots * 64;       // float4 per tile chunk
     // bf16: two LDS buffers of 16 KB, so that the next chunk goes to LDS while the other waves may still read the
     // current one, and one workgroup barrier per chunk does (floats: one buffer of 32 KB, two barriers).
-    constexpr int kBufs = BF16 ? 2 : 1;
+    constexpr int kBufs = BF16 || HALF ? 2 : 1;
     int buf = 0;  // the buffer that holds the chunk being computed
     const size_t tile_stride = (size_t)n_chunks * kChunkF4;  // float4 per packed tile
     const size_t block_stride = (size_t)n_chunks * kSlots * 64;  // float4 per 32-point block of a tile
@@ -1573,11 +2358,17 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     __shared__ int cnt[kMQ];
     __shared__ unsigned int hist_all[4][kWave];
     __shared__ float tmax_part[2];
+    __shared__ v4f beta_lds[HALF ? 2 * (kCT / 4) : 1];  // halves: what the accumulators start from, by parity of the tile
 
     const int tid = threadIdx.x;
     const int wave = tid >> 6, lane = tid & 63;
     const int qn = lane & 31, kh = lane >> 5;
     u64 *list = lists + (size_t)blockIdx.x * kMQ * cap;
+    const float half_s = HALF ? half_scale_factor(args.half_scale) : 1.0f, half_s2 = 0.5f * half_s * half_s;
+    const float half_back = -1.0f / half_s2;  // (a power of two)
+    const float *tile_beta = nullptr;         // of the query tile's frame
+    v4f stage_beta;
+    int parity = 0;
 
     // Chunk c of a candidate tile: global -> registers -> LDS.  Element e = 256 r + tid of the chunk is
     // float4 (e % 512) of block e / 512 = r / 2.
@@ -1588,10 +2379,13 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
 #pragma unroll
         for (int r = 0; r < kSlots; ++r)
             stage[r] = src[(size_t)((256 * r) / (64 * kSlots)) * block_stride + (256 * r) % (64 * kSlots)];
+        if (HALF && c == 0 && tid < kCT / 4) stage_beta = reinterpret_cast<const v4f *>(tile_beta + (size_t)tile * kCT)[tid];
     };
-    auto stash = [&](int b) {
+    // (first: of a tile)
+    auto stash = [&](int b, bool first) {
 #pragma unroll
         for (int r = 0; r < kSlots; ++r) a_lds[b * kChunkF4 + r * 256 + tid] = stage[r];
+        if (HALF && first && tid < kCT / 4) beta_lds[(parity ^ 1) * (kCT / 4) + tid] = stage_beta * -half_s2;
     };
     const int num_ctiles = (N + kCT - 1) / kCT;
 
@@ -1606,6 +2400,16 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             cnt[tid] = 0;
         }
         const float q_len = BF16 && q < N ? sqrtf(args.norms[q]) * (1.0f + 1e-6f) : 0.0f;  // |q|, rounded up
+        HalfQuery hq = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, -1};
+        int own_frame = 0;
+        if constexpr (HALF) {
+            const float2 len = args.point_len[q];
+            hq.len = len.x;
+            hq.eps = len.y;
+            hq.kap = 5.0f * (float)(D + 8) * 5.9604644775390625e-08f;
+            own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(args.tile_info[qt].z));
+            tile_beta = args.beta + (size_t)own_frame * args.beta_pitch;
+        }
         // This wave's block of the query-side copy.
         const v4f *bsrc = reinterpret_cast<const v4f *>(args.Bp) + (size_t)qt * tile_stride + (size_t)wave * block_stride + lane;
         v4f bcur[kSlots], bnext[kSlots];
@@ -1620,7 +2424,12 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
 #pragma unroll
             for (int b = 0; b < 4; ++b)
 #pragma unroll
-                for (int e = 0; e < 16; ++e) acc[b][e] = 0.0f;
+                for (int g = 0; g < 4; ++g) {
+                    v4f start = {0.0f, 0.0f, 0.0f, 0.0f};
+                    if constexpr (HALF) start = beta_lds[parity * (kCT / 4) + 8 * b + 2 * g + kh];
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) acc[b][4 * g + k] = start[k];
+                }
             // bf16: this lane's share of |q - m|^2 (m: the tile's centre), or all of it from the table
             float f_part = 0.0f;
             if constexpr (TABLE) f_part = args.centre_dist[(size_t)ct * args.centre_pitch + q];
@@ -1642,7 +2451,18 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
 #pragma unroll
                     for (int s4 = 0; s4 < kSlots; ++s4) bnext[s4] = bn[s4 * 64];
                 }
-                if constexpr (BF16) {
+                if constexpr (HALF) {
+#pragma unroll
+                    for (int step = 0; step < kSlots; ++step) {
+                        v4f x[4];
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) x[b] = a_lds[buf * kChunkF4 + (b * kSlots + step) * 64 + lane];
+                        const v8h qh = __builtin_bit_cast(v8h, bcur[step]);
+#pragma unroll
+                        for (int b = 0; b < 4; ++b)
+                            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, x[b]), qh, acc[b], 0, 0, 0);
+                    }
+                } else if constexpr (BF16) {
 #pragma unroll
                     for (int step = 0; step < kSteps16; ++step) {
                         v4f xh[4], xl[4];
@@ -1691,13 +2511,13 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                     }
                 }
                 if (!last) {
-                    if constexpr (BF16) {
-                        stash(buf ^ 1);  // (last read a chunk ago, before the barrier that ended that chunk)
+                    if constexpr (BF16 || HALF) {
+                        stash(buf ^ 1, false);  // (last read a chunk ago, before the barrier that ended that chunk)
                         __syncthreads();
                         buf ^= 1;
                     } else {
                         __syncthreads();  // all waves have read this chunk
-                        stash(0);
+                        stash(0, false);
                         __syncthreads();
                     }
 #pragma unroll
@@ -1714,6 +2534,17 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             // (the rounding of its sum, and, formed from the query's two terms, the 2^-16 |q| by which they miss q)
             // less the tile's error bound; the products are tested against the threshold less `off`, rounded up.
             float off = 0.0f, limit_acc = limit_d;
+            if constexpr (HALF) {
+                // Distance less its bound = off - product / half_s2; what is tested is the product.
+                const float4 info = args.tile_info[__builtin_amdgcn_readfirstlane(ct)];
+                const int frame = __builtin_amdgcn_readfirstlane(__float_as_int(info.z));
+                if (frame != hq.frame) {
+                    const float d2 = args.frame_d2[own_frame * kFrames + frame];
+                    enter_frame(hq, frame, args.beta[(size_t)frame * args.beta_pitch + q], d2, sqrtf(d2) * (1.0f + 1e-3f));
+                }
+                off = tile_offset(hq, info.x, info.y);
+                limit_acc = ((off - limit_d) - 4e-7f * (fabsf(off) + fabsf(limit_d))) * half_s2;
+            }
             if constexpr (BF16) {
                 const float f = TABLE ? f_part : f_part + __shfl_xor(f_part, 32);
                 off = f * (1.0f - (float)(D + 4) * 5.9604644775390625e-08f);
@@ -1722,7 +2553,10 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 limit_acc = limit_d - off;
                 limit_acc += 2.4e-7f * (fabsf(limit_d) + fabsf(off));
             }
-            const float lim = q < N ? fminf(limit_acc, 3.4028234663852886e38f) : -INFINITY;
+            // (halves: the accumulators fall as the distance grows, and everything is the other way round)
+            auto passes = [](float v, float limit) { return HALF ? v >= limit : v <= limit; };
+            constexpr float kNever = HALF ? -INFINITY : INFINITY, kMost = 3.4028234663852886e38f;
+            const float lim = q < N ? (HALF ? fmaxf(limit_acc, -kMost) : fminf(limit_acc, kMost)) : -kNever;
             const bool edge_tile = c0 + kCT > N || (unsigned int)(q0 - c0) < (unsigned int)kCT;
 #pragma unroll
             for (int cb = 0; cb < 4; cb += 2) {
@@ -1730,26 +2564,26 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 // Register v of lane l holds candidate row 8*(v/4) + 4*(l/32) + v%4 of the block, query column l%32.
                 float best = matrix_result(acc0[0]);
 #pragma unroll
-                for (int v = 1; v + 1 < 16; v += 2) best = min3(best, acc0[v], acc0[v + 1]);
-                best = min3(best, acc0[15], matrix_result(acc1[0]));
+                for (int v = 1; v + 1 < 16; v += 2) best = extreme3<HALF>(best, acc0[v], acc0[v + 1]);
+                best = extreme3<HALF>(best, acc0[15], matrix_result(acc1[0]));
 #pragma unroll
-                for (int v = 1; v + 1 < 16; v += 2) best = min3(best, acc1[v], acc1[v + 1]);
-                best = min2(best, acc1[15]);
-                if (best <= limit_acc) {
+                for (int v = 1; v + 1 < 16; v += 2) best = extreme3<HALF>(best, acc1[v], acc1[v + 1]);
+                best = extreme2<HALF>(best, acc1[15]);
+                if (passes(best, limit_acc)) {
                     const int jbase = c0 + cb * 32 + 4 * kh;  // element (half, v) is candidate jbase + 32 half + 8 (v / 4) + v % 4
                     // Candidates beyond N (last tile) and the query itself (its own tile) are raised to +inf.
                     if (edge_tile) {
 #pragma unroll
                         for (int e = 0; e < 16; ++e) {
                             const int j = jbase + 8 * (e >> 2) + (e & 3);
-                            if (j >= N || j == q) acc0[e] = INFINITY;
-                            if (j + 32 >= N || j + 32 == q) acc1[e] = INFINITY;
+                            if (j >= N || j == q) acc0[e] = kNever;
+                            if (j + 32 >= N || j + 32 == q) acc1[e] = kNever;
                         }
                     }
                     // Count, reserve the list slots with one LDS atomic, then store the keys.
                     int n = 0;
 #pragma unroll
-                    for (int e = 0; e < 32; ++e) n += ((e < 16 ? acc0[e & 15] : acc1[e & 15]) <= lim) ? 1 : 0;
+                    for (int e = 0; e < 32; ++e) n += passes(e < 16 ? acc0[e & 15] : acc1[e & 15], lim) ? 1 : 0;
                     if (n != 0) {
                         const int slot = atomicAdd(&cnt[wave * 32 + qn], n);
                         u64 *dst = list + (size_t)(wave * 32 + qn) * cap + slot;
@@ -1758,8 +2592,10 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
 #pragma unroll
                         for (int e = 0; e < 32; ++e) {
                             const float dist = e < 16 ? acc0[e & 15] : acc1[e & 15];
-                            if (dist <= lim2)
-                                *dst++ = pack_key(BF16 ? dist + off : dist, jbase + 32 * (e >> 4) + 8 * ((e & 15) >> 2) + (e & 3));
+                            const int j = jbase + 32 * (e >> 4) + 8 * ((e & 15) >> 2) + (e & 3);
+                            if (passes(dist, lim2))
+                                *dst++ = HALF ? pack_key_positive(fmaxf(fmaf(dist, half_back, off), 0.0f), j)
+                                              : pack_key(BF16 ? dist + off : dist, j);
                         }
                     }
                 }
@@ -1774,14 +2610,17 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                                 args.select_slack);
                 }
             }
-            if constexpr (BF16) {
-                if (next_ct >= 0) stash(buf ^ 1);
+            if constexpr (BF16 || HALF) {
+                if (next_ct >= 0) stash(buf ^ 1, true);
                 __syncthreads();  // the next tile's first chunk is in LDS; all waves are done with this tile's last
-                if (next_ct >= 0) buf ^= 1;
+                if (next_ct >= 0) {
+                    buf ^= 1;
+                    parity ^= 1;
+                }
             } else {
                 __syncthreads();  // all waves are done with the tile's last chunk
                 if (next_ct >= 0) {
-                    stash(0);
+                    stash(0, true);
                     __syncthreads();
                 }
             }
@@ -1809,7 +2648,10 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
         if (cur >= 0) fetch(cur, 0);
         __syncthreads();  // the previous query tile's last reads of the LDS chunk
         buf = 0;
-        if (cur >= 0) stash(0);
+        if (cur >= 0) {
+            stash(0, true);
+            parity ^= 1;
+        }
         __syncthreads();
         bool home = true;
         unsigned int swept = 0;
@@ -1832,7 +2674,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                     float v = -INFINITY;
                     if (q0 + tid < N) {
                         const u64 t = thr[tid];
-                        v = t == ~0ull ? INFINITY : key_distance(t) + (BF16 ? 0.0f : args.norms[q0 + tid]);
+                        v = t == ~0ull ? INFINITY : key_distance(t) + (BF16 || HALF ? 0.0f : args.norms[q0 + tid]);
                         v += 1e-5f * fabsf(v) + 1e-30f;
                     }
                     v = group_max<kWave>(v);
@@ -1849,7 +2691,8 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 nxt = next_tile();
                 if (nxt >= 0) {
                     fetch(nxt, 0);
-                    stash(buf);  // the barrier that ended the last tile freed the LDS chunks
+                    stash(buf, true);  // the barrier that ended the last tile freed the LDS chunks
+                    parity ^= 1;
                     __syncthreads();
                 }
                 __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0), as in the kernel above
@@ -2126,42 +2969,43 @@ int next_pow2(int v) {
     return n;
 }
 
-template <int KSTEPS, bool BF16>
-int launch_mfma_sweep(const SweepArgs &args, int grid, hipStream_t s) {
-    constexpr int S4 = BF16 ? 2 * KSTEPS : (KSTEPS + 3) / 4;
-    // one tile (bf16: with its centre block) + a sort buffer per wave + the visit bitmap
-    const size_t lds = sizeof(float4) * (4 * S4 * 64 + (BF16 ? 64 : 0)) + sizeof(u64) * 4 * args.cap +
-                       sizeof(unsigned int) * args.bitmap_words;
-    TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(knn_mfma_sweep_kernel<KSTEPS, BF16>),
-                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    knn_mfma_sweep_kernel<KSTEPS, BF16><<<grid, 256, lds, s>>>(args);
+// lds: SweepGeometry::lds_with
+template <int KSTEPS, Products PRODUCTS>
+int launch_mfma_sweep(const SweepArgs &args, int grid, size_t lds, hipStream_t s) {
+    void (*sweep)(const SweepArgs) = nullptr;
+    if constexpr (PRODUCTS == Products::kHalf)
+        sweep = knn_half_sweep_kernel<KSTEPS>;
+    else
+        sweep = knn_mfma_sweep_kernel<KSTEPS, PRODUCTS == Products::kBf16>;
+    TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sweep), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    sweep<<<grid, 256, lds, s>>>(args);
     TSNE_TRY(hipGetLastError());
     return 0;
 }
 
-// Steps of 16 dimensions of the bf16 sweep: up to 125 dimensions + the three |c|^2 terms.
-int dispatch_bf16_sweep(int steps, const SweepArgs &args, int grid, hipStream_t s) {
+// Steps of 16 dimensions, of the bf16 sweep (up to 125 dimensions + the three |c|^2 terms) or the one on halves.
+template <Products P>
+int dispatch_steps16(int steps, const SweepArgs &args, int grid, size_t lds, hipStream_t s) {
     switch (steps) {
-        case 1: return launch_mfma_sweep<1, true>(args, grid, s);
-        case 2: return launch_mfma_sweep<2, true>(args, grid, s);
-        case 3: return launch_mfma_sweep<3, true>(args, grid, s);
-        case 4: return launch_mfma_sweep<4, true>(args, grid, s);
-        case 5: return launch_mfma_sweep<5, true>(args, grid, s);
-        case 6: return launch_mfma_sweep<6, true>(args, grid, s);
-        case 7: return launch_mfma_sweep<7, true>(args, grid, s);
-        case 8: return launch_mfma_sweep<8, true>(args, grid, s);
+        case 1: return launch_mfma_sweep<1, P>(args, grid, lds, s);
+        case 2: return launch_mfma_sweep<2, P>(args, grid, lds, s);
+        case 3: return launch_mfma_sweep<3, P>(args, grid, lds, s);
+        case 4: return launch_mfma_sweep<4, P>(args, grid, lds, s);
+        case 5: return launch_mfma_sweep<5, P>(args, grid, lds, s);
+        case 6: return launch_mfma_sweep<6, P>(args, grid, lds, s);
+        case 7: return launch_mfma_sweep<7, P>(args, grid, lds, s);
+        case 8: return launch_mfma_sweep<8, P>(args, grid, lds, s);
         default:
-            set_error("knn: no bf16 matrix-instruction sweep for %d steps", steps);
+            set_error("knn: no matrix-instruction sweep for %d steps of 16 dimensions", steps);
             return 1;
     }
 }
 
-
 // Instantiated step counts: every count up to 32 (62 dimensions), then multiples of 4.
-int dispatch_mfma_sweep(int ksteps, const SweepArgs &args, int grid, hipStream_t s) {
+int dispatch_mfma_sweep(int ksteps, const SweepArgs &args, int grid, size_t lds, hipStream_t s) {
 #define TSNE_MFMA_CASE(KS) \
     case KS:               \
-        return launch_mfma_sweep<KS, false>(args, grid, s);
+        return launch_mfma_sweep<KS, Products::kFloats>(args, grid, lds, s);
     switch (ksteps) {
         TSNE_MFMA_CASE(2) TSNE_MFMA_CASE(3) TSNE_MFMA_CASE(4) TSNE_MFMA_CASE(5) TSNE_MFMA_CASE(6)
         TSNE_MFMA_CASE(7) TSNE_MFMA_CASE(8) TSNE_MFMA_CASE(9) TSNE_MFMA_CASE(10) TSNE_MFMA_CASE(11)
@@ -2183,39 +3027,49 @@ struct SweepGeometry {
     int Dnorm;           // |x|^2 row: first even row after the real dimensions
     int ksteps;          // k-steps incl. the augmented pair
     bool chunked;        // more dimensions than one wave's registers hold
+    bool half;           // one half per coordinate
     bool bf16, bf16_chunked;
     int n_chunks, steps16, num_tiles, bitmap_words;
+    int slots;           // 16-byte slots per lane and block of the packed points
+    size_t tile_float4;  // float4 per packed tile
     size_t tile_lds;
 
-    // Unless force_f32 asks for products of floats, the sweeps multiply bf16 terms (two per coordinate) of the
-    // points relative to their tile's centre; three more dimensions carry a per-point term.
-    SweepGeometry(int N, int D, bool force_f32) {
+    // Two bf16 terms per coordinate are of the points relative to their tile's centre; three more dimensions carry a
+    // per-point term, and 126 dimensions, the most the register-resident sweep takes, are multiplied as floats.
+    SweepGeometry(int N, int D, Products products) {
         Dnorm = (D + 1) & ~1;
         ksteps = (Dnorm + 2) / 2;
         chunked = ksteps > kMfmaMaxSteps;
-        bf16 = !chunked && !force_f32 && D + 3 <= 128;
-        bf16_chunked = chunked && !force_f32;
-        n_chunks = chunked ? (bf16_chunked ? div_up(D + 3, 32) : div_up(ksteps, kChunkSteps)) : 0;
+        half = products == Products::kHalf;
+        bf16 = !chunked && products == Products::kBf16 && D + 3 <= 128;
+        bf16_chunked = chunked && products == Products::kBf16;
+        n_chunks = !chunked ? 0 : half ? div_up(D, 64) : bf16_chunked ? div_up(D + 3, 32) : div_up(ksteps, kChunkSteps);
         if (chunked) ksteps = n_chunks * (bf16_chunked ? kChunkSteps / 2 : kChunkSteps);  // (slots of 16 bytes per lane x 4)
         else if (ksteps > 32) ksteps = (ksteps + 3) & ~3;
-        steps16 = div_up(D + 3, 16);
+        steps16 = half ? div_up(D, 16) : div_up(D + 3, 16);
         num_tiles = div_up(N, kCT);
         bitmap_words = div_up(num_tiles, 32);
-        tile_lds = chunked ? sizeof(float4) * kChunkFloat4 + sizeof(float) * D  // (bf16: two chunks of half the size)
-                           : sizeof(float4) * (bf16 ? 512 * steps16 + 64 : 4 * ((ksteps + 3) / 4) * 64);
+        slots = half ? (chunked ? 4 * n_chunks : steps16) : bf16 ? 2 * steps16 : (ksteps + 3) / 4;
+        tile_float4 = (size_t)kCT * slots * 2 + (bf16 ? 64 : 0);
+        // (the chunked sweeps on halves and bf16 terms keep two chunks of half the size)
+        tile_lds = chunked ? sizeof(float4) * kChunkFloat4 + sizeof(float) * D
+                           : sizeof(float4) * (half ? 2 * (size_t)half_tile_float4(steps16) : tile_float4);
     }
     size_t lds_with(int cap) const {
-        return tile_lds + sizeof(u64) * 4 * cap + sizeof(unsigned int) * bitmap_words;
+        return tile_lds + (half && !chunked ? 0 : sizeof(u64) * 4 * cap) + sizeof(unsigned int) * bitmap_words;
     }
     // Room for the candidates kept, as many again and one more tile where the LDS sort buffers of that
     // size fit: a list that is nearly full right after a selection would be selected again after every tile.
     int list_cap(int want) const {
+        if (half && !chunked) return kHalfCap;
         int cap = next_pow2(2 * want + kCT);
         if (cap > 4096 || lds_with(cap) > 150 * 1024) cap = next_pow2(want + kCT);
         return cap < 256 ? 256 : cap;
     }
     size_t sweep_lds(int want) const { return lds_with(list_cap(want)); }
-    bool fits(int want) const { return list_cap(want) <= 4096 && sweep_lds(want) <= 150 * 1024; }
+    bool fits(int want) const {
+        return (half && !chunked ? want <= kHalfWant : list_cap(want) <= 4096) && sweep_lds(want) <= 150 * 1024;
+    }
 };
 // Chunked sweep: the table of centre distances takes a pass of N^2 D / 128 and saves one in the sweep, and its launches
 // and memory (the square of the points: 80 MB at 50000) cost 0.2 ms.  Calls in a row without / with it, clustered and
@@ -2272,13 +3126,38 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
             pair_distances_kernel<4><<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
         TSNE_TRY(hipGetLastError());
         if (2 * (K - 1) <= 64 * 4)
-            select_row_kernel<4><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, indices,
-                                                                 sq_dist);
+            select_row_kernel<4><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, nullptr,
+                                                                 indices, sq_dist);
         else
-            select_row_kernel<8><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, indices,
-                                                                 sq_dist);
+            select_row_kernel<8><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, nullptr,
+                                                                 indices, sq_dist);
         TSNE_TRY(hipGetLastError());
     }
+    TSNE_TRY(hipStreamSynchronize(s));
+    return 0;
+}
+
+// A few queries (device list) of a moderate number of points: as above, their rows gathered first.  The vector sweep takes a
+// transposed copy of the points and three more launches for them: searches of 20000 x 50 with two such queries 3.4 -> 2.3 ms,
+// of 60000 x 784 with 100 of them 15.0 -> 12.2.
+constexpr int kListedPoints = 131072;  // (a wave reads a row of distances twice)
+int run_listed_search(const float *points, int N, int D, int K, const int *list, int count, int *indices, float *sq_dist,
+                      hipStream_t s) {
+    const int pitch = div_up(N, 64) * 64;
+    if (N > kListedPoints || K - 1 > kDirectNeighbors || (size_t)count * pitch > kDirectFloats) return kNoRoom;
+    DeviceMem dist, queries;
+    if (!dist.alloc_optional(sizeof(float) * (size_t)count * pitch) ||
+        !queries.alloc_optional(sizeof(float) * (size_t)count * D)) {
+        (void)hipGetLastError();
+        return kNoRoom;
+    }
+    if (launch_gather_rows(points, list, count, D, queries.as<float>(), s)) return 1;
+    pair_distances_kernel<4><<<dim3(div_up(N, 64), div_up(count, 64)), 256, 0, s>>>(
+        queries.as<float>(), count, points, N, D, 0, count, pitch, dist.as<float>());
+    TSNE_TRY(hipGetLastError());
+    const auto select = 2 * (K - 1) <= 64 * 4 ? select_row_kernel<4> : select_row_kernel<8>;
+    select<<<div_up(count, 4), 256, 0, s>>>(dist.as<float>(), N, 0, count, pitch, K, list, indices, sq_dist);
+    TSNE_TRY(hipGetLastError());
     TSNE_TRY(hipStreamSynchronize(s));
     return 0;
 }
@@ -2329,10 +3208,81 @@ int run_valu_sweep(const float *points, const float *Xt, int N, int Npad, int D,
     return 0;
 }
 
+// Fewer dimensions: a step of 16 dimensions is mostly padding, tiles are small beside their frame, and bf16 terms
+// relative to the tile's own centre keep more.
+constexpr int kHalfDims = 5;
+constexpr float kPartCost = 0.02f;  // of a round, per part
+// Halves relative to the frames lose more than two bf16 terms relative to the tiles where the points have structure that
+// kFrames frames do not follow.  Times as much as the sweep is let to be off by beside the other: one cloud in many
+// dimensions has 5 to 9 and verifies as well, hundreds of tight clusters 40 and more.
+constexpr float kHalfLoss = 16.0f;
+
+// What the sweeps on halves take beside the points: made in three steps.
+struct HalfOperands {
+    DeviceMem small, beta, point_len, tile_info;
+    int dims = 0, tiles = 0;
+    // `small`: kFrames keys, the scale, kFrames tile numbers, the frames' distances, the frames, the tiles' distance
+    // to theirs and its number.
+    u64 *best() const { return small.as<u64>(); }
+    HalfScale *scale() const { return reinterpret_cast<HalfScale *>(best() + kFrames); }
+    int *frame_tile() const { return reinterpret_cast<int *>(scale() + 1); }
+    float *frame_d2() const { return reinterpret_cast<float *>(frame_tile() + kFrames); }
+    float *frame_rows() const { return frame_d2() + kFrames * kFrames; }
+    float *nearest() const { return frame_rows() + (size_t)dims * kFrames; }
+    int *tile_frame() const { return reinterpret_cast<int *>(nearest() + tiles); }
+    void release() {
+        small.release();
+        beta.release();
+        point_len.release();
+        tile_info.release();
+    }
+    // Frames of the tiles; *pays: whether the sweeps should multiply halves (false also where there is no room).
+    int frames(const float *centers_t, const float *radius, int D, int T, bool *pays, hipStream_t s) {
+        *pays = false;
+        dims = D;
+        tiles = T;
+        const size_t keys = sizeof(u64) * kFrames + sizeof(HalfScale);
+        if (!small.alloc_optional(keys + sizeof(int) * (kFrames + kFrames * kFrames + (size_t)D * kFrames + 2 * (size_t)T))) {
+            (void)hipGetLastError();
+            return 0;
+        }
+        TSNE_TRY(hipMemsetAsync(small.p, 0, keys, s));
+        for (int f = 0; f < kFrames; f = f == 0 ? kSeedFrames : f + 1) {
+            frame_kernel<<<div_up(T, kFrameTiles), 1024, 0, s>>>(centers_t, radius, D, T, f, f == 0 ? kSeedFrames : f + 1, best(),
+                                                        frame_tile(), nearest(), tile_frame(), scale());
+            TSNE_TRY(hipGetLastError());
+        }
+        HalfScale host;
+        TSNE_TRY(hipMemcpyAsync(&host, scale(), sizeof(host), hipMemcpyDeviceToHost, s));
+        TSNE_TRY(hipStreamSynchronize(s));
+        // (a point that is not a number takes its tile with it, and which points those are the other sweep decides too)
+        // ... and one scale serves all: beside a few tiles that reach 2^16 times as far as most, those lose bits.
+        float reach;
+        std::memcpy(&reach, &host.reach, sizeof(reach));
+        *pays = host.not_finite == 0 && host.bound <= kHalfLoss * host.bound_bf16 &&
+                std::log2(std::max(reach, 1e-30f)) <= host.log_reach / (float)T + 16.0f;
+        return 0;
+    }
+    bool room(int N, const SweepGeometry &g) {
+        const size_t Npad = (size_t)g.num_tiles * kCT;
+        return beta.alloc_optional(sizeof(float) * kFrames * Npad) && point_len.alloc_optional(sizeof(float2) * Npad) &&
+               tile_info.alloc_optional(sizeof(float4) * g.num_tiles);
+    }
+    int pack(const float *points, const float *centers_t, int N, int D, const SweepGeometry &g, uint4 *Xh, hipStream_t s) {
+        frame_rows_kernel<<<1, 1024, 0, s>>>(centers_t, D, g.num_tiles, frame_tile(), frame_rows(), frame_d2());
+        TSNE_TRY(hipGetLastError());
+        half_pack_kernel<<<g.num_tiles, 256, 0, s>>>(points, N, D, g.slots, frame_rows(), tile_frame(), scale(),
+                                                     g.num_tiles * kCT, Xh, beta.as<float>(), point_len.as<float2>(),
+                                                     tile_info.as<float4>());
+        TSNE_TRY(hipGetLastError());
+        return 0;
+    }
+};
+
 }  // namespace
 
-// mode: 0 = choose, 1 = VALU sweep only, 2 = matrix-instruction sweep (error if the shape does not fit),
-// 3 = as 2 with the products on floats where 2 multiplies bf16 terms (every dimension count but 126).
+// mode: 0 = choose, 1 = VALU sweep only, 2 = matrix-instruction sweep on bf16 terms (on floats at 126 dimensions; error
+// if the shape does not fit), 3 = as 2 on floats whatever the dimension count.
 // stats (optional, 3 ints): [0] = 1 if the matrix-instruction sweep ran, [1] = queries redone by the VALU sweep,
 // [2] = per mille of the (query tile, candidate tile) pairs the matrix sweep computed.
 // renumbered != nullptr: `points` are a renumbered copy (point i is the caller's order[i]) and the result is in
@@ -2342,7 +3292,7 @@ struct KnnRenumbered {
     const float *caller_points;  // device
 };
 static int search(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s, int mode,
-                  int *stats, const KnnProbes *probes, const KnnRenumbered *renumbered) {
+                  int *stats, const KnnProbes *probes, const KnnRenumbered *renumbered, bool halves = true) {
     if (stats) stats[0] = stats[1] = stats[2] = 0;
     if (N <= 0 || D <= 0 || K <= 0) {
         set_error("knn: num_points, num_dims and num_neighbors must be positive (got %d, %d, %d)", N, D, K);
@@ -2366,12 +3316,9 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     TSNE_TRY(hipGetDevice(&device));
     TSNE_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
 
-    const bool force_f32 = mode == 3;
+    SweepGeometry geometry(N, D, mode == 3 ? Products::kFloats : Products::kBf16);
     if (mode == 3) mode = 2;
-    const SweepGeometry geometry(N, D, force_f32);
-    const bool chunked = geometry.chunked, bf16 = geometry.bf16, bf16_chunked = geometry.bf16_chunked;
-    const int Dnorm = geometry.Dnorm, ksteps = geometry.ksteps, n_chunks = geometry.n_chunks;
-    const int steps16 = geometry.steps16, num_tiles = geometry.num_tiles, bitmap_words = geometry.bitmap_words;
+    const bool chunked = geometry.chunked;
     int want = candidates_kept(N, K);
     const bool mfma_fits = geometry.fits(want);
     bool use_mfma = mode == 2 || (mode == 0 && mfma_fits && N >= kMatrixPoints);
@@ -2412,33 +3359,54 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
     }
 
-    const int S4 = bf16 ? 2 * steps16 : (ksteps + 3) / 4;  // 16-byte slots per lane and block of the packed points
+    const int num_qtiles = div_up(N, kMQ), num_tiles = geometry.num_tiles;
     DeviceMem Xp, Bp, norms, scal, fail_list, centers, radius;
-    const int num_qtiles = div_up(N, kMQ);
-    const size_t tile_float4 = bf16 ? 512 * (size_t)steps16 + 64 : (size_t)kCT * S4 * 2;  // float4 per packed tile
-    if (!Xp.alloc(sizeof(float4) * tile_float4 * num_tiles) || !norms.alloc(sizeof(float) * Npad) ||
-        (chunked && !Bp.alloc(sizeof(float4) * (size_t)Npad * S4 * 2)) ||
-        !scal.alloc(4 * sizeof(int)) || !fail_list.alloc(sizeof(int) * N) ||
-        !centers.alloc(sizeof(float) * (size_t)D * num_tiles) || !radius.alloc(sizeof(float) * num_tiles)) {
-        set_error("knn: out of device memory for the candidate buffers");
+    auto no_room = [](const char *what) {
+        set_error("knn: out of device memory for the %s", what);
         return kNoRoom;
-    }
+    };
+    if (!scal.alloc(4 * sizeof(int)) || !fail_list.alloc(sizeof(int) * N) ||
+        !centers.alloc(sizeof(float) * (size_t)D * num_tiles) || !radius.alloc(sizeof(float) * num_tiles))
+        return no_room("candidate buffers");
     TSNE_TRY(hipMemsetAsync(scal.p, 0, 4 * sizeof(int), s));  // [0] max |x|^2 (float bits), [1] fail count, [2..3] tiles swept (64-bit)
-    norms_kernel<<<div_up(Npad, 256), 256, 0, s>>>(points, N, D, Npad, norms.as<float>(), scal.as<float>());
-    TSNE_TRY(hipGetLastError());
-    if (!bf16 && !bf16_chunked) {
-        pack_points_kernel<<<div_up((int64_t)Npad * S4 * 2, 256), 256, 0, s>>>(points, norms.as<float>(), N, D, Dnorm,
-                                                                              S4, Npad, Xp.as<float4>(), false);
-        TSNE_TRY(hipGetLastError());
-    }
-    if (chunked && !bf16_chunked) {
-        pack_points_kernel<<<div_up((int64_t)Npad * S4 * 2, 256), 256, 0, s>>>(points, norms.as<float>(), N, D, Dnorm,
-                                                                              S4, Npad, Bp.as<float4>(), true);
-        TSNE_TRY(hipGetLastError());
-    }
     tile_balls_kernel<<<num_tiles, 128, sizeof(float) * D, s>>>(points, N, D, num_tiles, centers.as<float>(),
                                                                radius.as<float>());
     TSNE_TRY(hipGetLastError());
+    HalfOperands operands;
+    if (mode == 0 && halves && !probes && D >= kHalfDims) {
+        const SweepGeometry on_halves(N, D, Products::kHalf);
+        bool pays = false;
+        if (on_halves.fits(want))
+            if (const int rc = operands.frames(centers.as<float>(), radius.as<float>(), D, num_tiles, &pays, s)) return rc;
+        if (pays && operands.room(N, on_halves) && Xp.alloc_optional(sizeof(float4) * on_halves.tile_float4 * num_tiles)) {
+            geometry = on_halves;
+            if (operands.pack(points, centers.as<float>(), N, D, geometry, Xp.as<uint4>(), s)) return 1;
+        } else {
+            operands.release();
+            (void)hipGetLastError();  // (of an allocation that did not fit)
+        }
+    }
+    const bool half = geometry.half, bf16 = geometry.bf16, bf16_chunked = geometry.bf16_chunked;
+    const int Dnorm = geometry.Dnorm, ksteps = geometry.ksteps, n_chunks = geometry.n_chunks;
+    const int steps16 = geometry.steps16, bitmap_words = geometry.bitmap_words;
+    const int S4 = geometry.slots;
+    if (!half) {
+        if (!Xp.alloc(sizeof(float4) * geometry.tile_float4 * num_tiles) || !norms.alloc(sizeof(float) * Npad) ||
+            (chunked && !Bp.alloc(sizeof(float4) * (size_t)Npad * S4 * 2)))
+            return no_room("candidate buffers");
+        norms_kernel<<<div_up(Npad, 256), 256, 0, s>>>(points, N, D, Npad, norms.as<float>(), scal.as<float>());
+        TSNE_TRY(hipGetLastError());
+    }
+    if (!half && !bf16 && !bf16_chunked) {
+        pack_points_kernel<<<div_up((int64_t)Npad * S4 * 2, 256), 256, 0, s>>>(points, norms.as<float>(), N, D, Dnorm,
+                                                                              S4, Npad, Xp.as<float4>(), false);
+        TSNE_TRY(hipGetLastError());
+        if (chunked) {
+            pack_points_kernel<<<div_up((int64_t)Npad * S4 * 2, 256), 256, 0, s>>>(
+                points, norms.as<float>(), N, D, Dnorm, S4, Npad, Bp.as<float4>(), true);
+            TSNE_TRY(hipGetLastError());
+        }
+    }
     if (bf16) {
         pack_points_bf16_kernel<<<div_up((int64_t)Npad * steps16 * 4, 256), 256, 0, s>>>(
             points, centers.as<float>(), N, D, steps16, num_tiles, Npad, Xp.as<uint4>());
@@ -2488,18 +3456,32 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         // of dimensions, and the tiles differ in how many candidate tiles they can skip: unless there are
         // several query tiles per workgroup slot to even that out, the chunked kernel splits every tile's
         // candidates over up to 8 workgroups.
-        const int slots = cus * (bf16 ? bf16_sweep_occupancy(steps16) : (!chunked && ksteps <= 28 ? 3 : 2));
+        const int slots = cus * (chunked ? 2
+                                 : half  ? half_sweep_occupancy(steps16)
+                                 : bf16  ? bf16_sweep_occupancy(steps16)
+                                         : (ksteps <= 28 ? 3 : 2));
         int parts = 1;
         if (chunked)
             while (parts < 8 && count * parts < 3 * slots && parts * 2 * keep <= 2048 && parts * 2 <= num_tiles)
                 parts *= 2;
-        const int grid = std::min(count * parts, slots);
+        // On halves below that the last round of the workgroups counts: what does not fill one is swept by several
+        // workgroups per tile, in a launch of its own.
+        const int whole = half && !chunked ? count / slots * slots : count, rest = count - whole;
+        // (Time in rounds; every part sweeps its own neighbourhood and keeps its own list, which costs some.)
+        int rest_parts = 1;
+        if (rest > 0) {
+            auto rounds = [&](int p) { return (float)div_up(rest * p, slots) / (float)p + kPartCost * (float)p; };
+            for (int p = 2; p <= 16 && p * keep <= 2048 && p * 2 * (2 * kHomeTiles + 1) <= num_tiles; p *= 2)
+                if (rounds(p) < rounds(rest_parts)) rest_parts = p;
+        }
+        const int grid = std::min(std::max(whole * parts, rest * rest_parts), slots);
         const size_t n_slots = (size_t)(tile_list || step != 1 ? count * kMQ : N);
+        const size_t merged_rows = parts > 1 ? n_slots : rest_parts > 1 ? n_slots - (size_t)whole * kMQ : 0;
         DeviceMem lists, cand, tau, part_keys;
         auto alloc_lists = [&]() -> bool {
             return lists.alloc(sizeof(u64) * (size_t)grid * kMQ * cap) && cand.alloc(sizeof(int) * n_slots * keep) &&
                    tau.alloc(sizeof(float) * n_slots) &&
-                   (parts == 1 || part_keys.alloc(sizeof(u64) * n_slots * parts * keep));
+                   (merged_rows == 0 || part_keys.alloc(sizeof(u64) * merged_rows * std::max(parts, rest_parts) * keep));
         };
         bool room = alloc_lists();
         if (!room && centre_dist.p) {
@@ -2535,7 +3517,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         args.trigger = cap - kCT;  // as late as possible: a later selection costs the same and sees more candidates
         args.select_slack = (cap - kCT - keep) / 4;
         args.tiles_swept = reinterpret_cast<unsigned long long *>(scal.as<int>() + 2);
-        args.Bp = Bp.as<float4>();
+        args.Bp = half ? Xp.as<float4>() : Bp.as<float4>();
         args.n_chunks = n_chunks;
         args.qtile_list = tile_list;
         args.qtile_first = first;
@@ -2546,26 +3528,49 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         args.probe_list_words = probes ? probes->list_words : 0;
         args.probe_nlist = probes ? probes->nlist : 0;
         args.probe_list_tiles = probes ? probes->list_tiles : nullptr;
+        args.beta = operands.beta.as<float>();
+        args.beta_pitch = Npad;
+        args.point_len = operands.point_len.as<float2>();
+        args.tile_info = operands.tile_info.as<float4>();
+        args.frame_d2 = operands.frame_d2();
+        args.half_scale = operands.scale();
+        for (int k = 0; k < kRankRounds; ++k) {
+            const double share = (double)(K - 1 + 16 + (K - 1) / 8) / (double)(64 >> (2 * k));
+            args.ranks[k] = (int)std::ceil(share + 5.5 * std::sqrt(share) + 5.0);
+        }
+        const size_t lds = geometry.lds_with(cap);
         if (chunked) {
-            const size_t lds = geometry.sweep_lds(keep);
-            const auto sweep = !bf16_chunked          ? knn_mfma_chunked_sweep_kernel<false, false>
-                               : args.centre_dist ? knn_mfma_chunked_sweep_kernel<true, true>
-                                                  : knn_mfma_chunked_sweep_kernel<true, false>;
+            const auto sweep = half               ? knn_mfma_chunked_sweep_kernel<Products::kHalf, false>
+                               : !bf16_chunked    ? knn_mfma_chunked_sweep_kernel<Products::kFloats, false>
+                               : args.centre_dist ? knn_mfma_chunked_sweep_kernel<Products::kBf16, true>
+                                                  : knn_mfma_chunked_sweep_kernel<Products::kBf16, false>;
             TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(sweep),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
             sweep<<<grid, 256, lds, s>>>(args);
             TSNE_TRY(hipGetLastError());
-        } else if (bf16 ? dispatch_bf16_sweep(steps16, args, grid, s) : dispatch_mfma_sweep(ksteps, args, grid, s)) {
+        } else if (half) {
+            if (whole > 0) {
+                args.num_qtiles = whole;
+                if (dispatch_steps16<Products::kHalf>(steps16, args, std::min(whole, slots), lds, s)) return 1;
+            }
+            if (rest > 0) {
+                args.num_qtiles = rest;
+                args.qtile_first = first + whole * step;
+                args.parts = rest_parts;
+                if (dispatch_steps16<Products::kHalf>(steps16, args, std::min(rest * rest_parts, slots), lds, s)) return 1;
+            }
+        } else if (bf16 ? dispatch_steps16<Products::kBf16>(steps16, args, grid, lds, s)
+                        : dispatch_mfma_sweep(ksteps, args, grid, lds, s)) {
             return 1;
         }
-        if (parts > 1) {
+        if (merged_rows > 0) {
             // rows of a partial last tile are merged too: the sweep left them unwritten, the re-rank skips them
-            const size_t lds = sizeof(u64) * 4 * parts * keep;
+            const int merged = std::max(parts, rest_parts);
+            const size_t lds = sizeof(u64) * 4 * merged * keep, done = n_slots - merged_rows;
             TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(knn_merge_parts_kernel),
                                          hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-            knn_merge_parts_kernel<<<div_up((int)n_slots, 4), 256, lds, s>>>(part_keys.as<u64>(), parts, keep,
-                                                                            (int)n_slots, cand.as<int>(),
-                                                                            tau.as<float>());
+            knn_merge_parts_kernel<<<div_up((int)merged_rows, 4), 256, lds, s>>>(
+                part_keys.as<u64>(), merged, keep, (int)merged_rows, cand.as<int>() + done * keep, tau.as<float>() + done);
             TSNE_TRY(hipGetLastError());
         }
         const int sort_n = next_pow2(keep) < 64 ? 64 : next_pow2(keep);
@@ -2574,7 +3579,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         knn_rerank_kernel<<<div_up((int)n_slots, 4), 256, sizeof(u64) * 4 * sort_n, s>>>(
             points, norms.as<float>(), N, D, K, keep, sort_n, cand.as<int>(), tau.as<float>(), scal.as<float>(),
             indices, sq_dist, scal.as<int>() + 1, fail_list.as<int>(), tile_list, first, step, (int)n_slots,
-            bf16 || bf16_chunked ? 1 : 0, renumbered ? renumbered->order : nullptr);
+            half || bf16 || bf16_chunked ? 1 : 0, renumbered ? renumbered->order : nullptr);
         TSNE_TRY(hipGetLastError());
         int host_scal[4] = {0, 0, 0, 0};
         TSNE_TRY(hipMemcpyAsync(host_scal, scal.p, sizeof(host_scal), hipMemcpyDeviceToHost, s));
@@ -2586,6 +3591,13 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
 
     int failed = 0;
     unsigned long long swept = 0;
+    // Points that the halves cannot tell apart: everything once more on two bf16 terms.
+    auto without_halves = [&]() -> int {
+        Xp.release();
+        operands.release();
+        centers.release();
+        return search(points, N, D, K, indices, sq_dist, s, mode, stats, probes, renumbered, false);
+    };
     // The verification needs the distance gap between neighbour K and candidate K' to exceed the rounding
     // bound of the approximate distances, which grows with the dimension count and with the points'
     // distance from the origin.  With many dimensions the neighbour distances of a query lie close
@@ -2604,12 +3616,14 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
                 want = wider;
             }
         }
+        if (!verified && half) return without_halves();
         if (!verified && mode == 0) {
             if (const int rc = build_transposed()) return rc;
             return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
         }
     }
     if (const int rc = sweep_and_rerank(want, nullptr, 0, 1, num_qtiles, failed, swept)) return rc;
+    if (half && !chunked && failed > N / 64) return without_halves();
     if (stats) {
         stats[0] = 1;
         stats[1] = failed;
@@ -2643,11 +3657,13 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         }
     }
     if (failed > 0) {
-        if (const int rc = build_transposed()) return rc;
         if (renumbered) {
             rename_list_kernel<<<div_up(failed, 256), 256, 0, s>>>(renumbered->order, failed, fail_list.as<int>());
             TSNE_TRY(hipGetLastError());
         }
+        const int rc_listed = run_listed_search(caller_points, N, D, K, fail_list.as<int>(), failed, indices, sq_dist, s);
+        if (rc_listed != kNoRoom) return rc_listed;
+        if (const int rc = build_transposed()) return rc;
         return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, fail_list.as<int>(), failed, cus, indices, sq_dist, s);
     }
     return 0;
@@ -2742,7 +3758,7 @@ static int search_renumbered(const float *points, int N, int D, int K, int *indi
 int run_knn_any_order(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s,
                       int *stats) {
     if (K > 1 && D > 0 && K <= N && N > kDirectPoints && locality_pivot_count(N) > 0 &&
-        SweepGeometry(N, D, false).fits(candidates_kept(N, K))) {
+        SweepGeometry(N, D, Products::kBf16).fits(candidates_kept(N, K))) {
         bool pays = false, searched = false;
         int rc = 0;
         try {
