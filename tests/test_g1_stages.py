@@ -1509,3 +1509,45 @@ def test_knn_on_halves(stages, n, d, k, kind):
     assert stats[0] == 1
     idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("n,kind", [(2, "plain"), (640, "plain"), (7680, "plain"), (7681, "line"), (15361, "far"),
+                                    (20480, "one box"), (20481, "plain"), (9001, "equal"), (5003, "not a number"),
+                                    (12000, "boxes' edges")])
+def test_small_step_spread_without_grouping(stages, monkeypatch, n, kind):
+    """Steps of a small problem whose points are looked through by every row of boxes against steps that group them by tile
+    (TSNE_KEEP_GROUPING asks for those): the same bits, at the remainders of the chunks they are looked through in, up
+    to the most points, with all points but one in a box, on a line, in one place, far from the origin, on the edges of
+    the boxes, and with one that is not a number (which both forms take into the first box)."""
+    rng = np.random.default_rng(n)
+    k = min(n, 12)
+    idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
+    P = (rng.random((n, k)) / (n * k)).astype(np.float32)
+    y0 = rng.standard_normal((2, n)).astype(np.float32)
+    if kind == "line":
+        y0[0] = 0.25
+    elif kind == "far":
+        y0 += np.float32(1e4)
+    elif kind == "one box":
+        y0[:] = 1e-3 * y0
+        y0[:, 7] = 5.0
+    elif kind == "equal":
+        y0[:] = 0.5
+    elif kind == "not a number":
+        y0[0, 11] = np.nan
+    elif kind == "boxes' edges":
+        y0 = rng.integers(0, 131, size=(2, n)).astype(np.float32)
+
+    def run(asked):
+        monkeypatch.setenv("TSNE_KEEP_GROUPING", "1") if asked else monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
+        plan = stages.Plan(n, k)
+        plan.prepare_attractive(dev(P), dev(idx))
+        y = dev(y0.reshape(-1).copy())
+        gains, old = torch.ones_like(y), torch.zeros_like(y)
+        z = plan.iterate_(None, None, y, gains, old, 0, 5, eta=10.0)
+        torch.cuda.synchronize()
+        plan.close()
+        return [v.cpu().numpy() for v in (y, gains, old, z)]
+
+    for a, b in zip(run(False), run(True)):
+        assert same_bits(a, b)

@@ -195,9 +195,10 @@ int launch_step(tsne_hip_plan *p, const float *pij, const int *indices, float *e
         // A small problem's step is its launches one after the other.  Its attractive forces ride along with the
         // inverse row pass, whose workgroups leave most of the chip idle (kernel alone, us: 1203 points x 32 neighbours
         // 5.1 -> 0; 20011 x 50 8.3 -> 1.5; 50000 x 90 13.4 -> 12.8, the positions' cache lines; see forces_ride_along),
-        // and the two kernels that group the points by tile are only launched every kGroupingInterval steps.
+        // and its points are spread without a grouping by tile (up to kScanPoints), or the two kernels that make one are
+        // only launched every kGroupingInterval steps.
         if (!pij && !p->csr_row_ptr && p->row_entries && !p->profiling && !p->profiling_attractive) {
-            const SmallStep small = {p->attr, p->steps_to_grouping <= 0};
+            const SmallStep small = {p->attr, p->steps_to_grouping <= 0, !p->grouping_asked};
             p->steps_to_grouping = (small.may_group ? kGroupingInterval : p->steps_to_grouping) - 1;
             if (launch_repulsive(p, embedding, slot, p->rep, nullptr, nullptr, s, true, &small)) return 1;
             if (normalization && launch_finish_z(p, normalization, s)) return 1;
@@ -435,7 +436,10 @@ int tsne_hip_plan_create(tsne_hip_plan **plan, int num_points, int num_neighbors
     p->n_nodes = n_boxes_per_dim * kInterp;
     p->device = device;
     p->lagrange = make_lagrange();
-    if (const char *v = std::getenv("TSNE_KEEP_GROUPING")) p->keep_grouping = v[0] != '0';
+    if (const char *v = std::getenv("TSNE_KEEP_GROUPING")) {
+        p->keep_grouping = v[0] != '0';
+        p->grouping_asked = true;
+    }
     // The grid buffers hold the largest grid: tsne_hip_plan_set_boxes may change the size between steps.
     const size_t G2 = (size_t)(kMaxBoxes * kInterp) * (kMaxBoxes * kInterp);
     const size_t spec = (size_t)2 * kFft * kNodePad;
@@ -521,6 +525,7 @@ int tsne_hip_plan_create(tsne_hip_plan **plan, int num_points, int num_neighbors
          hipStreamCreateWithFlags(&p->loop_stream, hipStreamNonBlocking) == hipSuccess &&
          hipEventCreateWithFlags(&p->enter_event, hipEventDisableTiming) == hipSuccess &&
          hipEventCreateWithFlags(&p->leave_event, hipEventDisableTiming) == hipSuccess;
+    ok = ok && prepare_repulsive() == 0;
     if (!ok) {
         set_error("plan_create: device allocation or initialisation failed: %s",
                   hipGetErrorString(hipGetLastError()));

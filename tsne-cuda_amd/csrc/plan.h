@@ -53,6 +53,12 @@ inline bool forces_ride_along(int N, int K) {
     return N <= kSingleStreamPoints && K <= 512 && (int64_t)N * K <= 3000000 + 50 * (int64_t)N;
 }
 
+// Up to this many points such a step spreads them without grouping them (conv_rows_scan_kernel).  us per step, grouped /
+// scanned, from the start of a fit, late in one, and with every point but one in one box: 1203 points 58 / 48, 56 / 49,
+// 68 / 51; 5000 61 / 50, 59 / 52, 70 / 59; 10007 62 / 54, 58 / 55, 71 / 70; 20011 66 / 59, 59 / 58, 71 / 89;
+// 40001 71 / 74, 64 / 70, 76 / 133.
+constexpr int kScanPoints = 20480;
+
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
     kKernelTileCount = 0,
@@ -93,6 +99,7 @@ struct tsne_hip_plan {
     const float *loop_embedding = nullptr;  // where tsne_hip_iterate last left off: the buffer and the step after its last
     int loop_next_step = -1;
     bool keep_grouping = true;     // loops may carry the grouping by tile from step to step (TSNE_KEEP_GROUPING=0: never)
+    bool grouping_asked = false;   // TSNE_KEEP_GROUPING given: small problems group their points too
     // Box moments of the charge spreading, 64-bit fixed point (scale moment_scale): [x box][moment][y box].  All
     // zero between steps: the spread kernel adds to them, the forward row pass reads them, the column pass
     // clears them.  Sized for the largest grid.
@@ -204,7 +211,10 @@ int launch_bounds(tsne_hip_plan *p, const float *embedding, int slot, hipStream_
 struct SmallStep {
     float *attr;
     bool may_group;
+    bool may_scan;  // ... or spread them without a grouping
 };
+// Where a kernel needs to be told something once per device.
+int prepare_repulsive();
 int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *rep, float *point_potentials,
                      float *charges_out, hipStream_t s, bool keep_grouping = false,
                      const SmallStep *small = nullptr);

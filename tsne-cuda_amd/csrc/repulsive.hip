@@ -244,6 +244,15 @@ __device__ __forceinline__ void mixed_pass(float2 *s, int nfft, const float2 *tw
     __syncthreads();
 }
 
+// The roots of unity into LDS (the caller's next barrier makes them visible): the passes of a chain of short kernels wait
+// for them one after the other where they come from memory, whose caches every launch finds cold.  Costs 6400 bytes of
+// LDS, which the kernels that run beside the attractive kernel do not have.  (Alone: column pass 13.8 -> 12.8 us, inverse
+// row pass 8.0 -> 7.5.)
+template <int THREADS>
+__device__ __forceinline__ void stage_twiddles(float2 (&lds)[kFftShort], const float2 *__restrict__ tw, int tid) {
+    for (int e = tid; e < kFftShort; e += THREADS) lds[e] = tw[e];
+}
+
 // What the convolution's kernels need of a transform length: the slot of element i within a transform's N LDS
 // slots, the frequency held at a position of the forward transform's output, and the transforms themselves
 // (every pass ends with a barrier).
@@ -866,6 +875,50 @@ __device__ __forceinline__ void kernel_rows_block(int block, const LoopScalars *
 // provided those are in one piece (the loop enqueues the attractive kernel first for that reason).  One row per
 // workgroup (256 threads, 16 KB) measured 21 us against 17 us alone and 2 % fewer iterations per second.
 // ---------------------------------------------------------------------------
+// The monomial coefficients where a lane can pick its node's (an argument that lanes index goes to scratch memory).
+__device__ __forceinline__ void stage_monomials(double (&mono)[kInterp][3], const LagrangeMonomials &arg, int tid) {
+    if (tid == 0)
+#pragma unroll
+        for (int m = 0; m < kInterp; ++m)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) mono[m][i] = arg.c[m][i];
+}
+// Charges of node (gx, n) from its box's moments, `moment(m)` the m-th of them.
+template <class Moment>
+__device__ __forceinline__ float4 node_charges(int gx, int n, const Bounds &bd, const double (&mono)[kInterp][3],
+                                               Moment moment) {
+    const int bx = gx / kInterp, a = gx % kInterp, by = n / kInterp, b = n % kInterp;
+    double M[kMoments];
+#pragma unroll
+    for (int m = 0; m < kMoments; ++m) M[m] = moment(m);
+    double ca[3], cb[3];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        ca[i] = mono[a][i];
+        cb[i] = mono[b][i];
+    }
+    double s00 = 0.0, s10 = 0.0, s01 = 0.0, s20 = 0.0, s02 = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const double cc = ca[i] * cb[j];
+            s00 += cc * M[moment_index(i, j)];
+            s10 += cc * M[moment_index(i + 1, j)];
+            s01 += cc * M[moment_index(i, j + 1)];
+            s20 += cc * M[moment_index(i + 2, j)];
+            s02 += cc * M[moment_index(i, j + 2)];
+        }
+    const double bw = bd.box_width;
+    const double xl = box_lower(bx, bd), yl = box_lower(by, bd);
+    float4 v;
+    v.x = (float)s00;
+    v.y = (float)(xl * s00 + bw * s10);
+    v.z = (float)(yl * s00 + bw * s01);
+    v.w = (float)((xl * xl + yl * yl) * s00 + 2.0 * bw * (xl * s10 + yl * s01) + bw * bw * (s20 + s02));
+    return v;
+}
+
 template <int ROWS, int NFFT>
 __global__ __launch_bounds__(256 * ROWS) void conv_rows_forward_kernel(const unsigned long long *__restrict__ moments,
                                                                        double from_fixed, LagrangeMonomials mono,
@@ -892,42 +945,18 @@ __global__ __launch_bounds__(256 * ROWS) void conv_rows_forward_kernel(const uns
     const int m0 = row_block * ROWS;
     const float s3 = r2_plane_scale(sc, slot);
     const Bounds bd = load_bounds(sc, slot, n_boxes);
+    __shared__ double mono_lds[kInterp][3];
+    stage_monomials(mono_lds, mono, tid);
+    __syncthreads();
     for (int e = tid; e < ROWS * NFFT; e += kThreads) {
         const int r = e / NFFT, n = e - r * NFFT;
         float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
         if (n < G && m0 + r < G) {
             const int gx = m0 + r;
-            const int bx = gx / kInterp, a = gx % kInterp, by = n / kInterp, b = n % kInterp;
-            const unsigned long long *src = moments + (size_t)bx * kMoments * n_boxes + by;
-            if (src[0] != 0ull) {  // moment (0, 0) counts the points of the box
-                double M[kMoments];
-#pragma unroll
-                for (int m = 0; m < kMoments; ++m) M[m] = (double)(long long)src[(size_t)m * n_boxes] * from_fixed;
-                double ca[3], cb[3];
-#pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    ca[i] = a == 0 ? mono.c[0][i] : (a == 1 ? mono.c[1][i] : mono.c[2][i]);
-                    cb[i] = b == 0 ? mono.c[0][i] : (b == 1 ? mono.c[1][i] : mono.c[2][i]);
-                }
-                double s00 = 0.0, s10 = 0.0, s01 = 0.0, s20 = 0.0, s02 = 0.0;
-#pragma unroll
-                for (int i = 0; i < 3; ++i)
-#pragma unroll
-                    for (int j = 0; j < 3; ++j) {
-                        const double cc = ca[i] * cb[j];
-                        s00 += cc * M[moment_index(i, j)];
-                        s10 += cc * M[moment_index(i + 1, j)];
-                        s01 += cc * M[moment_index(i, j + 1)];
-                        s20 += cc * M[moment_index(i + 2, j)];
-                        s02 += cc * M[moment_index(i, j + 2)];
-                    }
-                const double bw = bd.box_width;
-                const double xl = box_lower(bx, bd), yl = box_lower(by, bd);
-                v.x = (float)s00;
-                v.y = (float)(xl * s00 + bw * s10);
-                v.z = (float)(yl * s00 + bw * s01);
-                v.w = (float)((xl * xl + yl * yl) * s00 + 2.0 * bw * (xl * s10 + yl * s01) + bw * bw * (s20 + s02));
-            }
+            const unsigned long long *src = moments + (size_t)(gx / kInterp) * kMoments * n_boxes + n / kInterp;
+            if (src[0] != 0ull)  // moment (0, 0) counts the points of the box
+                v = node_charges(gx, n, bd, mono_lds,
+                                 [&](int m) { return (double)(long long)src[(size_t)m * n_boxes] * from_fixed; });
             if (charges_out) charges_out[(size_t)gx * G + n] = v;
         }
         s[r * 2 + 0][T::slot(n)] = make_float2(v.x, v.w * s3);  // planes 1 and r^2 / m^2
@@ -944,6 +973,171 @@ __global__ __launch_bounds__(256 * ROWS) void conv_rows_forward_kernel(const uns
         } else {
             *dst = s[pair][T::slot(pos)];
         }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Spread and forward row pass of a small problem's step in one kernel, without any grouping of the points: a workgroup
+// has one row of boxes (three grid rows), looks through all points for those of its row, adds their moments to its
+// boxes' in LDS and transforms the three rows.  The same integers as the spread kernel's sums, so the same bits.  It
+// stands for three launches (tile count and scatter, every second step, and the spread), whose 7 to 18 us are latency and
+// atomics on the grid's moments, and reads the positions once per workgroup, from the L2: a chain of 130 row
+// workgroups leaves half the chip idle anyway.  What it adds to the row pass is two trips through memory, two barriers
+// per kScanChunk points and the spreading of the fullest row of boxes (1203 points: 15.4 us, row pass and spread before
+// 10.6 + 7.2 and the grouping's launches; the whole step 60.7 -> 48.4, kScanPoints has more).
+//
+// The workgroups past the rows produce the kernel's row spectra, as in conv_rows_forward_kernel.
+// Dynamic LDS: kScanCopies x kMoments x n_boxes moments (lanes take turns: points of one box meet on one word), then the
+// points found, up to kScanChunk, and in their place the six transforms.
+// ---------------------------------------------------------------------------
+constexpr int kScanThreads = 640;  // ten waves: 600 butterflies of the first pass of six transforms of 800 points
+constexpr int kScanPer = 12, kScanChunk = kScanPer * kScanThreads;  // points looked at between two barriers
+constexpr int kScanCopies = 2;
+inline size_t scan_lds(int n_boxes) {
+    return sizeof(unsigned long long) * kScanCopies * kMoments * n_boxes + sizeof(float2) * std::max(kScanChunk, 6 * kFftShort);
+}
+__global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const float *__restrict__ emb, int N, double to_fixed,
+                                                                      double from_fixed, LagrangeMonomials mono, int G,
+                                                                      int n_boxes, LoopScalars *sc, int slot, int next_slot,
+                                                                      const float2 *__restrict__ twiddles,
+                                                                      float2 *__restrict__ row_spectra,
+                                                                      float *__restrict__ kernel_rows) {
+    using T = Transform<kFftShort>;
+    constexpr int NFFT = kFftShort;
+    extern __shared__ __attribute__((aligned(16))) unsigned char scan_raw[];
+    __shared__ int found[2];
+    __shared__ double mono_lds[kInterp][3];
+    __shared__ float2 tw[kFftShort];
+    unsigned long long *acc = reinterpret_cast<unsigned long long *>(scan_raw);
+    const int words = kMoments * n_boxes;
+    float2 *list = reinterpret_cast<float2 *>(acc + kScanCopies * words);
+    float2(*s)[NFFT] = reinterpret_cast<float2(*)[NFFT]>(list);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    // The step's resets (see spread_kernel).
+    if (blockIdx.x == 0 && tid < kZParts) sc->z_part[tid] = 0ll;
+    if (blockIdx.x == 0 && tid == 0) {
+        sc->min_enc[next_slot] = 0xffffffffu;
+        sc->max_enc[next_slot] = 0u;
+    }
+    stage_twiddles<kScanThreads>(tw, twiddles, tid);
+    const int launched = kXcds * ((n_boxes + kXcds - 1) / kXcds);
+    if ((int)blockIdx.x >= launched) {
+        kernel_rows_block<kScanThreads, 2, NFFT>(blockIdx.x - launched, sc, slot, n_boxes, tw, kernel_rows, s);
+        return;
+    }
+    const int bx = xcd_row_block(blockIdx.x, n_boxes);
+    if (bx < 0) return;
+    float px[kScanPer], py[kScanPer];
+    auto fetch = [&](int first) {
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u) {
+            const int i = min(first + u * kScanThreads + tid, N - 1);
+            px[u] = emb[i];
+            py[u] = emb[N + i];
+        }
+    };
+    fetch(0);
+    for (int e = tid; e < kScanCopies * words; e += kScanThreads) acc[e] = 0ull;
+    if (tid < 2) found[tid] = 0;
+    stage_monomials(mono_lds, mono, tid);
+    const float s3 = r2_plane_scale(sc, slot);
+    const Bounds bd = load_bounds(sc, slot, n_boxes);
+    const unsigned long long below = (1ull << lane) - 1ull;
+    // A point is looked at with two comparisons; whether it lies in the row is settled, as everywhere, by the division,
+    // for the few that pass.  (On the distance from the lower bound, as the division, with a hundredth of a box to spare
+    // either side: division and products are rounded by 2^-24 of at most 133 boxes.  The outermost rows take what the
+    // binning clamps; a NaN lies in the first box.)
+    const float from = bx == 0 ? -INFINITY : ((float)bx - 0.01f) * bd.box_width;
+    const float to = bx == n_boxes - 1 ? INFINITY : ((float)bx + 1.01f) * bd.box_width;
+    const bool all = !(bd.box_width > 1e-30f);
+    // A thread's points of one box in a row are summed in registers: with every point in one box, as beside a far
+    // outlier, the additions in LDS would come one after the other (20011 points 235 us a step).
+    unsigned long long sum[kMoments];
+    int sum_box = -1;
+    auto flush = [&]() {
+        unsigned long long *dst = acc + (lane % kScanCopies) * words + sum_box;
+#pragma unroll
+        for (int m = 0; m < kMoments; ++m) atomicAdd(dst + m * n_boxes, sum[m]);
+    };
+    __syncthreads();
+    for (int first = 0, turn = 0; first < N; first += kScanChunk, turn ^= 1) {
+        unsigned long long mine[kScanPer];
+        int total = 0;
+#pragma unroll
+        for (int u = 0; u < kScanPer; ++u) {
+            mine[u] = __ballot(first + u * kScanThreads + tid < N && (all || (!(px[u] - bd.lo < from) && !(px[u] - bd.lo > to))));
+            total += __popcll(mine[u]);
+        }
+        if (total > 0) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&found[turn], total);
+            at = __builtin_amdgcn_readfirstlane(at);
+#pragma unroll
+            for (int u = 0; u < kScanPer; ++u) {
+                if ((mine[u] >> lane) & 1ull) list[at + __popcll(mine[u] & below)] = make_float2(px[u], py[u]);
+                at += __popcll(mine[u]);
+            }
+        }
+        if (first + kScanChunk < N) fetch(first + kScanChunk);
+        __syncthreads();
+        const int n = found[turn];
+        if (tid == 0) found[turn ^ 1] = 0;
+        for (int e = tid; e < n; e += kScanThreads) {
+            const float2 p = list[e];
+            int b, by;
+            float pu[5], pv[5];
+            pu[0] = pv[0] = 1.0f;
+            bin_and_coord(p.x, bd, n_boxes, b, pu[1]);
+            if (b != bx) continue;
+            bin_and_coord(p.y, bd, n_boxes, by, pv[1]);
+#pragma unroll
+            for (int k = 2; k < 5; ++k) {
+                pu[k] = pu[k - 1] * pu[1];
+                pv[k] = pv[k - 1] * pv[1];
+            }
+            const bool same = by == sum_box;
+            if (!same && sum_box >= 0) flush();
+            sum_box = by;
+#pragma unroll
+            for (int j = 0; j < 5; ++j)
+#pragma unroll
+                for (int i = 0; i < 5; ++i)
+                    if (j <= 2 || i <= 2) {
+                        unsigned long long &to_sum = sum[moment_index(i, j)];
+                        to_sum = (same ? to_sum : 0ull) + to_fixed_bits(pu[i] * pv[j], to_fixed);
+                    }
+        }
+        __syncthreads();
+    }
+    if (sum_box >= 0) flush();
+    __syncthreads();
+    double *moments = reinterpret_cast<double *>(acc);
+    for (int e = tid; e < words; e += kScanThreads) {
+        unsigned long long v = acc[e];
+#pragma unroll
+        for (int c = 1; c < kScanCopies; ++c) v += acc[c * words + e];
+        moments[e] = (double)(long long)v * from_fixed;
+    }
+    __syncthreads();
+    for (int e = tid; e < kInterp * G; e += kScanThreads) {
+        const int r = e / G, n = e - r * G;
+        const double *src = moments + n / kInterp;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (src[0] != 0.0) v = node_charges(bx * kInterp + r, n, bd, mono_lds, [&](int m) { return src[m * n_boxes]; });
+        s[r * 2 + 0][T::slot(n)] = make_float2(v.x, v.w * s3);  // planes 1 and r^2 / m^2
+        s[r * 2 + 1][T::slot(n)] = make_float2(v.y, v.z);       // planes x and y
+    }
+    for (int e = tid; e < 2 * kInterp * (NFFT - G); e += kScanThreads) {
+        const int f = e / (NFFT - G), n = G + e - f * (NFFT - G);
+        s[f][T::slot(n)] = make_float2(0.f, 0.f);
+    }
+    __syncthreads();
+    T::forward(&s[0][0], 2 * kInterp, tw, tid, kScanThreads);
+    for (int e = tid; e < 2 * NFFT; e += kScanThreads) {
+        const int pair = e / NFFT, pos = e - pair * NFFT;
+        float2 *dst = row_spectra + ((size_t)pair * NFFT + pos) * kNodePad + bx * kInterp;
+#pragma unroll
+        for (int r = 0; r < kInterp; ++r) dst[r] = s[r * 2 + pair][T::slot(pos)];
     }
 }
 
@@ -1047,7 +1241,7 @@ __global__ __launch_bounds__(512) void conv_columns_kernel(const float2 *__restr
 template <bool SLIM>
 __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *__restrict__ row_spectra, int G,
                                                                  const float *__restrict__ kernel_rows,
-                                                                 const float2 *__restrict__ tw,
+                                                                 const float2 *__restrict__ twiddles,
                                                                  float2 *__restrict__ col_results,
                                                                  unsigned long long *__restrict__ moments,
                                                                  int moment_words) {
@@ -1057,6 +1251,9 @@ __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *_
     constexpr int kKernelSlot = SLIM ? 0 : 4;
     __shared__ float2 s[SLIM ? 4 : 5][N];  // [pair * 2 + col]; SLIM = false: then the kernel's two columns
     const int tid = threadIdx.x;
+    __shared__ float2 staged[SLIM ? 1 : N];
+    if constexpr (!SLIM) stage_twiddles<512>(staged, twiddles, tid);  // (the first pass has its own from memory, with the data)
+    const float2 *tw = SLIM ? twiddles : staged;
     const int c0 = blockIdx.x * 2;
     int v0 = T::frequency(c0), v1 = T::frequency(c0 + 1);
     v0 = min(v0, N - v0);
@@ -1073,7 +1270,7 @@ __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *_
     };
     float kreg[10] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
     if constexpr (SLIM) {
-        mixed_pass_io<N, 800, 8, false>(1, tw, tid, 512, [&](int, int m, int) { return kernel_column(m); }, lds_store);
+        mixed_pass_io<N, 800, 8, false>(1, twiddles, tid, 512, [&](int, int m, int) { return kernel_column(m); }, lds_store);
         __syncthreads();
         mixed_pass<N, 100, 10, false>(&s[0][0], 1, tw, tid, 512);
         mixed_pass<N, 10, 10, false>(&s[0][0], 1, tw, tid, 512);
@@ -1086,11 +1283,11 @@ __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *_
             }
         }
         __syncthreads();
-        mixed_pass_io<N, 800, 8, false>(4, tw, tid, 512, [&](int f, int m, int) { return data_column(f, m); },
+        mixed_pass_io<N, 800, 8, false>(4, twiddles, tid, 512, [&](int f, int m, int) { return data_column(f, m); },
                                         lds_store);
     } else {
         mixed_pass_io<N, 800, 8, false>(
-            5, tw, tid, 512, [&](int f, int m, int) { return f < 4 ? data_column(f, m) : kernel_column(m); },
+            5, twiddles, tid, 512, [&](int f, int m, int) { return f < 4 ? data_column(f, m) : kernel_column(m); },
             lds_store);
     }
     __syncthreads();
@@ -1169,7 +1366,8 @@ __device__ __forceinline__ void row_forces_block(const RowForces &f, int block, 
 
 // With rows.entries set, the workgroups from rows.first_block on compute the attractive forces of a small problem
 // (nothing of this step but the update waits for either).
-template <int NFFT>
+// STAGED (800 points): the twiddles through LDS, where the attractive kernel does not run beside.
+template <int NFFT, bool STAGED>
 __global__ __launch_bounds__(kRowThreads) void conv_rows_inverse_kernel(const float2 *__restrict__ col_results, int G,
                                                                 const LoopScalars *sc, int slot,
                                                                 const float2 *__restrict__ twiddles,
@@ -1181,11 +1379,13 @@ __global__ __launch_bounds__(kRowThreads) void conv_rows_inverse_kernel(const fl
         return;
     }
     __shared__ float2 s[4][NFFT];  // [row * 2 + pair]
-    const float2 *tw = twiddles;
+    __shared__ float2 staged[STAGED ? kFftShort : 1];
+    const float2 *tw = STAGED ? staged : twiddles;
     const int tid = threadIdx.x;
     const int row_block = xcd_row_block(blockIdx.x, (G + 1) / 2);
     if (row_block < 0) return;
     const int m0 = row_block * 2;
+    if constexpr (STAGED) stage_twiddles<kRowThreads>(staged, twiddles, tid);
     for (int e = tid; e < 2 * NFFT; e += kRowThreads) {
         const int pair = e / NFFT, pos = e - pair * NFFT;
         const float4 v =
@@ -1308,6 +1508,12 @@ int launch_bounds(tsne_hip_plan *p, const float *embedding, int slot, hipStream_
     return 0;
 }
 
+int prepare_repulsive() {
+    TSNE_TRY(hipFuncSetAttribute(reinterpret_cast<const void *>(conv_rows_scan_kernel),
+                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)scan_lds(kFftShort / (2 * kInterp))));
+    return 0;
+}
+
 // All kernels of one repulsive-force evaluation.  Expects the bounds of
 // `embedding` in `slot`; leaves sum_i z_i in scalars->z_part and resets the other
 // bounds slot.  charges_out (optional) receives a copy of the node charges.
@@ -1317,12 +1523,18 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
     const bool group = !small || small->may_group || !keep;
     if (!group) keep = kKeepAlways;
     const int N = p->num_points, G = p->n_nodes, nb = p->n_boxes;
+    // Transform length: 800 points where the padded grid (2 G - 1) fits, else 1024 (TSNE_FFT=1024 forces the latter).
+    const char *fft_env = getenv("TSNE_FFT");  // (read on every call, like the column pass's switch below)
+    const bool long_only = fft_env && atoi(fft_env) == kFft;
+    const bool short_fft = 2 * G - 1 <= kFftShort && !long_only;
+    const bool scan = small && small->may_scan && short_fft && N <= kScanPoints;
+    if (scan) keep = 0;
     const int tiles_per_dim = (nb + kTileBoxes - 1) / kTileBoxes;
     // Few, large workgroups: every workgroup ends with one global atomic per tile counter, and
     // same-address atomics serialise (about a thousand per counter cost ~20 us).
     // (one point per thread until that many workgroups are in use)
     const int sort_blocks = std::min(div_up(N, 1024), kSortBlocks);
-    if (group) {
+    if (group && !scan) {
         if (profile_mark(p, kKernelTileCount, s)) return 1;
         TSNE_LOOP_KERNEL(p, (tile_count_kernel), sort_blocks, 1024, 0, s, embedding, N, p->scalars, slot, slot ^ 1, nb, p->tile_count,
                                                        p->tile_cursor, p->chunks, p->num_chunks, p->num_chunks + 1,
@@ -1334,24 +1546,26 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
                                                          p->scalars, keep);
         TSNE_LAUNCHED(s);
     }
-    if (profile_mark(p, kKernelSpread, s)) return 1;
-    // Resident workgroups share the chunk list (its length is only known on the device; with fewer chunks
-    // than workgroups the surplus ones exit at once).
-    const int spread_blocks =
-        xcd_launch_blocks(std::min(N / kChunkPoints + tiles_per_dim * tiles_per_dim + 1, p->spread_grid));
-    TSNE_LOOP_KERNEL(p, (spread_kernel), spread_blocks, kSpreadThreads, 0, s, p->tile_xy, p->tile_perm, p->yxy, p->chunks,
-                                                           p->num_chunks, p->scalars, slot, slot ^ 1, nb,
-                                                           p->moment_scale, p->box_moments, keep);
-    TSNE_LAUNCHED(s);
-    // Transform length: 800 points where the padded grid (2 G - 1) fits, else 1024 (TSNE_FFT=1024 forces the latter).
-    const char *fft_env = getenv("TSNE_FFT");  // (read on every call, like the column pass's switch below)
-    const bool long_only = fft_env && atoi(fft_env) == kFft;
-    const bool short_fft = 2 * G - 1 <= kFftShort && !long_only;
-    const int row_grid = xcd_launch_blocks(div_up(G, 2));
     const double from_fixed = 1.0 / p->moment_scale;
+    const int row_grid = xcd_launch_blocks(div_up(G, 2));
+    if (!scan) {
+        if (profile_mark(p, kKernelSpread, s)) return 1;
+        // Resident workgroups share the chunk list (its length is only known on the device; with fewer chunks
+        // than workgroups the surplus ones exit at once).
+        const int spread_blocks =
+            xcd_launch_blocks(std::min(N / kChunkPoints + tiles_per_dim * tiles_per_dim + 1, p->spread_grid));
+        TSNE_LOOP_KERNEL(p, (spread_kernel), spread_blocks, kSpreadThreads, 0, s, p->tile_xy, p->tile_perm, p->yxy, p->chunks,
+                                                               p->num_chunks, p->scalars, slot, slot ^ 1, nb,
+                                                               p->moment_scale, p->box_moments, keep);
+        TSNE_LAUNCHED(s);
+    }
     float4 *charges4 = reinterpret_cast<float4 *>(charges_out);
     if (profile_mark(p, kKernelConvRowsForward, s)) return 1;
-    if (short_fft)
+    if (scan)
+        TSNE_LOOP_KERNEL(p, (conv_rows_scan_kernel), xcd_launch_blocks(nb) + div_up(G, 8), kScanThreads, scan_lds(nb), s, embedding, N,
+                         p->moment_scale, from_fixed, p->monomials, G, nb, p->scalars, slot, slot ^ 1, p->twiddles_short,
+                         p->row_spectra, p->kernel_rows);
+    else if (short_fft)
         TSNE_LOOP_KERNEL(p, (conv_rows_forward_kernel<2, kFftShort>), row_grid + div_up(G, 8), 512, 0, s, p->box_moments, from_fixed, p->monomials, charges4, G, nb, p->scalars, slot, p->twiddles_short,
             p->row_spectra, p->kernel_rows);
     else
@@ -1362,7 +1576,7 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
     const char *slim_env = getenv("TSNE_SLIM_COLUMNS");
     const int slim_mode = slim_env ? atoi(slim_env) : -1;
     const bool slim = slim_mode < 0 ? (p->blocked_ready && p->strip_rows >= 1024) : slim_mode == 1;
-    const int moment_words = kMoments * nb * nb;
+    const int moment_words = scan ? 0 : kMoments * nb * nb;  // (to clear)
     if (short_fft && slim)
         TSNE_LOOP_KERNEL(p, (conv_columns_short_kernel<true>), kFftShort / 2, 512, 0, s, p->row_spectra, G, p->kernel_rows, p->twiddles_short, p->col_results, p->box_moments, moment_words);
     else if (short_fft)
@@ -1381,11 +1595,14 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
         rows = {p->row_entries, p->yxy, small->attr, N, p->num_neighbors, row_grid};
         inverse_grid += div_up(N, kRowThreads / kForceLanes);
     }
-    if (short_fft)
-        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFftShort>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
+    if (short_fft && small)
+        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFftShort, true>), inverse_grid, kRowThreads, 0, s, p->col_results, G,
+                         p->scalars, slot, p->twiddles_short, p->node_potentials, rows);
+    else if (short_fft)
+        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFftShort, false>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
                                                                             p->twiddles_short, p->node_potentials, rows);
     else
-        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFft>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
+        TSNE_LOOP_KERNEL(p, (conv_rows_inverse_kernel<kFft, false>), inverse_grid, kRowThreads, 0, s, p->col_results, G, p->scalars, slot,
                                                                        p->twiddles, p->node_potentials, rows);
     TSNE_LAUNCHED(s);
     if (profile_mark(p, kKernelGather, s)) return 1;
