@@ -289,6 +289,10 @@ int tsne_hip_repulsive_error(tsne_hip_plan *plan, const float *embedding, int sa
 int tsnecuda_trustworthiness(const float *points, const float *embedding, int num_points, int num_dims,
                              int n_neighbors, int max_sample, int device, double *trustworthiness, int *sample_out);
 
+/* Gives the device memory back that the library keeps between calls (blocks of 32 MB and more that its calls used as
+ * scratch, at most 2 GB per device; unused ones go after five seconds by themselves, at the next call). */
+int tsne_hip_release_scratch(void);
+
 /* Squared L2 norm of n device floats into the device scalar *out
  * (tsnecuda::util::L2NormDeviceVector without the root, src/util/math_utils.cu:51-57). */
 int tsne_hip_sum_squares(tsne_hip_plan *plan, const float *values, int64_t n, float *out, void *stream);

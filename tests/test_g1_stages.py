@@ -1551,3 +1551,44 @@ def test_small_step_spread_without_grouping(stages, monkeypatch, n, kind):
 
     for a, b in zip(run(False), run(True)):
         assert same_bits(a, b)
+
+
+def test_scratch_is_kept_bounded_and_given_back(stages):
+    """Large scratch of a call is kept for the next, at most 2 GB of it, and goes when asked; calls of several threads on
+    streams of their own, of sizes that take over each other's blocks, give what they give alone."""
+    import threading
+    problems = [(dev(np.random.default_rng(n).standard_normal((n, d)).astype(np.float32)), k)
+                for n, d, k in ((60000, 12, 45), (100003, 20, 33), (40000, 150, 90))]
+    torch.cuda.synchronize()
+    stages.release_scratch()
+    want = []
+    for x, k in problems:
+        want.append(stages.knn(x, k))
+        stages.release_scratch()
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    got = [None] * 6
+
+    def work(t):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for turn in range(2):
+                x, k = problems[(t + turn) % 3]
+                got[2 * t + turn] = ((t + turn) % 3, stages.knn(x, k))
+        stream.synchronize()
+
+    torch.cuda.synchronize()
+    threads = [threading.Thread(target=work, args=(t,)) for t in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    for which, (idx, d2) in got:
+        assert torch.equal(idx, want[which][0]) and torch.equal(d2, want[which][1])
+    del got, idx, d2
+    torch.cuda.empty_cache()
+    kept = free - torch.cuda.mem_get_info()[0]
+    assert kept <= (2 << 30) + (256 << 20)
+    stages.release_scratch()
+    assert free - torch.cuda.mem_get_info()[0] <= 256 << 20

@@ -39,7 +39,7 @@ hipError_t malloc_optional(void **p, size_t bytes) {
             *p = nullptr;
             return hipErrorOutOfMemory;
         }
-    return hipMalloc(p, bytes);
+    return scratch_malloc(p, bytes);
 }
 
 int profile_mark(tsne_hip_plan *p, int id, hipStream_t) {

@@ -850,11 +850,11 @@ void release_blocked(tsne_hip_plan *p) {
     (void)hipDeviceSynchronize();
     for (auto &g : p->step_graphs) (void)hipGraphExecDestroy(g.exec);
     p->step_graphs.clear();
-    (void)hipFree(p->ent_p);
+    scratch_free(p->ent_p);
     (void)hipFree(p->seg);
     (void)hipFree(p->strip_row0);
     (void)hipFree(p->wseg);
-    (void)hipFree(p->row_entries);
+    scratch_free(p->row_entries);
     p->wseg = nullptr;
     p->row_entries = nullptr;
     p->blocked_direct = false;
@@ -872,17 +872,15 @@ static int prepare_direct(tsne_hip_plan *p, const float *pij, const int *indices
     while ((1 << strip_bits) < p->n_strips) ++strip_bits;
     struct Scratch {
         void *ptr = nullptr;
-        ~Scratch() {
-            if (ptr) (void)hipFree(ptr);
-        }
+        ~Scratch() { scratch_free(ptr); }
     } keys, keys_alt, vals, vals_alt, hist, wpad;
     const int sort_tiles = div_up(nnz, radix_sort_tile());
-    if (hipMalloc(&keys.ptr, sizeof(u64) * (size_t)nnz) != hipSuccess ||
-        hipMalloc(&keys_alt.ptr, sizeof(u64) * (size_t)nnz) != hipSuccess ||
-        hipMalloc(&vals.ptr, sizeof(float) * (size_t)nnz) != hipSuccess ||
-        hipMalloc(&vals_alt.ptr, sizeof(float) * (size_t)nnz) != hipSuccess ||
-        hipMalloc(&hist.ptr, sizeof(unsigned int) * 256 * ((size_t)sort_tiles + 1)) != hipSuccess ||
-        hipMalloc(&wpad.ptr, sizeof(unsigned int) * (size_t)p->n_strips * (kMaxWindows + 1)) != hipSuccess) {
+    if (scratch_malloc(&keys.ptr, sizeof(u64) * (size_t)nnz) != hipSuccess ||
+        scratch_malloc(&keys_alt.ptr, sizeof(u64) * (size_t)nnz) != hipSuccess ||
+        scratch_malloc(&vals.ptr, sizeof(float) * (size_t)nnz) != hipSuccess ||
+        scratch_malloc(&vals_alt.ptr, sizeof(float) * (size_t)nnz) != hipSuccess ||
+        scratch_malloc(&hist.ptr, sizeof(unsigned int) * 256 * ((size_t)sort_tiles + 1)) != hipSuccess ||
+        scratch_malloc(&wpad.ptr, sizeof(unsigned int) * (size_t)p->n_strips * (kMaxWindows + 1)) != hipSuccess) {
         set_error("attractive_prepare: out of device memory for sorting %lld entries", nnz);
         return 1;
     }
@@ -994,7 +992,7 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
     const size_t item_entries = p->blocked_direct ? kDirectItem : kItemEntries;
     const size_t items_per_strip = (strip_entries + item_entries - 1) / item_entries;
     const size_t nnz = items_per_strip * p->n_strips * item_entries;
-    bool ok = hipMalloc(&p->ent_p, 2 * sizeof(float) * nnz) == hipSuccess &&
+    bool ok = scratch_malloc(reinterpret_cast<void **>(&p->ent_p), 2 * sizeof(float) * nnz) == hipSuccess &&
               hipMalloc(&p->seg, p->blocked_direct ? sizeof(unsigned int)
                                                    : sizeof(unsigned int) * (size_t)p->n_strips * p->seg_stride) == hipSuccess &&
               (!p->blocked_direct ||

@@ -22,6 +22,10 @@ bool sync_kernels_enabled();
 // hipMalloc for memory that a faster form of a stage uses and a slower one does without.  TSNE_SCRATCH_LIMIT=<bytes>
 // (read on every call; for measurements and tests of the slower forms): more than that is never there.
 hipError_t malloc_optional(void **p, size_t bytes);
+// hipMalloc and hipFree for a call's scratch: large blocks are kept for the next call (scratch.hip).  What malloc_optional
+// returned goes back through scratch_free too.
+hipError_t scratch_malloc(void **p, size_t bytes);
+void scratch_free(void *p);
 
 #define TSNE_TRY(expr)                                                                              \
     do {                                                                                            \

@@ -45,12 +45,12 @@ void hip_or_die(hipError_t e, const char *what) {
 struct DeviceBuffer {
     void *ptr = nullptr;
     DeviceBuffer() {}
-    explicit DeviceBuffer(size_t bytes) { hip_or_die(hipMalloc(&ptr, bytes ? bytes : 1), "device allocation"); }
+    explicit DeviceBuffer(size_t bytes) { hip_or_die(tsnehip::scratch_malloc(&ptr, bytes), "device allocation"); }
     DeviceBuffer(const DeviceBuffer &) = delete;
     DeviceBuffer &operator=(const DeviceBuffer &) = delete;
     ~DeviceBuffer() { release(); }
     void release() {
-        if (ptr) (void)hipFree(ptr);
+        tsnehip::scratch_free(ptr);
         ptr = nullptr;
     }
     void swap(DeviceBuffer &other) { std::swap(ptr, other.ptr); }

@@ -2945,12 +2945,12 @@ struct DeviceMem {
     void *p = nullptr;
     ~DeviceMem() { release(); }
     void release() {
-        if (p) (void)hipFree(p);  // (waits for the kernels that use it)
+        scratch_free(p);  // (waits for the kernels that use it)
         p = nullptr;
     }
     bool alloc(size_t bytes) {
         release();
-        return hipMalloc(&p, bytes ? bytes : 1) == hipSuccess;
+        return scratch_malloc(&p, bytes) == hipSuccess;
     }
     // (of a form that the call can do without)
     bool alloc_optional(size_t bytes) {

@@ -99,10 +99,10 @@ __global__ void gather_rows_kernel(const float *__restrict__ src, const int *__r
 
 struct Scratch {
     void *p = nullptr;
-    ~Scratch() { (void)hipFree(p); }
+    ~Scratch() { scratch_free(p); }
     bool alloc(size_t bytes, bool optional) {
         if (!bytes) bytes = 1;
-        return (optional ? malloc_optional(&p, bytes) : hipMalloc(&p, bytes)) == hipSuccess;
+        return (optional ? malloc_optional(&p, bytes) : scratch_malloc(&p, bytes)) == hipSuccess;
     }
     template <typename T>
     T *as() { return static_cast<T *>(p); }

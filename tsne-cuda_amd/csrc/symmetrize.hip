@@ -301,7 +301,7 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
             }
             if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
             if (e == hipSuccess) e = hipStreamSynchronize(s);  // the tables go
-            (void)hipFree(memory);
+            scratch_free(memory);
             if (e != hipSuccess) {
                 set_error("symmetrize: %s", hipGetErrorString(e));
                 return 1;

@@ -76,7 +76,7 @@ def lib():
                      "profile_attractive_end"):
             getattr(L, "tsne_hip_" + name).restype = c_int
         for name in ("locality_order", "gather_rows", "knn", "max_normalize", "perplexity", "symmetrize", "plan_create", "attractive",
-                     "repulsive", "update", "iterate", "sum_squares"):
+                     "repulsive", "update", "iterate", "sum_squares", "release_scratch"):
             getattr(L, "tsne_hip_" + name).restype = c_int
         _lib = L
     return _lib
@@ -98,6 +98,11 @@ def _stream():
 def _f32(t):
     assert t.is_cuda and t.dtype == torch.float32 and t.is_contiguous()
     return t
+
+
+def release_scratch():
+    """Gives back the device memory that the library keeps between calls."""
+    _check(lib().tsne_hip_release_scratch())
 
 
 def knn(points, num_neighbors):
