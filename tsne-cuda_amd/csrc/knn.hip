@@ -1188,7 +1188,8 @@ struct HalfScale {
     int not_finite;         // tiles without a finite ball
     float bound, bound_bf16;  // sums over the tiles of about what a distance within the tile may be off by, on either operand
     float log_reach;        // sum over the tiles of log2 of the most a point of theirs lies from the frame
-    float pad[3];
+    int unsure;             // sampled queries whose neighbours the bound may not tell from the rest (gap_kernel)
+    float pad[2];
 };
 
 // Frames first .. last - 1: distances of all tile centres to them, and every tile's nearest frame so far.  The first
@@ -1277,6 +1278,55 @@ __global__ __launch_bounds__(1024) void frame_kernel(const float *__restrict__ c
         atomicAdd(&scale->bound, sb);
         atomicAdd(&scale->bound_bf16, sb16);
         atomicAdd(&scale->log_reach, sl);
+    }
+}
+
+// Whether the bound leaves room between a query's K-th neighbour and the last candidate kept of it: for one point of each
+// sampled tile (`step` apart), the distances to the points of its neighbourhood in the numbering, the K-th and the
+// `want`-th smallest of them, and the tile's bound.  The gap among all points is smaller than that, a third to all of it.
+// One workgroup of 256 threads per sampled tile.
+__global__ __launch_bounds__(256) void gap_kernel(const float *__restrict__ X, int N, int D, int T, int step, int K, int want,
+                                                  const float *__restrict__ nearest, const float *__restrict__ radius,
+                                                  HalfScale *scale) {
+    constexpr int kEach = (2 * kHomeTiles + 1) * kCT / 256 + 1;
+    __shared__ int below[2];
+    const int tid = threadIdx.x, tile = min((int)blockIdx.x * step + step / 2, T - 1);
+    const int q = min(tile * kCT + 5, N - 1);
+    const int first = max(tile - kHomeTiles, 0) * kCT, last = min((tile + kHomeTiles + 1) * kCT, N);
+    const float *xq = X + (size_t)q * D;
+    unsigned int dist[kEach];
+#pragma unroll
+    for (int u = 0; u < kEach; ++u) {
+        const int j = first + u * 256 + tid;
+        const float *x = X + (size_t)min(j, last - 1) * D;
+        float sum = 0.0f;
+#pragma unroll 4
+        for (int d = 0; d < D; ++d) {
+            const float diff = xq[d] - x[d];
+            sum = fmaf(diff, diff, sum);
+        }
+        dist[u] = j < last && j != q ? __float_as_uint(sum) : ~0u;  // (not negative: ordered as its bits)
+    }
+    // The largest value that fewer than `rank` distances lie below.
+    auto ranked = [&](int rank) {
+        unsigned int value = 0u;
+        for (int b = 30, turn = 0; b >= 8; --b, turn ^= 1) {  // (23 bits: a relative 3e-5)
+            const unsigned int trial = value | (1u << b);
+            if (tid == 0) below[turn] = 0;
+            __syncthreads();
+            int c = 0;
+#pragma unroll
+            for (int u = 0; u < kEach; ++u) c += __popcll(__ballot(dist[u] < trial));
+            if ((tid & (kWave - 1)) == 0) atomicAdd(&below[turn], c);
+            __syncthreads();
+            if (below[turn] < rank) value = trial;
+        }
+        return __uint_as_float(value);
+    };
+    const float near_d = ranked(K - 1), far_d = ranked(want);
+    if (tid == 0) {
+        const float reach = sqrtf(nearest[tile]) + radius[tile];
+        if (!(4.0f * 4.0f / 4096.0f * reach * reach < far_d - near_d)) atomicAdd(&scale->unsure, 1);
     }
 }
 
@@ -3211,10 +3261,11 @@ int run_valu_sweep(const float *points, const float *Xt, int N, int Npad, int D,
 // Fewer dimensions: a step of 16 dimensions is mostly padding, tiles are small beside their frame, and bf16 terms
 // relative to the tile's own centre keep more.
 constexpr int kHalfDims = 5;
-constexpr float kPartCost = 0.02f;  // of a round, per part
+constexpr int kGapSamples = 128;
 // Halves relative to the frames lose more than two bf16 terms relative to the tiles where the points have structure that
-// kFrames frames do not follow.  Times as much as the sweep is let to be off by beside the other: one cloud in many
-// dimensions has 5 to 9 and verifies as well, hundreds of tight clusters 40 and more.
+// kFrames frames do not follow.  What counts is whether neighbours can be told from the rest, which a sample says (at
+// most one in 32 may be in doubt: 60000 x 20 in 300 clusters, 617 queries failed and were searched again, 4.5 ms, 2.5 on
+// bf16 terms); and beyond this many times the other sweep's bound that one is the better try.
 constexpr float kHalfLoss = 16.0f;
 
 // What the sweeps on halves take beside the points: made in three steps.
@@ -3237,7 +3288,9 @@ struct HalfOperands {
         tile_info.release();
     }
     // Frames of the tiles; *pays: whether the sweeps should multiply halves (false also where there is no room).
-    int frames(const float *centers_t, const float *radius, int D, int T, bool *pays, hipStream_t s) {
+    // (points of more dimensions than a wave holds are tried on a sample of query tiles anyway: `sample` false)
+    int frames(const float *points, const float *centers_t, const float *radius, int N, int D, int T, int K, int want, bool sample,
+               bool *pays, hipStream_t s) {
         *pays = false;
         dims = D;
         tiles = T;
@@ -3252,6 +3305,11 @@ struct HalfOperands {
                                                         frame_tile(), nearest(), tile_frame(), scale());
             TSNE_TRY(hipGetLastError());
         }
+        const int sampled = std::min(T, kGapSamples);
+        if (sample) {
+            gap_kernel<<<sampled, 256, 0, s>>>(points, N, D, T, T / sampled, K, want, nearest(), radius, scale());
+            TSNE_TRY(hipGetLastError());
+        }
         HalfScale host;
         TSNE_TRY(hipMemcpyAsync(&host, scale(), sizeof(host), hipMemcpyDeviceToHost, s));
         TSNE_TRY(hipStreamSynchronize(s));
@@ -3259,7 +3317,7 @@ struct HalfOperands {
         // ... and one scale serves all: beside a few tiles that reach 2^16 times as far as most, those lose bits.
         float reach;
         std::memcpy(&reach, &host.reach, sizeof(reach));
-        *pays = host.not_finite == 0 && host.bound <= kHalfLoss * host.bound_bf16 &&
+        *pays = host.not_finite == 0 && host.unsure * 32 <= sampled && host.bound <= kHalfLoss * host.bound_bf16 &&
                 std::log2(std::max(reach, 1e-30f)) <= host.log_reach / (float)T + 16.0f;
         return 0;
     }
@@ -3377,7 +3435,9 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         const SweepGeometry on_halves(N, D, Products::kHalf);
         bool pays = false;
         if (on_halves.fits(want))
-            if (const int rc = operands.frames(centers.as<float>(), radius.as<float>(), D, num_tiles, &pays, s)) return rc;
+            if (const int rc = operands.frames(points, centers.as<float>(), radius.as<float>(), N, D, num_tiles, K, want,
+                                               !chunked, &pays, s))
+                return rc;
         if (pays && operands.room(N, on_halves) && Xp.alloc_optional(sizeof(float4) * on_halves.tile_float4 * num_tiles)) {
             geometry = on_halves;
             if (operands.pack(points, centers.as<float>(), N, D, geometry, Xp.as<uint4>(), s)) return 1;
@@ -3467,13 +3527,15 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         // On halves below that the last round of the workgroups counts: what does not fill one is swept by several
         // workgroups per tile, in a launch of its own.
         const int whole = half && !chunked ? count / slots * slots : count, rest = count - whole;
-        // (Time in rounds; every part sweeps its own neighbourhood and keeps its own list, which costs some.)
+        // Every part sweeps a neighbourhood and keeps lists of its own, so parts only pay where they run beside each
+        // other on a chip that is half empty.  Whole searches, ms, in 1 / 2 / 4 / 8 parts: 157 tiles on 768 slots 1.58 /
+        // 1.33 / 1.43 / 1.77, 313 2.31 / 1.99 / 2.26 / 3.04, 424 2.68 / 2.55 / 3.06 / 3.81, 469 without structure 3.79 / 4.97 /
+        // 5.69 / 7.53; what 768 leave of 938 6.79 / 6.64 / 6.69 / 7.43, of 1172 6.81 / 6.15 / 6.33 / 7.18.
         int rest_parts = 1;
-        if (rest > 0) {
-            auto rounds = [&](int p) { return (float)div_up(rest * p, slots) / (float)p + kPartCost * (float)p; };
-            for (int p = 2; p <= 16 && p * keep <= 2048 && p * 2 * (2 * kHomeTiles + 1) <= num_tiles; p *= 2)
-                if (rounds(p) < rounds(rest_parts)) rest_parts = p;
-        }
+        if (rest > 0)
+            while (rest_parts < (whole > 0 ? 16 : 2) && rest * rest_parts * 2 <= slots + slots / 16 &&
+                   rest_parts * 2 * keep <= 2048 && rest_parts * 4 * (2 * kHomeTiles + 1) <= num_tiles)
+                rest_parts *= 2;
         const int grid = std::min(std::max(whole * parts, rest * rest_parts), slots);
         const size_t n_slots = (size_t)(tile_list || step != 1 ? count * kMQ : N);
         const size_t merged_rows = parts > 1 ? n_slots : rest_parts > 1 ? n_slots - (size_t)whole * kMQ : 0;
