@@ -12,7 +12,7 @@
 //     next, built in LDS by a group of lanes per row); a non-zero looks for its row
 //     number in the table of row j.  Large tables hold a byte of each column's hash
 //     and its place in the row instead: 16 bytes of a bucket answer most lookups,
-//     and the row itself the others;
+//     the row itself the others, and a pair is looked up once for both its entries;
 //   * scanning (small problems, more than 1638 neighbours, rows that name a column
 //     twice, or when the tables do not fit in memory): a group of lanes owns row i
 //     and the whole group scans each row j
@@ -151,29 +151,16 @@ __global__ __launch_bounds__(256) void build_tables_kernel(const float *__restri
     }
 }
 
-// 0x80 in every byte of w that is zero.
-__device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
-    return ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w | 0x7f7f7f7fu);
-}
-
-// Bound by the cache lines that the lookups touch, random ones.  TAGS: a lookup reads its bucket's tags first and ends
-// there unless one matches (50-dimensional Gaussians: one lookup in four finds its column); the match's place leads to
-// the row's own column and value.  Tags and places of a million rows of 90 neighbours are 256 MB where slots are 1 GB.
-// What that saves is not the kernels' time alone (lookups 2970 us in slots, 2340 in this form, 2580 with tags and
-// places in two arrays; 1547 with tags beside the slots, 1.15 GB) but the memory: a call that takes and returns over a
-// gigabyte waits for the driver to clear what the call before returned.  1,000,000 x 90, affinities called one after the other: 17.3 ms with tags beside the slots
-// (4.6 for a single call), 8.4 with slots alone, 5.4 in this form.
 constexpr size_t kTaggedBytes = (size_t)512 << 20;  // slots of more bytes than this are replaced by tags and places
-template <bool TAGS, typename PLACE>
+
+// Tables of slots.  Bound by the cache lines that the lookups touch, random ones.
 __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__restrict__ p, const int *__restrict__ idx,
                                                                 int N, int K, int log2_slots,
                                                                 const Slot *__restrict__ table,
-                                                                const Tagged<PLACE> *__restrict__ tagged,
                                                                 const int *__restrict__ flags, float *__restrict__ P) {
     if (flags[0] | flags[1]) return;  // (a column out of range: P stays as it is; one named twice: the scan writes it)
     const size_t nnz = (size_t)N * K;
     const double denom = 2.0 * (double)N;
-    const unsigned int buckets = 1u << (log2_slots - 4);
     for (size_t e0 = (size_t)blockIdx.x * 256; e0 < nnz; e0 += (size_t)gridDim.x * 256) {
         const size_t row0 = e0 / (unsigned int)K, e = e0 + threadIdx.x;
         if (e >= nnz) return;
@@ -181,7 +168,7 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
         const int j = idx[e];
         const float own = p[e];
         float found = 0.0f;
-        if (!TAGS && (unsigned int)j < (unsigned int)N) {
+        if ((unsigned int)j < (unsigned int)N) {
             const Slot *theirs = table + ((size_t)j << log2_slots);
             unsigned int at = hash_of(row) >> (32 - log2_slots);
             for (int seen = 1;; ++seen) {  // (an empty slot is always met)
@@ -194,19 +181,85 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
                 at = next_slot(at, seen, log2_slots);
             }
         }
-        if (TAGS && (unsigned int)j < (unsigned int)N) {
-            const unsigned int hash = hash_of(row), tag = tag_of(hash) * 0x01010101u;
+        P[e] = (float)((double)(own + found) / denom);
+    }
+}
+
+// Tables of tags and places, in two kernels.  A pair that both rows name has one value, p[i,j] + p[j,i] over 2 N, at two
+// places: it is looked up once, by the row of the smaller number, which finds the other place and writes both.  Before
+// that every entry is written as if its pair were named once (a point that names itself: twice its own).
+__global__ __launch_bounds__(256) void halve_entries_kernel(const float *__restrict__ p, const int *__restrict__ idx, int N, int K,
+                                                            const int *__restrict__ flags, float *__restrict__ P) {
+    if (flags[0] | flags[1]) return;  // (as above)
+    const size_t nnz = (size_t)N * K;
+    const double denom = 2.0 * (double)N;
+    for (size_t e0 = (size_t)blockIdx.x * 1024; e0 < nnz; e0 += (size_t)gridDim.x * 1024) {
+        const size_t row0 = e0 / (unsigned int)K;
+        const unsigned int in_row0 = (unsigned int)(e0 - row0 * K);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const unsigned int t = u * 256 + threadIdx.x;
+            if (e0 + t >= nnz) break;
+            const float own = p[e0 + t];
+            const bool self = idx[e0 + t] == (int)row0 + (int)((in_row0 + t) / (unsigned int)K);
+            P[e0 + t] = (float)((double)(own + (self ? own : 0.0f)) / denom);
+        }
+    }
+}
+
+// 0x80 in every byte of w that is zero.
+__device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
+    return ~(((w & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w | 0x7f7f7f7fu);
+}
+
+// Bound by the cache lines that the lookups touch, random ones, four lookups of a thread in flight.  A lookup reads its
+// bucket's tags first and ends there unless one matches (50-dimensional Gaussians: one lookup in four finds its column); the
+// match's place leads to the row's own column and value.  Tags and places of a million rows of 90 neighbours are 256 MB
+// where slots are 1 GB.  1,000,000 x 90, us: lookups in slots 2970; of every entry in this form 2340;
+// of a pair once 1397, and 187 for the entries as if named once.  (Tags beside the slots: 1547 and 1.15 GB.)
+constexpr int kLookups = 4;
+template <typename PLACE>
+__global__ __launch_bounds__(256) void symmetrize_pairs_kernel(const float *__restrict__ p, const int *__restrict__ idx, int N,
+                                                               int K, int log2_slots, const Tagged<PLACE> *__restrict__ tagged,
+                                                               const int *__restrict__ flags, float *__restrict__ P) {
+    if (flags[0] | flags[1]) return;  // (as above)
+    const size_t nnz = (size_t)N * K;
+    const double denom = 2.0 * (double)N;
+    const unsigned int buckets = 1u << (log2_slots - 4);
+    for (size_t e0 = (size_t)blockIdx.x * (256 * kLookups); e0 < nnz; e0 += (size_t)gridDim.x * (256 * kLookups)) {
+        const size_t row0 = e0 / (unsigned int)K;
+        const unsigned int in_row0 = (unsigned int)(e0 - row0 * K);
+        int row[kLookups], col[kLookups];  // (col < 0: nothing to look up)
+        uint4 first[kLookups];
+#pragma unroll
+        for (int u = 0; u < kLookups; ++u) {
+            const unsigned int t = u * 256 + threadIdx.x;
+            row[u] = (int)row0 + (int)((in_row0 + t) / (unsigned int)K);
+            col[u] = e0 + t < nnz ? idx[e0 + t] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < kLookups; ++u) {
+            if (col[u] <= row[u] || col[u] >= N) col[u] = -1;
+            const unsigned int bucket = (hash_of(row[u]) >> (32 - log2_slots)) / kBucket;
+            first[u] = make_uint4(0u, 0u, 0u, 0u);
+            if (col[u] >= 0)
+                first[u] = *reinterpret_cast<const uint4 *>(tagged[((size_t)col[u] << (log2_slots - 4)) + bucket].tags);
+        }
+#pragma unroll
+        for (int u = 0; u < kLookups; ++u) {
+            if (col[u] < 0) continue;
+            const unsigned int hash = hash_of(row[u]), tag = tag_of(hash) * 0x01010101u;
             unsigned int bucket = (hash >> (32 - log2_slots)) / kBucket;
-            const Tagged<PLACE> *theirs = tagged + ((size_t)j << (log2_slots - 4));
-            const size_t their_row = (size_t)j * K;
-            for (unsigned int visited = 0; visited < buckets; ++visited) {
-                const uint4 t = *reinterpret_cast<const uint4 *>(theirs[bucket].tags);
+            const Tagged<PLACE> *theirs = tagged + ((size_t)col[u] << (log2_slots - 4));
+            const size_t their_row = (size_t)col[u] * K;
+            uint4 t = first[u];
+            for (unsigned int visited = 0;;) {
                 const unsigned int w[4] = {t.x, t.y, t.z, t.w};
                 unsigned int empty = 0u, matches = 0u;  // (matches: a bit per slot of the bucket)
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    empty |= zero_bytes(w[u]);
-                    matches |= (((zero_bytes(w[u] ^ tag) >> 7) * 0x10204080u) >> 28) << (4 * u);
+                for (int k = 0; k < 4; ++k) {
+                    empty |= zero_bytes(w[k]);
+                    matches |= (((zero_bytes(w[k] ^ tag) >> 7) * 0x10204080u) >> 28) << (4 * k);
                 }
                 bool hit = false;
                 while (matches && !hit) {
@@ -214,16 +267,17 @@ __global__ __launch_bounds__(256) void symmetrize_hashed_kernel(const float *__r
                     matches &= matches - 1u;
                     const int key = idx[at];
                     const float value = p[at];
-                    if (key == row) {
-                        found = value;
+                    if (key == row[u]) {
+                        const size_t e = e0 + u * 256 + threadIdx.x;
+                        P[e] = P[at] = (float)((double)(p[e] + value) / denom);
                         hit = true;
                     }
                 }
-                if (hit || empty) break;
+                if (hit || empty || ++visited == buckets) break;
                 bucket = (bucket + 1u) & (buckets - 1u);
+                t = *reinterpret_cast<const uint4 *>(theirs[bucket].tags);
             }
         }
-        P[e] = (float)((double)(own + found) / denom);
     }
 }
 
@@ -291,12 +345,16 @@ int launch_symmetrize(const float *p, const int *idx, int N, int K, float *P, hi
                     build_tables_kernel<64><<<div_up(N, 4), 256, sizeof(Slot) * 4 << log2_slots, s>>>(
                         p, idx, N, K, log2_slots, table, words, flags);
                 const int grid = (int)std::min<int64_t>(div_up((int64_t)N * K, 256), 1 << 20);
-                if (!tagged)
-                    symmetrize_hashed_kernel<false><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, flags, P);
-                else if (narrow)
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, bytes, flags, P);
-                else
-                    symmetrize_hashed_kernel<true><<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, words, flags, P);
+                if (!tagged) {
+                    symmetrize_hashed_kernel<<<grid, 256, 0, s>>>(p, idx, N, K, log2_slots, table, flags, P);
+                } else {
+                    const int by_four = (int)std::min<int64_t>(div_up((int64_t)N * K, 1024), 1 << 18);
+                    halve_entries_kernel<<<by_four, 256, 0, s>>>(p, idx, N, K, flags, P);
+                    if (narrow)
+                        symmetrize_pairs_kernel<<<by_four, 256, 0, s>>>(p, idx, N, K, log2_slots, bytes, flags, P);
+                    else
+                        symmetrize_pairs_kernel<<<by_four, 256, 0, s>>>(p, idx, N, K, log2_slots, words, flags, P);
+                }
                 e = hipGetLastError();
             }
             if (e == hipSuccess) e = hipMemcpyAsync(raised, flags, sizeof(raised), hipMemcpyDeviceToHost, s);
