@@ -216,7 +216,7 @@ __device__ __forceinline__ unsigned int zero_bytes(unsigned int w) {
 // bucket's tags first and ends there unless one matches (50-dimensional Gaussians: one lookup in four finds its column); the
 // match's place leads to the row's own column and value.  Tags and places of a million rows of 90 neighbours are 256 MB
 // where slots are 1 GB.  1,000,000 x 90, us: lookups in slots 2970; of every entry in this form 2340;
-// of a pair once 1397, and 187 for the entries as if named once.  (Tags beside the slots: 1547 and 1.15 GB.)
+// of a pair once 1397, and 187 for the entries as if named once.
 constexpr int kLookups = 4;
 template <typename PLACE>
 __global__ __launch_bounds__(256) void symmetrize_pairs_kernel(const float *__restrict__ p, const int *__restrict__ idx, int N,
