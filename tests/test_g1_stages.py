@@ -1511,6 +1511,22 @@ def test_knn_on_halves(stages, n, d, k, kind):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("k", [45, 90, 150, 172])
+def test_knn_on_halves_with_many_equal_points(stages, k):
+    """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles
+    ends and the next begins with as many candidates as a list has room for, and few enough tiles are involved that no rank
+    among them lowers the threshold.  The rows are the vector sweep's all the same."""
+    n, d = 200000, 8
+    rng = np.random.default_rng(k)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    ends = np.r_[0:1536, n - 1536:n]
+    X[ends[np.arange(ends.size) % 50 != 0]] = X[100000]
+    idx, d2, stats = stages.knn_select(dev(X), k, 0)
+    assert stats[0] == 1
+    idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
 @pytest.mark.parametrize("n,kind", [(2, "plain"), (640, "plain"), (7680, "plain"), (7681, "line"), (15361, "far"),
                                     (20480, "one box"), (20481, "plain"), (9001, "equal"), (5003, "not a number"),
                                     (12000, "boxes' edges")])

@@ -2279,10 +2279,13 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
                 const u64 crowded = __ballot(my_fill() > half - kCT / 2);
                 mask = (unsigned int)(crowded | (crowded >> 32));  // lanes l, l+32 share a query
             }
-            const bool rank = round_over && nxt >= 0;
-            if (mask) {
+            // (A list whose counted entries are too few for a rank keeps all it has, full or not, and so may one whose
+            // entries are equally far: those are compacted like any other before the next tile.)
+            for (bool rank = round_over && nxt >= 0; mask; rank = false) {
                 const int slack = cold()->select_slack;
                 select_queries(mask, rank ? cold()->ranks[round - 1] : want, rank || nxt < 0 ? 0 : slack, rank);
+                const u64 crowded = rank ? __ballot(my_fill() > half - kCT / 2) : 0ull;
+                mask = (unsigned int)(crowded | (crowded >> 32));
             }
             if (home_done) {
                 home = false;
