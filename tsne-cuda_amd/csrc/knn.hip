@@ -653,7 +653,9 @@ __device__ __forceinline__ int select_halves(u64 *list, int want, int slack, boo
         }
         limit = hi;
         if (at_hi > want + slack && !counted) ties = want - at_under;  // (equal distances: as many of them as there is room for)
-        if (lane == 0) *thr = ((u64)limit << 32) | 0xffffffffull;
+        // (Entries pass up to 4e-7 beyond the threshold of the moment: with fewer than `want` within it, as a rank among
+        // few leaves them, the want-th may be one of those.)
+        if (lane == 0) *thr = min(*thr, ((u64)limit << 32) | 0xffffffffull);
     }
     int base = 0, equal = 0;
 #pragma unroll
