@@ -1482,21 +1482,28 @@ def test_loop_and_symmetrisation_without_room_for_the_faster_form(stages, monkey
         assert same_bits(a, b)
 
 
-@pytest.mark.parametrize("n,d,k,kind", [
-    (16500, 5, 2, "plain"), (16513, 16, 20, "grid"), (17003, 17, 33, "clusters"), (17003, 64, 172, "plain"),
-    (17003, 65, 173, "plain"), (16640, 126, 129, "clusters"), (16500, 127, 20, "grid"), (16500, 192, 20, "clusters"),
-    (16500, 193, 33, "plain"), (20000, 30, 25, "far"), (20000, 30, 25, "one far point"), (98304, 12, 60, "grid"),
-    (98433, 8, 20, "plain"), (100003, 20, 90, "clumps"), (131200, 24, 33, "clusters"), (100003, 3, 45, "clumps")])
-def test_knn_on_halves(stages, n, d, k, kind):
+@pytest.mark.parametrize("n,d,k,kind,halves", [
+    (16500, 5, 2, "plain", True), (16513, 16, 20, "grid", True), (17003, 17, 33, "clusters", True),
+    (17003, 64, 172, "plain", True), (17003, 65, 172, "plain", True), (17003, 65, 173, "plain", False),
+    (16640, 126, 129, "clusters", True), (16500, 127, 20, "grid", True), (16500, 192, 20, "clusters", True),
+    (16500, 193, 33, "plain", True), (20000, 30, 25, "far", True), (20000, 30, 25, "one far point", False),
+    (98304, 12, 60, "grid", True), (98433, 8, 20, "plain", True), (100003, 20, 33, "clumps", True),
+    (100003, 20, 90, "clumps", False), (131200, 24, 33, "clusters", True), (100003, 3, 45, "clumps", False),
+    (60000, 20, 45, "300 clusters", False)])
+def test_knn_on_halves(stages, monkeypatch, n, d, k, kind, halves):
     """The search's own choice of sweep - on halves relative to frames, beyond four dimensions - gives the vector sweep's
     rows, bit for bit: at the remainders of a step of 16 dimensions and of a chunk of 64, at the most neighbours the
     register-resident form keeps, with whole rounds of query tiles and what is left of one (from 98304 points on, where
-    thresholds are set ahead of the lists), with equal distances, neighbours that lie forty to a tile, points far from
-    the origin and one point far from all others."""
+    thresholds are set ahead of the lists), with equal distances, neighbours that lie forty to a tile and points far from
+    the origin.  It is the sweep on halves that ran (TSNE_KNN_PRODUCTS=half makes anything else an error), with few
+    queries to redo; and it does not run where it keeps too few candidates, in three dimensions, beside one point far from
+    all others, among more clusters than there are frames and where the neighbours fill two clumps and a part of a third."""
     rng = np.random.default_rng(n + d)
     X = rng.standard_normal((n, d)).astype(np.float32)
     if kind == "clusters":
         X += (8.0 * rng.standard_normal((5, d)))[np.arange(n) * 5 // n].astype(np.float32)
+    elif kind == "300 clusters":
+        X += (30.0 * rng.standard_normal((300, d)))[np.arange(n) * 300 // n].astype(np.float32)
     elif kind == "grid":
         X = np.round(2.0 * X).astype(np.float32)
     elif kind == "clumps":
@@ -1505,22 +1512,32 @@ def test_knn_on_halves(stages, n, d, k, kind):
         X += np.float32(300.0)
     elif kind == "one far point":
         X[7] = 1e9
-    idx, d2, stats = stages.knn_select(dev(X), k, 0)
-    assert stats[0] == 1
-    idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+    dX = dev(X)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    if halves:
+        idx, d2, stats = stages.knn_select(dX, k, 0)
+        assert stats[0] == 1 and stats[1] <= (n // 256 if kind == "plain" else n // 10)
+    else:
+        with pytest.raises(RuntimeError, match="TSNE_KNN_PRODUCTS"):
+            stages.knn_select(dX, k, 0)
+        monkeypatch.delenv("TSNE_KNN_PRODUCTS")
+        idx, d2, _ = stages.knn_select(dX, k, 0)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
 @pytest.mark.parametrize("k", [45, 90, 150, 172])
-def test_knn_on_halves_with_many_equal_points(stages, k):
+def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles
     ends and the next begins with as many candidates as a list has room for, and few enough tiles are involved that no rank
-    among them lowers the threshold.  The rows are the vector sweep's all the same."""
+    among them lowers the threshold.  The rows are the vector sweep's all the same, those of the sweep on halves among them."""
     n, d = 200000, 8
     rng = np.random.default_rng(k)
     X = rng.standard_normal((n, d)).astype(np.float32)
     ends = np.r_[0:1536, n - 1536:n]
     X[ends[np.arange(ends.size) % 50 != 0]] = X[100000]
+    if k < 172:  # (for so many neighbours more queries fail than the sweep on halves may leave: bf16 terms after it)
+        monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
     idx, d2, stats = stages.knn_select(dev(X), k, 0)
     assert stats[0] == 1
     idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)

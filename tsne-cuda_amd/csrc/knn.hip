@@ -3379,6 +3379,15 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     TSNE_TRY(hipGetDevice(&device));
     TSNE_TRY(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
 
+    // TSNE_KNN_PRODUCTS (measurements and tests of the search's own choice): bf16 never multiplies halves, half is an
+    // error wherever the rows would not all come from a sweep on halves and its re-rank.
+    const char *products = mode == 0 && !probes ? std::getenv("TSNE_KNN_PRODUCTS") : nullptr;
+    const bool halves_only = products && std::strcmp(products, "half") == 0;
+    if (products && std::strcmp(products, "bf16") == 0) halves = false;
+    auto not_on_halves = [](const char *why) {
+        set_error("knn: TSNE_KNN_PRODUCTS=half, but this search %s", why);
+        return 1;
+    };
     SweepGeometry geometry(N, D, mode == 3 ? Products::kFloats : Products::kBf16);
     if (mode == 3) mode = 2;
     const bool chunked = geometry.chunked;
@@ -3413,6 +3422,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         TSNE_TRY(hipGetLastError());
         return 0;
     };
+    if (halves_only && (!use_mfma || direct_search_pays(N, K))) return not_on_halves("is of few points or many neighbours");
     if (mode == 0 && direct_search_pays(N, K) && K - 1 <= kDirectNeighbors) {
         const int rc = run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
         if (rc != kNoRoom) return rc;
@@ -3452,6 +3462,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         }
     }
     const bool half = geometry.half, bf16 = geometry.bf16, bf16_chunked = geometry.bf16_chunked;
+    if (halves_only && !half) return not_on_halves("does not choose them");
     const int Dnorm = geometry.Dnorm, ksteps = geometry.ksteps, n_chunks = geometry.n_chunks;
     const int steps16 = geometry.steps16, bitmap_words = geometry.bitmap_words;
     const int S4 = geometry.slots;
@@ -3660,6 +3671,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     unsigned long long swept = 0;
     // Points that the halves cannot tell apart: everything once more on two bf16 terms.
     auto without_halves = [&]() -> int {
+        if (halves_only) return not_on_halves("returns from them");
         Xp.release();
         operands.release();
         centers.release();
