@@ -1544,6 +1544,22 @@ def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("n,d,size", [(16500, 5, 1e-19), (16500, 5, 2e-20), (17003, 20, 1e-15), (16500, 130, 1e-19),
+                                      (17003, 20, 1e-10)])
+def test_knn_of_points_whose_squares_underflow(stages, monkeypatch, n, d, size):
+    """Points so near each other that their squared coordinates lose bits or vanish are not searched on halves, whose bound
+    rests on those; the vector sweep's rows, bit for bit (also where all is large enough, 1e-10)."""
+    x = (size * np.random.default_rng(n).standard_normal((n, d))).astype(np.float32)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    if size < 1e-12:
+        with pytest.raises(RuntimeError, match="does not choose them"):
+            stages.knn(dev(x), 20)
+        monkeypatch.delenv("TSNE_KNN_PRODUCTS")
+    idx, d2 = stages.knn(dev(x), 20)
+    idx_v, d2_v, _ = stages.knn_select(dev(x), 20, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
 @pytest.mark.parametrize("n,kind", [(2, "plain"), (640, "plain"), (7680, "plain"), (7681, "line"), (15361, "far"),
                                     (20480, "one box"), (20481, "plain"), (9001, "equal"), (5003, "not a number"),
                                     (12000, "boxes' edges")])

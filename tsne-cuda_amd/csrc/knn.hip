@@ -55,6 +55,7 @@
 //    every tile's candidates over several workgroups; a merge kernel reduces
 //    their lists to what a single list would have kept.
 #include "common.h"
+#include "half_bound.h"
 #include "stages.h"
 
 #include <algorithm>
@@ -1370,7 +1371,7 @@ __device__ __forceinline__ float half_scale_factor(const HalfScale *scale) {
 // One workgroup per tile.  Xh: [tile][block of 32 points (4)][step of 16 dimensions (S)][lane (64)] 8 halves, lane = 32 *
 // (dimension % 16 / 8) + point % 32, element = dimension % 8 (the layout of pack_points_bf16_kernel, one term).
 // beta: row f of `pitch` floats holds beta_f of every point.  point_len: |x'| and |x' - what the halves stand for|,
-// rounded up.  tile_info: the largest of the second and of |x'| among a tile's points, and the tile's frame.
+// rounded up (half_bound.h has what the sweeps make of them).  tile_info: the largest of the second and of |x'| among a tile's points, and the tile's frame.
 __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict__ X, int N, int D, int S,
                                                         const float *__restrict__ frames, const int *__restrict__ tile_frame,
                                                         const HalfScale *scale, int pitch, uint4 *__restrict__ Xh,
@@ -1414,7 +1415,7 @@ __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict_
         const float other = dot[f] + __shfl_xor(dot[f], 32, kWave);
         if ((f & 1) == h) beta[(size_t)f * pitch + i] = fmaf(-2.0f, other, len);
     }
-    const float xl = sqrtf(len) * (1.0f + 1e-3f), xe = sqrtf(eps) * (1.0f + 1e-3f);
+    const float xl = length_bound(len, D), xe = length_bound(eps, D);
     if (h == 0) point_len[i] = make_float2(xl, xe);
     const float me = group_max<kWave>(xe), ml = group_max<kWave>(xl);
     if (lane == 0) {
@@ -1426,30 +1427,6 @@ __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict_
         tile_info[tile] = make_float4(fmaxf(fmaxf(wave_eps[0], wave_eps[1]), fmaxf(wave_eps[2], wave_eps[3])),
                                       fmaxf(fmaxf(wave_len[0], wave_len[1]), fmaxf(wave_len[2], wave_len[3])),
                                       __int_as_float(own), 0.0f);
-}
-
-// A query's side of the bound: what is subtracted from a distance of the sweep on halves to make it a lower bound.
-//  - q' and x' are kept as halves: |q'.x' - (their halves)| <= |q'| e_x + e_q (|x'| + e_x), e what the halves lose;
-//  - D products are accumulated in fp32 onto -beta / 2, in the matrix unit's order, and beta itself is a sum of D
-//    rounded terms: 5 (D + 8) 2^-24 (the factor covers that order) times the magnitudes, 2 |q'||x'| + |x'|^2 + 2 |f - c||x'|;
-//  - |q - c|^2 is a sum of D rounded terms too, (|q'| + |f - c|)^2 at most, taken in a known order: 1.25 (D + 8) 2^-24.
-struct HalfQuery {
-    float len, eps, kap;      // |q'|, what its halves lose, 5 (D + 8) 2^-24
-    float off, frame_len;     // lower bound of |q - c|^2, and |f - c|, of the candidate frame at hand
-    int frame;                // that frame (-1: none yet)
-};
-// (d2, frame_len: |f - c|^2, and |f - c| rounded up)
-__device__ __forceinline__ void enter_frame(HalfQuery &hq, int frame, float beta_q, float d2, float frame_len) {
-    hq.frame = frame;
-    hq.frame_len = frame_len;
-    const float reach = hq.len + hq.frame_len;
-    hq.off = beta_q + d2 - 0.25f * hq.kap * reach * reach;
-}
-// |q - c|^2 less the bound for a tile (its tile_info).
-__device__ __forceinline__ float tile_offset(const HalfQuery &hq, float tile_eps, float tile_len) {
-    const float split = hq.len * tile_eps + hq.eps * (tile_len + tile_eps);
-    const float sums = tile_len * (2.0f * hq.len + tile_len + 2.0f * hq.frame_len);
-    return hq.off - (2.02f * split + hq.kap * sums);
 }
 
 constexpr int kRankRounds = 3;
@@ -2091,7 +2068,7 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
             for (int k = 0; k < S; ++k) bq[k] = __builtin_bit_cast(v8h, src[k * 64]);
         }
         const float2 len = cold()->point_len[q];
-        hq = {len.x, len.y, 5.0f * (float)(D + 8) * 5.9604644775390625e-08f, 0.0f, 0.0f, -1};
+        hq = half_query(len.x, len.y, D, back);
         const int own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(args.tile_info[qt].z));
         tile_beta = args.beta + (size_t)own_frame * args.beta_pitch;
 
@@ -2102,7 +2079,7 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
         float next_beta = 0.0f;
         const float *const query_beta = args.beta + q;
         const float my_d2 = args.frame_d2[own_frame * kFrames + (lane & (kFrames - 1))];  // a frame per lane
-        const float my_frame_len = sqrtf(my_d2) * (1.0f + 1e-3f);
+        const float my_frame_len = length_bound(my_d2, D);
         auto fetch_info = [&](int tile) {
             const int t = __builtin_amdgcn_readfirstlane(tile);
             ConstFloat *of_tile = as_const(args.tile_info) + 4 * (size_t)t;  // (scalar loads)
@@ -2455,13 +2432,11 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             cnt[tid] = 0;
         }
         const float q_len = BF16 && q < N ? sqrtf(args.norms[q]) * (1.0f + 1e-6f) : 0.0f;  // |q|, rounded up
-        HalfQuery hq = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, -1};
+        HalfQuery hq = {};
         int own_frame = 0;
         if constexpr (HALF) {
             const float2 len = args.point_len[q];
-            hq.len = len.x;
-            hq.eps = len.y;
-            hq.kap = 5.0f * (float)(D + 8) * 5.9604644775390625e-08f;
+            hq = half_query(len.x, len.y, D, half_back);
             own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(args.tile_info[qt].z));
             tile_beta = args.beta + (size_t)own_frame * args.beta_pitch;
         }
@@ -2595,7 +2570,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 const int frame = __builtin_amdgcn_readfirstlane(__float_as_int(info.z));
                 if (frame != hq.frame) {
                     const float d2 = args.frame_d2[own_frame * kFrames + frame];
-                    enter_frame(hq, frame, args.beta[(size_t)frame * args.beta_pitch + q], d2, sqrtf(d2) * (1.0f + 1e-3f));
+                    enter_frame(hq, frame, args.beta[(size_t)frame * args.beta_pitch + q], d2, length_bound(d2, D));
                 }
                 off = tile_offset(hq, info.x, info.y);
                 limit_acc = ((off - limit_d) - 4e-7f * (fabsf(off) + fabsf(limit_d))) * half_s2;
@@ -3322,8 +3297,9 @@ struct HalfOperands {
         // ... and one scale serves all: beside a few tiles that reach 2^16 times as far as most, those lose bits.
         float reach;
         std::memcpy(&reach, &host.reach, sizeof(reach));
+        // ... and points mostly within 1e-12 of their frames lose their squares to underflow, and the bound its grip.
         *pays = host.not_finite == 0 && host.unsure * 32 <= sampled && host.bound <= kHalfLoss * host.bound_bf16 &&
-                std::log2(std::max(reach, 1e-30f)) <= host.log_reach / (float)T + 16.0f;
+                std::log2(std::max(reach, 1e-30f)) <= host.log_reach / (float)T + 16.0f && host.log_reach >= -40.0f * (float)T;
         return 0;
     }
     bool room(int N, const SweepGeometry &g) {
