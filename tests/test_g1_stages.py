@@ -1544,6 +1544,23 @@ def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("n,d,k", [(20000, 30, 25), (100003, 12, 90), (20011, 150, 33)])
+def test_knn_on_halves_without_room_for_its_lists(stages, monkeypatch, n, d, k):
+    """Room for the operands of the sweep on halves but not for its lists, the largest of what it takes: the search does
+    without halves instead of failing."""
+    rng = np.random.default_rng(n)
+    dX = dev((rng.standard_normal((n, d)) + (8.0 * rng.standard_normal((5, d)))[np.arange(n) * 5 // n]).astype(np.float32))
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    stages.knn(dX, k)
+    monkeypatch.setenv("TSNE_SCRATCH_LIMIT", str(40 << 20))
+    with pytest.raises(RuntimeError, match="returns from them"):
+        stages.knn(dX, k)
+    monkeypatch.delenv("TSNE_KNN_PRODUCTS")
+    idx, d2 = stages.knn(dX, k)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
 @pytest.mark.parametrize("n,d,size", [(16500, 5, 1e-19), (16500, 5, 2e-20), (17003, 20, 1e-15), (16500, 130, 1e-19),
                                       (17003, 20, 1e-10)])
 def test_knn_of_points_whose_squares_underflow(stages, monkeypatch, n, d, size):

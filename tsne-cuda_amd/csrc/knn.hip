@@ -3532,10 +3532,12 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         const size_t n_slots = (size_t)(tile_list || step != 1 ? count * kMQ : N);
         const size_t merged_rows = parts > 1 ? n_slots : rest_parts > 1 ? n_slots - (size_t)whole * kMQ : 0;
         DeviceMem lists, cand, tau, part_keys;
+        // (on halves the lists are longer than on bf16 terms, up to three times, and the search goes on without them)
         auto alloc_lists = [&]() -> bool {
-            return lists.alloc(sizeof(u64) * (size_t)grid * kMQ * cap) && cand.alloc(sizeof(int) * n_slots * keep) &&
-                   tau.alloc(sizeof(float) * n_slots) &&
-                   (merged_rows == 0 || part_keys.alloc(sizeof(u64) * merged_rows * std::max(parts, rest_parts) * keep));
+            const auto get = [&](DeviceMem &m, size_t bytes) { return half ? m.alloc_optional(bytes) : m.alloc(bytes); };
+            return get(lists, sizeof(u64) * (size_t)grid * kMQ * cap) && get(cand, sizeof(int) * n_slots * keep) &&
+                   get(tau, sizeof(float) * n_slots) &&
+                   (merged_rows == 0 || get(part_keys, sizeof(u64) * merged_rows * std::max(parts, rest_parts) * keep));
         };
         bool room = alloc_lists();
         if (!room && centre_dist.p) {
@@ -3544,8 +3546,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
             room = alloc_lists();
         }
         if (!room) {
-            set_error("knn: out of device memory for the candidate lists");
-            return kNoRoom;
+            (void)hipGetLastError();
+            return no_room("candidate lists");
         }
         TSNE_TRY(hipMemsetAsync(scal.as<int>() + 1, 0, 3 * sizeof(int), s));
         SweepArgs args;
@@ -3645,12 +3647,11 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
 
     int failed = 0;
     unsigned long long swept = 0;
-    // Points that the halves cannot tell apart: everything once more on two bf16 terms.
+    // Points that the halves cannot tell apart, or no room for their lists: everything once more on two bf16 terms.
     auto without_halves = [&]() -> int {
         if (halves_only) return not_on_halves("returns from them");
-        Xp.release();
+        for (DeviceMem *m : {&Xp, &centers, &radius, &scal, &fail_list}) m->release();
         operands.release();
-        centers.release();
         return search(points, N, D, K, indices, sq_dist, s, mode, stats, probes, renumbered, false);
     };
     // The verification needs the distance gap between neighbour K and candidate K' to exceed the rounding
@@ -3662,7 +3663,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         const int sample_tiles = 16, step = num_qtiles / sample_tiles;
         bool verified = false;
         for (int attempt = 0; attempt < 3 && !verified; ++attempt) {
-            if (const int rc = sweep_and_rerank(want, nullptr, step / 2, step, sample_tiles, failed, swept)) return rc;
+            if (const int rc = sweep_and_rerank(want, nullptr, step / 2, step, sample_tiles, failed, swept))
+                return rc == kNoRoom && half ? without_halves() : rc;
             if (failed * 10 <= sample_tiles * kMQ) {
                 verified = true;
             } else {
@@ -3677,7 +3679,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
             return run_valu_sweep(caller_points, Xt.as<float>(), N, Npad, D, K, nullptr, N, cus, indices, sq_dist, s);
         }
     }
-    if (const int rc = sweep_and_rerank(want, nullptr, 0, 1, num_qtiles, failed, swept)) return rc;
+    if (const int rc = sweep_and_rerank(want, nullptr, 0, 1, num_qtiles, failed, swept))
+        return rc == kNoRoom && half ? without_halves() : rc;
     if (half && !chunked && failed > N / 64) return without_halves();
     if (stats) {
         stats[0] = 1;
@@ -3707,11 +3710,14 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
                 unsigned long long swept_again = 0;
                 if (const int rc =
                         sweep_and_rerank(wider, tile_list.as<int>(), 0, 1, (int)tiles.size(), failed, swept_again))
-                    return rc;
+                    return rc == kNoRoom && half ? without_halves() : rc;
             }
         }
     }
     if (failed > 0) {
+        Xp.release();  // (room for what follows)
+        Bp.release();
+        operands.release();
         if (renumbered) {
             rename_list_kernel<<<div_up(failed, 256), 256, 0, s>>>(renumbered->order, failed, fail_list.as<int>());
             TSNE_TRY(hipGetLastError());
