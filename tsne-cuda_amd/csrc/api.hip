@@ -346,7 +346,7 @@ int tsne_hip_max_normalize(float *values, int64_t n, void *stream) {
     TSNE_REQUIRE(values && n > 0, "max_normalize: need a non-empty array");
     hipStream_t s = (hipStream_t)stream;
     float *scratch = nullptr;
-    TSNE_TRY(hipMalloc(&scratch, sizeof(float)));
+    TSNE_TRY(device_malloc(&scratch, sizeof(float)));
     int rc = launch_max_normalize(values, n, scratch, s);
     if (!rc && hipStreamSynchronize(s) != hipSuccess) {
         set_error("max_normalize: stream synchronisation failed");
@@ -474,26 +474,26 @@ int tsne_hip_plan_create(tsne_hip_plan **plan, int num_points, int num_neighbors
         p->stream_grid = cus + cus / 2;
     }
     // yxy carries one spare pair so that two-point (float4) loads may straddle the end.
-    bool ok = hipMalloc(&p->yxy, sizeof(float2) * (N + 2)) == hipSuccess &&
-              hipMalloc(&p->tile_xy, sizeof(float2) * N) == hipSuccess &&
-              hipMalloc(&p->tile_perm, sizeof(int) * N) == hipSuccess &&
-              hipMalloc(&p->tile_count, sizeof(int) * kMaxTiles) == hipSuccess &&
-              hipMalloc(&p->tile_cursor, sizeof(int) * kMaxTiles) == hipSuccess &&
-              hipMalloc(&p->point_code, sizeof(unsigned int) * N) == hipSuccess &&
-              hipMalloc(&p->wg_tile_base, sizeof(int) * (size_t)kSortBlocks * kMaxTiles) == hipSuccess &&
-              hipMalloc(&p->chunks, sizeof(int4) * p->max_chunks) == hipSuccess &&
-              hipMalloc(&p->num_chunks, 2 * sizeof(int)) == hipSuccess &&
-              hipMalloc(&p->box_moments, moment_bytes) == hipSuccess &&
-              hipMalloc(&p->centre_parts, sizeof(double2) * 2 * kMaxCentreParts) == hipSuccess &&
-              hipMalloc(&p->node_potentials, sizeof(float4) * G2) == hipSuccess &&
-              hipMalloc(&p->row_spectra, sizeof(float2) * spec) == hipSuccess &&
-              hipMalloc(&p->col_results, sizeof(float2) * spec) == hipSuccess &&
-              hipMalloc(&p->kernel_rows, sizeof(float) * (size_t)(kFft / 2 + 1) * kNodePad) == hipSuccess &&
-              hipMalloc(&p->twiddles, sizeof(float2) * kFft) == hipSuccess &&
-              hipMalloc(&p->twiddles_short, sizeof(float2) * kFftShort) == hipSuccess &&
-              hipMalloc(&p->scalars, sizeof(LoopScalars)) == hipSuccess &&
-              hipMalloc(&p->attr, sizeof(float) * 2 * N) == hipSuccess &&
-              hipMalloc(&p->rep, sizeof(float) * 2 * N) == hipSuccess;
+    bool ok = device_malloc(&p->yxy, sizeof(float2) * (N + 2)) == hipSuccess &&
+              device_malloc(&p->tile_xy, sizeof(float2) * N) == hipSuccess &&
+              device_malloc(&p->tile_perm, sizeof(int) * N) == hipSuccess &&
+              device_malloc(&p->tile_count, sizeof(int) * kMaxTiles) == hipSuccess &&
+              device_malloc(&p->tile_cursor, sizeof(int) * kMaxTiles) == hipSuccess &&
+              device_malloc(&p->point_code, sizeof(unsigned int) * N) == hipSuccess &&
+              device_malloc(&p->wg_tile_base, sizeof(int) * (size_t)kSortBlocks * kMaxTiles) == hipSuccess &&
+              device_malloc(&p->chunks, sizeof(int4) * p->max_chunks) == hipSuccess &&
+              device_malloc(&p->num_chunks, 2 * sizeof(int)) == hipSuccess &&
+              device_malloc(&p->box_moments, moment_bytes) == hipSuccess &&
+              device_malloc(&p->centre_parts, sizeof(double2) * 2 * kMaxCentreParts) == hipSuccess &&
+              device_malloc(&p->node_potentials, sizeof(float4) * G2) == hipSuccess &&
+              device_malloc(&p->row_spectra, sizeof(float2) * spec) == hipSuccess &&
+              device_malloc(&p->col_results, sizeof(float2) * spec) == hipSuccess &&
+              device_malloc(&p->kernel_rows, sizeof(float) * (size_t)(kFft / 2 + 1) * kNodePad) == hipSuccess &&
+              device_malloc(&p->twiddles, sizeof(float2) * kFft) == hipSuccess &&
+              device_malloc(&p->twiddles_short, sizeof(float2) * kFftShort) == hipSuccess &&
+              device_malloc(&p->scalars, sizeof(LoopScalars)) == hipSuccess &&
+              device_malloc(&p->attr, sizeof(float) * 2 * N) == hipSuccess &&
+              device_malloc(&p->rep, sizeof(float) * 2 * N) == hipSuccess;
     if (ok) {
         std::vector<float2> tw(kFft), tws(kFftShort);
         for (int k = 0; k < kFft; ++k) {

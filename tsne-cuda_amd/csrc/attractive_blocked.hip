@@ -800,7 +800,7 @@ static int balanced_strips(const int *indices, int N, int K, int n_parts, int ma
                            hipStream_t s) {
     const int micro = div_up(N, kMicroRows), words = div_up(n_parts, 32);
     unsigned int *d_bits = nullptr;
-    TSNE_TRY(hipMalloc(&d_bits, sizeof(unsigned int) * (size_t)micro * words));
+    TSNE_TRY(device_malloc(&d_bits, sizeof(unsigned int) * (size_t)micro * words));
     micro_strip_parts_kernel<<<micro, 256, sizeof(unsigned int) * words, s>>>(indices, N, K, words, d_bits);
     std::vector<unsigned int> bits((size_t)micro * words);
     hipError_t err = hipGetLastError();
@@ -946,7 +946,7 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
     // A strip's list: the run starts (padded: the force kernel reads two past the last run) and the partitions.
     p->list_words = (n_parts + 4 + 3) & ~3;
     p->seg_stride = 4 + p->list_words + ((n_parts + 3) & ~3);
-    if (hipMalloc(&p->strip_row0, sizeof(int) * row0.size()) != hipSuccess ||
+    if (device_malloc(&p->strip_row0, sizeof(int) * row0.size()) != hipSuccess ||
         hipMemcpy(p->strip_row0, row0.data(), sizeof(int) * row0.size(), hipMemcpyHostToDevice) != hipSuccess) {
         release_blocked(p);
         set_error("attractive_prepare: out of device memory for the strip boundaries");
@@ -981,7 +981,7 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
         p->strip_rows = strip_rows = std::min(N, direct_uniform_rows);
         (void)hipFree(p->strip_row0);
         p->strip_row0 = nullptr;
-        if (hipMalloc(&p->strip_row0, sizeof(int) * row0.size()) != hipSuccess ||
+        if (device_malloc(&p->strip_row0, sizeof(int) * row0.size()) != hipSuccess ||
             hipMemcpy(p->strip_row0, row0.data(), sizeof(int) * row0.size(), hipMemcpyHostToDevice) != hipSuccess) {
             release_blocked(p);
             set_error("attractive_prepare: out of device memory for the strip boundaries");
@@ -997,10 +997,10 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
     const size_t items_per_strip = (strip_entries + item_entries - 1) / item_entries;
     const size_t nnz = items_per_strip * p->n_strips * item_entries;
     bool ok = scratch_malloc(reinterpret_cast<void **>(&p->ent_p), 2 * sizeof(float) * nnz) == hipSuccess &&
-              hipMalloc(&p->seg, p->blocked_direct ? sizeof(unsigned int)
+              device_malloc(&p->seg, p->blocked_direct ? sizeof(unsigned int)
                                                    : sizeof(unsigned int) * (size_t)p->n_strips * p->seg_stride) == hipSuccess &&
               (!p->blocked_direct ||
-               hipMalloc(&p->wseg, sizeof(unsigned int) * (size_t)p->n_strips * p->wseg_stride) == hipSuccess);
+               device_malloc(&p->wseg, sizeof(unsigned int) * (size_t)p->n_strips * p->wseg_stride) == hipSuccess);
     if (!ok) {
         release_blocked(p);
         set_error("attractive_prepare: out of device memory for the re-blocked pattern (%zu bytes)", nnz * 8);

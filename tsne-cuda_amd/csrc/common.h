@@ -19,11 +19,18 @@ const char *last_error();
 // TSNE_MAYBE_SYNC does (src/include/util/cuda_utils.h:46-70).
 bool sync_kernels_enabled();
 
-// hipMalloc for memory that a faster form of a stage uses and a slower one does without.  TSNE_SCRATCH_LIMIT=<bytes>
+// hipMalloc, as everything here allocates: where there is no room, the scratch that is kept between calls goes first
+// (scratch.hip).
+hipError_t device_malloc_bytes(void **p, size_t bytes);
+template <typename T>
+inline hipError_t device_malloc(T **p, size_t bytes) {
+    return device_malloc_bytes(reinterpret_cast<void **>(p), bytes);
+}
+// The same for memory that a faster form of a stage uses and a slower one does without.  TSNE_SCRATCH_LIMIT=<bytes>
 // (read on every call; for measurements and tests of the slower forms): more than that is never there.
 hipError_t malloc_optional(void **p, size_t bytes);
-// hipMalloc and hipFree for a call's scratch: large blocks are kept for the next call (scratch.hip).  What malloc_optional
-// returned goes back through scratch_free too.
+// ... and for a call's scratch, whose large blocks are kept for the next call.  What these two return goes back through
+// scratch_free.
 hipError_t scratch_malloc(void **p, size_t bytes);
 void scratch_free(void *p);
 

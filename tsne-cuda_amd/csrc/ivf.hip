@@ -46,7 +46,7 @@ struct Buffer {
     ~Buffer() {
         if (ptr) (void)hipFree(ptr);
     }
-    bool alloc(size_t bytes) { return hipMalloc(&ptr, bytes ? bytes : 1) == hipSuccess; }
+    bool alloc(size_t bytes) { return device_malloc(&ptr, bytes ? bytes : 1) == hipSuccess; }
     template <typename T>
     T *as() const {
         return static_cast<T *>(ptr);

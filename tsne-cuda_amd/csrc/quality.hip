@@ -41,7 +41,7 @@ struct DeviceArray {
     ~DeviceArray() {
         if (ptr) (void)hipFree(ptr);
     }
-    bool alloc(size_t bytes) { return hipMalloc(&ptr, bytes ? bytes : 1) == hipSuccess; }
+    bool alloc(size_t bytes) { return device_malloc(&ptr, bytes ? bytes : 1) == hipSuccess; }
     template <typename T>
     T *as() const {
         return static_cast<T *>(ptr);

@@ -296,7 +296,7 @@ __global__ __launch_bounds__(256) void index_range_kernel(const int *__restrict_
 // set.  Synchronises the stream.
 int validate_indices(const int *idx, int64_t n, int N, const char *who, hipStream_t s) {
     int *flag = nullptr;
-    TSNE_TRY(hipMalloc(&flag, sizeof(int)));
+    TSNE_TRY(device_malloc(&flag, sizeof(int)));
     int host = 0;
     hipError_t e = hipMemsetAsync(flag, 0, sizeof(int), s);
     if (e == hipSuccess) {
