@@ -1310,10 +1310,12 @@ __global__ __launch_bounds__(256) void gap_kernel(const float *__restrict__ X, i
         }
         dist[u] = j < last && j != q ? __float_as_uint(sum) : ~0u;  // (not negative: ordered as its bits)
     }
-    // The largest value that fewer than `rank` distances lie below.
+    // The largest value that fewer than `rank` distances lie below.  (turn: over both calls, whose last and first counts
+    // would otherwise share a word, cleared while it is still read)
+    int turn = 0;
     auto ranked = [&](int rank) {
         unsigned int value = 0u;
-        for (int b = 30, turn = 0; b >= 8; --b, turn ^= 1) {  // (23 bits: a relative 3e-5)
+        for (int b = 30; b >= 8; --b, turn ^= 1) {  // (23 bits: a relative 3e-5)
             const unsigned int trial = value | (1u << b);
             if (tid == 0) below[turn] = 0;
             __syncthreads();
