@@ -1489,7 +1489,8 @@ def test_loop_and_symmetrisation_without_room_for_the_faster_form(stages, monkey
     (16500, 193, 33, "plain", True), (20000, 30, 25, "far", True), (20000, 30, 25, "one far point", False),
     (98304, 12, 60, "grid", True), (98433, 8, 20, "plain", True), (100003, 20, 33, "clumps", True),
     (100003, 20, 90, "clumps", False), (131200, 24, 33, "clusters", True), (100003, 3, 45, "clumps", False),
-    (60000, 20, 45, "300 clusters", False)])
+    (60000, 20, 45, "300 clusters", False), (20011, 150, 90, "18 clusters", False), (16500, 200, 20, "60 clusters", False),
+    (16500, 400, 20, "60 clusters", False)])
 def test_knn_on_halves(stages, monkeypatch, n, d, k, kind, halves):
     """The search's own choice of sweep - on halves relative to frames, beyond four dimensions - gives the vector sweep's
     rows, bit for bit: at the remainders of a step of 16 dimensions and of a chunk of 64, at the most neighbours the
@@ -1502,8 +1503,9 @@ def test_knn_on_halves(stages, monkeypatch, n, d, k, kind, halves):
     X = rng.standard_normal((n, d)).astype(np.float32)
     if kind == "clusters":
         X += (8.0 * rng.standard_normal((5, d)))[np.arange(n) * 5 // n].astype(np.float32)
-    elif kind == "300 clusters":
-        X += (30.0 * rng.standard_normal((300, d)))[np.arange(n) * 300 // n].astype(np.float32)
+    elif kind.endswith(" clusters"):
+        c = int(kind.split()[0])
+        X += (30.0 * rng.standard_normal((c, d)))[np.arange(n) * c // n].astype(np.float32)
     elif kind == "grid":
         X = np.round(2.0 * X).astype(np.float32)
     elif kind == "clumps":

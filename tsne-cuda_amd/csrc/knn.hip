@@ -1284,54 +1284,110 @@ __global__ __launch_bounds__(1024) void frame_kernel(const float *__restrict__ c
     }
 }
 
+// A sampled tile's query and its neighbourhood in the numbering.
+constexpr int kGapMost = (2 * kHomeTiles + 1) * kCT;
+constexpr int kGapStride = 2, kGapGiven = kGapMost / kGapStride;  // gap_distances_kernel: every second point of it
+struct GapQuery {
+    int tile, q, first, last;
+    __device__ GapQuery(int sample, int step, int N, int T) {
+        tile = min(sample * step + step / 2, T - 1);
+        q = min(tile * kCT + 5, N - 1);
+        first = max(tile - kHomeTiles, 0) * kCT;
+        last = min((tile + kHomeTiles + 1) * kCT, N);
+    }
+};
+// Squared distances of the sampled queries to their neighbourhoods where rows are long (as bits; all ones beyond the
+// points there are, and for the query): four rows per wave and turn, kGapSplit workgroups per sample.  Bound by the rows it
+// reads (64 samples of 2176 rows of 784 dimensions 76 us, 5.7 TB/s; a workgroup per sample 0.3 ms): hence every second one.
+constexpr int kGapSplit = 8;
+__global__ __launch_bounds__(1024) void gap_distances_kernel(const float *__restrict__ X, int N, int D, int T, int step,
+                                                             unsigned int *__restrict__ dist) {
+    constexpr int kAtOnce = 4, kRows = kGapGiven / kGapSplit;
+    static_assert(kRows % kAtOnce == 0 && kGapGiven % kGapSplit == 0, "whole turns");
+    const GapQuery g((int)blockIdx.y, step, N, T);
+    const int lane = threadIdx.x & (kWave - 1), row0 = (int)blockIdx.x * kRows;
+    const float *xq = X + (size_t)g.q * D;
+    for (int p = threadIdx.x / kWave * kAtOnce; p < kRows; p += 1024 / kWave * kAtOnce) {
+        float sum[kAtOnce];
+        const float *x[kAtOnce];
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u) {
+            sum[u] = 0.0f;
+            x[u] = X + (size_t)min(g.first + kGapStride * (row0 + p + u), g.last - 1) * D;
+        }
+#pragma unroll 8
+        for (int d = lane; d < D; d += kWave) {
+            const float v = xq[d];
+#pragma unroll
+            for (int u = 0; u < kAtOnce; ++u) {
+                const float diff = v - x[u][d];
+                sum[u] = fmaf(diff, diff, sum[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kAtOnce; ++u) {
+            const int j = g.first + kGapStride * (row0 + p + u);
+            const float total = group_sum<kWave>(sum[u]);
+            if (lane == 0) dist[(size_t)blockIdx.y * kGapGiven + row0 + p + u] = j < g.last && j != g.q ? __float_as_uint(total) : ~0u;
+        }
+    }
+}
+
 // Whether the bound leaves room between a query's K-th neighbour and the last candidate kept of it: for one point of each
-// sampled tile (`step` apart), the distances to the points of its neighbourhood in the numbering, the K-th and the
-// `want`-th smallest of them, and the tile's bound.  The gap among all points is smaller than that, a third to all of it.
-// One workgroup of 256 threads per sampled tile.
-__global__ __launch_bounds__(256) void gap_kernel(const float *__restrict__ X, int N, int D, int T, int step, int K, int want,
+// sampled tile (`step` apart), the distances to the points of its neighbourhood in the numbering (`given`, or formed here),
+// those of the ranks `near_rank` and `far_rank` among them, and `loss` times the squared reach of the tile from its frame.  The
+// gap among all points is smaller than that, a third to all of it.  One workgroup of 256 threads per sampled tile.
+__global__ __launch_bounds__(256) void gap_kernel(const float *__restrict__ X, int N, int D, int T, int step, int near_rank,
+                                                  int far_rank, float loss, const unsigned int *__restrict__ given,
                                                   const float *__restrict__ nearest, const float *__restrict__ radius,
                                                   HalfScale *scale) {
-    constexpr int kEach = (2 * kHomeTiles + 1) * kCT / 256 + 1;
-    __shared__ int below[2];
-    const int tid = threadIdx.x, tile = min((int)blockIdx.x * step + step / 2, T - 1);
-    const int q = min(tile * kCT + 5, N - 1);
-    const int first = max(tile - kHomeTiles, 0) * kCT, last = min((tile + kHomeTiles + 1) * kCT, N);
-    const float *xq = X + (size_t)q * D;
+    constexpr int kEach = (kGapMost + 255) / 256;
+    __shared__ int below[2][2];
+    const int tid = threadIdx.x;
+    const GapQuery g((int)blockIdx.x, step, N, T);
+    const float *xq = X + (size_t)g.q * D;
     unsigned int dist[kEach];
 #pragma unroll
     for (int u = 0; u < kEach; ++u) {
-        const int j = first + u * 256 + tid;
-        const float *x = X + (size_t)min(j, last - 1) * D;
+        const int r = u * 256 + tid, j = g.first + r;
+        if (given) {
+            dist[u] = r < kGapGiven ? given[(size_t)blockIdx.x * kGapGiven + r] : ~0u;
+            continue;
+        }
+        const float *x = X + (size_t)min(j, g.last - 1) * D;
         float sum = 0.0f;
 #pragma unroll 4
         for (int d = 0; d < D; ++d) {
             const float diff = xq[d] - x[d];
             sum = fmaf(diff, diff, sum);
         }
-        dist[u] = j < last && j != q ? __float_as_uint(sum) : ~0u;  // (not negative: ordered as its bits)
+        dist[u] = j < g.last && j != g.q ? __float_as_uint(sum) : ~0u;  // (not negative: ordered as its bits)
     }
-    // The largest value that fewer than `rank` distances lie below.  (turn: over both calls, whose last and first counts
-    // would otherwise share a word, cleared while it is still read)
-    int turn = 0;
-    auto ranked = [&](int rank) {
-        unsigned int value = 0u;
-        for (int b = 30; b >= 8; --b, turn ^= 1) {  // (23 bits: a relative 3e-5)
-            const unsigned int trial = value | (1u << b);
-            if (tid == 0) below[turn] = 0;
-            __syncthreads();
-            int c = 0;
+    // The largest values that fewer distances than the ranks lie below, bit by bit, side by side.
+    unsigned int near_bits = 0u, far_bits = 0u;
+    for (int b = 30, turn = 0; b >= 8; --b, turn ^= 1) {  // (23 bits: a relative 3e-5)
+        const unsigned int near_trial = near_bits | (1u << b), far_trial = far_bits | (1u << b);
+        if (tid < 2) below[turn][tid] = 0;
+        __syncthreads();
+        int c_near = 0, c_far = 0;
 #pragma unroll
-            for (int u = 0; u < kEach; ++u) c += __popcll(__ballot(dist[u] < trial));
-            if ((tid & (kWave - 1)) == 0) atomicAdd(&below[turn], c);
-            __syncthreads();
-            if (below[turn] < rank) value = trial;
+        for (int u = 0; u < kEach; ++u) {
+            c_near += __popcll(__ballot(dist[u] < near_trial));
+            c_far += __popcll(__ballot(dist[u] < far_trial));
         }
-        return __uint_as_float(value);
-    };
-    const float near_d = ranked(K - 1), far_d = ranked(want);
+        if ((tid & (kWave - 1)) == 0) {
+            atomicAdd(&below[turn][0], c_near);
+            atomicAdd(&below[turn][1], c_far);
+        }
+        __syncthreads();  // (these words are cleared two turns on, past the barrier of the next)
+        if (below[turn][0] < near_rank) near_bits = near_trial;
+        if (below[turn][1] < far_rank) far_bits = far_trial;
+    }
     if (tid == 0) {
-        const float reach = sqrtf(nearest[tile]) + radius[tile];
-        if (!(4.0f * 4.0f / 4096.0f * reach * reach < far_d - near_d)) atomicAdd(&scale->unsure, 1);
+        const float near_d = __uint_as_float(near_bits), far_d = __uint_as_float(far_bits);
+        // (in many dimensions a point lies about across from the frame, seen from the tile's centre)
+        const float r = radius[g.tile], reach = sqrtf(nearest[g.tile]) + r, reach2 = given ? nearest[g.tile] + r * r : reach * reach;
+        if (!(loss * reach2 < far_d - near_d)) atomicAdd(&scale->unsure, 1);
     }
 }
 
@@ -3243,11 +3299,34 @@ int run_valu_sweep(const float *points, const float *Xt, int N, int Npad, int D,
 // Fewer dimensions: a step of 16 dimensions is mostly padding, tiles are small beside their frame, and bf16 terms
 // relative to the tile's own centre keep more.
 constexpr int kHalfDims = 5;
-constexpr int kGapSamples = 128;
 // Halves relative to the frames lose more than two bf16 terms relative to the tiles where the points have structure that
-// kFrames frames do not follow.  What counts is whether neighbours can be told from the rest, which a sample says (at
-// most one in 32 may be in doubt: 60000 x 20 in 300 clusters, 617 queries failed and were searched again, 4.5 ms, 2.5 on
-// bf16 terms); and beyond this many times the other sweep's bound that one is the better try.
+// kFrames frames do not follow.  What counts is whether neighbours can be told from the rest, which a sample says (60000 x
+// 20 in 300 clusters, 617 queries failed and were searched again, 4.5 ms, 2.5 on bf16 terms); and beyond kHalfLoss times the
+// other sweep's bound that one is the better try.
+// The chunked sweep widens its margin until a sample of query tiles verifies, and finds there what it has to, but three
+// sweeps of a sample and a return to bf16 terms cost up to as much as the search: it is asked what twice the candidates
+// would tell apart, or four times from kWideDims dimensions on, where halves save 40 % of a sweep and wider lists pay as well.
+// ms, on bf16 terms / without this sample / with it, clusters 20 deviations apart in their order: 20000 x 150, 90
+// neighbours, 18 clusters 8.3 / 15.7 / 8.3, 60 clusters 8.4 / 14.4 / 8.3; 60000 x 200, 45: 18 clusters 13.9 / 19.4 / 14.4, 60
+// clusters 21.4 / 28.4 / 21.9, 300 clusters 10 apart 16.9 / 14.2 / 14.4; 60000 x 784, 45: 300 clusters 4 apart 37.9 / 24.5 /
+// 24.7, pixel vectors 21.8 / 13.6 / 13.7.  With more dimensions more queries may be in doubt, which the vector sweep takes
+// (60000 x 784, 17 clusters of which one has no frame, 105 / 46.4 / 46.8: bf16 terms cannot tell those neighbours apart
+// either).
+struct GapSample {
+    int tiles, near_rank, far_rank;
+    int most_in_doubt;  // one in so many may be
+    float loss;
+};
+constexpr int kWideDims = 400;
+inline GapSample gap_sample(int D, int T, int K, int want, bool chunked) {
+    if (!chunked) return {std::min(T, 128), K - 1, want, 32, 4.0f * 4.0f / 4096.0f};
+    const bool wide = D >= kWideDims;
+    // (no more than a neighbourhood at either end of the numbering has; for more neighbours nothing is sampled)
+    const int asked = std::min((wide ? 4 : 2) * want, kHomeTiles * kCT);
+    // (the bound of half_bound.h at |q'| = |x'|: a coordinate's half is off by 0.4 of 2^-12 in the mean square)
+    const float loss = 1.8f / 4096.0f + 15.0f * (float)(D + 8) * 5.9604644775390625e-08f;
+    return {asked > want ? std::min(T, 48) : 0, std::max((K - 1) / kGapStride, 1), asked / kGapStride, wide ? 8 : 32, loss};
+}
 constexpr float kHalfLoss = 16.0f;
 
 // What the sweeps on halves take beside the points: made in three steps.
@@ -3255,7 +3334,7 @@ struct HalfOperands {
     DeviceMem small, beta, point_len, tile_info;
     int dims = 0, tiles = 0;
     // `small`: kFrames keys, the scale, kFrames tile numbers, the frames' distances, the frames, the tiles' distance
-    // to theirs and its number.
+    // to theirs and its number, and in the chunked form the sampled distances.
     u64 *best() const { return small.as<u64>(); }
     HalfScale *scale() const { return reinterpret_cast<HalfScale *>(best() + kFrames); }
     int *frame_tile() const { return reinterpret_cast<int *>(scale() + 1); }
@@ -3270,14 +3349,15 @@ struct HalfOperands {
         tile_info.release();
     }
     // Frames of the tiles; *pays: whether the sweeps should multiply halves (false also where there is no room).
-    // (points of more dimensions than a wave holds are tried on a sample of query tiles anyway: `sample` false)
-    int frames(const float *points, const float *centers_t, const float *radius, int N, int D, int T, int K, int want, bool sample,
-               bool *pays, hipStream_t s) {
+    int frames(const float *points, const float *centers_t, const float *radius, int N, int D, int T, int K, int want,
+               bool chunked, bool *pays, hipStream_t s) {
         *pays = false;
         dims = D;
         tiles = T;
         const size_t keys = sizeof(u64) * kFrames + sizeof(HalfScale);
-        if (!small.alloc_optional(keys + sizeof(int) * (kFrames + kFrames * kFrames + (size_t)D * kFrames + 2 * (size_t)T))) {
+        const GapSample sample = gap_sample(D, T, K, want, chunked);
+        const size_t given = chunked ? (size_t)sample.tiles * kGapGiven : 0;
+        if (!small.alloc_optional(keys + sizeof(int) * (kFrames + kFrames * kFrames + (size_t)D * kFrames + 2 * (size_t)T + given))) {
             (void)hipGetLastError();
             return 0;
         }
@@ -3287,9 +3367,12 @@ struct HalfOperands {
                                                         frame_tile(), nearest(), tile_frame(), scale());
             TSNE_TRY(hipGetLastError());
         }
-        const int sampled = std::min(T, kGapSamples);
-        if (sample) {
-            gap_kernel<<<sampled, 256, 0, s>>>(points, N, D, T, T / sampled, K, want, nearest(), radius, scale());
+        if (sample.tiles > 0) {
+            const int step = T / sample.tiles;
+            unsigned int *dist = given ? reinterpret_cast<unsigned int *>(tile_frame() + tiles) : nullptr;
+            if (given) gap_distances_kernel<<<dim3(kGapSplit, sample.tiles), 1024, 0, s>>>(points, N, D, T, step, dist);
+            gap_kernel<<<sample.tiles, 256, 0, s>>>(points, N, D, T, step, sample.near_rank, sample.far_rank, sample.loss, dist,
+                                                    nearest(), radius, scale());
             TSNE_TRY(hipGetLastError());
         }
         HalfScale host;
@@ -3300,7 +3383,7 @@ struct HalfOperands {
         float reach;
         std::memcpy(&reach, &host.reach, sizeof(reach));
         // ... and points mostly within 1e-12 of their frames lose their squares to underflow, and the bound its grip.
-        *pays = host.not_finite == 0 && host.unsure * 32 <= sampled && host.bound <= kHalfLoss * host.bound_bf16 &&
+        *pays = host.not_finite == 0 && host.unsure * sample.most_in_doubt <= sample.tiles && host.bound <= kHalfLoss * host.bound_bf16 &&
                 std::log2(std::max(reach, 1e-30f)) <= host.log_reach / (float)T + 16.0f && host.log_reach >= -40.0f * (float)T;
         return 0;
     }
@@ -3429,7 +3512,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         bool pays = false;
         if (on_halves.fits(want))
             if (const int rc = operands.frames(points, centers.as<float>(), radius.as<float>(), N, D, num_tiles, K, want,
-                                               !chunked, &pays, s))
+                                               chunked, &pays, s))
                 return rc;
         if (pays && operands.room(N, on_halves) && Xp.alloc_optional(sizeof(float4) * on_halves.tile_float4 * num_tiles)) {
             geometry = on_halves;
@@ -3664,7 +3747,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     if (chunked && num_qtiles >= 64) {
         const int sample_tiles = 16, step = num_qtiles / sample_tiles;
         bool verified = false;
-        for (int attempt = 0; attempt < 3 && !verified; ++attempt) {
+        const int attempts = half && D < kWideDims ? 2 : 3;  // (see GapSample)
+        for (int attempt = 0; attempt < attempts && !verified; ++attempt) {
             if (const int rc = sweep_and_rerank(want, nullptr, step / 2, step, sample_tiles, failed, swept))
                 return rc == kNoRoom && half ? without_halves() : rc;
             if (failed * 10 <= sample_tiles * kMQ) {
