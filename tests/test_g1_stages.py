@@ -1583,10 +1583,11 @@ def test_knn_of_points_whose_squares_underflow(stages, monkeypatch, n, d, size):
                                     (20480, "one box"), (20481, "plain"), (9001, "equal"), (5003, "not a number"),
                                     (12000, "boxes' edges")])
 def test_small_step_spread_without_grouping(stages, monkeypatch, n, kind):
-    """Steps of a small problem whose points are looked through by every row of boxes against steps that group them by tile
-    (TSNE_KEEP_GROUPING asks for those): the same bits, at the remainders of the chunks they are looked through in, up
-    to the most points, with all points but one in a box, on a line, in one place, far from the origin, on the edges of
-    the boxes, and with one that is not a number (which both forms take into the first box)."""
+    """Steps of a small problem whose points are looked through by every row of boxes (up to 20480 of them) against steps
+    that group them by tile, every step or most (TSNE_KEEP_GROUPING=0 and 1 ask for those; with more points the second is
+    what runs anyway): the same bits, at the remainders of the chunks they are looked through in, with all points but one
+    in a box, on a line, in one place, far from the origin, on the edges of the boxes, and with one that is not a number
+    (which all forms take into the first box)."""
     rng = np.random.default_rng(n)
     k = min(n, 12)
     idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
@@ -1607,7 +1608,7 @@ def test_small_step_spread_without_grouping(stages, monkeypatch, n, kind):
         y0 = rng.integers(0, 131, size=(2, n)).astype(np.float32)
 
     def run(asked):
-        monkeypatch.setenv("TSNE_KEEP_GROUPING", "1") if asked else monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
+        monkeypatch.setenv("TSNE_KEEP_GROUPING", asked) if asked else monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
         plan = stages.Plan(n, k)
         plan.prepare_attractive(dev(P), dev(idx))
         y = dev(y0.reshape(-1).copy())
@@ -1617,8 +1618,10 @@ def test_small_step_spread_without_grouping(stages, monkeypatch, n, kind):
         plan.close()
         return [v.cpu().numpy() for v in (y, gains, old, z)]
 
-    for a, b in zip(run(False), run(True)):
-        assert same_bits(a, b)
+    want = run(None)
+    for asked in ("1", "0"):
+        for a, b in zip(want, run(asked)):
+            assert same_bits(a, b)
 
 
 def test_scratch_is_kept_bounded_and_given_back(stages):

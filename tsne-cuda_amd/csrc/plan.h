@@ -53,10 +53,12 @@ inline bool forces_ride_along(int N, int K) {
     return N <= kSingleStreamPoints && K <= 512 && (int64_t)N * K <= 3000000 + 50 * (int64_t)N;
 }
 
-// Up to this many points such a step spreads them without grouping them (conv_rows_scan_kernel).  us per step, grouped /
-// scanned, from the start of a fit, late in one, and with every point but one in one box: 1203 points 58 / 48, 56 / 49,
-// 68 / 51; 5000 61 / 50, 59 / 52, 70 / 59; 10007 62 / 54, 58 / 55, 71 / 70; 20011 66 / 59, 59 / 58, 71 / 89;
-// 40001 71 / 74, 64 / 70, 76 / 133.
+// Up to this many points such a step spreads them without grouping them (conv_rows_scan_kernel).  Whole loops of 1000 steps
+// of clustered points, ms, grouped / scanned: 5000 points 57.6 / 49.3, 7680 57.8 / 50.6, 10007 58.5 / 53.1, 13001 58.4 / 53.8,
+// 15361 59.1 / 56.1, 20011 at three learning rates 59.3 / 58.0, 58.0 / 58.0, 59.4 / 56.7.  What the scan costs grows with the
+// fullest row of boxes, which one workgroup spreads alone; us per step of embeddings that no fit was seen in, every point but
+// one in one box, and tails of two degrees of freedom: 1203 points 64 / 47, 49 / 45; 5000 66 / 53, 51 / 48; 10007 67 / 62,
+// 65 / 71; 15361 68 / 71, 59 / 71; 20011 69 / 78, 66 / 99.
 constexpr int kScanPoints = 20480;
 
 // Kernels of one gradient step, in launch order (profiling slots).

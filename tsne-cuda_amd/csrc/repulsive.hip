@@ -560,11 +560,14 @@ __global__ __launch_bounds__(1024) void tile_scatter_kernel(const float *__restr
 
 constexpr int kSpreadThreads = 512;  // two points of a 1024-point chunk per thread
 
-// v * scale rounded to a 64-bit integer (|v * scale| < 2^51).
-__device__ __forceinline__ unsigned long long to_fixed_bits(float v, double scale) {
+// v * scale rounded to a 64-bit integer (|v * scale| < 2^51), more by kFixedOffset.
+constexpr unsigned long long kFixedOffset = 0x4338000000000000ull;  // the bits of 1.5 * 2^52
+__device__ __forceinline__ unsigned long long to_offset_bits(float v, double scale) {
     const double magic = 6755399441055744.0;  // 1.5 * 2^52: adding it rounds a double to an integer
-    const double r = fma((double)v, scale, magic);
-    return (unsigned long long)(__double_as_longlong(r) - __double_as_longlong(magic));
+    return (unsigned long long)__double_as_longlong(fma((double)v, scale, magic));
+}
+__device__ __forceinline__ unsigned long long to_fixed_bits(float v, double scale) {
+    return to_offset_bits(v, scale) - kFixedOffset;
 }
 // 64-bit fixed-point add of v * scale to an LDS (or global) word.
 __device__ __forceinline__ void add_fixed(unsigned long long *dst, float v, double scale) {
@@ -1051,13 +1054,15 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
     const float to = bx == n_boxes - 1 ? INFINITY : ((float)bx + 1.01f) * bd.box_width;
     const bool all = !(bd.box_width > 1e-30f);
     // A thread's points of one box in a row are summed in registers: with every point in one box, as beside a far
-    // outlier, the additions in LDS would come one after the other (20011 points 235 us a step).
-    unsigned long long sum[kMoments];
+    // outlier, the additions in LDS would come one after the other (20011 points 235 us a step).  There one workgroup's
+    // arithmetic is what a step waits for, so a sum takes no more of it than need be: what every addend is too large by goes
+    // at the end, and the sums are cleared where a box ends (20011 points 87 -> 78 us a step).
+    unsigned long long sum[kMoments], count = 0ull;
     int sum_box = -1;
     auto flush = [&]() {
         unsigned long long *dst = acc + (lane % kScanCopies) * words + sum_box;
 #pragma unroll
-        for (int m = 0; m < kMoments; ++m) atomicAdd(dst + m * n_boxes, sum[m]);
+        for (int m = 0; m < kMoments; ++m) atomicAdd(dst + m * n_boxes, sum[m] - count * kFixedOffset);
     };
     __syncthreads();
     for (int first = 0, turn = 0; first < N; first += kScanChunk, turn ^= 1) {
@@ -1095,17 +1100,19 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
                 pu[k] = pu[k - 1] * pu[1];
                 pv[k] = pv[k - 1] * pv[1];
             }
-            const bool same = by == sum_box;
-            if (!same && sum_box >= 0) flush();
-            sum_box = by;
+            if (by != sum_box) {
+                if (sum_box >= 0) flush();
+                sum_box = by;
+                count = 0ull;
+#pragma unroll
+                for (int m = 0; m < kMoments; ++m) sum[m] = 0ull;
+            }
+            ++count;
 #pragma unroll
             for (int j = 0; j < 5; ++j)
 #pragma unroll
                 for (int i = 0; i < 5; ++i)
-                    if (j <= 2 || i <= 2) {
-                        unsigned long long &to_sum = sum[moment_index(i, j)];
-                        to_sum = (same ? to_sum : 0ull) + to_fixed_bits(pu[i] * pv[j], to_fixed);
-                    }
+                    if (j <= 2 || i <= 2) sum[moment_index(i, j)] += to_offset_bits(pu[i] * pv[j], to_fixed);
         }
         __syncthreads();
     }
