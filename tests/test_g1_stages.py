@@ -1267,18 +1267,21 @@ def test_knn_of_points_in_no_order(stages, n, d, k, kind):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
-@pytest.mark.parametrize("n,k", [(2, 2), (63, 5), (65, 1), (130, 129), (1203, 32), (2049, 33), (20011, 50), (300, 300)])
-def test_small_step_forms(stages, n, k):
-    """The step of a small problem takes its attractive forces in spare workgroups of the inverse row pass and
-    launches the grouping kernels every second step only; with per-kernel timing on it launches every kernel by
-    itself on every step.  Same bits, at the remainders of the rows of a workgroup and of the entries of a lane."""
+@pytest.mark.parametrize("n,k", [(2, 2), (63, 5), (65, 1), (130, 129), (1203, 32), (2049, 33), (20011, 50), (300, 300),
+                                 (20481, 20), (40003, 33)])
+def test_small_step_forms(stages, monkeypatch, n, k):
+    """The step of a small problem takes its attractive forces in spare workgroups of the inverse row pass and spreads
+    its points without a grouping (up to 20480 points), or launches the grouping kernels every second step only (beyond,
+    and where TSNE_KEEP_GROUPING asks for it); with per-kernel timing on it launches every kernel by itself on every step.
+    Same bits, at the remainders of the rows of a workgroup and of the entries of a lane."""
     rng = np.random.default_rng(n)
     idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
     idx[:, 0] = np.arange(n)
     P = (rng.random((n, k)) / (n * k)).astype(np.float32)
     y0 = rng.standard_normal(2 * n).astype(np.float32)
 
-    def run(timed):
+    def run(timed, asked=None):
+        monkeypatch.setenv("TSNE_KEEP_GROUPING", asked) if asked else monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
         plan = stages.Plan(n, k)
         plan.prepare_attractive(dev(P), dev(idx))
         if timed:
@@ -1293,16 +1296,23 @@ def test_small_step_forms(stages, n, k):
         plan.close()
         return [v.cpu().numpy() for v in (y, gains, old, z)]
 
-    for a, b in zip(run(False), run(True)):
-        assert same_bits(a, b)
+    want = run(True)
+    for asked in (None, "1"):
+        for a, b in zip(want, run(False, asked)):
+            assert same_bits(a, b)
 
 
-def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch):
+@pytest.mark.parametrize("n,asked", [(3000, True), (20481, False), (3000, False)])
+def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch, n, asked):
     """Steps of a small problem that do not launch the grouping kernels only ever follow one of the same call that
     does: a captured pair of steps replayed for a new start finds that start's grouping (no point strays), a call
-    that was captured and not run leaves the next one to group for itself, and replays of it start afresh each time."""
+    that was captured and not run leaves the next one to group for itself, and replays of it start afresh each time.
+    So it is where TSNE_KEEP_GROUPING asks for a grouping and where there are too many points to do without; steps
+    without one (no point can stray) replay as they should too."""
     monkeypatch.setenv("TSNE_OVERLAP", "0")
-    n, k = 3000, 20
+    if asked:
+        monkeypatch.setenv("TSNE_KEEP_GROUPING", "1")
+    k = 20
     rng = np.random.default_rng(11)
     idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
     idx[:, 0] = np.arange(n)
@@ -1660,6 +1670,6 @@ def test_scratch_is_kept_bounded_and_given_back(stages):
     del got, idx, d2
     torch.cuda.empty_cache()
     kept = free - torch.cuda.mem_get_info()[0]
-    assert kept <= (2 << 30) + (256 << 20)
+    assert 32 << 20 <= kept <= (2 << 30) + (256 << 20)
     stages.release_scratch()
     assert free - torch.cuda.mem_get_info()[0] <= 256 << 20
