@@ -41,6 +41,8 @@ struct World {
     bool known = true, waits_well = true;
     double clock = 0.0;
     char *next = reinterpret_cast<char *>(4096);
+    void (*meanwhile)(void *) = nullptr;  // what another thread does while this one asks for its device
+    void *with = nullptr;
 };
 struct Device {
     World *w;
@@ -65,7 +67,14 @@ struct Device {
         w->room[w->live[p].second] += w->live[p].first;
         w->live.erase(p);
     }
-    int current() { return w->known ? w->here : -1; }
+    int current() {
+        if (w->meanwhile) {
+            auto act = w->meanwhile;
+            w->meanwhile = nullptr;
+            act(w->with);
+        }
+        return w->known ? w->here : -1;
+    }
     bool idle() {
         ++w->waits;
         return w->waits_well;
@@ -135,6 +144,17 @@ int main() {
                 void *c;
                 EXPECT((scratch ? pool.take(&c, 2 * GB) : pool.plain(&c, 2 * GB)) == 2 && !c && w.errors);
             }
+    }
+    {  // ... also where another thread gives it, just after this one found none
+        World w;
+        w.room[0] = 1 * GB;
+        Pool pool(Device{&w});
+        void *a, *b;
+        EXPECT(!pool.take(&a, 1 * GB));
+        pool.put(a);
+        w.with = &pool;
+        w.meanwhile = [](void *p) { static_cast<Pool *>(p)->release(); };
+        EXPECT(!pool.plain(&b, 4096) && w.errors == 0);
     }
     {  // returned from another device, or while the device cannot be waited for: freed
         World w;

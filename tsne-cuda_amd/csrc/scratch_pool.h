@@ -27,8 +27,9 @@ class ScratchPool {
         const int e = device_.alloc(p, bytes);
         if (!e) return 0;
         const int here = device_.current();
+        if (here < 0) return e;
         std::lock_guard<std::mutex> hold(lock_);
-        if (here < 0 || !give_back(here, 0)) return e;
+        give_back(here, 0);  // (tried again also if that gave nothing: another thread may just have given it)
         device_.forgive();
         return device_.alloc(p, bytes);
     }
@@ -102,13 +103,12 @@ class ScratchPool {
     };
 
     // Frees what has been kept too long, the longest unused while more than `most` bytes are kept on `device`, and, for
-    // device < 0, everything.  Whether anything went.
-    bool give_back(int device, size_t most) {
+    // device < 0, everything.
+    void give_back(int device, size_t most) {
         const double now = device_.now();
         size_t total = 0;
         for (const Block &b : kept_)
             if (b.device == device) total += b.bytes;
-        bool any = false;
         for (size_t k = 0; k < kept_.size();) {  // (in the order they were returned)
             const Block b = kept_[k];
             if (now - b.since <= kKeptSeconds && device >= 0 && !(b.device == device && total > most)) {
@@ -118,9 +118,7 @@ class ScratchPool {
             if (b.device == device) total -= b.bytes;
             device_.free(b.p);
             kept_.erase(kept_.begin() + (long)k);
-            any = true;
         }
-        return any;
     }
 
     // Both lists have a place for every block there is and one more, so that no other push_back allocates.
