@@ -289,7 +289,7 @@ int tsne_hip_repulsive_error(tsne_hip_plan *plan, const float *embedding, int sa
 int tsnecuda_trustworthiness(const float *points, const float *embedding, int num_points, int num_dims,
                              int n_neighbors, int max_sample, int device, double *trustworthiness, int *sample_out);
 
-/* Gives the device memory back that the library keeps between calls (blocks of 32 MB and more that its calls used as
+/* Gives the device memory back that the library keeps between calls (blocks of 2 MB and more that its calls used as
  * scratch, at most 2 GB per device; unused ones go after five seconds by themselves, at the next call). */
 int tsne_hip_release_scratch(void);
 

@@ -14,7 +14,7 @@
 
 namespace tsnehip {
 
-constexpr size_t kKeptLeast = (size_t)32 << 20, kKeptMost = (size_t)2 << 30;
+constexpr size_t kKeptLeast = (size_t)2 << 20, kKeptMost = (size_t)2 << 30;
 constexpr double kKeptSeconds = 5.0;
 
 template <class Device>
