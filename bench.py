@@ -124,6 +124,17 @@ def main():
     dXs, gather_s = timed(lambda: stages.gather_rows(dX, order))
     del dX
     (idx, d2, knn_stats), knn_s = timed(lambda: stages.knn_select(dXs, k, 0))  # 0: what tsne_hip_knn does
+    # Whether that swept on halves, for its roofline: asked for nothing else, a search that would not is an error.
+    asked = os.environ.get("TSNE_KNN_PRODUCTS")
+    os.environ["TSNE_KNN_PRODUCTS"] = "half"
+    try:
+        knn_on_halves = asked != "bf16" and bool(stages.knn_select(dXs, k, 0))
+    except RuntimeError:
+        knn_on_halves = False
+    if asked is None:
+        del os.environ["TSNE_KNN_PRODUCTS"]
+    else:
+        os.environ["TSNE_KNN_PRODUCTS"] = asked
     # The optional approximate search (inverted file, floor(sqrt(N)) lists as the reference's FAISS index, 100
     # lists probed per list: what TSNE_KNN=ivf runs): training and search timed, recall against the exact rows.
     approx = None
@@ -217,11 +228,15 @@ def main():
                "frac": b / (kernels_us[name] * 1e-6) / 1e9 / HBM_PEAK_GBS}
         for name, b in loop_bytes.items() if kernels_us.get(name)}
     if knn_stats[0] == 1:
-        # Flop the matrix sweep executed per tile pair it did not skip: three products of bf16 terms
-        # (v_mfma_f32_32x32x16_bf16) over the dimensions + 3, padded to 16 (up to 125 dimensions) or to 32 (chunked
-        # sweep, beyond 126); at exactly 126 dimensions float products over 128 (v_mfma_f32_32x32x2_f32).
+        # Flop the matrix sweep executed per tile pair it did not skip: one product of halves
+        # (v_mfma_f32_32x32x16_f16) over the dimensions, padded to 16 (up to 126 of them) or to 64 (chunked sweep); or three
+        # of bf16 terms (v_mfma_f32_32x32x16_bf16) over the dimensions + 3, padded to 16 (up to 125) or to 32 (chunked,
+        # beyond 126); at exactly 126 dimensions float products over 128 (v_mfma_f32_32x32x2_f32).
         tiles = -(-n // 128)
-        if d == 126:
+        if knn_on_halves:
+            pad = 16 if d <= 126 else 64
+            per_pair, peak, pipe = 2.0 * 128 * 128 * (-(-d // pad) * pad), 2500.0, "f16"
+        elif d == 126:
             per_pair, peak, pipe = 2.0 * 128 * 128 * 128, 157.3, "fp32"
         else:
             pad = 16 if d + 3 <= 128 else 32
