@@ -646,8 +646,10 @@ __global__ __launch_bounds__(kDirectThreads) void attractive_direct_kernel(const
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     // Neighbouring strips, whose entries name the same columns, go to workgroups of one XCD (dealt out round robin by
-    // their number), 32 of each round of 256: they walk the columns at one pace, and its L2 fetches a position once
-    // (2,500,001 points x 45 late in a fit 346 -> 330 us beside the repulsive chain, steps 463 -> 450).
+    // their number), 32 of each whole round of 256: they walk the columns at one pace, and its L2 fetches a position once
+    // (2,500,001 points x 45 late in a fit, 508 strips of which the first 256 are dealt so: 346 -> 330 us beside the
+    // repulsive chain, steps 463 -> 450).  The strips of a last round that is not whole go out by their number: up to some
+    // 1.7 million points that is all of them.
     const int round = blockIdx.x & ~255, in_round = blockIdx.x & 255;
     const int strip = round + 256 <= (int)gridDim.x ? round + (in_round % 8) * 32 + in_round / 8 : (int)blockIdx.x;
     typedef const __attribute__((address_space(4))) unsigned int *ConstWords;

@@ -1429,7 +1429,8 @@ __device__ __forceinline__ float half_scale_factor(const HalfScale *scale) {
 // One workgroup per tile.  Xh: [tile][block of 32 points (4)][step of 16 dimensions (S)][lane (64)] 8 halves, lane = 32 *
 // (dimension % 16 / 8) + point % 32, element = dimension % 8 (the layout of pack_points_bf16_kernel, one term).
 // beta: row f of `pitch` floats holds beta_f of every point.  point_len: |x'| and |x' - what the halves stand for|,
-// rounded up (half_bound.h has what the sweeps make of them).  tile_info: the largest of the second and of |x'| among a tile's points, and the tile's frame.
+// rounded up (half_bound.h has what the sweeps make of them).  tile_info: the largest of the second and of |x'| among a
+// tile's points, and the tile's frame.
 __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict__ X, int N, int D, int S,
                                                         const float *__restrict__ frames, const int *__restrict__ tile_frame,
                                                         const HalfScale *scale, int pitch, uint4 *__restrict__ Xh,
@@ -1993,8 +1994,9 @@ __global__ __launch_bounds__(256, (sweep_occupancy<KSTEPS, BF16>())) void knn_mf
 // What bounds the kernel is the latency of a wave's own chain (the products are a sixth of its time): runs of results
 // in which some lane passes, stores to the lists, selections over them, the barrier that ends a tile.  So: three waves
 // per SIMD, nothing of the tile loop in scratch memory (a wait for a spilled register is a wait for the next tile's loads
-// too: four waves of 128 registers took 115 ms where three of 168 take 92), no sort buffers (a selection holds the list
-// in registers), two LDS tiles and one barrier per tile, what a tile's bound takes fetched a tile ahead.
+// too: four waves of 128 registers took 115 ms where three of 168 take 92; with five steps two registers lie there, read once per
+// query tile), no sort buffers (a selection holds the list in registers), two LDS tiles and one barrier per
+// tile, what a tile's bound takes fetched a tile ahead.
 // Whole searches, ms, on two bf16 terms / here: 1,000,000 x 50 in four clusters, 90 neighbours 163 / 91; 300000 x 50 without
 // structure 57 / 30; 300000 x 100, 45 neighbours 41 / 24; 199999 x 30, 33 neighbours 11.7 / 9.3; 300000 x 10, 30 neighbours
 // 21.8 / 19.9.
