@@ -1538,6 +1538,25 @@ def test_knn_on_halves(stages, monkeypatch, n, d, k, kind, halves):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("n,d,k", [
+    (40007, 16, 30), (40007, 17, 150), (36000, 33, 90), (33001, 64, 90), (34003, 65, 45), (33333, 81, 20),
+    (33333, 97, 33), (33100, 113, 60), (33100, 126, 90), (33100, 40, 172), (70001, 12, 90), (16500, 20, 90)])
+def test_knn_on_halves_measured_first(stages, monkeypatch, n, d, k):
+    """Thresholds measured before entries are stored, at every count of steps of 16 dimensions: neighbour counts whose
+    candidates the neighbourhood's runs are enough for and not (240 candidates kept and more), tiles enough to sample beyond
+    it and not, either end of the numbering (a shorter neighbourhood), a last tile of few points.  The vector sweep's rows."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    X[n // 2 :] += 1.5 * rng.standard_normal(d).astype(np.float32)
+    dX = dev(X)
+    dX = stages.gather_rows(dX, stages.locality_order(dX))
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    idx, d2, stats = stages.knn_select(dX, k, 0)
+    assert stats[0] == 1 and stats[1] <= 64
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
 @pytest.mark.parametrize("k", [45, 90, 150, 172])
 def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles

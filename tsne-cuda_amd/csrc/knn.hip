@@ -72,6 +72,8 @@ namespace {
 typedef unsigned long long u64;
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v8f __attribute__((ext_vector_type(8)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 
@@ -84,6 +86,24 @@ constexpr int kDC = 32;   // VALU sweep: dimensions staged per chunk
 constexpr int kMQ = 128;  // MFMA sweep: queries per workgroup (4 waves x 32)
 constexpr int kMfmaMaxSteps = 64;  // k-steps of 2 dimensions: up to 126 dimensions + 2 augmented
 static_assert(kMQ == kCT, "query tiles and candidate tiles share the packed layout");
+
+// From memory to LDS with no register in between: lane l's 16 bytes, at src + its offset, go to dst + 16 l.  The
+// compiler knows nothing of the load: s_waitcnt vmcnt(0) and a barrier stand between it and the words' readers, a barrier
+// between their last readers and it.  (As a builtin, every read of LDS that follows waits for it.)
+typedef __attribute__((address_space(3))) unsigned char LdsByte;
+__device__ __forceinline__ void load_to_lds(const void *src, unsigned int offset, unsigned int dst) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(src), "v"(offset), "s"(dst) : "memory");
+}
+// (The builtin: a wait inside inline assembly leaves the compiler waiting once more for loads it knows of, and with them
+// for those it does not.)
+__device__ __forceinline__ void wait_for_loads() {
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    asm volatile("" ::: "memory");
+}
+
+// Of a branch, where it stands: the path that is seldom taken is laid out elsewhere, and the other runs straight on.
+#define TSNE_LIKELY(c) __builtin_expect(!!(c), 1)
+#define TSNE_UNLIKELY(c) __builtin_expect(!!(c), 0)
 
 // v_min3_f32 / v_min_f32 without the quieting moves the library fminf adds for signalling NaNs.
 // The compiler's wait states between a matrix instruction and a vector instruction that reads its result do
@@ -610,6 +630,42 @@ __device__ __forceinline__ void load_halves(const u64 *list, int half, int c0, i
         if (e < n) key[u] = list[e < c0 ? e : half + e - c0];
     }
 }
+// A value that at least `want` of the wave's `ranked` rated words (of 64 NK; all bits set: not rated) do not exceed, and, but
+// for equal ones, at most want + slack.  at_under: how many lie below it, at_hi: how many do not exceed it.
+template <int NK>
+__device__ __forceinline__ unsigned int ranked_limit(const unsigned int (&rated)[NK], int ranked, int want, int slack,
+                                                     int &at_under, int &at_hi) {
+    unsigned int lo = ~0u, hi = 0u;
+#pragma unroll
+    for (int u = 0; u < NK; ++u) {
+        lo = min(lo, rated[u]);
+        hi = max(hi, rated[u] == ~0u ? 0u : rated[u]);
+    }
+    lo = wave_extreme<true>(lo);
+    hi = wave_extreme<false>(hi);
+    // Fewer than `want` lie below or at `lo - 1` (at_under of them), at least `want` at or below hi (at_hi of them).
+    unsigned int under = lo - 1u;
+    at_under = 0;
+    at_hi = ranked;
+    for (int round = 0; at_hi > want + slack && hi - under > 1u; ++round) {
+        const float share = (round & 1) ? 0.5f : (float)(want + slack / 2 - at_under) * __builtin_amdgcn_rcpf((float)(at_hi - at_under));
+        const unsigned int span = hi - under;
+        unsigned int step = (unsigned int)((float)span * share);
+        step = min(max(step, 1u), span - 1u);
+        const unsigned int trial = __builtin_amdgcn_readfirstlane(under + step);
+        int c = 0;
+#pragma unroll
+        for (int u = 0; u < NK; ++u) c += __popcll(__ballot(rated[u] <= trial));
+        if (c >= want) {
+            hi = trial;
+            at_hi = c;
+        } else {
+            under = trial;
+            at_under = c;
+        }
+    }
+    return hi;
+}
 template <int NK>
 __device__ __forceinline__ int select_halves(u64 *list, int want, int slack, bool counted, int half, int n, u64 *thr,
                                              int lane, const u64 (&key)[NK]) {
@@ -624,35 +680,8 @@ __device__ __forceinline__ int select_halves(u64 *list, int want, int slack, boo
     unsigned int limit = ~0u;  // distances up to this are kept ...
     int ties = INT_MAX;        // ... of those equal to it so many
     if (ranked >= want) {
-        unsigned int lo = ~0u, hi = 0u;
-#pragma unroll
-        for (int u = 0; u < NK; ++u) {
-            lo = min(lo, rated[u]);
-            hi = max(hi, rated[u] == ~0u ? 0u : rated[u]);
-        }
-        lo = wave_extreme<true>(lo);
-        hi = wave_extreme<false>(hi);
-        // Fewer than `want` lie below or at `lo - 1` (at_lo of them), at least `want` at or below hi (at_hi of them).
-        unsigned int under = lo - 1u;
-        int at_under = 0, at_hi = ranked;
-        for (int round = 0; at_hi > want + slack && hi - under > 1u; ++round) {
-            const float share = (round & 1) ? 0.5f : (float)(want + slack / 2 - at_under) / (float)(at_hi - at_under);
-            const unsigned int span = hi - under;
-            unsigned int step = (unsigned int)((float)span * share);
-            step = min(max(step, 1u), span - 1u);
-            const unsigned int trial = __builtin_amdgcn_readfirstlane(under + step);
-            int c = 0;
-#pragma unroll
-            for (int u = 0; u < NK; ++u) c += __popcll(__ballot(rated[u] <= trial));
-            if (c >= want) {
-                hi = trial;
-                at_hi = c;
-            } else {
-                under = trial;
-                at_under = c;
-            }
-        }
-        limit = hi;
+        int at_under, at_hi;
+        limit = ranked_limit<NK>(rated, ranked, want, slack, at_under, at_hi);
         if (at_hi > want + slack && !counted) ties = want - at_under;  // (equal distances: as many of them as there is room for)
         // (Entries pass up to 4e-7 beyond the threshold of the moment: with fewer than `want` within it, as a rank among
         // few leaves them, the want-th may be one of those.)
@@ -1428,7 +1457,8 @@ __device__ __forceinline__ float half_scale_factor(const HalfScale *scale) {
 
 // One workgroup per tile.  Xh: [tile][block of 32 points (4)][step of 16 dimensions (S)][lane (64)] 8 halves, lane = 32 *
 // (dimension % 16 / 8) + point % 32, element = dimension % 8 (the layout of pack_points_bf16_kernel, one term).
-// beta: row f of `pitch` floats holds beta_f of every point.  point_len: |x'| and |x' - what the halves stand for|,
+// beta: row f of `pitch` floats holds beta_f of every point times -s^2 / 2 (s: the halves' scale), which is what the
+// accumulators start from; -infinity beyond the points there are, so that nothing passes there.  point_len: |x'| and |x' - what the halves stand for|,
 // rounded up (half_bound.h has what the sweeps make of them).  tile_info: the largest of the second and of |x'| among a
 // tile's points, and the tile's frame.
 __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict__ X, int N, int D, int S,
@@ -1472,7 +1502,7 @@ __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict_
 #pragma unroll
     for (int f = 0; f < kFrames; ++f) {
         const float other = dot[f] + __shfl_xor(dot[f], 32, kWave);
-        if ((f & 1) == h) beta[(size_t)f * pitch + i] = fmaf(-2.0f, other, len);
+        if ((f & 1) == h) beta[(size_t)f * pitch + i] = (i < N ? fmaf(-2.0f, other, len) : INFINITY) * (-0.5f * s * s);
     }
     const float xl = length_bound(len, D), xe = length_bound(eps, D);
     if (h == 0) point_len[i] = make_float2(xl, xe);
@@ -1488,7 +1518,7 @@ __global__ __launch_bounds__(256) void half_pack_kernel(const float *__restrict_
                                       __int_as_float(own), 0.0f);
 }
 
-constexpr int kRankRounds = 3;
+constexpr int kRankRounds = 4;  // (every 256th, 64th, 16th, 4th tile; then all)
 // Memory that no kernel writes while this one runs: with a uniform address, loads on the scalar unit.
 typedef const __attribute__((address_space(4))) float ConstFloat;
 __device__ __forceinline__ ConstFloat *as_const(const void *p) { return (ConstFloat *)p; }
@@ -1991,42 +2021,51 @@ __global__ __launch_bounds__(256, (sweep_occupancy<KSTEPS, BF16>())) void knn_mf
 // output are those of knn_mfma_sweep_kernel; the accumulators start from the candidates' betas and fall as the
 // distance grows, so what is looked for is the largest.
 //
-// What bounds the kernel is the latency of a wave's own chain (the products are a sixth of its time): runs of results
-// in which some lane passes, stores to the lists, selections over them, the barrier that ends a tile.  So: three waves
-// per SIMD, nothing of the tile loop in scratch memory (a wait for a spilled register is a wait for the next tile's loads
-// too: four waves of 128 registers took 115 ms where three of 168 take 92; with five steps two registers lie there, read once per
-// query tile), no sort buffers (a selection holds the list in registers), two LDS tiles and one barrier per
-// tile, what a tile's bound takes fetched a tile ahead.
-// Whole searches, ms, on two bf16 terms / here: 1,000,000 x 50 in four clusters, 90 neighbours 163 / 91; 300000 x 50 without
-// structure 57 / 30; 300000 x 100, 45 neighbours 41 / 24; 199999 x 30, 33 neighbours 11.7 / 9.3; 300000 x 10, 30 neighbours
-// 21.8 / 19.9.
+// What bounds the kernel: about 240 vector instructions a wave and tile, 1000 cycles of a SIMD, and 640 of the matrix unit,
+// which hide less of each other than three waves per SIMD might; a wave waits 44 % of its time.  So: three waves, nothing of
+// the tile loop in scratch memory (a wait for a spilled register is a wait for the next tile's loads too: one of them took
+// the sweep of 1,000,000 x 50 from 74 to 100 ms; four waves of 128 registers 86), and to that end what is seldom run takes
+// its arguments and its lane number where it stands (`cold`, `here`).  Tiles go from memory to LDS without registers; all
+// operands of a pair of blocks are asked for ahead of its products, and all products are under way before the first results
+// are looked at; seldom taken paths lie outside the straight run of the loop.
+// Whole searches, ms, with staging through registers, thresholds from the lists alone and the accumulators loaded from LDS /
+// here: 1,000,000 x 50 in four clusters, 90 neighbours 82.8 / 71.6; 300000 x 50 without structure 28.3 / 25.3;
+// 300000 x 100, 45 neighbours 40.3 / 33.4; 199999 x 30, 33 neighbours 7.6 / 6.3; 300000 x 10, 30 neighbours 11.7 / 10.0.
 //
 // Thresholds ahead of the lists.  A list's own threshold, the `want`-th best of what has been seen, lets 133 ln(N / n)
 // candidates of a query with 90 neighbours through (more, as it is only lowered when a list is full), ten times what is
-// wanted in the end, and each costs a store and a share of the selections.  So after the neighbourhood the tiles are
-// visited in four rounds, every 64th, 16th and 4th tile first: the r-th nearest point of a share p of the tiles is
-// farther than the wanted number of all of them unless r or more of those lie in that share, and ranks[] has the r for
-// which that does not happen (p wanted + 5.5 sqrt(p wanted) + 5: about 1e-8).  Neighbours may lie many to a tile, so at
-// most one entry per query, tile and lane counts, the first that passes: r entries are in r halves of tiles then, and
-// all tiles have r / p with one at least as near.  A query for which it happens all the same is left with too few
-// candidates, fails its verification and is searched again.
+// wanted in the end, and each costs a store and a share of the selections.  So tiles are measured before any entry is
+// stored.  The neighbourhood: of each run of eight results the smallest distance is kept, and the want-th of those that hold
+// a candidate is a threshold that `want` candidates meet.  Then a sample of the tiles beyond it, every 16th (64th, 256th of
+// many): the smallest distance of each tile and lane, and the r-th of those is the threshold: the r-th nearest point of a
+// share p of the tiles is farther than the wanted number of all of them unless r or more of those lie in that share, and
+// ranks[] has the r for which that does not happen (p wanted + 5.5 sqrt(p wanted) + 5: about 1e-8).  The lists are filled
+// after that, round by round: every 4th tile (16th, 64th) first, with another such threshold from the entries after it.
+// Neighbours may lie many to a tile, so at most one entry per query, tile and lane counts, the first that passes: r entries
+// are in r halves of tiles then, and all tiles have r / p with one at least as near.  A query for which it happens all the
+// same is left with too few candidates, fails its verification and is searched again.  Entries per query of the 1,000,000 x
+// 50 search: 1050 from lists and rounds alone, 530 so, for 122 more tiles; selections 8 and 3.
 //
 // Parts: as in the chunked sweep (no rounds: a part's threshold must be that of a list that lacks nothing).
 // Dynamic LDS: two candidate tiles, each
-//   a[cand block (4)][step (S)][lane (64)] 8 halves, 128 betas (times -s^2 / 2)
+//   a[cand block (4)][step (S)][lane (64)] 8 halves, 128 betas (times -s^2 / 2), its tile_info
 // and the visit bitmap.
 // ---------------------------------------------------------------------------
-constexpr int kRoundTiles = 256;  // fewer tiles to visit after the neighbourhood: no rounds
+constexpr int kRoundTiles = 256;   // fewer tiles to visit after the neighbourhood: no rounds
+constexpr int kSampleTiles = 240;  // measured beyond the neighbourhood, about, at most (a lane has room for kHalfCap / 2 distances)
 // Entries of a list, which a selection holds in registers (eight per lane; with sixteen the tile loop's own go to
 // memory: 20000 x 8, 300 neighbours 3.1 ms on bf16 terms, 3.8), and the most candidates kept of them.
 constexpr int kHalfCap = 512, kHalfWant = 256;
 // Workgroups per compute unit the register budget is set for.
 constexpr int half_sweep_occupancy(int steps) { return steps <= 5 ? 3 : 2; }
-constexpr int half_tile_float4(int steps) { return 256 * steps + kCT / 4; }
+constexpr int half_tile_float4(int steps) { return 256 * steps + kCT / 4 + 1; }
 template <int S>
 __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_kernel(const SweepArgs args) {
     constexpr int cap = kHalfCap, half = cap / 2, NK = cap / kWave;
-    const int N = args.N, D = args.D, want = args.want;
+    const int N = args.N, want = args.want;
+    // (loaded once)
+    const float4 *tile_info = args.tile_info, *points = args.Xp;
+    asm volatile("" : "+s"(tile_info), "+s"(points));
     constexpr int kMain = 256 * S, kTile = half_tile_float4(S);
     // Arguments of the code outside the tile loop, read where they are used: kept in registers from the start, they push
     // those of the loop out.
@@ -2037,33 +2076,43 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
         return p;
     };
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    v4f *tiles = reinterpret_cast<v4f *>(lds_raw);
-    unsigned int *bitmap = reinterpret_cast<unsigned int *>(tiles + 2 * kTile);
+    unsigned int *bitmap = reinterpret_cast<unsigned int *>(lds_raw + 2 * kTile * 16);
     __shared__ u64 thr[kMQ];
     __shared__ int fill[256];  // entries in each lane's region of its query's list, around a selection
     __shared__ float qcenter[128];
     __shared__ float tmax_part[2];
 
+    // (A copy that the compiler takes for a new value: what is seldom run forms its addresses from that where it stands, or
+    // they would be formed ahead of the loops and held in the tile loop's registers.)
+    auto here = [](int v) {
+        asm volatile("" : "+v"(v));
+        return v;
+    };
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int qn = lane & 31, kh = lane >> 5;
     u64 *list = args.lists + (size_t)blockIdx.x * kMQ * cap;
-    const float s = half_scale_factor(cold()->half_scale), s2 = 0.5f * s * s, back = -1.0f / s2;  // (powers of two)
+    // (The same in every lane: kept on the scalar side.)
+    auto uniform = [](float v) { return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(v))); };
+    const float s = half_scale_factor(cold()->half_scale), s2 = uniform(0.5f * s * s), back = uniform(-1.0f / s2);  // (powers of two)
     const int T = (N + kCT - 1) / kCT, P = args.parts;
 
-    v4f stage[S], stage_more;
+    // A candidate tile goes to LDS without a register in between: every wave its blocks of 64 slots of 16 bytes, the first
+    // wave the betas (lanes 0 .. 31) and what the tile's bound takes (lane 0) as well.
+    const unsigned int lds_base = __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(LdsByte *)lds_raw);
+    const unsigned int lane_byte = (unsigned int)(wave * 64 + lane) * 16u;
     const float *tile_beta = nullptr;  // of the query tile's frame
-    auto fetch = [&](int tile) {
-        const v4f *src = reinterpret_cast<const v4f *>(args.Xp) + (size_t)tile * kMain + tid;
+    const unsigned int wave_dst = lds_base + (unsigned int)wave * 1024u;
+    auto fetch = [&](int tile, unsigned int buf) {
+        unsigned int to = wave_dst + buf;
+        asm volatile("" : "+s"(to));  // (what is added to it is, where it is used)
 #pragma unroll
-        for (int r = 0; r < S; ++r) stage[r] = src[r * 256];
-        if (tid < kCT / 4) stage_more = reinterpret_cast<const v4f *>(tile_beta + (size_t)tile * kCT)[tid];
-    };
-    auto stash = [&](int buf) {
-        v4f *dst = tiles + buf * kTile + tid;
-#pragma unroll
-        for (int r = 0; r < S; ++r) dst[r * 256] = stage[r];
-        if (tid < kCT / 4) dst[kMain] = stage_more * -s2;
+        for (int r = 0; r < S; ++r) load_to_lds(points + (size_t)tile * kMain + r * 256, lane_byte, to + r * 4096u);
+        if (wave == 0) {
+            const unsigned int dst = lds_base + buf + kMain * 16;
+            if (lane < kCT / 4) load_to_lds(tile_beta + (size_t)tile * kCT, lane_byte, dst);
+            if (lane == 0) load_to_lds(tile_info + tile, lane_byte, dst + kCT * 4);
+        }
     };
 
     for (int w = blockIdx.x; w < args.num_qtiles * P; w += gridDim.x) {
@@ -2080,9 +2129,14 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
         float limit_d = INFINITY;  // the query's threshold
         unsigned int not_counted = (unsigned int)kNotCounted;  // of the next entry of this lane
         bool home = true;
+        // Measuring: of each lane's results only the smallest distances, of runs of eight (in the neighbourhood) or of the
+        // tile, go to the second half of its region, `minima` of them so far, and nothing to the list.
+        bool measure = false;
+        int minima = 0;
         auto my_fill = [&]() { return (int)((my_at - region) / (unsigned int)sizeof(u64)); };
         // Selections over the lists of this wave's queries in `mask`, the next list on its way into registers meanwhile.
         auto select_queries = [&](unsigned int mask, int rank, int slack, bool counted) {
+            const int tid = here(threadIdx.x), lane = tid & 63, qn = lane & 31;
             fill[tid] = my_fill();
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             auto counts = [&](int b, int &c0, int &n) {
@@ -2123,257 +2177,318 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
         v8h bq[S];
         HalfQuery hq;
         {
-            const v4f *src = reinterpret_cast<const v4f *>(args.Xp) + (size_t)qt * kMain + (size_t)wave * S * 64 + lane;
+            const v4f *src = reinterpret_cast<const v4f *>(points) + (size_t)qt * kMain + (size_t)wave * S * 64 + lane;
 #pragma unroll
             for (int k = 0; k < S; ++k) bq[k] = __builtin_bit_cast(v8h, src[k * 64]);
         }
         const float2 len = cold()->point_len[q];
-        hq = half_query(len.x, len.y, D, back);
-        const int own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(args.tile_info[qt].z));
-        tile_beta = args.beta + (size_t)own_frame * args.beta_pitch;
+        hq = half_query(len.x, len.y, cold()->D, back);
+        hq.kap = uniform(hq.kap);
+        hq.least = uniform(hq.least);
+        const int own_frame = __builtin_amdgcn_readfirstlane(__float_as_int(cold()->tile_info[qt].z));
+        tile_beta = cold()->beta + (size_t)own_frame * cold()->beta_pitch;
+        // The query's betas: the two lanes of a query have the even and the odd frames'.
+        v8f query_beta;
+        const int odd = here(kh);
+#pragma unroll
+        for (int f = 0; f < kFrames / 2; ++f) query_beta[f] = cold()->beta[(size_t)(2 * f + odd) * cold()->beta_pitch + q];
+        const float my_d2 = cold()->frame_d2[own_frame * kFrames + (lane & (kFrames - 1))];  // a frame per lane
+        const float my_frame_len = length_bound(my_d2, cold()->D);
 
-        int buf = 0;
-        // What the bound of a tile takes, and the query's distance from its frame: fetched a tile ahead.
-        float2 info, next_info;
-        int next_frame = -1;
-        float next_beta = 0.0f;
-        const float *const query_beta = args.beta + q;
-        const float my_d2 = args.frame_d2[own_frame * kFrames + (lane & (kFrames - 1))];  // a frame per lane
-        const float my_frame_len = length_bound(my_d2, D);
-        auto fetch_info = [&](int tile) {
-            const int t = __builtin_amdgcn_readfirstlane(tile);
-            ConstFloat *of_tile = as_const(args.tile_info) + 4 * (size_t)t;  // (scalar loads)
-            next_info = make_float2(of_tile[0], of_tile[1]);
-            next_frame = __float_as_int(of_tile[2]);
-        };
-        auto fetch_beta = [&]() { next_beta = query_beta[(size_t)next_frame * args.beta_pitch]; };
-        // One tile: compute it from LDS buffer `buf` while the next one travels through registers into the other.
+        unsigned int buf = 0;  // byte offset of the LDS buffer that holds the tile at hand: 0 or kTile * 16
+        // One tile: compute it from LDS buffer `buf` while the next one travels into the other.
         auto process = [&](int ct, int next_ct) {
             const int c0 = ct * kCT;
-            info = next_info;
-            if (next_frame != hq.frame)
-                enter_frame(hq, next_frame, next_beta, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_d2), next_frame)),
-                            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_frame_len), next_frame)));
-            if (next_ct >= 0) {
-                fetch(next_ct);
-                fetch_info(next_ct);
+            const v4f *tile = reinterpret_cast<const v4f *>(lds_raw + buf);
+            // All operands of the first two blocks of candidates are asked for before their first product, those of the others
+            // as registers come free; and all products are under way before the first result is looked at: the filter of
+            // the first two blocks runs beside the products of the others.
+            v4f a[4][S];
+            float start[2];
+            auto load_start = [&](int pair) { start[pair] = reinterpret_cast<const float *>(tile + kMain)[64 * pair + lane]; };
+            auto load_step = [&](int pair, int k) {
+                a[2 * pair][k] = tile[(2 * pair * S + k) * 64 + lane];
+                a[2 * pair + 1][k] = tile[((2 * pair + 1) * S + k) * 64 + lane];
+            };
+            // The accumulators start from the betas by a product of a column of them and a row of ones: one word of LDS per
+            // lane and two blocks, where loading every lane's sixteen of a block takes as much of the LDS as the operands.
+            v16f acc[4];
+            auto multiply = [&](int pair) {
+                const v32f both = __builtin_amdgcn_mfma_f32_32x32x1f32(start[pair], 1.0f, v32f{}, 0, 0, 0);
+                acc[2 * pair] = __builtin_shufflevector(both, both, 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
+                acc[2 * pair + 1] = __builtin_shufflevector(both, both, 16, 17, 18, 19, 20, 21, 22, 23, 24, 25, 26, 27, 28, 29, 30, 31);
+                if (pair == 0) load_start(1);
+#pragma unroll
+                for (int k = 0; k < S; ++k) {
+#pragma unroll
+                    for (int b = 2 * pair; b < 2 * pair + 2; ++b)
+                        acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[b][k]), bq[k], acc[b], 0, 0, 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (pair == 0) load_step(1, k);
+                }
+            };
+            load_start(0);
+#pragma unroll
+            for (int k = 0; k < S; ++k) load_step(0, k);
+            const v4f info = tile[kMain + kCT / 4];
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(next_ct >= 0 ? next_ct : ct, kTile * 16 - buf);  // (last read a tile ago, before the barrier that ended that tile)
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(1);
+            __builtin_amdgcn_sched_barrier(0);
+            const int frame = __builtin_amdgcn_readfirstlane(__float_as_int(info[2]));
+            if (frame != hq.frame) {
+                const unsigned int mine = __float_as_uint(query_beta[frame >> 1]);
+                const auto halves = __builtin_amdgcn_permlane32_swap(mine, mine, false, false);
+                const float beta = __uint_as_float((frame & 1) ? halves[1] : halves[0]) * back;
+                enter_frame(hq, frame, beta, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_d2), frame)),
+                            __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_frame_len), frame)));
             }
-            const v4f *tile = tiles + buf * kTile;
             // Distance less its bound = off + product * back; what is tested is the product.  (Never -inf: excluded
             // elements must fail also while the query has no threshold.)
             not_counted = home ? (unsigned int)kNotCounted : 0u;
-            const float off = tile_offset(hq, info.x, info.y);
+            const float off = tile_offset(hq, info[0], info[1]);
             const float limit_acc = ((off - limit_d) - 4e-7f * (fabsf(off) + fabsf(limit_d))) * s2;
             const float lim = live ? fmaxf(limit_acc, -3.4028234663852886e38f) : INFINITY;
-            const bool edge = c0 + kCT > N || (unsigned int)(q0 - c0) < (unsigned int)kCT;
-            auto multiply = [&](int cb, v16f &acc0, v16f &acc1) {
-                const v4f *b0 = tile + (size_t)cb * S * 64 + lane, *b1 = b0 + S * 64;
-                // (register v of the result is candidate 8 (v / 4) + 4 (lane / 32) + v % 4 of the block)
-                const v4f *start = tile + kMain + 8 * cb + kh;
+            // The largest of each run of eight results: a run in which no lane of the wave passes is skipped.  (Element v of
+            // run r is candidate c0 + 16 r + 4 kh + v + (v & 4).)
+            float run_max[8];
 #pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const v4f t0 = start[2 * g], t1 = start[8 + 2 * g];
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        acc0[4 * g + k] = t0[k];
-                        acc1[4 * g + k] = t1[k];
-                    }
+            for (int r = 0; r < 8; ++r) {
+                const v16f &x = acc[r >> 1];
+                const int o = 8 * (r & 1);
+                float m = matrix_result(x[o + 7]);
+                m = max3(m, x[o], x[o + 1]);
+                m = max3(m, x[o + 2], x[o + 3]);
+                m = max3(m, x[o + 4], x[o + 5]);
+                run_max[r] = max2(m, x[o + 6]);
+            }
+            if (TSNE_UNLIKELY(measure)) {
+                float *to = reinterpret_cast<float *>(reinterpret_cast<char *>(list) + region + half * (sizeof(u64) / 2)) + min(minima, half - 1);
+                auto key = [&](float p) { return fmaxf(fmaf(p, back, off), 0.0f); };
+                if (home) {
+                    v4f *const to4 = reinterpret_cast<v4f *>(to);
+                    to4[0] = v4f{key(run_max[0]), key(run_max[1]), key(run_max[2]), key(run_max[3])};
+                    to4[1] = v4f{key(run_max[4]), key(run_max[5]), key(run_max[6]), key(run_max[7])};
+                    minima += 8;
+                } else {
+                    float m = max3(run_max[0], run_max[1], run_max[2]);
+                    m = max3(m, run_max[3], run_max[4]);
+                    *to = key(max2(max3(m, run_max[5], run_max[6]), run_max[7]));
+                    ++minima;
                 }
-                v4f next[2] = {b0[0], b1[0]};
+            } else {
 #pragma unroll
-                for (int k = 0; k < S; ++k) {
-                    const v8h x = __builtin_bit_cast(v8h, next[0]), y = __builtin_bit_cast(v8h, next[1]);
-                    if (k + 1 < S) {
-                        next[0] = b0[(k + 1) * 64];
-                        next[1] = b1[(k + 1) * 64];
-                    }
-                    acc0 = __builtin_amdgcn_mfma_f32_32x32x16_f16(x, bq[k], acc0, 0, 0, 0);
-                    acc1 = __builtin_amdgcn_mfma_f32_32x32x16_f16(y, bq[k], acc1, 0, 0, 0);
-                }
-            };
-            auto filter = [&](int cb, v16f &acc0, v16f &acc1) {
-                // The largest of each run of eight results: a run in which no lane of the wave passes is skipped.
-                float run_max[4];
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const v16f &a = g < 2 ? acc0 : acc1;
-                    const int o = 8 * (g & 1);
-                    float m = matrix_result(a[o + 7]);
-                    m = max3(m, a[o], a[o + 1]);
-                    m = max3(m, a[o + 2], a[o + 3]);
-                    m = max3(m, a[o + 4], a[o + 5]);
-                    run_max[g] = max2(m, a[o + 6]);
-                }
-                const int jbase = c0 + cb * 32 + 4 * kh;  // element (half, v) is candidate jbase + 32 half + 8 (v / 4) + v % 4
-                // Only the last tile has candidates beyond N and only the query's own tile holds the query.
-                if (edge) {
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        int j = jbase + 8 * (e >> 2) + (e & 3);
-                        asm volatile("" : "+v"(j));  // (one after the other: thirty comparisons at a time take every register)
-                        if (j >= N || j == q) acc0[e] = -INFINITY;
-                        if (j + 32 >= N || j + 32 == q) acc1[e] = -INFINITY;
-                    }
-                }
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    // (the maxima are from before the exclusions: upper bounds, which is all this needs)
-                    if (__ballot(run_max[g] >= lim) == 0) continue;
+                for (int r = 0; r < 8; ++r) {
+                    if (TSNE_LIKELY(__ballot(run_max[r] >= lim) == 0)) continue;
+                    const v16f &x = acc[r >> 1];
+                    const int o = 8 * (r & 1);
                     // All eight comparisons first: a branch on a comparison just made waits for it.
                     u64 any[8];
 #pragma unroll
-                    for (int v = 0; v < 8; ++v) any[v] = __ballot((g < 2 ? acc0 : acc1)[8 * (g & 1) + v] >= lim);
+                    for (int v = 0; v < 8; ++v) any[v] = __ballot(x[o + v] >= lim);
 #pragma unroll
                     for (int v = 0; v < 8; ++v) {
-                        if (any[v] == 0) continue;
+                        if (TSNE_LIKELY(any[v] == 0)) continue;
                         asm volatile("");  // (a scalar branch, not a condition more for the lanes)
-                        const int e = 8 * (g & 1) + v;
-                        const float p = (g < 2 ? acc0 : acc1)[e];
-                        if (p >= lim) {
-                            int jb = jbase;
-                            asm volatile("" : "+v"(jb));  // the index is formed here, not held in 32 registers
+                        const float p = x[o + v];
+                        const int j = c0 + 16 * r + 4 * (here(lane) >> 5) + v + (v & 4);  // (formed here, not held in registers)
+                        if (p >= lim && j != q) {
                             *reinterpret_cast<u64 *>(reinterpret_cast<char *>(list) + my_at) =
-                                pack_key_positive(fmaxf(fmaf(p, back, off), 0.0f),
-                                                  (int)((unsigned int)(jb + 32 * (g >> 1) + 8 * (e >> 2) + (e & 3)) | not_counted));
+                                pack_key_positive(fmaxf(fmaf(p, back, off), 0.0f), (int)((unsigned int)j | not_counted));
                             my_at += (unsigned int)sizeof(u64);
                             not_counted = (unsigned int)kNotCounted;
                         }
                     }
                 }
-            };
-            v16f acc0, acc1;
-            multiply(0, acc0, acc1);
-            if (next_ct >= 0) fetch_beta();
-            filter(0, acc0, acc1);
-            multiply(2, acc0, acc1);
-            if (next_ct >= 0) stash(buf ^ 1);  // (last read a tile ago, before the barrier that ended that tile)
-            filter(2, acc0, acc1);
+            }
+            wait_for_loads();  // (the next tile is in LDS)
             __syncthreads();
-            if (next_ct >= 0) buf ^= 1;
+            buf = kTile * 16 - buf;
         };
 
-        // Phase 1: the query tile's neighbourhood; phase 2: the tiles the bitmap keeps.
         const int reach = max(kHomeTiles / P, 2) * P;  // (at least two tiles either side of every part)
         const int h0 = max(qt - reach, 0), h1 = min(qt + reach, T - 1);
         int word_idx = -1;
         unsigned int cur_word = 0u;
-        // Next set bit of the bitmap, ascending within a round; every wave walks the same words.  Round k takes the
-        // tiles that are `first` modulo 64, 16, 4 and 1, without those of the rounds before it.
-        int round = kRankRounds;
-        bool in_rounds = false;
-        const int first = (int)((unsigned int)qt * 0x9E3779B1u >> 26);
+        // Next set bit of the bitmap, ascending within a round; every wave walks the same words, sixty-four at a time.  Round
+        // k takes the tiles that are `first` modulo 256, 64, 16, 4 and 1, without those of the rounds before it.
+        int round = kRankRounds, first_round = kRankRounds, last_round = kRankRounds;
+        const int first = (int)((unsigned int)(w / (int)gridDim.x) * 0x9E3779B1u >> 24);
         auto round_mask = [&](int k, int word) -> unsigned int {
-            return k < 0   ? 0u
-                   : k == 0 ? ((word & 1) == first >> 5 ? 1u << (first & 31) : 0u)
-                   : k == 1 ? 0x00010001u << (first & 15)
-                   : k == 2 ? 0x11111111u << (first & 3)
+            return k == 0   ? ((word & 7) == first >> 5 ? 1u << (first & 31) : 0u)
+                   : k == 1 ? ((word & 1) == ((first >> 5) & 1) ? 1u << (first & 31) : 0u)
+                   : k == 2 ? 0x00010001u << (first & 15)
+                   : k == 3 ? 0x11111111u << (first & 3)
                             : ~0u;
         };
         bool round_over = false;  // the tile returned last was the last of its round
         auto next_tile = [&]() -> int {
-            for (;;) {
-                while (cur_word == 0u) {
-                    ++word_idx;
-                    if (word_idx >= args.bitmap_words) {
-                        if (round == kRankRounds) return -1;
+            if (TSNE_UNLIKELY(cur_word == 0u)) {
+                const int lane = here(threadIdx.x) & 63;
+                for (;;) {
+                    const int word = word_idx + 1 + lane;
+                    unsigned int bits = word < cold()->bitmap_words ? bitmap[word] : 0u;
+                    bits &= round_mask(round, word) & ~(round > first_round ? round_mask(round - 1, word) : 0u);
+                    const u64 some = __ballot(bits != 0u);
+                    if (some) {
+                        const int l = __ffsll((long long)some) - 1;
+                        cur_word = (unsigned int)__builtin_amdgcn_readlane((int)bits, l);
+                        word_idx += 1 + l;
+                        break;
+                    }
+                    word_idx += kWave;
+                    if (word_idx + 1 >= cold()->bitmap_words) {
+                        if (round == last_round) return -1;
                         ++round;
                         round_over = true;
                         word_idx = -1;
-                        continue;
                     }
-                    cur_word = bitmap[word_idx];
-                    if (in_rounds) cur_word &= round_mask(round, word_idx) & ~round_mask(round - 1, word_idx);
                 }
-                const int b = __ffs((int)cur_word) - 1;
-                cur_word &= cur_word - 1u;
-                return word_idx * 32 + b;
             }
+            const int b = __ffs((int)cur_word) - 1;
+            cur_word &= cur_word - 1u;
+            return word_idx * 32 + b;
         };
-        int cur = h0 + (part - h0 % P + P) % P;  // this part's first tile of the neighbourhood
-        if (cur > h1) cur = -1;  // fewer tiles than parts: nothing for this part, its lists stay empty
-        if (cur >= 0) {
-            fetch(cur);
-            fetch_info(cur);
-            fetch_beta();
-        }
-        __syncthreads();
-        if (cur >= 0) stash(0);
-        __syncthreads();
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): see below
-        unsigned int swept = 0;
-        for (bool done = false; !done; ) {
-            int nxt = -1;
+        // From rounds `from` to `to`: the first tile of theirs.
+        auto start_rounds = [&](int from, int to) -> int {
+            home = false;
+            round = first_round = from;
+            last_round = to;
+            word_idx = -1;
+            cur_word = 0u;
+            const int t = next_tile();
             round_over = false;
-            if (cur >= 0) {
-                ++swept;
-                nxt = home ? (cur + P <= h1 ? cur + P : -1) : next_tile();
-                process(cur, nxt);
-            }
-            const bool home_done = cur >= 0 && nxt < 0 && home && (h0 > 0 || h1 < T - 1);
-            done = nxt < 0 && !home_done;
-            // Lists that a further tile could overflow are compacted by their own wave, right away (a region takes at
-            // most 64 entries per tile); all of them after the neighbourhood, for thresholds, and at the end.
-            unsigned int mask = all_queries;
-            if (nxt >= 0 && !round_over) {
-                const u64 crowded = __ballot(my_fill() > half - kCT / 2);
-                mask = (unsigned int)(crowded | (crowded >> 32));  // lanes l, l+32 share a query
-            }
-            // (A list whose counted entries are too few for a rank keeps all it has, full or not, and so may one whose
-            // entries are equally far: those are compacted like any other before the next tile.)
-            for (bool rank = round_over && nxt >= 0; mask; rank = false) {
-                const int slack = cold()->select_slack;
-                select_queries(mask, rank ? cold()->ranks[round - 1] : want, rank || nxt < 0 ? 0 : slack, rank);
-                const u64 crowded = rank ? __ballot(my_fill() > half - kCT / 2) : 0ull;
-                mask = (unsigned int)(crowded | (crowded >> 32));
-            }
-            if (home_done) {
-                home = false;
-                for (int k = tid; k < args.bitmap_words; k += 256) bitmap[k] = 0u;
-                if (tid < args.D) qcenter[tid] = cold()->centers_t[(size_t)tid * T + qt];
-                __syncthreads();
-                if (tid < kMQ) {
-                    // Largest squared distance any query of the tile would still accept (rounded up).
-                    float v = -INFINITY;
-                    if (q0 + tid < N) {
-                        const u64 t = thr[tid];
-                        v = t == ~0ull ? INFINITY : key_distance(t);
-                        v += 1e-5f * fabsf(v) + 1e-30f;
-                    }
-                    v = group_max<kWave>(v);
-                    if (lane == 0) tmax_part[wave] = v;
+            return t;
+        };
+        // Thresholds from the measured distances: the one of rank `rank` of a query's two lanes'.
+        auto take_thresholds = [&](int rank) {
+            asm volatile("" ::: "memory");
+            minima = min(minima, half);
+            const int lane = here(threadIdx.x) & 63;
+            for (int b = 0; b < valid; ++b) {
+                const unsigned int *from = reinterpret_cast<const unsigned int *>(list + (size_t)(wave * 32 + b) * cap + half / 2);
+                unsigned int rated[NK];
+                int ranked = 0;
+#pragma unroll
+                for (int u = 0; u < NK; ++u) {
+                    const int e = u * kWave + lane;
+                    rated[u] = ~0u;
+                    if (e < 2 * minima) rated[u] = from[e < minima ? e : 2 * half + e - minima] | 0x80000000u;
+                    if (rated[u] >= 0xff800000u) rated[u] = ~0u;  // (no candidate in it)
+                    ranked += __popcll(__ballot(rated[u] != ~0u));
                 }
-                __syncthreads();
-                const float tmax = fmaxf(tmax_part[0], tmax_part[1]);
-                const float *radius = cold()->radius, *centers_t = cold()->centers_t;
-                const float ra = radius[qt];
-                for (int t = tid; t < T; t += 256)
-                    if ((t < h0 || t > h1) && t % P == part && tile_may_matter(qcenter, ra, centers_t, radius, D, T, t, tmax))
-                        atomicOr(&bitmap[t >> 5], 1u << (t & 31));
-                __syncthreads();
-                int visits = 0;
-                for (int k = lane; k < args.bitmap_words; k += kWave) visits += __popc(bitmap[k]);
-                visits = __builtin_amdgcn_readfirstlane(group_sum_int(visits));
-                if (P == 1 && visits >= kRoundTiles) {
-                    in_rounds = true;
-                    round = 0;
-                }
-                nxt = next_tile();
-                round_over = false;
-                done = nxt < 0;
-                if (nxt >= 0) {
-                    fetch(nxt);
-                    fetch_info(nxt);
-                    fetch_beta();
-                    stash(buf);  // the barrier that ended the last tile freed both buffers
-                    __syncthreads();
-                }
-                // (nothing left in flight as far as the compiler can tell, as in the kernel above)
-                __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+                if (ranked < rank) continue;
+                int at_under, at_hi;
+                const unsigned int limit = ranked_limit<NK>(rated, ranked, rank, rank / 16, at_under, at_hi);
+                if (lane == 0) thr[wave * 32 + b] = min(thr[wave * 32 + b], ((u64)limit << 32) | 0xffffffffull);
             }
+            minima = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const u64 limit = thr[wave * 32 + (lane & 31)];
+            limit_d = limit == ~0ull ? INFINITY : key_distance(limit);
+        };
+        // The tiles that some query of the tile may want, by the thresholds so far: their number.
+        auto map_tiles = [&]() -> int {
+            const int tid = here(threadIdx.x), lane = tid & 63;
+            for (int k = tid; k < cold()->bitmap_words; k += 256) bitmap[k] = 0u;
+            if (tid < cold()->D) qcenter[tid] = cold()->centers_t[(size_t)tid * T + qt];
+            __syncthreads();
+            if (tid < kMQ) {
+                // Largest squared distance any query of the tile would still accept (rounded up).
+                float v = -INFINITY;
+                if (q0 + tid < N) {
+                    const u64 t = thr[tid];
+                    v = t == ~0ull ? INFINITY : key_distance(t);
+                    v += 1e-5f * fabsf(v) + 1e-30f;
+                }
+                v = group_max<kWave>(v);
+                if (lane == 0) tmax_part[tid >> 6] = v;
+            }
+            __syncthreads();
+            const float tmax = fmaxf(tmax_part[0], tmax_part[1]);
+            const float *radius = cold()->radius, *centers_t = cold()->centers_t;
+            const float ra = radius[qt];
+            for (int t = tid; t < T; t += 256)
+                if ((t < h0 || t > h1) && t % P == part && tile_may_matter(qcenter, ra, centers_t, radius, cold()->D, T, t, tmax))
+                    atomicOr(&bitmap[t >> 5], 1u << (t & 31));
+            __syncthreads();
+            int visits = 0;
+            for (int k = lane; k < cold()->bitmap_words; k += kWave) visits += __popc(bitmap[k]);
+            return __builtin_amdgcn_readfirstlane(group_sum_int(visits));
+        };
+        const int home_first = h0 + (part - h0 % P + P) % P;  // this part's first tile of the neighbourhood
+        int cur = home_first <= h1 ? home_first : -1;          // (fewer tiles than parts: nothing for this part, its lists stay empty)
+        const bool beyond = h0 > 0 || h1 < T - 1;
+        // The passes over a query tile's tiles.  The neighbourhood is measured first, where that gives distances enough, so
+        // that the lists begin with a threshold, and so is, where there are many of them, a sample of the tiles beyond.
+        enum { kMeasureHome, kListHome, kMeasureRounds, kListRounds, kDone };
+        int pass = beyond && cur >= 0 && 16 * ((h1 - home_first) / P + 1) > want + want / 8 ? kMeasureHome : kListHome;
+        measure = pass == kMeasureHome;
+        int sample = kRankRounds;  // the round whose tiles are measured (kRankRounds: none)
+        if (cur >= 0) fetch(cur, 0);
+        wait_for_loads();
+        __syncthreads();
+        unsigned int swept = 0;
+        while (cur >= 0) {
+            round_over = false;
+            int nxt;
+            if (TSNE_UNLIKELY(home)) nxt = cur + P <= h1 ? cur + P : -1;
+            else nxt = next_tile();
+            process(cur, nxt);
+            swept += measure ? 0 : 1;
+            if (TSNE_LIKELY(nxt >= 0 && !round_over && __ballot(my_fill() > half - kCT / 2) == 0)) {
+                cur = nxt;
+                continue;
+            }
+            if (nxt >= 0) {
+                // Lists that a further tile could overflow are compacted by their own wave, right away (a region takes at
+                // most 64 entries per tile); all of them after a round, for thresholds.  (A list whose counted entries are
+                // too few for a rank keeps all it has, full or not, and so may one whose entries are equally far: those are
+                // compacted like any other before the next tile.)
+                const auto crowded = [&]() -> unsigned int {
+                    const u64 lanes = __ballot(my_fill() > half - kCT / 2);
+                    return (unsigned int)(lanes | (lanes >> 32));  // lanes l, l+32 share a query
+                };
+                if (round_over) select_queries(all_queries, cold()->ranks[round - 1], 0, true);
+                const unsigned int mask = crowded();
+                if (mask) select_queries(mask, want, cold()->select_slack, false);
+                cur = nxt;
+                continue;
+            }
+            // A pass is over: on to the next that has tiles.
+            while (nxt < 0 && pass != kDone) {
+                measure = false;
+                if (pass == kMeasureHome) {
+                    take_thresholds(want + 1);  // (the query itself is the nearest of one run)
+                    pass = kListHome;
+                    nxt = home_first;
+                } else if (pass == kListHome && beyond) {
+                    select_queries(all_queries, want, 0, false);
+                    const int visits = map_tiles();
+                    if (P == 1 && visits >= kRoundTiles) sample = visits <= 16 * kSampleTiles ? 2 : visits <= 64 * kSampleTiles ? 1 : 0;
+                    measure = sample < kRankRounds;
+                    pass = measure ? kMeasureRounds : kListRounds;
+                    nxt = start_rounds(sample, sample);
+                } else if (pass == kMeasureRounds) {
+                    take_thresholds(cold()->ranks[sample]);
+                    pass = kListRounds;
+                    nxt = start_rounds(sample + 1, kRankRounds);
+                } else {
+                    pass = kDone;
+                }
+            }
+            if (nxt >= 0) fetch(nxt, buf);  // the barrier that ended the last tile freed both buffers
+            wait_for_loads();
+            __syncthreads();
             cur = nxt;
         }
+        select_queries(all_queries, want, 0, false);
         if (tid == 0) atomicAdd(cold()->tiles_swept, (unsigned long long)swept);
         // Output, every wave for its own queries.
+        const int lane = here(threadIdx.x) & 63;
         for (int b = 0; b < valid; ++b) {
             const int ql = wave * 32 + b;
             const int n = fill[wave * 64 + b] + fill[wave * 64 + b + 32];
@@ -2477,7 +2592,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     auto stash = [&](int b, bool first) {
 #pragma unroll
         for (int r = 0; r < kSlots; ++r) a_lds[b * kChunkF4 + r * 256 + tid] = stage[r];
-        if (HALF && first && tid < kCT / 4) beta_lds[(parity ^ 1) * (kCT / 4) + tid] = stage_beta * -half_s2;
+        if (HALF && first && tid < kCT / 4) beta_lds[(parity ^ 1) * (kCT / 4) + tid] = stage_beta;
     };
     const int num_ctiles = (N + kCT - 1) / kCT;
 
@@ -2630,7 +2745,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 const int frame = __builtin_amdgcn_readfirstlane(__float_as_int(info.z));
                 if (frame != hq.frame) {
                     const float d2 = args.frame_d2[own_frame * kFrames + frame];
-                    enter_frame(hq, frame, args.beta[(size_t)frame * args.beta_pitch + q], d2, length_bound(d2, D));
+                    enter_frame(hq, frame, args.beta[(size_t)frame * args.beta_pitch + q] * half_back, d2, length_bound(d2, D));
                 }
                 off = tile_offset(hq, info.x, info.y);
                 limit_acc = ((off - limit_d) - 4e-7f * (fabsf(off) + fabsf(limit_d))) * half_s2;
@@ -3678,7 +3793,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         args.frame_d2 = operands.frame_d2();
         args.half_scale = operands.scale();
         for (int k = 0; k < kRankRounds; ++k) {
-            const double share = (double)(K - 1 + 16 + (K - 1) / 8) / (double)(64 >> (2 * k));
+            const double share = (double)(K - 1 + 16 + (K - 1) / 8) / (double)(256 >> (2 * k));
             args.ranks[k] = (int)std::ceil(share + 5.5 * std::sqrt(share) + 5.0);
         }
         const size_t lds = geometry.lds_with(cap);
