@@ -60,6 +60,8 @@ inline bool forces_ride_along(int N, int K) {
 // one in one box, and tails of two degrees of freedom: 1203 points 64 / 47, 49 / 45; 5000 66 / 53, 51 / 48; 10007 67 / 62,
 // 65 / 71; 15361 68 / 71, 59 / 71; 20011 69 / 78, 66 / 99.
 constexpr int kScanPoints = 20480;
+static_assert(kScanPoints <= 65536, "point numbers of 16 bits (row_points)");
+constexpr int kScanRows = kFftShort / (2 * kInterp);  // most boxes per side of an 800-point transform's grid
 
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
@@ -135,6 +137,10 @@ struct tsne_hip_plan {
     // Small problems (one stream, see api.hip): the pattern once more, row by row, {probability, neighbour} in the
     // caller's order of neighbours; the inverse row pass computes the attractive forces from it in spare workgroups.
     uint2 *row_entries = nullptr;
+    // ... and, up to kScanPoints points, for each row of boxes the points that the spreading scan found there (num_points of
+    // them at most) and their number, for the gathering at the end of the same step's chain.
+    unsigned short *row_points = nullptr;
+    int *row_counts = nullptr;
     int steps_to_grouping = 0;      // steps of that form until the grouping kernels are launched again, in this call
     int spin_limit = 0;             // polls before a wave of the attractive kernel gives up a wait
     bool blocked_ready = false;
