@@ -63,6 +63,7 @@
 #include <cmath>
 #include <cstring>
 #include <new>
+#include <type_traits>
 #include <vector>
 
 namespace tsnehip {
@@ -2535,6 +2536,7 @@ constexpr int kChunkFloat4 = 4 * kChunkS4 * 64;      // float4 per tile chunk
 // forms it chunk by chunk from the query's own two terms and the centre's chunk, which is five vector instructions
 // per coordinate and 16 registers beside the matrix instructions (sweeps of 50000 x 1024: 27.5 -> 24.3 ms and 1.2 for
 // the table; 60000 x 784: 13.7 -> 11.9 and 1.1).
+constexpr int kSweepXcds = 8;
 template <Products PRODUCTS, bool TABLE>
 __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const SweepArgs args) {
     constexpr bool BF16 = PRODUCTS == Products::kBf16, HALF = PRODUCTS == Products::kHalf;
@@ -2546,7 +2548,9 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     // Slots of 16 bytes per lane, block and chunk: 8 groups of four k-steps (64 dimensions) on floats; on bf16
     // terms 2 terms x 2 steps of 16 dimensions (32 dimensions: with 64 the chunk loop's registers did not fit
     // and the compiler spilled the prefetched chunks the moment they were loaded).
-    // halves 4 steps of 16 dimensions (64): sweeps of 50000 x 1024 21.8 -> 11.9 ms, of 60000 x 784 9.2 -> 5.7.
+    // halves 4 steps of 16 dimensions (64): sweeps of 50000 x 1024 21.8 -> 11.9 ms, of 60000 x 784 9.2 -> 5.7.  Straight into
+    // LDS and with a step's operands ahead of the products of the one before, searches of 60000 x 784 10.5 -> 10.0, of
+    // 40000 x 200 5.8 -> 5.5.
     constexpr int kSlots = BF16 || HALF ? 4 : kChunkS4;
     constexpr int kSteps16 = 2;                     // bf16: steps of 16 dimensions per chunk
     constexpr int kChunkF4 = 4 * kSlots * 64;       // float4 per tile chunk
@@ -2574,31 +2578,48 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     const float half_s = HALF ? half_scale_factor(args.half_scale) : 1.0f, half_s2 = 0.5f * half_s * half_s;
     const float half_back = -1.0f / half_s2;  // (a power of two)
     const float *tile_beta = nullptr;         // of the query tile's frame
-    v4f stage_beta;
     int parity = 0;
 
     // Chunk c of a candidate tile: global -> registers -> LDS.  Element e = 256 r + tid of the chunk is
-    // float4 (e % 512) of block e / 512 = r / 2.
-    v4f stage[kSlots];
+    // float4 (e % 512) of block e / 512 = r / 2.  (Halves: straight into LDS buffer b, block r by the 256 threads' r-th
+    // load; with a tile's first chunk its betas, by the first wave.)
+    v4f stage[HALF ? 1 : kSlots];
+    const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+    const unsigned int lane_byte = (unsigned int)tid * 16u;
+    auto fetch_half = [&](int tile, int c, int b) {
+        const float4 *src = args.Xp + (size_t)tile * tile_stride + (size_t)c * (kSlots * 64);
+        unsigned int to = __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(LdsByte *)lds_raw) + (unsigned int)(b * kChunkF4 * 16 + wave_u * 1024);
+        asm volatile("" : "+s"(to));
+#pragma unroll
+        for (int r = 0; r < 4; ++r) load_to_lds(src + r * block_stride, lane_byte, to + r * 4096u);
+        if (c == 0 && wave_u == 0 && lane < kCT / 4)
+            load_to_lds(tile_beta + (size_t)tile * kCT, lane_byte,
+                        __builtin_amdgcn_readfirstlane((unsigned int)(size_t)(LdsByte *)beta_lds) + (unsigned int)(parity ^ 1) * (kCT * 4));
+    };
     auto fetch = [&](int tile, int c) {
         const v4f *src = reinterpret_cast<const v4f *>(args.Xp) + (size_t)tile * tile_stride + (size_t)c * (kSlots * 64) + tid;
         // element 256 r + tid of the chunk: block (256 r + tid) / (64 kSlots), float4 (256 r + tid) % (64 kSlots) of it
 #pragma unroll
         for (int r = 0; r < kSlots; ++r)
             stage[r] = src[(size_t)((256 * r) / (64 * kSlots)) * block_stride + (256 * r) % (64 * kSlots)];
-        if (HALF && c == 0 && tid < kCT / 4) stage_beta = reinterpret_cast<const v4f *>(tile_beta + (size_t)tile * kCT)[tid];
     };
-    // (first: of a tile)
-    auto stash = [&](int b, bool first) {
+    auto stash = [&](int b) {
 #pragma unroll
         for (int r = 0; r < kSlots; ++r) a_lds[b * kChunkF4 + r * 256 + tid] = stage[r];
-        if (HALF && first && tid < kCT / 4) beta_lds[(parity ^ 1) * (kCT / 4) + tid] = stage_beta;
     };
     const int num_ctiles = (N + kCT - 1) / kCT;
 
     const int P = args.parts;
-    for (int w = blockIdx.x; w < num_qtiles * P; w += gridDim.x) {
-        const int qi = w / P, part = w - qi * P;
+    // The parts of a query tile go to workgroups of one XCD, which read the tile's operands at about the same time, and so do
+    // query tiles next to each other, which visit much the same candidate tiles.  (Workgroups go to the XCDs round robin; the
+    // grid is a multiple of their number times P.  50000 x 1024: 65 % of the requests missed the L2 with the parts dealt to all
+    // XCDs, and the sweep went at the rate of the cache behind it, 7 TB/s; 46 % so, 12.0 -> 10.3 ms.)
+    const int round_tiles = (int)gridDim.x / P, xcd = (int)blockIdx.x % kSweepXcds;
+    const int in_xcd = (int)blockIdx.x / kSweepXcds, part = in_xcd % P;
+    for (int round = 0; round < num_qtiles; round += round_tiles) {
+        const int tiles = min(round_tiles, num_qtiles - round);  // of this round, dealt out evenly
+        const int qi = round + xcd * tiles / kSweepXcds + in_xcd / P;
+        if (qi >= round + (xcd + 1) * tiles / kSweepXcds) continue;
         const int qt = args.qtile_list ? args.qtile_list[qi] : args.qtile_first + qi * args.qtile_step;
         const int q0 = qt * kMQ;
         const int q = q0 + wave * 32 + qn;  // this lane's query (>= N in the last tile: padded zeros)
@@ -2625,6 +2646,8 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
         // for next_ct on exit.
         auto process = [&](int ct, int next_ct) {
             const int c0 = ct * kCT;
+            // (nothing is in flight as far as the compiler can tell, or it waits in the chunk loop, and for the loads to LDS too)
+            if constexpr (HALF) wait_for_loads();
             v16f acc[4];
 #pragma unroll
             for (int b = 0; b < 4; ++b)
@@ -2638,8 +2661,9 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             // bf16: this lane's share of |q - m|^2 (m: the tile's centre), or all of it from the table
             float f_part = 0.0f;
             if constexpr (TABLE) f_part = args.centre_dist[(size_t)ct * args.centre_pitch + q];
-            for (int c = 0; c < n_chunks; ++c) {
-                const bool last = c + 1 == n_chunks;
+            // (`last` a type of its own on halves: with one body for all chunks there is a path, never taken, from the last
+            // chunk's loads to the next chunk, and on it the compiler waits for all loads there)
+            auto chunk = [&](int c, auto last) {
                 v4f mc[2 * kSteps16];  // bf16: the centre's 16 coordinates that go with this lane's 16 of the chunk
                 if constexpr (BF16 && !TABLE) {
                     const v4f *msrc = reinterpret_cast<const v4f *>(args.centres_p) + (size_t)ct * (8 * n_chunks) + 8 * c + 2 * kh;
@@ -2649,23 +2673,37 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                         mc[2 * step + 1] = msrc[4 * step + 1];
                     }
                 }
-                if (!last) fetch(ct, c + 1);
-                else if (next_ct >= 0) fetch(next_ct, 0);
+                if constexpr (HALF) {
+                    // (the buffer was last read a chunk ago, before the barrier that ended that chunk)
+                    if (!last || next_ct >= 0) fetch_half(last ? next_ct : ct, last ? 0 : c + 1, buf ^ 1);
+                } else {
+                    if (!last) fetch(ct, c + 1);
+                    else if (next_ct >= 0) fetch(next_ct, 0);
+                }
                 {
                     const v4f *bn = bsrc + (size_t)(last ? 0 : c + 1) * (kSlots * 64);
 #pragma unroll
                     for (int s4 = 0; s4 < kSlots; ++s4) bnext[s4] = bn[s4 * 64];
                 }
                 if constexpr (HALF) {
+                    // (a step's operands are asked for ahead of the products of the step before)
+                    v4f x[2][4];
+                    auto load_step = [&](int step) {
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) x[step & 1][b] = a_lds[buf * kChunkF4 + (b * kSlots + step) * 64 + lane];
+                    };
+                    load_step(0);
+                    load_step(1);
+                    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                     for (int step = 0; step < kSlots; ++step) {
-                        v4f x[4];
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) x[b] = a_lds[buf * kChunkF4 + (b * kSlots + step) * 64 + lane];
                         const v8h qh = __builtin_bit_cast(v8h, bcur[step]);
 #pragma unroll
                         for (int b = 0; b < 4; ++b)
-                            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, x[b]), qh, acc[b], 0, 0, 0);
+                            acc[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, x[step & 1][b]), qh, acc[b], 0, 0, 0);
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (step + 2 < kSlots) load_step(step + 2);
+                        __builtin_amdgcn_sched_barrier(0);
                     }
                 } else if constexpr (BF16) {
 #pragma unroll
@@ -2716,18 +2754,28 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                     }
                 }
                 if (!last) {
-                    if constexpr (BF16 || HALF) {
-                        stash(buf ^ 1, false);  // (last read a chunk ago, before the barrier that ended that chunk)
+                    if constexpr (HALF) {
+                        wait_for_loads();  // (the next chunk is in LDS)
+                        __syncthreads();
+                        buf ^= 1;
+                    } else if constexpr (BF16) {
+                        stash(buf ^ 1);  // (last read a chunk ago, before the barrier that ended that chunk)
                         __syncthreads();
                         buf ^= 1;
                     } else {
                         __syncthreads();  // all waves have read this chunk
-                        stash(0, false);
+                        stash(0);
                         __syncthreads();
                     }
 #pragma unroll
                     for (int s4 = 0; s4 < kSlots; ++s4) bcur[s4] = bnext[s4];
                 }
+            };
+            if constexpr (HALF) {
+                for (int c = 0; c + 1 < n_chunks; ++c) chunk(c, std::false_type());
+                chunk(n_chunks - 1, std::true_type());
+            } else {
+                for (int c = 0; c < n_chunks; ++c) chunk(c, c + 1 == n_chunks);
             }
             const u64 limit = thr[wave * 32 + qn];
             // ~0 is "no threshold yet": its distance field does not decode to a number.
@@ -2816,7 +2864,8 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 }
             }
             if constexpr (BF16 || HALF) {
-                if (next_ct >= 0) stash(buf ^ 1, true);
+                if constexpr (HALF) wait_for_loads();
+                else if (next_ct >= 0) stash(buf ^ 1);
                 __syncthreads();  // the next tile's first chunk is in LDS; all waves are done with this tile's last
                 if (next_ct >= 0) {
                     buf ^= 1;
@@ -2825,7 +2874,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
             } else {
                 __syncthreads();  // all waves are done with the tile's last chunk
                 if (next_ct >= 0) {
-                    stash(0, true);
+                    stash(0);
                     __syncthreads();
                 }
             }
@@ -2850,13 +2899,16 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
         };
         int cur = h0 + (part - h0 % P + P) % P;  // this part's first tile of the neighbourhood
         if (cur > h1) cur = -1;  // fewer tiles than parts: nothing for this part, its lists stay empty
-        if (cur >= 0) fetch(cur, 0);
+        if constexpr (!HALF)
+            if (cur >= 0) fetch(cur, 0);
         __syncthreads();  // the previous query tile's last reads of the LDS chunk
         buf = 0;
         if (cur >= 0) {
-            stash(0, true);
+            if constexpr (HALF) fetch_half(cur, 0, 0);
+            else stash(0);
             parity ^= 1;
         }
+        wait_for_loads();
         __syncthreads();
         bool home = true;
         unsigned int swept = 0;
@@ -2895,8 +2947,13 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
                 __syncthreads();
                 nxt = next_tile();
                 if (nxt >= 0) {
-                    fetch(nxt, 0);
-                    stash(buf, true);  // the barrier that ended the last tile freed the LDS chunks
+                    if constexpr (HALF) {
+                        fetch_half(nxt, 0, buf);  // the barrier that ended the last tile freed the LDS chunks
+                        wait_for_loads();
+                    } else {
+                        fetch(nxt, 0);
+                        stash(buf);
+                    }
                     parity ^= 1;
                     __syncthreads();
                 }
@@ -3730,7 +3787,9 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
             while (rest_parts < (whole > 0 ? 16 : 2) && rest * rest_parts * 2 <= slots + slots / 16 &&
                    rest_parts * 2 * keep <= 2048 && rest_parts * 4 * (2 * kHomeTiles + 1) <= num_tiles)
                 rest_parts *= 2;
-        const int grid = std::min(std::max(whole * parts, rest * rest_parts), slots);
+        // (chunked: whole rounds of the XCDs, some of which may find nothing to do at the end)
+        const int grid = chunked ? std::min(div_up(count, kSweepXcds) * kSweepXcds * parts, std::max(slots / (kSweepXcds * parts), 1) * (kSweepXcds * parts))
+                                 : std::min(std::max(whole * parts, rest * rest_parts), slots);
         const size_t n_slots = (size_t)(tile_list || step != 1 ? count * kMQ : N);
         const size_t merged_rows = parts > 1 ? n_slots : rest_parts > 1 ? n_slots - (size_t)whole * kMQ : 0;
         DeviceMem lists, cand, tau, part_keys;
