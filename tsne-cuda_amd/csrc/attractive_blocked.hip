@@ -861,11 +861,8 @@ void release_blocked(tsne_hip_plan *p) {
     (void)hipFree(p->strip_row0);
     (void)hipFree(p->wseg);
     scratch_free(p->row_entries);
-    scratch_free(p->row_counts);
     p->wseg = nullptr;
     p->row_entries = nullptr;
-    p->row_points = nullptr;
-    p->row_counts = nullptr;
     p->blocked_direct = false;
     p->ent_p = nullptr;
     p->seg = nullptr;
@@ -1039,16 +1036,6 @@ int prepare_blocked(tsne_hip_plan *p, const float *pij, const int *indices, hipS
             TSNE_LAUNCHED(s);
         } else {
             p->row_entries = nullptr;  // (no room: the steps then launch the attractive kernel by itself)
-            (void)hipGetLastError();
-        }
-    }
-    if (p->row_entries && N <= kScanPoints) {
-        constexpr int kCounts = (kScanRows + 63) / 64 * 64;
-        if (malloc_optional(reinterpret_cast<void **>(&p->row_counts),
-                            sizeof(int) * kCounts + sizeof(unsigned short) * (size_t)kScanRows * N) == hipSuccess) {
-            p->row_points = reinterpret_cast<unsigned short *>(p->row_counts + kCounts);
-        } else {
-            p->row_counts = nullptr;  // (no room: the steps gather in a kernel of its own)
             (void)hipGetLastError();
         }
     }

@@ -62,6 +62,8 @@ inline bool forces_ride_along(int N, int K) {
 constexpr int kScanPoints = 20480;
 static_assert(kScanPoints <= 65536, "point numbers of 16 bits (row_points)");
 constexpr int kScanRows = kFftShort / (2 * kInterp);  // most boxes per side of an 800-point transform's grid
+constexpr int kScanRowsPad = (kScanRows + 63) / 64 * 64;
+inline size_t row_lists_bytes(size_t N) { return sizeof(int) * kScanRowsPad + sizeof(unsigned short) * kScanRows * N; }
 
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
@@ -111,7 +113,11 @@ struct tsne_hip_plan {
     double moment_scale = 0.0;          // 2^s with N 2^s < 2^62: a box can hold every point
     double z_scale = 0.0;               // fixed-point scale of the partial sums of z (4 N^2 z_scale < 2^63)
     tsnehip::LagrangeMonomials monomials;
-    float4 *node_potentials = nullptr;  // n_nodes^2
+    // n_nodes^2; in steps of up to kScanPoints points whose potentials stay in LDS, instead, the points that the spreading scan
+    // found in each row of boxes (row_points) and their number.
+    float4 *node_potentials = nullptr;
+    int *row_counts() const { return reinterpret_cast<int *>(node_potentials); }
+    unsigned short *row_points() const { return reinterpret_cast<unsigned short *>(row_counts() + tsnehip::kScanRowsPad); }
     float2 *row_spectra = nullptr;      // 2 plane pairs x kFft x kNodePad (transposed)
     float2 *col_results = nullptr;      // same shape
     float *kernel_rows = nullptr;       // (kFft/2+1) x kNodePad: row spectra of the Cauchy kernel
@@ -137,10 +143,6 @@ struct tsne_hip_plan {
     // Small problems (one stream, see api.hip): the pattern once more, row by row, {probability, neighbour} in the
     // caller's order of neighbours; the inverse row pass computes the attractive forces from it in spare workgroups.
     uint2 *row_entries = nullptr;
-    // ... and, up to kScanPoints points, for each row of boxes the points that the spreading scan found there (num_points of
-    // them at most) and their number, for the gathering at the end of the same step's chain.
-    unsigned short *row_points = nullptr;
-    int *row_counts = nullptr;
     int steps_to_grouping = 0;      // steps of that form until the grouping kernels are launched again, in this call
     int spin_limit = 0;             // polls before a wave of the attractive kernel gives up a wait
     bool blocked_ready = false;

@@ -221,7 +221,7 @@ __device__ __forceinline__ void small_dft(float2 (&x)[R]) {
 // is unrolled), store(f, i, j, v) takes it back: the LDS in the middle of a transform, memory at either end of it
 // where a kernel fuses its loads and stores into the first and last pass.  USED: of a butterfly's R elements the last
 // R - USED are zero (not loaded); KEPT: only the first KEPT results are stored.  The grids fill at most half of a transform:
-// the first pass forwards and the last one of the inverse do half the work of whole ones (column pass 12.9 -> 11.8 us, a
+// the first pass forwards does half the work of a whole one and the last one of the inverse half the stores (column pass 12.9 -> 11.8 us, a
 // small problem's step 58.2 -> 56.5).
 template <int N, int L, int R, bool INVERSE, int USED = R, int KEPT = R, class Load, class Store>
 __device__ __forceinline__ void mixed_pass_io(int nfft, const float2 *tw, int tid, int nthreads, Load load,
@@ -245,6 +245,10 @@ __device__ __forceinline__ void mixed_pass_io(int nfft, const float2 *tw, int ti
         }
 #pragma unroll
         for (int j = 0; j < KEPT; ++j) store(f, i0 + j * Q, j, x[j]);
+        // (the others are formed all the same: a product that goes into one sum only is fused with it, and the kept results
+        // would be others in their last bits)
+#pragma unroll
+        for (int j = KEPT; j < R; ++j) asm volatile("" : : "v"(x[j].x), "v"(x[j].y));
     }
 }
 template <int N, int L, int R, bool INVERSE, int USED = R, int KEPT = R>
@@ -1094,7 +1098,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
         for (int m = 0; m < kMoments; ++m) atomicAdd(dst + m * n_boxes, sum[m] - count * kFixedOffset);
     };
     // The points found are listed for the step's gathering kernel, too.
-    unsigned short *listed = row_points ? row_points + (size_t)bx * N : nullptr;
+    unsigned short *listed = row_points + (size_t)bx * N;
     __syncthreads();
     for (int first = 0, turn = 0; first < N; first += kScanChunk, turn ^= 1) {
         unsigned long long mine[kScanPer];
@@ -1113,7 +1117,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
                 if ((mine[u] >> lane) & 1ull) {
                     const int to = at + __popcll(mine[u] & below);
                     list[to] = make_float2(px[u], py[u]);
-                    if (listed) listed[to] = (unsigned short)(first + u * kScanThreads + tid);
+                    listed[to] = (unsigned short)(first + u * kScanThreads + tid);
                 }
                 at += __popcll(mine[u]);
             }
@@ -1122,7 +1126,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
         __syncthreads();
         const int n = found[turn];
         if (tid == 0) found[turn ^ 1] = 0;
-        if (listed) listed += n;
+        listed += n;
         for (int e = tid; e < n; e += kScanThreads) {
             const float2 p = list[e];
             int b, by;
@@ -1153,7 +1157,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
         __syncthreads();
     }
     if (sum_box >= 0) flush();
-    if (listed && tid == 0) row_counts[bx] = (int)(listed - (row_points + (size_t)bx * N));
+    if (tid == 0) row_counts[bx] = (int)(listed - (row_points + (size_t)bx * N));
     __syncthreads();
     double *moments = reinterpret_cast<double *>(acc);
     for (int e = tid; e < words; e += kScanThreads) {
@@ -1712,7 +1716,7 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
     if (scan)
         TSNE_LOOP_KERNEL(p, (conv_rows_scan_kernel), xcd_launch_blocks(nb) + div_up(G, 8), kScanThreads, scan_lds(nb), s, embedding, N,
                          p->moment_scale, from_fixed, p->monomials, G, nb, p->scalars, slot, slot ^ 1, p->twiddles_short,
-                         p->row_spectra, p->kernel_rows, p->row_points, p->row_counts);
+                         p->row_spectra, p->kernel_rows, p->row_points(), p->row_counts());
     else if (short_fft)
         TSNE_LOOP_KERNEL(p, (conv_rows_forward_kernel<2, kFftShort>), row_grid + div_up(G, 8), 512, 0, s, p->box_moments, from_fixed, p->monomials, charges4, G, nb, p->scalars, slot, p->twiddles_short,
             p->row_spectra, p->kernel_rows);
@@ -1736,11 +1740,11 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
         TSNE_LOOP_KERNEL(p, (conv_columns_kernel<false, kFft>), kFft / 2, 512, 0, s, p->row_spectra, G, p->kernel_rows, p->twiddles,
                                                                   p->col_results, p->box_moments, moment_words);
     TSNE_LAUNCHED(s);
-    if (scan && p->row_points) {
+    if (scan) {
         const int row_blocks = xcd_launch_blocks(nb);
         const RowForces forces = {p->row_entries, p->yxy, small->attr, N, p->num_neighbors, row_blocks};
         conv_rows_gather_kernel<<<row_blocks + div_up(N, kScanThreads / kForceLanes), kScanThreads, 0, s>>>(
-            p->col_results, embedding, N, p->scalars, slot, nb, p->lagrange, p->twiddles_short, p->row_points, p->row_counts,
+            p->col_results, embedding, N, p->scalars, slot, nb, p->lagrange, p->twiddles_short, p->row_points(), p->row_counts(),
             rep, p->scalars, p->z_scale, forces);
         TSNE_LAUNCHED(s);
         return 0;
