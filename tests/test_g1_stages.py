@@ -1302,11 +1302,12 @@ def test_small_step_forms(stages, monkeypatch, n, k):
             assert same_bits(a, b)
 
 
-@pytest.mark.parametrize("n", [2, 639, 641, 5003, 7681, 20480])
-def test_small_step_without_room_for_the_rows_points(stages, monkeypatch, n):
+@pytest.mark.parametrize("n", [2, 639, 641, 5003, 7681, 15700, 20480])
+def test_small_step_gathers_in_its_row_pass(stages, monkeypatch, n):
     """A small problem's step gathers in its inverse row pass, at the points that the spreading scan listed for each row of
-    boxes, or, without room for those lists, in a kernel of its own: the same bits, at the remainders of a workgroup's points
-    and of the chunks that the scan looks through, in more boxes than the reference's and in fewer."""
+    boxes; one that groups the points (TSNE_KEEP_GROUPING) in a kernel of its own.  The same bits, at the remainders of a
+    workgroup's points and of the chunks that the scan looks through, where the lists need more room than the potentials
+    whose place they take, and in more boxes than the reference's and in fewer."""
     rng = np.random.default_rng(n)
     k = min(n, 12)
     idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
@@ -1324,9 +1325,9 @@ def test_small_step_without_room_for_the_rows_points(stages, monkeypatch, n):
         return [v.cpu().numpy() for v in (y, gains, old, z)]
 
     for boxes in (130, 133, 7):
-        monkeypatch.delenv("TSNE_SCRATCH_LIMIT", raising=False)
+        monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
         want = run(boxes)
-        monkeypatch.setenv("TSNE_SCRATCH_LIMIT", str(8 * n * k + 64))  # (the pattern row by row, but no lists)
+        monkeypatch.setenv("TSNE_KEEP_GROUPING", "1")
         for a, b in zip(run(boxes), want):
             assert same_bits(a, b)
 
@@ -1437,6 +1438,23 @@ def test_knn_at_the_lines_of_the_direct_search(stages, n, d, k):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
     if n <= 11003:
         X[[5, n - 1], 2] = np.nan, -np.inf
+        idx, d2 = stages.knn(dev(X), k)
+        idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+        assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
+
+
+@pytest.mark.parametrize("n,d,k", [(1024, 7, 20), (1025, 16, 33), (1087, 1, 5), (1089, 33, 129), (4096, 8, 20),
+                                   (4225, 5, 33), (9001, 3, 12)])
+def test_knn_direct_search_mirrors_its_tiles(stages, n, d, k):
+    """Distances of pairs of tiles are formed once and written twice from 1025 points on: the vector sweep's rows at the edges of
+    tiles and of blocks of rows, with equal distances, with overflowing ones and with points that are not numbers, whose
+    distances have the sign that the order of the difference gives them."""
+    rng = np.random.default_rng(n + d)
+    X = np.round(2.0 * rng.standard_normal((n, d))).astype(np.float32)
+    X[n // 2] *= np.float32(1e30)
+    for bad in (False, True):
+        if bad:
+            X[[3, n // 3, n - 1], 0] = np.nan, np.inf, -np.nan
         idx, d2 = stages.knn(dev(X), k)
         idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
         assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))

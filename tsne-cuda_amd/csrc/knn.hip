@@ -988,7 +988,10 @@ constexpr int kDirectDims = 16;  // dimensions staged per chunk
 // A workgroup computes a square tile, R x R distances per thread, both operands staged in LDS a chunk of
 // dimensions ahead; same fma chain as everywhere (dimensions past D are zeros on both sides, which leave a sum
 // as it is).  Bound by the vector ALU, two instructions per pair and dimension.
-template <int R>
+//
+// MIRROR (Q = X): of the square of the rows' own columns only the tiles on and above the diagonal are formed, and those above
+// it are written a second time, mirrored: (a - b)^2 is (b - a)^2, bit for bit, and so are the sums, but for the sign of what is not a number.
+template <int R, bool MIRROR>
 __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__restrict__ Q, int NQ,
                                                              const float *__restrict__ X, int N, int D, int row0,
                                                              int rows, int pitch, float *__restrict__ dist) {
@@ -998,6 +1001,7 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__rest
     __shared__ __attribute__((aligned(16))) float xs[2][2][kDirectDims][kRow];
     const int tid = threadIdx.x, tq = tid >> 4, tc = tid & 15;
     const int q0 = row0 + blockIdx.y * kSide, c0 = blockIdx.x * kSide;
+    if (MIRROR && c0 >= row0 && c0 < q0) return;  // (row0 is a multiple of the side)
     const bool wide =
         (D & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) | reinterpret_cast<uintptr_t>(Q)) & 15) == 0;
     float4 ahead[2][kLoads];
@@ -1075,6 +1079,38 @@ __global__ __launch_bounds__(256) void pair_distances_kernel(const float *__rest
 #pragma unroll
         for (int b = 0; b < R; b += 4)
             *reinterpret_cast<float4 *>(dst + 16 * b) = float4{acc[a][b], acc[a][b + 1], acc[a][b + 2], acc[a][b + 3]};
+    }
+    if (MIRROR && c0 > q0 && c0 < row0 + rows) {
+        bool numbers = true;
+#pragma unroll
+        for (int a = 0; a < R; ++a)
+#pragma unroll
+            for (int b = 0; b < R; ++b) numbers = numbers && acc[a][b] == acc[a][b];
+        if (!numbers) {
+            // (where it is not a number its sign, which tells first from last neighbours, is that of the difference's order)
+#pragma unroll 1
+            for (int e = 0; e < R * R; ++e) {
+                const int a = e / R, b = e % R, r = c0 - row0 + tc * 4 + 16 * (b & ~3) + (b & 3), c = q0 + tq * R + a;
+                if (r >= rows) continue;
+                const float *x = Q + (size_t)(row0 + r) * D, *y = X + (size_t)c * D;  // (c < r + row0: both are points)
+                float sum = 0.0f;
+                for (int d = 0; d < D; ++d) {
+                    const float df = x[d] - y[d];
+                    sum = fmaf(df, df, sum);
+                }
+                dist[(size_t)r * pitch + c] = sum;
+            }
+            return;
+        }
+#pragma unroll
+        for (int b = 0; b < R; ++b) {
+            const int r = c0 - row0 + tc * 4 + 16 * (b & ~3) + (b & 3);
+            if (r >= rows) continue;
+            float *dst = dist + (size_t)r * pitch + q0 + tq * R;
+#pragma unroll
+            for (int a = 0; a < R; a += 4)
+                *reinterpret_cast<float4 *>(dst + a) = float4{acc[a][b], acc[a + 1][b], acc[a + 2][b], acc[a + 3][b]};
+        }
     }
 }
 
@@ -3368,11 +3404,13 @@ constexpr int kDirectNeighbors = 256;  // most K - 1 that select_row_kernel<8> t
 constexpr size_t kDirectFloats = (size_t)1 << 24;
 
 // (kNoRoom: nothing done, the sweeps need less memory)
-int run_direct_search(const float *points, int N, int D, int K, int cus, int *indices, float *sq_dist, hipStream_t s) {
+int run_direct_search(const float *points, int N, int D, int K, int *indices, float *sq_dist, hipStream_t s) {
     const int pitch = div_up(N, 128) * 128;
-    // Tiles of 128 points a side where they fill the chip, of 64 otherwise.
-    const bool large = (int64_t)(pitch / 128) * (pitch / 128) >= 2 * (int64_t)cus;
-    const int side = large ? 128 : 64;
+    // Tiles of 64 points a side: of 128, with which a thread loads half as much per pair, half of them mirrored leave the chip
+    // unevenly filled.  Whole searches, us, every tile formed with the better of the two / mirrored, 64 / 128 a side:
+    // 3000 x 64, 91 neighbours 88 / 71 / 79; 4000 x 126, 90: 149 / 121 / 144; 6000 x 200, 45: 445 / 369 / 429;
+    // 8000 x 126, 60: 532 / 492 / 518; 12000 x 40, 33: 731 / 697 / 737.
+    constexpr int side = 64;
     const int block = std::min(div_up(N, 128) * 128, std::max(128, (int)(kDirectFloats / pitch) / 128 * 128));
     DeviceMem dist;
     if (!dist.alloc_optional(sizeof(float) * (size_t)std::min(block, N) * pitch)) {
@@ -3382,10 +3420,9 @@ int run_direct_search(const float *points, int N, int D, int K, int cus, int *in
     for (int row0 = 0; row0 < N; row0 += block) {
         const int rows = std::min(block, N - row0);
         const dim3 grid(div_up(N, side), div_up(rows, side));
-        if (large)
-            pair_distances_kernel<8><<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
-        else
-            pair_distances_kernel<4><<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
+        // (up to 1024 points there is no more than a tile per compute unit: 1003 x 20, 32 neighbours 38.6 us, mirrored 39.6)
+        const auto distances = N <= 1024 ? pair_distances_kernel<4, false> : pair_distances_kernel<4, true>;
+        distances<<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
         TSNE_TRY(hipGetLastError());
         if (2 * (K - 1) <= 64 * 4)
             select_row_kernel<4><<<div_up(rows, 4), 256, 0, s>>>(dist.as<float>(), N, row0, rows, pitch, K, nullptr,
@@ -3414,7 +3451,7 @@ int run_listed_search(const float *points, int N, int D, int K, const int *list,
         return kNoRoom;
     }
     if (launch_gather_rows(points, list, count, D, queries.as<float>(), s)) return 1;
-    pair_distances_kernel<4><<<dim3(div_up(N, 64), div_up(count, 64)), 256, 0, s>>>(
+    pair_distances_kernel<4, false><<<dim3(div_up(N, 64), div_up(count, 64)), 256, 0, s>>>(
         queries.as<float>(), count, points, N, D, 0, count, pitch, dist.as<float>());
     TSNE_TRY(hipGetLastError());
     const auto select = 2 * (K - 1) <= 64 * 4 ? select_row_kernel<4> : select_row_kernel<8>;
@@ -3659,7 +3696,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     };
     if (halves_only && (!use_mfma || direct_search_pays(N, K))) return not_on_halves("is of few points or many neighbours");
     if (mode == 0 && direct_search_pays(N, K) && K - 1 <= kDirectNeighbors) {
-        const int rc = run_direct_search(points, N, D, K, cus, indices, sq_dist, s);
+        const int rc = run_direct_search(points, N, D, K, indices, sq_dist, s);
         if (rc != kNoRoom) return rc;
     }
     if (!use_mfma) {
@@ -3749,7 +3786,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
             transpose_points_kernel<<<dim3(div_up(D, 32), div_up(num_tiles, 32)), 256, 0, s>>>(
                 centers.as<float>(), D, num_tiles, D, centre_rows.as<float>());
             TSNE_TRY(hipGetLastError());
-            pair_distances_kernel<8><<<dim3(div_up(N, 128), div_up(num_tiles, 128)), 256, 0, s>>>(
+            pair_distances_kernel<8, false><<<dim3(div_up(N, 128), div_up(num_tiles, 128)), 256, 0, s>>>(
                 centre_rows.as<float>(), num_tiles, points, N, D, 0, num_tiles, Npad, centre_dist.as<float>());
             TSNE_TRY(hipGetLastError());
         } else {
