@@ -1302,36 +1302,6 @@ def test_small_step_forms(stages, monkeypatch, n, k):
             assert same_bits(a, b)
 
 
-@pytest.mark.parametrize("n", [2, 639, 641, 5003, 7681, 15700, 20480])
-def test_small_step_gathers_in_its_row_pass(stages, monkeypatch, n):
-    """A small problem's step gathers in its inverse row pass, at the points that the spreading scan listed for each row of
-    boxes; one that groups the points (TSNE_KEEP_GROUPING) in a kernel of its own.  The same bits, at the remainders of a
-    workgroup's points and of the chunks that the scan looks through, where the lists need more room than the potentials
-    whose place they take, and in more boxes than the reference's and in fewer."""
-    rng = np.random.default_rng(n)
-    k = min(n, 12)
-    idx = rng.integers(0, n, size=(n, k), dtype=np.int32)
-    P = (rng.random((n, k)) / (n * k)).astype(np.float32)
-    y0 = rng.standard_normal(2 * n).astype(np.float32)
-
-    def run(boxes):
-        plan = stages.Plan(n, k, boxes)
-        plan.prepare_attractive(dev(P), dev(idx))
-        y = dev(y0.copy())
-        gains, old = torch.ones_like(y), torch.zeros_like(y)
-        z = plan.iterate_(None, None, y, gains, old, 0, 4, eta=10.0)
-        torch.cuda.synchronize()
-        plan.close()
-        return [v.cpu().numpy() for v in (y, gains, old, z)]
-
-    for boxes in (130, 133, 7):
-        monkeypatch.delenv("TSNE_KEEP_GROUPING", raising=False)
-        want = run(boxes)
-        monkeypatch.setenv("TSNE_KEEP_GROUPING", "1")
-        for a, b in zip(run(boxes), want):
-            assert same_bits(a, b)
-
-
 @pytest.mark.parametrize("n,asked", [(3000, True), (20481, False), (3000, False)])
 def test_small_step_grouping_is_decided_on_the_device(stages, monkeypatch, n, asked):
     """Steps of a small problem that do not launch the grouping kernels only ever follow one of the same call that

@@ -444,7 +444,6 @@ int tsne_hip_plan_create(tsne_hip_plan **plan, int num_points, int num_neighbors
     const size_t G2 = (size_t)(kMaxBoxes * kInterp) * (kMaxBoxes * kInterp);
     const size_t spec = (size_t)2 * kFft * kNodePad;
     const size_t N = (size_t)num_points;
-    const size_t potential_bytes = std::max(sizeof(float4) * G2, N <= (size_t)kScanPoints ? row_lists_bytes(N) : 0);
     const size_t moment_bytes = sizeof(unsigned long long) * kMoments * kMaxBoxes * kMaxBoxes;
     {
         // Fixed-point scales.  Moments are sums of values in [0, 1], at most N of them in a box, and at most 4096
@@ -486,7 +485,7 @@ int tsne_hip_plan_create(tsne_hip_plan **plan, int num_points, int num_neighbors
               device_malloc(&p->num_chunks, 2 * sizeof(int)) == hipSuccess &&
               device_malloc(&p->box_moments, moment_bytes) == hipSuccess &&
               device_malloc(&p->centre_parts, sizeof(double2) * 2 * kMaxCentreParts) == hipSuccess &&
-              device_malloc(&p->node_potentials, potential_bytes) == hipSuccess &&
+              device_malloc(&p->node_potentials, sizeof(float4) * G2) == hipSuccess &&
               device_malloc(&p->row_spectra, sizeof(float2) * spec) == hipSuccess &&
               device_malloc(&p->col_results, sizeof(float2) * spec) == hipSuccess &&
               device_malloc(&p->kernel_rows, sizeof(float) * (size_t)(kFft / 2 + 1) * kNodePad) == hipSuccess &&

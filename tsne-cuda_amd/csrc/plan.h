@@ -60,10 +60,6 @@ inline bool forces_ride_along(int N, int K) {
 // one in one box, and tails of two degrees of freedom: 1203 points 64 / 47, 49 / 45; 5000 66 / 53, 51 / 48; 10007 67 / 62,
 // 65 / 71; 15361 68 / 71, 59 / 71; 20011 69 / 78, 66 / 99.
 constexpr int kScanPoints = 20480;
-static_assert(kScanPoints <= 65536, "point numbers of 16 bits (row_points)");
-constexpr int kScanRows = kFftShort / (2 * kInterp);  // most boxes per side of an 800-point transform's grid
-constexpr int kScanRowsPad = (kScanRows + 63) / 64 * 64;
-inline size_t row_lists_bytes(size_t N) { return sizeof(int) * kScanRowsPad + sizeof(unsigned short) * kScanRows * N; }
 
 // Kernels of one gradient step, in launch order (profiling slots).
 enum LoopKernel {
@@ -113,11 +109,7 @@ struct tsne_hip_plan {
     double moment_scale = 0.0;          // 2^s with N 2^s < 2^62: a box can hold every point
     double z_scale = 0.0;               // fixed-point scale of the partial sums of z (4 N^2 z_scale < 2^63)
     tsnehip::LagrangeMonomials monomials;
-    // n_nodes^2; in steps of up to kScanPoints points whose potentials stay in LDS, instead, the points that the spreading scan
-    // found in each row of boxes (row_points) and their number.
-    float4 *node_potentials = nullptr;
-    int *row_counts() const { return reinterpret_cast<int *>(node_potentials); }
-    unsigned short *row_points() const { return reinterpret_cast<unsigned short *>(row_counts() + tsnehip::kScanRowsPad); }
+    float4 *node_potentials = nullptr;  // n_nodes^2
     float2 *row_spectra = nullptr;      // 2 plane pairs x kFft x kNodePad (transposed)
     float2 *col_results = nullptr;      // same shape
     float *kernel_rows = nullptr;       // (kFft/2+1) x kNodePad: row spectra of the Cauchy kernel

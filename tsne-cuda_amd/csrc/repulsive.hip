@@ -221,8 +221,8 @@ __device__ __forceinline__ void small_dft(float2 (&x)[R]) {
 // is unrolled), store(f, i, j, v) takes it back: the LDS in the middle of a transform, memory at either end of it
 // where a kernel fuses its loads and stores into the first and last pass.  USED: of a butterfly's R elements the last
 // R - USED are zero (not loaded); KEPT: only the first KEPT results are stored.  The grids fill at most half of a transform:
-// the first pass forwards does half the work of a whole one and the last one of the inverse half the stores (column pass 12.9 -> 11.8 us, a
-// small problem's step 58.2 -> 56.5).
+// the first pass forwards does half the work of a whole one and the last one of the inverse half the stores (column
+// pass 12.9 -> 11.8 us, a small problem's step 58.2 -> 56.5).
 template <int N, int L, int R, bool INVERSE, int USED = R, int KEPT = R, class Load, class Store>
 __device__ __forceinline__ void mixed_pass_io(int nfft, const float2 *tw, int tid, int nthreads, Load load,
                                               Store store) {
@@ -1035,9 +1035,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
                                                                       int n_boxes, LoopScalars *sc, int slot, int next_slot,
                                                                       const float2 *__restrict__ twiddles,
                                                                       float2 *__restrict__ row_spectra,
-                                                                      float *__restrict__ kernel_rows,
-                                                                      unsigned short *__restrict__ row_points,
-                                                                      int *__restrict__ row_counts) {
+                                                                      float *__restrict__ kernel_rows) {
     using T = Transform<kFftShort>;
     constexpr int NFFT = kFftShort;
     extern __shared__ __attribute__((aligned(16))) unsigned char scan_raw[];
@@ -1097,8 +1095,6 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
 #pragma unroll
         for (int m = 0; m < kMoments; ++m) atomicAdd(dst + m * n_boxes, sum[m] - count * kFixedOffset);
     };
-    // The points found are listed for the step's gathering kernel, too.
-    unsigned short *listed = row_points + (size_t)bx * N;
     __syncthreads();
     for (int first = 0, turn = 0; first < N; first += kScanChunk, turn ^= 1) {
         unsigned long long mine[kScanPer];
@@ -1114,11 +1110,7 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
             at = __builtin_amdgcn_readfirstlane(at);
 #pragma unroll
             for (int u = 0; u < kScanPer; ++u) {
-                if ((mine[u] >> lane) & 1ull) {
-                    const int to = at + __popcll(mine[u] & below);
-                    list[to] = make_float2(px[u], py[u]);
-                    listed[to] = (unsigned short)(first + u * kScanThreads + tid);
-                }
+                if ((mine[u] >> lane) & 1ull) list[at + __popcll(mine[u] & below)] = make_float2(px[u], py[u]);
                 at += __popcll(mine[u]);
             }
         }
@@ -1126,7 +1118,6 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
         __syncthreads();
         const int n = found[turn];
         if (tid == 0) found[turn ^ 1] = 0;
-        listed += n;
         for (int e = tid; e < n; e += kScanThreads) {
             const float2 p = list[e];
             int b, by;
@@ -1157,7 +1148,6 @@ __global__ __launch_bounds__(kScanThreads, 3) void conv_rows_scan_kernel(const f
         __syncthreads();
     }
     if (sum_box >= 0) flush();
-    if (tid == 0) row_counts[bx] = (int)(listed - (row_points + (size_t)bx * N));
     __syncthreads();
     double *moments = reinterpret_cast<double *>(acc);
     for (int e = tid; e < words; e += kScanThreads) {
@@ -1369,7 +1359,7 @@ __global__ __launch_bounds__(512) void conv_columns_short_kernel(const float2 *_
 // produces node potentials in natural order, scaled by 1 / (transform length)^2.
 // ---------------------------------------------------------------------------
 
-// Attractive forces of THREADS / kForceLanes rows from the row-ordered pattern: kForceLanes lanes per row, four
+// Attractive forces of kRowThreads / kForceLanes rows from the row-ordered pattern: kForceLanes lanes per row, four
 // entries of a lane in flight, the same fixed-point sums as the re-blocked kernel's (the same bits).
 constexpr int kForceLanes = 8;
 struct RowForces {
@@ -1379,9 +1369,8 @@ struct RowForces {
     int N, K;
     int first_block;  // (a multiple of the XCD count: the workgroups before it are the row pass's)
 };
-template <int THREADS>
 __device__ __forceinline__ void row_forces_block(const RowForces &f, int block, float p_max) {
-    const int row = block * (THREADS / kForceLanes) + (int)threadIdx.x / kForceLanes;
+    const int row = block * (kRowThreads / kForceLanes) + (int)threadIdx.x / kForceLanes;
     const int lane = threadIdx.x % kForceLanes;
     const bool live = row < f.N;
     const uint2 *mine = f.entries + (size_t)(live ? row : 0) * f.K;
@@ -1426,7 +1415,7 @@ __global__ __launch_bounds__(kRowThreads) void conv_rows_inverse_kernel(const fl
                                                                 RowForces rows) {
     using T = Transform<NFFT>;
     if (rows.entries && (int)blockIdx.x >= rows.first_block) {
-        row_forces_block<kRowThreads>(rows, blockIdx.x - rows.first_block, sc->vmax);
+        row_forces_block(rows, blockIdx.x - rows.first_block, sc->vmax);
         return;
     }
     __shared__ float2 s[4][NFFT];  // [row * 2 + pair]
@@ -1464,45 +1453,6 @@ __global__ __launch_bounds__(kRowThreads) void conv_rows_inverse_kernel(const fl
 // (src/kernels/nbodyfft.cu:141-173, src/kernels/rep_forces.cu:3-31).  Block
 // partial sums of z_i go to the device scalar with one atomic per block.
 // ---------------------------------------------------------------------------
-// Last kernel of the chain: whether the next step keeps this step's grouping of the points by tile.  (The spread kernel has
-// finished counting; the chain's kernels of this step have all read the flag.)
-__device__ __forceinline__ void close_chain(LoopScalars *sc, int N, int keep_grouping) {
-    const bool reused = keep_grouping == kKeepAlways || (keep_grouping && sc->reuse_sort);
-    const int age = reused ? sc->sort_age + 1 : 0;
-    const unsigned int strays = sc->strays;
-    sc->strays = 0u;
-    sc->sort_age = age;
-    sc->chain_runs += 1u;
-    sc->chain_sorts += reused ? 0u : 1u;
-    sc->strays_total += strays;
-    sc->reuse_sort = (keep_grouping && strays <= (unsigned int)max(N >> kStrayShift, kStrayFloor) && age < kMaxSortAge) ? 1 : 0;
-}
-
-// Potentials at a point, `node(a, b)` those of the nodes of its box: phi_i = sum_{a,b} Lx_a Ly_b y~[node].
-template <class Node>
-__device__ __forceinline__ float4 point_potential(const float (&Lx)[kInterp], const float (&Ly)[kInterp], Node node) {
-    float4 phi = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-    for (int a = 0; a < kInterp; ++a) {
-#pragma unroll
-        for (int b = 0; b < kInterp; ++b) {
-            const float lw = Lx[a] * Ly[b];
-            const float4 yt = node(a, b);
-            phi.x += lw * yt.x;
-            phi.y += lw * yt.y;
-            phi.z += lw * yt.z;
-            phi.w += lw * yt.w;
-        }
-    }
-    return phi;
-}
-__device__ __forceinline__ float point_z(float x, float y, const float4 &phi) {
-    return (1 + x * x + y * y) * phi.x - 2 * (x * phi.y + y * phi.z) + phi.w;
-}
-
-// EACH_POINT: the z_i are added up as fixed-point numbers, one by one, where the points are not always gathered by the same
-// workgroups (up to kScanPoints points: see conv_rows_gather_kernel); otherwise a workgroup's are added as floats.
-template <bool EACH_POINT>
 __global__ __launch_bounds__(256) void gather_forces_kernel(const float *__restrict__ emb, int N,
                                                             const LoopScalars *sc_in, int slot, int n_boxes,
                                                             LagrangeConsts lc,
@@ -1510,11 +1460,22 @@ __global__ __launch_bounds__(256) void gather_forces_kernel(const float *__restr
                                                             float *__restrict__ rep, float *__restrict__ phi_out,
                                                             LoopScalars *sc, int keep_grouping, double z_scale) {
     __shared__ float partial[256 / kWave];
-    if (blockIdx.x == 0 && threadIdx.x == 0) close_chain(sc, N, keep_grouping);
+    // Last kernel of the chain: whether the next step keeps this step's grouping of the points by tile.  (The
+    // spread kernel has finished counting; the chain's kernels of this step have all read the flag.)
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        const bool reused = keep_grouping == kKeepAlways || (keep_grouping && sc->reuse_sort);
+        const int age = reused ? sc->sort_age + 1 : 0;
+        const unsigned int strays = sc->strays;
+        sc->strays = 0u;
+        sc->sort_age = age;
+        sc->chain_runs += 1u;
+        sc->chain_sorts += reused ? 0u : 1u;
+        sc->strays_total += strays;
+        sc->reuse_sort = (keep_grouping && strays <= (unsigned int)max(N >> kStrayShift, kStrayFloor) && age < kMaxSortAge) ? 1 : 0;
+    }
     const Bounds bd = load_bounds(sc_in, slot, n_boxes);
     const int G = n_boxes * kInterp;
     float z = 0.0f;
-    long long z_fixed = 0ll;
     // Grid-stride: the workgroup count stays small because every workgroup ends with an atomic on
     // the one Z accumulator, and same-address atomics serialise.
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) {
@@ -1523,22 +1484,23 @@ __global__ __launch_bounds__(256) void gather_forces_kernel(const float *__restr
         float Lx[kInterp], Ly[kInterp];
         bin_and_weights(x, bd, n_boxes, lc, bx, Lx);
         bin_and_weights(y, bd, n_boxes, lc, by, Ly);
-        const float4 phi = point_potential(
-            Lx, Ly, [&](int a, int b) { return node_potentials[(size_t)(bx * kInterp + a) * G + (by * kInterp + b)]; });
-        if (EACH_POINT)
-            z_fixed += __double2ll_rn((double)point_z(x, y, phi) * z_scale);
-        else
-            z += point_z(x, y, phi);
+        float4 phi = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int a = 0; a < kInterp; ++a) {
+#pragma unroll
+            for (int b = 0; b < kInterp; ++b) {
+                const float lw = Lx[a] * Ly[b];
+                const float4 yt = node_potentials[(size_t)(bx * kInterp + a) * G + (by * kInterp + b)];
+                phi.x += lw * yt.x;
+                phi.y += lw * yt.y;
+                phi.z += lw * yt.z;
+                phi.w += lw * yt.w;
+            }
+        }
+        z += (1 + x * x + y * y) * phi.x - 2 * (x * phi.y + y * phi.z) + phi.w;
         rep[i] = x * phi.x - phi.y;
         rep[N + i] = y * phi.x - phi.z;
         if (phi_out) reinterpret_cast<float4 *>(phi_out)[i] = phi;
-    }
-    if (EACH_POINT) {
-#pragma unroll
-        for (int m = kWave / 2; m >= 1; m >>= 1) z_fixed += __shfl_xor(z_fixed, m, kWave);
-        if ((threadIdx.x & (kWave - 1)) == 0 && z_fixed != 0ll)
-            atomicAdd(reinterpret_cast<unsigned long long *>(&sc->z_part[blockIdx.x % kZParts]), (unsigned long long)z_fixed);
-        return;
     }
     z = group_sum<kWave>(z);
     if ((threadIdx.x & (kWave - 1)) == 0) partial[threadIdx.x / kWave] = z;
@@ -1551,80 +1513,6 @@ __global__ __launch_bounds__(256) void gather_forces_kernel(const float *__restr
         atomicAdd(reinterpret_cast<unsigned long long *>(&sc->z_part[blockIdx.x % kZParts]),
                   (unsigned long long)__double2ll_rn((double)t * z_scale));
     }
-}
-
-// Inverse row pass and gathering of a small problem's step in one kernel (see conv_rows_scan_kernel): a workgroup takes the
-// three grid rows of one row of boxes, whose potentials stay in LDS, and gathers at the points that the scan found there.  The
-// workgroups past the rows compute attractive forces, as in conv_rows_inverse_kernel.  It stands for two launches and the
-// potentials' trip through memory, and its own row pass is longer by the third row and the points of the fullest row of boxes:
-// 20011 points 12.4 us for 9.6 + 4.6 (a step 56.5 -> 55.3); 5000 points a step 1 % shorter.  The same bits as the two kernels'.
-__global__ __launch_bounds__(kScanThreads, 3) void conv_rows_gather_kernel(const float2 *__restrict__ col_results,
-                                                                        const float *__restrict__ emb, int N,
-                                                                        const LoopScalars *sc_in, int slot, int n_boxes,
-                                                                        LagrangeConsts lc,
-                                                                        const float2 *__restrict__ twiddles,
-                                                                        const unsigned short *__restrict__ row_points,
-                                                                        const int *__restrict__ row_counts,
-                                                                        float *__restrict__ rep, LoopScalars *sc,
-                                                                        double z_scale, RowForces rows) {
-    using T = Transform<kFftShort>;
-    constexpr int NFFT = kFftShort;
-    if ((int)blockIdx.x >= rows.first_block) {
-        row_forces_block<kScanThreads>(rows, blockIdx.x - rows.first_block, sc_in->vmax);
-        return;
-    }
-    __shared__ float2 s[2 * kInterp][NFFT];  // [row * 2 + pair]
-    __shared__ float2 tw[kFftShort];
-    __shared__ unsigned long long z_sum;
-    const int tid = threadIdx.x;
-    if (blockIdx.x == 0 && tid == 0) close_chain(sc, N, 0);
-    const int bx = xcd_row_block(blockIdx.x, n_boxes);
-    if (bx < 0) return;
-    if (tid == 0) z_sum = 0ull;
-    stage_twiddles<kScanThreads>(tw, twiddles, tid);
-    for (int e = tid; e < 2 * NFFT; e += kScanThreads) {
-        const int pair = e / NFFT, pos = e - pair * NFFT;
-        const float2 *src = col_results + ((size_t)pair * NFFT + pos) * kNodePad + bx * kInterp;
-#pragma unroll
-        for (int r = 0; r < kInterp; ++r) s[r * 2 + pair][T::slot(pos)] = src[r];
-    }
-    // The first points, on their way during the transforms.
-    const int n = row_counts[bx];
-    const unsigned short *points = row_points + (size_t)bx * N;
-    int i = tid < n ? points[tid] : 0;
-    float x = emb[i], y = emb[N + i];
-    const Bounds bd = load_bounds(sc_in, slot, n_boxes);
-    const float scale = 1.0f / ((float)NFFT * (float)NFFT);
-    const float scale3 = scale / r2_plane_scale(sc_in, slot);
-    __syncthreads();
-    T::inverse_grid(&s[0][0], 2 * kInterp, tw, tid, kScanThreads);
-    long long z_fixed = 0ll;
-    for (int e = tid; e < n; e += kScanThreads) {
-        int b, by;
-        float Lx[kInterp], Ly[kInterp];
-        bin_and_weights(x, bd, n_boxes, lc, b, Lx);
-        bin_and_weights(y, bd, n_boxes, lc, by, Ly);
-        if (b == bx) {  // (what was found near the row's edges may lie in the next)
-            const float4 phi = point_potential(Lx, Ly, [&](int a, int c) {
-                const float2 p0 = s[a * 2 + 0][T::slot(by * kInterp + c)], p1 = s[a * 2 + 1][T::slot(by * kInterp + c)];
-                return make_float4(p0.x * scale, p1.x * scale, p1.y * scale, p0.y * scale3);
-            });
-            z_fixed += __double2ll_rn((double)point_z(x, y, phi) * z_scale);
-            rep[i] = x * phi.x - phi.y;
-            rep[N + i] = y * phi.x - phi.z;
-        }
-        if (e + kScanThreads < n) {
-            i = points[e + kScanThreads];
-            x = emb[i];
-            y = emb[N + i];
-        }
-    }
-#pragma unroll
-    for (int m = kWave / 2; m >= 1; m >>= 1) z_fixed += __shfl_xor(z_fixed, m, kWave);
-    if ((tid & (kWave - 1)) == 0 && z_fixed != 0ll) atomicAdd(&z_sum, (unsigned long long)z_fixed);
-    __syncthreads();
-    if (tid == 0)
-        atomicAdd(reinterpret_cast<unsigned long long *>(&sc->z_part[blockIdx.x % kZParts]), z_sum);
 }
 
 __global__ void finish_z_kernel(const LoopScalars *sc, int N, double z_inv_scale, float *out) {
@@ -1716,7 +1604,7 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
     if (scan)
         TSNE_LOOP_KERNEL(p, (conv_rows_scan_kernel), xcd_launch_blocks(nb) + div_up(G, 8), kScanThreads, scan_lds(nb), s, embedding, N,
                          p->moment_scale, from_fixed, p->monomials, G, nb, p->scalars, slot, slot ^ 1, p->twiddles_short,
-                         p->row_spectra, p->kernel_rows, p->row_points(), p->row_counts());
+                         p->row_spectra, p->kernel_rows);
     else if (short_fft)
         TSNE_LOOP_KERNEL(p, (conv_rows_forward_kernel<2, kFftShort>), row_grid + div_up(G, 8), 512, 0, s, p->box_moments, from_fixed, p->monomials, charges4, G, nb, p->scalars, slot, p->twiddles_short,
             p->row_spectra, p->kernel_rows);
@@ -1740,15 +1628,6 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
         TSNE_LOOP_KERNEL(p, (conv_columns_kernel<false, kFft>), kFft / 2, 512, 0, s, p->row_spectra, G, p->kernel_rows, p->twiddles,
                                                                   p->col_results, p->box_moments, moment_words);
     TSNE_LAUNCHED(s);
-    if (scan) {
-        const int row_blocks = xcd_launch_blocks(nb);
-        const RowForces forces = {p->row_entries, p->yxy, small->attr, N, p->num_neighbors, row_blocks};
-        conv_rows_gather_kernel<<<row_blocks + div_up(N, kScanThreads / kForceLanes), kScanThreads, 0, s>>>(
-            p->col_results, embedding, N, p->scalars, slot, nb, p->lagrange, p->twiddles_short, p->row_points(), p->row_counts(),
-            rep, p->scalars, p->z_scale, forces);
-        TSNE_LAUNCHED(s);
-        return 0;
-    }
     if (profile_mark(p, kKernelConvRowsInverse, s)) return 1;
     RowForces rows = {nullptr, nullptr, nullptr, 0, 0, 0};
     int inverse_grid = row_grid;
@@ -1767,12 +1646,9 @@ int launch_repulsive(tsne_hip_plan *p, const float *embedding, int slot, float *
                                                                        p->twiddles, p->node_potentials, rows);
     TSNE_LAUNCHED(s);
     if (profile_mark(p, kKernelGather, s)) return 1;
-    if (N <= kScanPoints)
-        TSNE_LOOP_KERNEL(p, (gather_forces_kernel<true>), std::min(div_up(N, 256), 1024), 256, 0, s, embedding, N, p->scalars, slot, nb,
-                         p->lagrange, p->node_potentials, rep, point_potentials, p->scalars, keep, p->z_scale);
-    else
-        TSNE_LOOP_KERNEL(p, (gather_forces_kernel<false>), std::min(div_up(N, 256), 1024), 256, 0, s, embedding, N, p->scalars, slot, nb,
-                         p->lagrange, p->node_potentials, rep, point_potentials, p->scalars, keep, p->z_scale);
+    TSNE_LOOP_KERNEL(p, (gather_forces_kernel), std::min(div_up(N, 256), 1024), 256, 0, s, embedding, N, p->scalars, slot, nb, p->lagrange,
+                                                        p->node_potentials, rep, point_potentials, p->scalars, keep,
+                                                        p->z_scale);
     TSNE_LAUNCHED(s);
     return 0;
 }
