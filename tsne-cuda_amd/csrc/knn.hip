@@ -91,10 +91,18 @@ static_assert(kMQ == kCT, "query tiles and candidate tiles share the packed layo
 // From memory to LDS with no register in between: lane l's 16 bytes, at src + its offset, go to dst + 16 l.  The
 // compiler knows nothing of the load: s_waitcnt vmcnt(0) and a barrier stand between it and the words' readers, a barrier
 // between their last readers and it.  (As a builtin, every read of LDS that follows waits for it.)
+// The address is copied here, on the scalar unit: a memory instruction may not read a scalar register within five wait states
+// of the vector instruction that wrote it (a readfirstlane of an address, say), and the compiler counts those for instructions
+// it knows only.  The copy is also the wait state between M0's writing and its use.  (M0 is a reserved register: naming it tells
+// the compiler that it is written, and draws a warning that it would not be saved, which nobody asks for.)
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"
 typedef __attribute__((address_space(3))) unsigned char LdsByte;
 __device__ __forceinline__ void load_to_lds(const void *src, unsigned int offset, unsigned int dst) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %0" : : "s"(src), "v"(offset), "s"(dst) : "memory");
+    const void *at;
+    asm volatile("s_mov_b32 m0, %3\n\ts_mov_b64 %0, %1\n\tglobal_load_lds_dwordx4 %2, %0" : "=&s"(at) : "s"(src), "v"(offset), "s"(dst) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // (The builtin: a wait inside inline assembly leaves the compiler waiting once more for loads it knows of, and with them
 // for those it does not.)
 __device__ __forceinline__ void wait_for_loads() {
