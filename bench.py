@@ -228,7 +228,8 @@ def main():
                "frac": b / (kernels_us[name] * 1e-6) / 1e9 / HBM_PEAK_GBS}
         for name, b in loop_bytes.items() if kernels_us.get(name)}
     if knn_stats[0] == 1:
-        # Flop the matrix sweep executed per tile pair it did not skip: one product of halves
+        # Flop of the matrix sweep for every tile pair it did not skip, once each (on halves the neighbourhood and a sample are
+        # multiplied twice, for thresholds: those products are not counted): one product of halves
         # (v_mfma_f32_32x32x16_f16) over the dimensions, padded to 16 (up to 126 of them) or to 64 (chunked sweep); or three
         # of bf16 terms (v_mfma_f32_32x32x16_bf16) over the dimensions + 3, padded to 16 (up to 125) or to 32 (chunked,
         # beyond 126); at exactly 126 dimensions float products over 128 (v_mfma_f32_32x32x2_f32).
@@ -244,7 +245,8 @@ def main():
         flop = per_pair * tiles * tiles * knn_stats[2] / 1000.0
         phase_rooflines["knn"] = {"bound": "mfma", "flop": flop, "achieved": flop / knn_s / 1e12, "unit": "TFLOP/s",
                                   "frac": flop / knn_s / 1e12 / peak, "tile_pairs_per_mille": knn_stats[2],
-                                  "note": pipe + " matrix peak; time of the whole kNN call (sweep, re-rank, packing)"}
+                                  "note": pipe + " matrix peak; tile pairs not skipped, once each; time of the whole kNN call (sweep, "
+                                          "re-rank, packing)"}
 
     # One-shot stages that are HBM problems (algorithmic bytes: what the stage must read and write once).
     nnz = float(n) * k

@@ -55,10 +55,12 @@ int tsne_hip_knn(const float *points, int num_points, int num_dims, int num_neig
  * (host pointer to three ints, may be NULL): [0] = 1 if the matrix sweep ran,
  * [1] = queries that failed the verification of the sweep over all query tiles
  * (they are swept again with a wider margin or by the vector sweep), [2] = per
- * mille of the (query tile, candidate tile) pairs the matrix sweep computed (it
- * skips candidate tiles whose bounding ball lies beyond every threshold of the
- * query tile, which pays on locality-ordered points).  Same reference
- * counterpart as tsne_hip_knn. */
+ * mille of the (query tile, candidate tile) pairs that the matrix sweep did not
+ * skip (it skips candidate tiles whose bounding ball lies beyond every threshold
+ * of the query tile, which pays on locality-ordered points).  A pair counts once,
+ * also where the sweep's own choice (sweep 0) computes it twice, first for a
+ * threshold and then for its candidates: up to 17 tiles around a query tile, and
+ * about 240 or less of a sample.  Same reference counterpart as tsne_hip_knn. */
 int tsne_hip_knn_select(const float *points, int num_points, int num_dims, int num_neighbors, int *indices,
                         float *sq_dist, void *stream, int sweep, int *stats);
 

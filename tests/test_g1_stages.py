@@ -1574,6 +1574,20 @@ def test_knn_on_halves_measured_first(stages, monkeypatch, n, d, k):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
+@pytest.mark.parametrize("n,kind", [(16500, "blob"), (70001, "blob"), (33000, "runs")])
+def test_knn_on_halves_counts_a_pair_of_tiles_once(stages, monkeypatch, n, kind):
+    """The statistic is of the pairs that were not skipped, as on bf16 terms: also where pairs are measured for a threshold
+    before they are swept (70001 points without structure: beyond the neighbourhood too)."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 20)).astype(np.float32)
+    if kind == "runs":
+        X += (6.0 * rng.standard_normal((5, 20)))[np.arange(n) * 5 // n].astype(np.float32)
+    _, _, stats_bf16 = stages.knn_select(dev(X), 33, 2)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    _, _, stats = stages.knn_select(dev(X), 33, 0)
+    assert stats[0] == 1 and stats[2] == stats_bf16[2] and (stats[2] == 1000 if kind == "blob" else stats[2] < 500)
+
+
 @pytest.mark.parametrize("k", [45, 90, 150, 172])
 def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles

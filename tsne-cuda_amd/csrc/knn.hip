@@ -1584,7 +1584,7 @@ struct SweepArgs {
     const float *radius;     // T tile radii (upper bounds)
     int bitmap_words;        // ceil(T / 32)
     int trigger;             // a list longer than this is compacted after the tile (<= cap - kCT)
-    unsigned long long *tiles_swept;  // statistics: (query tile, candidate tile) pairs computed
+    unsigned long long *tiles_swept;  // statistics: (query tile, candidate tile) pairs that were not skipped, each once
     const float4 *Bp;  // chunked sweep only: query-side packed copy (-2 x_d, 1 in the |c|^2 row)
     int n_chunks;      // chunked sweep only: chunks of kChunkSteps k-steps per point
     // Chunked sweep only.  The num_qtiles query tiles are qtile_list[i], or first + i step without a list.
@@ -2483,7 +2483,7 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
             if (TSNE_UNLIKELY(home)) nxt = cur + P <= h1 ? cur + P : -1;
             else nxt = next_tile();
             process(cur, nxt);
-            swept += measure ? 0 : 1;
+            swept += measure ? 0 : 1;  // (those measured first are not skipped later, and counted then)
             if (TSNE_LIKELY(nxt >= 0 && !round_over && __ballot(my_fill() > half - kCT / 2) == 0)) {
                 cur = nxt;
                 continue;
@@ -3634,7 +3634,8 @@ struct HalfOperands {
 // mode: 0 = choose, 1 = VALU sweep only, 2 = matrix-instruction sweep on bf16 terms (on floats at 126 dimensions; error
 // if the shape does not fit), 3 = as 2 on floats whatever the dimension count.
 // stats (optional, 3 ints): [0] = 1 if the matrix-instruction sweep ran, [1] = queries redone by the VALU sweep,
-// [2] = per mille of the (query tile, candidate tile) pairs the matrix sweep computed.
+// [2] = per mille of the (query tile, candidate tile) pairs the matrix sweep did not skip, each counted once: on halves those of
+// the neighbourhood and of a sample are computed twice (SweepArgs::tiles_swept).
 // renumbered != nullptr: `points` are a renumbered copy (point i is the caller's order[i]) and the result is in
 // the caller's numbering.  Returns kNoRoom where memory is what it lacks.
 struct KnnRenumbered {
@@ -3811,7 +3812,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
 
     // Sweep + re-rank of `count` query tiles: those of tile_list (device), or first, first + step, ... without a
     // list.  Keeps `keep` candidates per query and part.  failed = queries of those tiles whose verification
-    // failed (listed in fail_list), swept = tile pairs computed.
+    // failed (listed in fail_list), swept = tile pairs not skipped.
     auto sweep_and_rerank = [&](int keep, const int *tile_list, int first, int step, int count, int &failed,
                                 unsigned long long &swept) -> int {
         const int cap = geometry.list_cap(keep);

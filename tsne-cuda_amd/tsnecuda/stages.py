@@ -118,7 +118,7 @@ def knn_select(points, num_neighbors, sweep):
     """knn() with an explicit sweep (1 = vector ALU, 2 = matrix instructions,
     3 = matrix instructions with the products on floats instead of bf16 terms).
     Returns (indices, sq_dist, stats) with stats = (matrix sweep ran, queries redone,
-    per mille of tile pairs computed)."""
+    per mille of tile pairs not skipped, each counted once)."""
     points = _f32(points)
     n, d = points.shape
     idx = torch.empty((n, num_neighbors), dtype=torch.int32, device=points.device)
