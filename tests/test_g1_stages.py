@@ -1588,6 +1588,22 @@ def test_knn_on_halves_counts_a_pair_of_tiles_once(stages, monkeypatch, n, kind)
     assert stats[0] == 1 and stats[2] == stats_bf16[2] and (stats[2] == 1000 if kind == "blob" else stats[2] < 500)
 
 
+@pytest.mark.parametrize("n,d", [(30000, 300), (30000, 1000), (20011, 784)])
+def test_knn_of_clusters_in_many_dimensions_keeps_its_margin(stages, n, d):
+    """For 90 neighbours 133 candidates are kept, or 128 where those do as well: where they do not - the sample of query tiles
+    fails, and the margin is doubled until it does not - the sweep skips as many tiles as for 94 neighbours, whose 139
+    candidates are never trimmed.  The vector sweep's rows."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    X += (4.0 * rng.standard_normal((20, d)))[np.arange(n) * 20 // n].astype(np.float32)
+    idx, d2, stats = stages.knn_select(dev(X), 90, 0)
+    _, _, stats_more = stages.knn_select(dev(X), 94, 0)
+    print("n=%d d=%d: %s, 94 neighbours %s" % (n, d, stats, stats_more))
+    assert stats[0] == stats_more[0] == 1 and stats[2] <= stats_more[2] + 20
+    idx_v, d2_v, _ = stages.knn_select(dev(X), 90, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
 @pytest.mark.parametrize("k", [45, 90, 150, 172])
 def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles

@@ -1647,9 +1647,11 @@ struct SweepArgs {
 // bytes of spills (300,000 points, 64 / 90 / 100 dimensions: 0.040 -> 0.027 s, 0.044 -> 0.033 s,
 // 0.045 -> 0.040 s); at 8 steps two tiles of 66 KB do not fit a compute unit's LDS.
 constexpr int bf16_sweep_occupancy(int steps) { return steps <= 2 ? 3 : (steps <= 7 ? 2 : 1); }
+constexpr size_t kUnitLds = 160 * 1024, kSweepLds = 4112;  // bytes of a compute unit, and of a workgroup beside its dynamic ones
+constexpr int float_sweep_occupancy(int ksteps) { return ksteps <= 28 ? 3 : 1; }
 template <int KSTEPS, bool BF16>
 constexpr int sweep_occupancy() {
-    return BF16 ? bf16_sweep_occupancy(KSTEPS) : (KSTEPS <= 28 ? 3 : 1);
+    return BF16 ? bf16_sweep_occupancy(KSTEPS) : float_sweep_occupancy(KSTEPS);
 }
 
 template <int KSTEPS, bool BF16>
@@ -3387,13 +3389,15 @@ inline bool centre_table_pays(int N, int D) { return (double)N * N * D >= 3e11; 
 constexpr size_t kMaxCentreTable = (size_t)128 << 20;  // (64896 points)
 constexpr int kMatrixPoints = 8192;  // fewer points: vector sweep
 // K' candidates kept per query.
-inline int candidates_kept(int N, int K) {
-    int want = (K - 1) + std::max(32, (K - 1) / 2);
-    // The re-rank takes 64 of them at a time, and as long for a few as for 64: up to eight beyond a multiple are left out.  Of
-    // many points more queries then fail and are searched again.  90 neighbours, ms, 133 / 128 kept: 100000 x 30 4.45 / 4.28,
-    // 200000 x 20 7.84 / 7.49, 300000 x 50 25.3 / 25.2, 1,000,000 x 50 71.1 / 73.3; 50000 x 1024 17.3 / 16.6.
-    if (N <= 262144 && want < 256 && want % kWave <= 8 && want / kWave * kWave >= (K - 1) + 32) want -= want % kWave;
-    return std::min(N - 1, want);
+inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2)); }
+// The re-rank takes 64 of them at a time, and as long for a few as for 64: up to eight beyond a multiple may be left out (87 to
+// 92 and 130 to 134 neighbours).  Of many points more queries then fail and are searched again.  90 neighbours, on halves, ms, 133 /
+// 128 kept: 100000 x 30 4.45 / 4.28, 200000 x 20 7.84 / 7.49, 300000 x 50 25.3 / 25.2, 1,000,000 x 50 71.1 / 73.3.
+// Where that is no gain the search keeps them all (see there): which products tell the neighbours apart, how long the lists are and
+// whether a sample verifies are questions of margins, and an answer that eight candidates turn round costs more than they do.
+inline int candidates_trimmed(int N, int K) {
+    const int want = candidates_kept(N, K), whole = want / kWave * kWave;
+    return N <= 262144 && want < 256 && want - whole <= 8 && whole >= (K - 1) + 32 ? whole : want;
 }
 
 int valu_cap(int K) {
@@ -3680,6 +3684,7 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
     if (mode == 3) mode = 2;
     const bool chunked = geometry.chunked;
     int want = candidates_kept(N, K);
+    const int trimmed = candidates_trimmed(N, K);
     const bool mfma_fits = geometry.fits(want);
     bool use_mfma = mode == 2 || (mode == 0 && mfma_fits && N >= kMatrixPoints);
     if (mode == 2 && !mfma_fits) {
@@ -3738,8 +3743,8 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         const SweepGeometry on_halves(N, D, Products::kHalf);
         bool pays = false;
         if (on_halves.fits(want))
-            if (const int rc = operands.frames(points, centers.as<float>(), radius.as<float>(), N, D, num_tiles, K, want,
-                                               chunked, &pays, s))
+            if (const int rc = operands.frames(points, centers.as<float>(), radius.as<float>(), N, D, num_tiles, K,
+                                               chunked ? want : trimmed, chunked, &pays, s))
                 return rc;
         if (pays && operands.room(N, on_halves) && Xp.alloc_optional(sizeof(float4) * on_halves.tile_float4 * num_tiles)) {
             geometry = on_halves;
@@ -3750,6 +3755,16 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
         }
     }
     const bool half = geometry.half, bf16 = geometry.bf16, bf16_chunked = geometry.bf16_chunked;
+    // On bf16 terms and on floats the candidates kept set the lists' length, and trimmed from 198 to 192 (130 to 134 neighbours) lists
+    // are half as long and selected from twice as often: only where another workgroup then fits on a compute unit.  132 neighbours, all /
+    // trimmed, ms: where none does 20000 x 20 2.21 / 2.42, in 20 clusters 1.43 / 1.56, 120000 x 125 42.5 / 44.6 and 20.7 / 21.2, on
+    // floats 60000 x 126 15.7 / 16.2; where one does 60000 x 100 11.2 / 7.6, 5.2 / 4.7.  (200000 x 30 37.1 / 35.2, 11.0 / 10.9: points
+    // without structure, which would gain there, are searched on halves.)
+    if (!chunked && trimmed < want) {
+        const int most = bf16 ? bf16_sweep_occupancy(geometry.steps16) : float_sweep_occupancy(geometry.ksteps);
+        const auto workgroups = [&](int keep) { return std::min(most, (int)(kUnitLds / (geometry.sweep_lds(keep) + kSweepLds))); };
+        if (geometry.list_cap(trimmed) == geometry.list_cap(want) || workgroups(trimmed) > workgroups(want)) want = trimmed;
+    }
     if (halves_only && !half) return not_on_halves("does not choose them");
     const int Dnorm = geometry.Dnorm, ksteps = geometry.ksteps, n_chunks = geometry.n_chunks;
     const int steps16 = geometry.steps16, bitmap_words = geometry.bitmap_words;
@@ -3982,6 +3997,12 @@ static int search(const float *points, int N, int D, int K, int *indices, float 
                 return rc == kNoRoom && half ? without_halves() : rc;
             if (failed * 10 <= sample_tiles * kMQ) {
                 verified = true;
+                // Sampled with all, and trimmed for the search itself where few queries of the sample fail (trimmed, up to 1.7 times as
+                // many do, which stays below the tenth).  Points in 20 clusters, all throughout / trimmed throughout, ms: where that
+                // doubled the margin once more, 90 neighbours, 30000 x 300 7.7 / 11.4, 50000 x 784 24.8 / 29.8, 30000 x 1000 19.1 /
+                // 28.0; with 134 neighbours 50000 x 784 (6.6 % of the queries fail) 26.8 / 36.1; with 132 40000 x 200 (3.7 %) 12.7 /
+                // 10.2.  Without structure 50000 x 1024 17.3 / 16.6, 30000 x 300 with 132 8.3 / 7.7.
+                if (attempt == 0 && failed * 20 <= sample_tiles * kMQ) want = trimmed;
             } else {
                 const int wider = std::min(N - 1, 2 * want);
                 if (wider == want || !geometry.fits(wider)) break;
