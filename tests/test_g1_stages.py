@@ -1430,6 +1430,20 @@ def test_knn_direct_search_mirrors_its_tiles(stages, n, d, k):
         assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
 
 
+@pytest.mark.parametrize("n,d,k", [(1025, 5, 33), (4225, 17, 20), (8321, 3, 60)])
+def test_knn_direct_search_with_tiles_formed_twice(stages, n, d, k):
+    """A fifth of the points not numbers, of either sign, and some infinite: pairs of tiles in which no distance, some distances or all
+    of a row are not numbers, at edges of tiles and of blocks of rows.  The vector sweep's rows, signs included."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    bad = rng.random(n) < 0.2
+    bad[n // 3 : n // 2] = False
+    X[bad, rng.integers(0, d, bad.sum())] = rng.choice(np.array([np.nan, -np.nan, np.inf, -np.inf], np.float32), bad.sum())
+    idx, d2 = stages.knn(dev(X), k)
+    idx_v, d2_v, _ = stages.knn_select(dev(X), k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
+
+
 @pytest.mark.parametrize("value", [np.nan, np.inf])
 @pytest.mark.parametrize("row", ["pivot 0", "another pivot", "no pivot"])
 def test_knn_of_points_in_no_order_that_are_not_numbers(stages, row, value):
