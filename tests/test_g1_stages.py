@@ -1413,12 +1413,13 @@ def test_knn_at_the_lines_of_the_direct_search(stages, n, d, k):
         assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
 
 
-@pytest.mark.parametrize("n,d,k", [(1024, 7, 20), (1025, 16, 33), (1087, 1, 5), (1089, 33, 129), (4096, 8, 20),
+@pytest.mark.parametrize("n,d,k", [(1024, 7, 20), (1025, 16, 33), (1087, 1, 5), (1089, 33, 129), (1408, 32, 20),
+                                   (1409, 32, 20), (1471, 33, 33), (2048, 31, 20), (2049, 31, 20), (2111, 1, 5), (4096, 8, 20),
                                    (4225, 5, 33), (9001, 3, 12)])
 def test_knn_direct_search_mirrors_its_tiles(stages, n, d, k):
-    """Distances of pairs of tiles are formed once and written twice from 1025 points on: the vector sweep's rows at the edges of
-    tiles and of blocks of rows, with equal distances, with overflowing ones and with points that are not numbers, whose
-    distances have the sign that the order of the difference gives them."""
+    """Distances of pairs of tiles are formed once and written twice, from 1409 or 2049 points on (by dimensions): the vector
+    sweep's rows at the edges of tiles and of blocks of rows, with equal distances, with overflowing ones and with points
+    that are not numbers, whose distances have the sign that the order of the difference gives them."""
     rng = np.random.default_rng(n + d)
     X = np.round(2.0 * rng.standard_normal((n, d))).astype(np.float32)
     X[n // 2] *= np.float32(1e30)
@@ -1430,7 +1431,7 @@ def test_knn_direct_search_mirrors_its_tiles(stages, n, d, k):
         assert torch.equal(idx, idx_v) and torch.equal(d2.view(torch.int32), d2_v.view(torch.int32))
 
 
-@pytest.mark.parametrize("n,d,k", [(1025, 5, 33), (4225, 17, 20), (8321, 3, 60)])
+@pytest.mark.parametrize("n,d,k", [(1025, 5, 33), (1409, 32, 33), (4225, 17, 20), (8321, 3, 60)])
 def test_knn_direct_search_with_tiles_formed_twice(stages, n, d, k):
     """A fifth of the points not numbers, of either sign, and some infinite: pairs of tiles in which no distance, some distances or all
     of a row are not numbers, at edges of tiles and of blocks of rows.  The vector sweep's rows, signs included."""

@@ -3436,8 +3436,10 @@ int run_direct_search(const float *points, int N, int D, int K, int *indices, fl
     for (int row0 = 0; row0 < N; row0 += block) {
         const int rows = std::min(block, N - row0);
         const dim3 grid(div_up(N, side), div_up(rows, side));
-        // (up to 1024 points there is no more than a tile per compute unit: 1003 x 20, 32 neighbours 38.6 us, mirrored 39.6)
-        const auto distances = N <= 1024 ? pair_distances_kernel<4, false> : pair_distances_kernel<4, true>;
+        // Mirrored where the tiles are more than two per compute unit (22 a side), and of short rows from 2048 points on: every tile formed /
+        // mirrored, 32 neighbours, us, 1025 x 20 40.8 / 41.9; 1408 x 4 41.3 / 42.7, x 100 51.8 / 52.5; 1536 x 20 44.6 / 45.0, x 50
+        // 50.8 / 49.2, x 200 68.8 / 63.1; 1900 x 4 44.9 / 46.0, x 20 47.7 / 48.0; 2200 x 20 53.5 / 53.4, x 200 90.1 / 80.7.
+        const auto distances = N <= 1408 || (N <= 2048 && D < 32) ? pair_distances_kernel<4, false> : pair_distances_kernel<4, true>;
         distances<<<grid, 256, 0, s>>>(points, N, points, N, D, row0, rows, pitch, dist.as<float>());
         TSNE_TRY(hipGetLastError());
         if (2 * (K - 1) <= 64 * 4)
