@@ -1574,9 +1574,10 @@ def test_knn_on_halves(stages, monkeypatch, n, d, k, kind, halves):
     (40007, 16, 30), (40007, 17, 150), (36000, 33, 90), (33001, 64, 90), (34003, 65, 45), (33333, 81, 20),
     (33333, 97, 33), (33100, 113, 60), (33100, 126, 90), (33100, 40, 172), (70001, 12, 90), (16500, 20, 90)])
 def test_knn_on_halves_measured_first(stages, monkeypatch, n, d, k):
-    """Thresholds measured before entries are stored, at every count of steps of 16 dimensions: neighbour counts whose
-    candidates the neighbourhood's runs are enough for and not (240 candidates kept and more), tiles enough to sample beyond
-    it and not, either end of the numbering (a shorter neighbourhood), a last tile of few points.  The vector sweep's rows."""
+    """Thresholds measured in the neighbourhood before entries are stored, at every count of steps of 16 dimensions: neighbour
+    counts whose candidates the neighbourhood's runs are enough for and not (240 candidates kept and more), either end of the
+    numbering (a shorter neighbourhood), a last tile of few points; and, of 70001 points alone, in a sample of the tiles
+    beyond (the query tiles of the others do not fill half the chip, and each is swept in two parts).  The vector sweep's rows."""
     rng = np.random.default_rng(n + d)
     X = rng.standard_normal((n, d)).astype(np.float32)
     X[n // 2 :] += 1.5 * rng.standard_normal(d).astype(np.float32)
@@ -1587,6 +1588,41 @@ def test_knn_on_halves_measured_first(stages, monkeypatch, n, d, k):
     idx, d2, stats = stages.knn_select(dX, k, 0)
     assert stats[0] == 1 and stats[1] <= 64
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+@pytest.mark.parametrize("n,d,k", [
+    (53000, 16, 20), (54001, 17, 150), (53003, 33, 90), (53000, 50, 90), (61000, 64, 30), (53333, 80, 45), (36003, 96, 172),
+    (36001, 100, 90), (36007, 126, 60), (98433, 50, 90), (520003, 20, 33)])
+def test_knn_on_halves_samples_tiles(stages, monkeypatch, n, d, k):
+    """Points without structure and query tiles enough that each is swept in one part: with 256 to 3840 tiles beyond the
+    neighbourhood every 16th is measured, and every 4th swept ahead of the rest, at every count of steps of 16 dimensions; with
+    more (520003 points) every 64th, and every 16th and 4th swept first.  The vector sweep's rows, and few queries without."""
+    X = np.random.default_rng(n + d).standard_normal((n, d)).astype(np.float32)
+    dX = dev(X)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    idx, d2, stats = stages.knn_select(dX, k, 0)
+    tiles = -(-n // 128)
+    slots = torch.cuda.get_device_properties(0).multi_processor_count * (3 if d <= 80 else 2)
+    assert 2 * tiles > slots + slots // 16  # (or each would be swept in two parts, without a sample)
+    assert stats[0] == 1 and stats[1] <= 64 and tiles * stats[2] >= 1000 * ((3840 if n > 500000 else 256) + 17)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+def test_knn_on_halves_samples_tiles_of_many_points(stages, monkeypatch):
+    """More than 15360 tiles beyond the neighbourhood: every 256th is measured, and every 64th, 16th and 4th swept first.  Of a
+    sample of rows the exact distances, of all of them few without enough candidates."""
+    n, d, k = 1990003, 20, 12
+    X = torch.randn((n, d), device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    idx, d2, stats = stages.knn_select(X, k, 0)
+    tiles = -(-n // 128)
+    assert stats[0] == 1 and stats[1] <= 256 and tiles * stats[2] >= 1000 * (15360 + 17)
+    for q in torch.linspace(0, n - 1, 41).long().tolist():
+        exact = (X - X[q]).double().square().sum(1)
+        want = torch.topk(exact, k, largest=False).values
+        assert torch.allclose(d2[q].double(), want, rtol=1e-5, atol=0.0)  # (sums of 20 squares in 32 bits: 20 half ulps)
+        assert torch.allclose(exact[idx[q].long()], want, rtol=1e-5, atol=0.0)
 
 
 @pytest.mark.parametrize("n,kind", [(16500, "blob"), (70001, "blob"), (33000, "runs")])
