@@ -1590,71 +1590,6 @@ def test_knn_on_halves_measured_first(stages, monkeypatch, n, d, k):
     assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
 
 
-@pytest.mark.parametrize("n,d,k", [
-    (53000, 16, 20), (54001, 17, 150), (53003, 33, 90), (53000, 50, 90), (61000, 64, 30), (53333, 80, 45), (36003, 96, 172),
-    (36001, 100, 90), (36007, 126, 60), (98433, 50, 90), (520003, 20, 33)])
-def test_knn_on_halves_samples_tiles(stages, monkeypatch, n, d, k):
-    """Points without structure and query tiles enough that each is swept in one part: with 256 to 3840 tiles beyond the
-    neighbourhood every 16th is measured, and every 4th swept ahead of the rest, at every count of steps of 16 dimensions; with
-    more (520003 points) every 64th, and every 16th and 4th swept first.  The vector sweep's rows, and few queries without."""
-    X = np.random.default_rng(n + d).standard_normal((n, d)).astype(np.float32)
-    dX = dev(X)
-    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
-    idx, d2, stats = stages.knn_select(dX, k, 0)
-    tiles = -(-n // 128)
-    slots = torch.cuda.get_device_properties(0).multi_processor_count * (3 if d <= 80 else 2)
-    assert 2 * tiles > slots + slots // 16  # (or each would be swept in two parts, without a sample)
-    assert stats[0] == 1 and stats[1] <= 64 and tiles * stats[2] >= 1000 * ((3840 if n > 500000 else 256) + 17)
-    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
-    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
-
-
-def test_knn_on_halves_samples_tiles_of_many_points(stages, monkeypatch):
-    """More than 15360 tiles beyond the neighbourhood: every 256th is measured, and every 64th, 16th and 4th swept first.  Of a
-    sample of rows the exact distances, of all of them few without enough candidates."""
-    n, d, k = 1990003, 20, 12
-    X = torch.randn((n, d), device="cuda", generator=torch.Generator("cuda").manual_seed(n))
-    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
-    idx, d2, stats = stages.knn_select(X, k, 0)
-    tiles = -(-n // 128)
-    assert stats[0] == 1 and stats[1] <= 256 and tiles * stats[2] >= 1000 * (15360 + 17)
-    for q in torch.linspace(0, n - 1, 41).long().tolist():
-        exact = (X - X[q]).double().square().sum(1)
-        want = torch.topk(exact, k, largest=False).values
-        assert torch.allclose(d2[q].double(), want, rtol=1e-5, atol=0.0)  # (sums of 20 squares in 32 bits: 20 half ulps)
-        assert torch.allclose(exact[idx[q].long()], want, rtol=1e-5, atol=0.0)
-
-
-@pytest.mark.parametrize("n,kind", [(16500, "blob"), (70001, "blob"), (33000, "runs")])
-def test_knn_on_halves_counts_a_pair_of_tiles_once(stages, monkeypatch, n, kind):
-    """The statistic is of the pairs that were not skipped, as on bf16 terms: also where pairs are measured for a threshold
-    before they are swept (70001 points without structure: beyond the neighbourhood too)."""
-    rng = np.random.default_rng(n)
-    X = rng.standard_normal((n, 20)).astype(np.float32)
-    if kind == "runs":
-        X += (6.0 * rng.standard_normal((5, 20)))[np.arange(n) * 5 // n].astype(np.float32)
-    _, _, stats_bf16 = stages.knn_select(dev(X), 33, 2)
-    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
-    _, _, stats = stages.knn_select(dev(X), 33, 0)
-    assert stats[0] == 1 and stats[2] == stats_bf16[2] and (stats[2] == 1000 if kind == "blob" else stats[2] < 500)
-
-
-@pytest.mark.parametrize("n,d", [(30000, 300), (30000, 1000), (20011, 784)])
-def test_knn_of_clusters_in_many_dimensions_keeps_its_margin(stages, n, d):
-    """For 90 neighbours 133 candidates are kept, or 128 where those do as well: where they do not - the sample of query tiles
-    fails, and the margin is doubled until it does not - the sweep skips as many tiles as for 94 neighbours, whose 139
-    candidates are never trimmed.  The vector sweep's rows."""
-    rng = np.random.default_rng(n + d)
-    X = rng.standard_normal((n, d)).astype(np.float32)
-    X += (4.0 * rng.standard_normal((20, d)))[np.arange(n) * 20 // n].astype(np.float32)
-    idx, d2, stats = stages.knn_select(dev(X), 90, 0)
-    _, _, stats_more = stages.knn_select(dev(X), 94, 0)
-    print("n=%d d=%d: %s, 94 neighbours %s" % (n, d, stats, stats_more))
-    assert stats[0] == stats_more[0] == 1 and stats[2] <= stats_more[2] + 20
-    idx_v, d2_v, _ = stages.knn_select(dev(X), 90, 1)
-    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
-
-
 @pytest.mark.parametrize("k", [45, 90, 150, 172])
 def test_knn_on_halves_with_many_equal_points(stages, monkeypatch, k):
     """Equal points in tiles of their own at either end of the numbering, but for every fiftieth point: a round of tiles
@@ -1790,3 +1725,70 @@ def test_scratch_is_kept_bounded_and_given_back(stages):
     assert 32 << 20 <= kept <= (2 << 30) + (256 << 20)
     stages.release_scratch()
     assert free - torch.cuda.mem_get_info()[0] <= 256 << 20
+
+
+@pytest.mark.parametrize("n,d,k", [
+    (53000, 16, 20), (54001, 17, 150), (53003, 33, 90), (53000, 50, 90), (61000, 64, 30), (53333, 80, 45), (36003, 96, 172),
+    (36001, 100, 90), (36007, 126, 60), (98433, 50, 90), (520003, 20, 33)])
+def test_knn_on_halves_samples_tiles(stages, monkeypatch, n, d, k):
+    """Points without structure and query tiles enough that each is swept in one part: with 256 to 3840 tiles beyond the
+    neighbourhood every 16th is measured, and every 4th swept ahead of the rest, at every count of steps of 16 dimensions; with
+    more (520003 points) every 64th, and every 16th and 4th swept first.  The vector sweep's rows, and few queries without."""
+    X = np.random.default_rng(n + d).standard_normal((n, d)).astype(np.float32)
+    dX = dev(X)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    idx, d2, stats = stages.knn_select(dX, k, 0)
+    tiles = -(-n // 128)
+    slots = torch.cuda.get_device_properties(0).multi_processor_count * (3 if d <= 80 else 2)
+    assert 2 * tiles > slots + slots // 16  # (or each would be swept in two parts, without a sample)
+    assert stats[0] == 1 and stats[1] <= 64 and tiles * stats[2] >= 1000 * ((3840 if n > 500000 else 256) + 17)
+    idx_v, d2_v, _ = stages.knn_select(dX, k, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
+
+
+def test_knn_on_halves_samples_tiles_of_many_points(stages, monkeypatch):
+    """More than 15360 tiles beyond the neighbourhood: every 256th is measured, and every 64th, 16th and 4th swept first.  Of a
+    sample of rows the exact distances, of all of them few without enough candidates."""
+    n, d, k = 1990003, 20, 12
+    X = torch.randn((n, d), device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    idx, d2, stats = stages.knn_select(X, k, 0)
+    tiles = -(-n // 128)
+    assert stats[0] == 1 and stats[1] <= 256 and tiles * stats[2] >= 1000 * (15360 + 17)
+    for q in torch.linspace(0, n - 1, 41).long().tolist():
+        exact = (X - X[q]).double().square().sum(1)
+        want = torch.topk(exact, k, largest=False).values
+        assert torch.allclose(d2[q].double(), want, rtol=1e-5, atol=0.0)  # (sums of 20 squares in 32 bits: 20 half ulps)
+        assert torch.allclose(exact[idx[q].long()], want, rtol=1e-5, atol=0.0)
+    del X, idx, d2, exact, want
+    torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("n,kind", [(16500, "blob"), (70001, "blob"), (33000, "runs")])
+def test_knn_on_halves_counts_a_pair_of_tiles_once(stages, monkeypatch, n, kind):
+    """The statistic is of the pairs that were not skipped, as on bf16 terms: also where pairs are measured for a threshold
+    before they are swept (70001 points without structure: beyond the neighbourhood too)."""
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, 20)).astype(np.float32)
+    if kind == "runs":
+        X += (6.0 * rng.standard_normal((5, 20)))[np.arange(n) * 5 // n].astype(np.float32)
+    _, _, stats_bf16 = stages.knn_select(dev(X), 33, 2)
+    monkeypatch.setenv("TSNE_KNN_PRODUCTS", "half")
+    _, _, stats = stages.knn_select(dev(X), 33, 0)
+    assert stats[0] == 1 and stats[2] == stats_bf16[2] and (stats[2] == 1000 if kind == "blob" else stats[2] < 500)
+
+
+@pytest.mark.parametrize("n,d", [(30000, 300), (30000, 1000), (20011, 784)])
+def test_knn_of_clusters_in_many_dimensions_keeps_its_margin(stages, n, d):
+    """For 90 neighbours 133 candidates are kept, or 128 where those do as well: where they do not - the sample of query tiles
+    fails, and the margin is doubled until it does not - the sweep skips as many tiles as for 94 neighbours, whose 139
+    candidates are never trimmed.  The vector sweep's rows."""
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    X += (4.0 * rng.standard_normal((20, d)))[np.arange(n) * 20 // n].astype(np.float32)
+    idx, d2, stats = stages.knn_select(dev(X), 90, 0)
+    _, _, stats_more = stages.knn_select(dev(X), 94, 0)
+    print("n=%d d=%d: %s, 94 neighbours %s" % (n, d, stats, stats_more))
+    assert stats[0] == stats_more[0] == 1 and stats[2] <= stats_more[2] + 20
+    idx_v, d2_v, _ = stages.knn_select(dev(X), 90, 1)
+    assert torch.equal(idx, idx_v) and torch.equal(d2, d2_v)
