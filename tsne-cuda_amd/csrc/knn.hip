@@ -2065,8 +2065,8 @@ __global__ __launch_bounds__(256, (sweep_occupancy<KSTEPS, BF16>())) void knn_mf
 // output are those of knn_mfma_sweep_kernel; the accumulators start from the candidates' betas and fall as the
 // distance grows, so what is looked for is the largest.
 //
-// What bounds the kernel: about 240 vector instructions a wave and tile, 1000 cycles of a SIMD, and 640 of the matrix unit,
-// which hide less of each other than three waves per SIMD might; a wave waits 44 % of its time.  So: three waves, nothing of
+// What bounds the kernel (1,000,000 x 50): 220 vector instructions a wave and tile, 880 cycles of a SIMD, and 640 of the matrix
+// unit, of the 2100 that pass, so they hide little of each other; a wave waits 44 % of its time.  So: three waves, nothing of
 // the tile loop in scratch memory (a wait for a spilled register is a wait for the next tile's loads too: one of them took
 // the sweep of 1,000,000 x 50 from 74 to 100 ms; four waves of 128 registers 86), and to that end what is seldom run takes
 // its arguments and its lane number where it stands (`cold`, `here`).  Tiles go from memory to LDS without registers; all
@@ -2557,18 +2557,22 @@ __global__ __launch_bounds__(256, half_sweep_occupancy(S)) void knn_half_sweep_k
 // ---------------------------------------------------------------------------
 // MFMA sweep for more dimensions than one wave's registers hold (more than 126).
 // The k-steps are cut into chunks of kChunkSteps (64 dimensions).  Per candidate tile and chunk the
-// workgroup keeps the chunk of the tile in LDS (32 KB, layout [block (4)][step group (8)][lane (64)]
+// workgroup keeps the chunk of the tile in LDS (on floats 32 KB, layout [block (4)][step group (8)][lane (64)]
 // float4, copied verbatim from the packed points), every wave loads the same chunk of its 32 queries
 // from the packed query-side copy (already scaled: -2 q_d, 1 in the |c|^2 row) and the products of
-// all four candidate blocks accumulate over the chunks in 64 registers.  The next chunk of the tile
-// (or the first of the next tile) and of the queries travel through registers meanwhile.  Visiting
-// order, tile skipping, filter, lists and output are those of the kernel above.
+// all four candidate blocks accumulate over the chunks in 64 registers.  The next chunk of the queries travels
+// into registers meanwhile, and so, on floats and bf16 terms, does the next of the tile (or the first of the next tile); on
+// halves that goes straight into a second LDS buffer.  Visiting order, tile skipping, filter, lists and output are those of
+// the kernel above.
+// Halves: a chunk is 64 dimensions, 16 KB (two LDS buffers) as [block (4)][step of 16 dimensions (4)][lane (64)] 8 halves, one
+// product a step, for either side of the products the same packed points (half_pack_kernel), and the accumulators start from
+// the betas.
 // BF16 = true: a chunk is 32 dimensions, 16 KB (two LDS buffers) as [block (4)][term (2)][step of 16 dimensions (2)][lane (64)]
 // 8 x bf16 of the points relative to their tile's centre, the query side two terms of -2 q likewise, and the
 // products are those of the kernel above (three v_mfma_f32_32x32x16_bf16 per step); |q - centre|^2 is summed
 // over the chunks from the query side's two terms and the centre's chunk (pack_chunked_centres_kernel), and
 // the keys are lower bounds of the distances as there.
-// Dynamic LDS: one tile chunk, one sort buffer (cap keys) per wave, the visit bitmap, D floats
+// Dynamic LDS: 32 KB for one tile chunk or two, one sort buffer (cap keys) per wave, the visit bitmap, D floats
 // (centre of the query tile's ball).
 // ---------------------------------------------------------------------------
 constexpr int kChunkSteps = 32;
@@ -2597,7 +2601,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     constexpr int kSlots = BF16 || HALF ? 4 : kChunkS4;
     constexpr int kSteps16 = 2;                     // bf16: steps of 16 dimensions per chunk
     constexpr int kChunkF4 = 4 * kSlots * 64;       // float4 per tile chunk
-    // bf16: two LDS buffers of 16 KB, so that the next chunk goes to LDS while the other waves may still read the
+    // bf16 and halves: two LDS buffers of 16 KB, so that the next chunk goes to LDS while the other waves may still read the
     // current one, and one workgroup barrier per chunk does (floats: one buffer of 32 KB, two barriers).
     constexpr int kBufs = BF16 || HALF ? 2 : 1;
     int buf = 0;  // the buffer that holds the chunk being computed
@@ -2655,7 +2659,7 @@ __global__ __launch_bounds__(256, 2) void knn_mfma_chunked_sweep_kernel(const Sw
     const int P = args.parts;
     // The parts of a query tile go to workgroups of one XCD, which read the tile's operands at about the same time, and so do
     // query tiles next to each other, which visit much the same candidate tiles.  (Workgroups go to the XCDs round robin; the
-    // grid is a multiple of their number times P.  50000 x 1024: 65 % of the requests missed the L2 with the parts dealt to all
+    // grid is a multiple of their number times P.  50000 x 1024: 64 % of the requests missed the L2 with the parts dealt to all
     // XCDs, and the sweep went at the rate of the cache behind it, 7 TB/s; 46 % so, 12.0 -> 10.3 ms.)
     const int round_tiles = (int)gridDim.x / P, xcd = (int)blockIdx.x % kSweepXcds;
     const int in_xcd = (int)blockIdx.x / kSweepXcds, part = in_xcd % P;
@@ -3389,7 +3393,8 @@ constexpr int kMatrixPoints = 8192;  // fewer points: vector sweep
 inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std::max(32, (K - 1) / 2)); }
 // The re-rank takes 64 of them at a time, and as long for a few as for 64: up to eight beyond a multiple may be left out (87 to
 // 92 and 130 to 134 neighbours).  Of many points more queries then fail and are searched again.  90 neighbours, on halves, ms, 133 /
-// 128 kept: 100000 x 30 4.45 / 4.28, 200000 x 20 7.84 / 7.49, 300000 x 50 25.3 / 25.2, 1,000,000 x 50 71.1 / 73.3.
+// 128 kept: 100000 x 30 4.45 / 4.28, 200000 x 20 7.84 / 7.49, 300000 x 50 25.3 / 25.2, 1,000,000 x 50 in four clusters 71.1 /
+// 73.3; 270000 to 1,000,000 points without structure, 90 and 132 neighbours, within 1 % of each other.
 // Where that is no gain the search keeps them all (see there): which products tell the neighbours apart, how long the lists are and
 // whether a sample verifies are questions of margins, and an answer that eight candidates turn round costs more than they do.
 inline int candidates_trimmed(int N, int K) {
