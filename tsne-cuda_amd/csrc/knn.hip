@@ -3395,8 +3395,8 @@ inline int candidates_kept(int N, int K) { return std::min(N - 1, (K - 1) + std:
 // 92 and 130 to 134 neighbours).  Of many points more queries then fail and are searched again.  90 neighbours, on halves, ms, 133 /
 // 128 kept: 100000 x 30 4.45 / 4.28, 200000 x 20 7.84 / 7.49, 300000 x 50 25.3 / 25.2, 1,000,000 x 50 in four clusters 71.1 /
 // 73.3; 270000 to 1,000,000 points without structure, 90 and 132 neighbours, within 1 % of each other.
-// Where that is no gain the search keeps them all (see there): which products tell the neighbours apart, how long the lists are and
-// whether a sample verifies are questions of margins, and an answer that eight candidates turn round costs more than they do.
+// Where they decide more than that the search keeps them all (see there): how long lists are and whether a sample verifies are
+// questions of margins, and an answer that eight candidates turn round costs more than they do.
 inline int candidates_trimmed(int N, int K) {
     const int want = candidates_kept(N, K), whole = want / kWave * kWave;
     return N <= 262144 && want < 256 && want - whole <= 8 && whole >= (K - 1) + 32 ? whole : want;
